@@ -19,6 +19,7 @@ LIB_PATH = Path(os.environ.get("DWMI_LIB", Path(__file__).resolve().parent / "li
 
 DW_FP32, DW_BF16X3, DW_BF16, DW_FP64 = 0, 1, 2, 3
 PRECISIONS = {"fp32": DW_FP32, "bf16x3": DW_BF16X3, "bf16": DW_BF16, "fp64": DW_FP64}
+LAP_SPLIT, LAP_FP32 = 0, 1
 FLAG_NONFINITE, FLAG_FP64_DET, FLAG_FORCED_ACCEPT = 1, 2, 4
 TIMER_GEMM_1EL_LAP, TIMER_DET_LAP, TIMER_FORWARD, TIMER_LOCAL_ENERGY = 0, 1, 2, 3
 PROPOSALS = {"normal": 0, "local": 1, "langevin": 2, "normal_one_el": 3, "local_one_el": 4}
@@ -74,6 +75,7 @@ SIGNATURES = {
                          ctypes.POINTER(ctypes.c_int64)], ctypes.c_int),
     "dw_workspace_size": ([_vp, _i32, _i32], ctypes.c_size_t),
     "dw_model_set_chunk": ([_vp, _i32], ctypes.c_int),
+    "dw_model_set_lap_form": ([_vp, _i32], ctypes.c_int),
     "dw_model_set_workspace": ([_vp, _vp, ctypes.c_size_t], ctypes.c_int),
     "dw_model_set_tuning": ([_vp, ctypes.POINTER(Tuning)], ctypes.c_int),
     "dw_model_get_tuning": ([_vp, ctypes.POINTER(Tuning)], ctypes.c_int),
@@ -139,6 +141,7 @@ class NativeModel:
         _check(self.lib.dw_model_create(ctypes.byref(desc), ctypes.byref(h)))
         self.handle = h
         self._param_token = None
+        self._lap_form = LAP_SPLIT
         if chunk:
             _check(self.lib.dw_model_set_chunk(self.handle, int(chunk)))
 
@@ -211,6 +214,12 @@ class NativeModel:
             return
         _check(self.lib.dw_model_set_workspace(self.handle, ctypes.c_void_p(buf.data_ptr()), buf.numel() * buf.element_size()))
         self._ws = buf
+
+    def set_lap_form(self, form: int) -> int:
+        """dw_model_set_lap_form: LAP_SPLIT (default) or LAP_FP32.  Returns the form before."""
+        _check(self.lib.dw_model_set_lap_form(self.handle, int(form)))
+        old, self._lap_form = self._lap_form, int(form)
+        return old
 
     def set_chunk(self, walkers: int) -> None:
         _check(self.lib.dw_model_set_chunk(self.handle, int(walkers)))

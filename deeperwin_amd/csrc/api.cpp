@@ -112,15 +112,18 @@ struct Weights {
   std::vector<DevBuf> Wmain, Wmu, bias, Wmain_hi, Wmain_lo, Wmu_hi, Wmu_lo;
   std::vector<DevBuf> WmainT, WmuT;  // transposed copies for the gradient pass ([pad128(K)][W1])
   DevBuf W2e, b2e, Wo[2], Wo_hi[2], Wo_lo[2], WoT[2], kappa, wenv;
+  // FP32 form: the three BF16 parts of Wmain / Wo in MFMA lane order (derivative channels, gemm_split.hip)
+  std::vector<DevBuf> WmainS;
+  DevBuf WoS[2];
   // dpe4: pair-stream sets, el-ion stream, ion maps, ion table; h_map GEMM operands per iteration
   DevBuf Wp, bp, Wei, bei, Whim, bhim, table;
   std::vector<DevBuf> WhmT, WhmT_hi, WhmT_lo, bhm, WhmB;  // WhmB: h_map w [pad128(Kh)][32] (gradient pass)
   void release() {
     for (auto* v : {&Wmain, &Wmu, &bias, &Wmain_hi, &Wmain_lo, &Wmu_hi, &Wmu_lo, &WmainT, &WmuT, &WhmT, &WhmT_hi,
-                    &WhmT_lo, &bhm, &WhmB})
+                    &WhmT_lo, &bhm, &WhmB, &WmainS})
       for (auto& b : *v) b.release();
     for (DevBuf* b : {&W2e, &b2e, &Wo[0], &Wo[1], &Wo_hi[0], &Wo_hi[1], &Wo_lo[0], &Wo_lo[1], &WoT[0], &WoT[1], &kappa,
-                      &wenv, &Wp, &bp, &Wei, &bei, &Whim, &bhim, &table})
+                      &wenv, &Wp, &bp, &Wei, &bei, &Whim, &bhim, &table, &WoS[0], &WoS[1]})
       b->release();
     ready = false;
   }
@@ -163,6 +166,7 @@ struct dw_model {
   std::vector<std::pair<std::string, std::vector<int64_t>>> expected;
   bool dirty = true;
   int chunk = 0;
+  int lap_form = DW_LAP_SPLIT;  // dw_model_set_lap_form
   dw_tuning tune{-1, -1, 0, -1, -1, 0, 0};
   void* ext_ws = nullptr;  // caller-owned workspace (dw_model_set_workspace)
   size_t ext_ws_bytes = 0;
@@ -328,13 +332,23 @@ dw_status prepare_dpe4(dw_model* m, Weights& W, bool dbl, bool split) {
   return DW_OK;
 }
 
+// The split parts of device weights Bt [rows >= cols, K] (packed on the device from the FP32 layout).
+dw_status pack_split(DevBuf& out, const DevBuf& Bt, int cols, int K) {
+  HIP_TRY(out.ensure(split_pack_bytes(cols, K)));
+  launch_split_pack(Bt.as<float>(), K, cols, K, out.p, nullptr);
+  HIP_TRY(hipGetLastError());
+  return DW_OK;
+}
+
 // Build the device layouts of all weights from the host leaves, in float or double.
 dw_status prepare_weights(dw_model* m, Weights& W, bool dbl) {
   for (auto& e : m->expected)
     if (!m->leaves[e.first].set) return fail(DW_ERR_STATE, "parameter not set: " + e.first);
   const int W1 = m->W1, W2 = m->W2;
   const bool split = !dbl && m->prec != GEMM_F32;
-  for (auto* v : {&W.Wmain, &W.Wmu, &W.bias, &W.Wmain_hi, &W.Wmain_lo, &W.Wmu_hi, &W.Wmu_lo, &W.WmainT, &W.WmuT})
+  const bool parts3 = !dbl && m->prec == GEMM_F32;
+  for (auto* v : {&W.Wmain, &W.Wmu, &W.bias, &W.Wmain_hi, &W.Wmain_lo, &W.Wmu_hi, &W.Wmu_lo, &W.WmainT, &W.WmuT,
+                  &W.WmainS})
     v->resize(m->L);
   auto up = [&](DevBuf& b, const std::vector<float>& v) { return dbl ? upload_as<double>(b, v) : upload(b, v); };
   for (int l = 0; l < m->L; ++l) {
@@ -364,6 +378,7 @@ dw_status prepare_weights(dw_model* m, Weights& W, bool dbl) {
     if ((st = up(W.WmainT[l], wmT))) return st;
     if ((st = up(W.WmuT[l], wuT))) return st;
     if ((st = up(W.bias[l], b.data))) return st;
+    if (parts3 && (st = pack_split(W.WmainS[l], W.Wmain[l], W1, Kx))) return st;
     if (split) {
       if ((st = upload_split(W.Wmain_hi[l], W.Wmain_lo[l], wm))) return st;
       if ((st = upload_split(W.Wmu_hi[l], W.Wmu_lo[l], wu))) return st;
@@ -404,6 +419,7 @@ dw_status prepare_weights(dw_model* m, Weights& W, bool dbl) {
     dw_status st;
     if ((st = up(W.Wo[s], wo))) return st;
     if ((st = up(W.WoT[s], woT))) return st;
+    if (parts3 && (st = pack_split(W.WoS[s], W.Wo[s], m->NOp, W1))) return st;
     if (split && (st = upload_split(W.Wo_hi[s], W.Wo_lo[s], wo))) return st;
     const Leaf& a = m->leaves[leaf_key("envelope_orbitals", ak[s])];
     const Leaf& we = m->leaves[leaf_key("envelope_orbitals", wk[s])];
@@ -570,6 +586,9 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
   const int Cp = rows_per_electron(C);
   Shape sh{(int)B, m->n, m->u, m->I, m->D, C, Cp, m->W1, m->W2, m->L};
   const long rows = B * m->n * Cp;
+  // below 32768 rows a pass is launches and latency, and the value channel's own launches cost more than the
+  // split saves (16,384 rows of 256 LiH walkers: 760 us a call against 741)
+  const bool split = !DBL && C > 1 && m->prec == GEMM_F32 && m->lap_form == DW_LAP_SPLIT && rows >= 32768;
   Timed pass_timer(m, C > 1 ? DW_TIMER_LOCAL_ENERGY : DW_TIMER_FORWARD, s);
   T* const* X = ws.X;
   if (prop) {  // the pass runs on the Gaussian proposal, formed and stored by the features kernel
@@ -658,6 +677,18 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
         gemm_t(m, X[l], m->Kx[l], W.Wmain[l].as<T>(), W.Wmain_hi[l], W.Wmain_lo[l], m->Kx[l], ws.Z, m->W1,
                rows, m->W1, m->Kx[l], em, s);
         launch_tanh_rule<T>(ws.Z, outp, ldo, last ? 1 : 0, sh, s);
+      } else if (split) {
+        // value channel (row 0 of each electron) as in the value pass, then the derivative channels
+        GemmEpi e0 = em;
+        e0.C = 1;
+        e0.nC = m->n;
+        e0.ldv = Cp * m->W1;
+        e0.act_tanh = 1;
+        e0.permute = last ? 1 : 0;
+        gemm(GEMM_F32, X[l], Cp * m->Kx[l], W.Wmain[l].as<float>(), nullptr, nullptr, m->Kx[l], outp, Cp * ldo,
+             (int)(B * m->n), m->W1, m->Kx[l], e0, s);
+        split_lap(X[l], m->Kx[l], W.WmainS[l].p, m->Kx[l], ws.V, m->W1, outp, ldo, last ? 1 : 0, sh,
+                  m->tune.lap_electrons, m->tune.lap_cols, s);
       } else {
         gemm_lap(m->prec, X[l], m->Kx[l], W.Wmain[l].as<float>(), W.Wmain_hi[l].as<uint16_t>(),
                  W.Wmain_lo[l].as<uint16_t>(), m->Kx[l], ws.V, m->W1, outp, ldo, last ? 1 : 0, sh,
@@ -669,10 +700,20 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
   const long up_rows = B * m->u * Cp, dn_rows = B * m->dn * Cp;
   GemmEpiT<T> e0;
   e0.tile = C == 1 ? m->tune.fwd_orb_tile : m->tune.lap_orb_tile;
-  gemm_t(m, ws.H, m->W1, W.Wo[0].as<T>(), W.Wo_hi[0], W.Wo_lo[0], m->W1, ws.O, m->NO, up_rows, m->NO,
-         m->W1, e0, s);
-  gemm_t(m, ws.H + up_rows * m->W1, m->W1, W.Wo[1].as<T>(), W.Wo_hi[1], W.Wo_lo[1], m->W1,
-         ws.O + up_rows * m->NO, m->NO, dn_rows, m->NO, m->W1, e0, s);
+  for (int sp = 0; sp < 2; ++sp) {
+    const long rows0 = sp ? up_rows : 0, nr = sp ? dn_rows : up_rows;
+    if constexpr (!DBL) {
+      if (split) {  // every channel from the split form, then the value rows in FP32
+        split_gemm(ws.H + rows0 * m->W1, m->W1, W.WoS[sp].p, ws.O + rows0 * m->NO, m->NO, (int)nr, m->NO, m->W1,
+                   m->tune.lap_orb_tile, s);
+        gemm(GEMM_F32, ws.H + rows0 * m->W1, Cp * m->W1, W.Wo[sp].as<float>(), nullptr, nullptr, m->W1,
+             ws.O + rows0 * m->NO, Cp * m->NO, (int)(nr / Cp), m->NO, m->W1, GemmEpi{}, s);
+        continue;
+      }
+    }
+    gemm_t(m, ws.H + rows0 * m->W1, m->W1, W.Wo[sp].as<T>(), W.Wo_hi[sp], W.Wo_lo[sp], m->W1, ws.O + rows0 * m->NO,
+           m->NO, nr, m->NO, m->W1, e0, s);
+  }
   const OrbSrc<T> src{ws.O, m->NO, r, R, W.kappa.as<T>(), W.wenv.as<T>()};
   if (!det_reads_orbitals(m->n, C))
     launch_envelope<T>(ws.O, m->NO, r, R, W.kappa.as<T>(), W.wenv.as<T>(), ws.A, sh, s);
@@ -1213,6 +1254,13 @@ dw_status dw_model_set_tuning(dw_model* m, const dw_tuning* t) {
 dw_status dw_model_get_tuning(const dw_model* m, dw_tuning* out) {
   if (!m || !out) return fail(DW_ERR_INVALID, "null argument");
   *out = m->tune;
+  return DW_OK;
+}
+
+dw_status dw_model_set_lap_form(dw_model* m, int32_t form) {
+  if (!m) return fail(DW_ERR_INVALID, "null model");
+  if (form != DW_LAP_SPLIT && form != DW_LAP_FP32) return fail(DW_ERR_INVALID, "unknown Laplacian form");
+  m->lap_form = form;
   return DW_OK;
 }
 

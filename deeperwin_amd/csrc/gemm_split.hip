@@ -1,0 +1,354 @@
+// FP32 GEMMs of the Laplacian pass's derivative channels on BF16 MFMA.
+//
+// Every FP32 operand is the exact sum of three BF16 numbers (x = h + m + l: h = bf16(x), m = bf16(x - h),
+// l = x - h - m; 8 + 8 + 8 significant bits), so a product a b is the sum of nine BF16 products.  The three
+// below 2^-26 |a b| (m l, l m, l l) are left out, the other six accumulate in FP32, smallest first:
+//   l h + h l + m m + m h + h m + h h.
+// What is left out is under the rounding of one FP32 multiply-add, and a 32-wide K slice rounds the
+// accumulator six times where the FP32 MFMA (16x16x4) rounds it at least eight times.
+// v_mfma_f32_16x16x32_bf16 runs at 16 times the FP32 rate, so six products cost 6 / 16 of the FP32 form.
+// Measured against 64 bits (E_loc of 256 to 2048 walkers, 4 to 42 electrons, both models): the same relative
+// error as the FP32 form to two digits (4e-6 to 6e-5, set by the value channel), 2e-7 to 6e-7 between the two.
+//
+// Only derivative channels (tangents, Laplacian) come from here.  The value channel of the pass (the first row
+// of an electron) keeps the FP32 MFMA of the value pass: log|psi|, the orbital matrices and their inverses
+// amplify its rounding by the walker's conditioning, the derivative channels enter E_loc linearly.
+#include "common.h"
+#include "kernels.h"
+
+namespace dwmi {
+
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+
+// ------------------------------------------------------------------------------------------------
+// Operand parts
+// ------------------------------------------------------------------------------------------------
+__device__ __forceinline__ unsigned pack_bf16(float a, float b) {  // v_cvt_pk_bf16_f32 (nearest even)
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(v2f{a, b}, v2bf));
+}
+__device__ __forceinline__ float lo_f(unsigned u) { return __uint_as_float(u << 16); }
+__device__ __forceinline__ float hi_f(unsigned u) { return __uint_as_float(u & 0xFFFF0000u); }
+
+// Four floats -> the three parts of each, packed in 8 bytes per part.
+__device__ __forceinline__ void split4(v4f x, uint2 (&p)[3]) {
+  const unsigned h0 = pack_bf16(x[0], x[1]), h1 = pack_bf16(x[2], x[3]);
+  const float r0 = x[0] - lo_f(h0), r1 = x[1] - hi_f(h0), r2 = x[2] - lo_f(h1), r3 = x[3] - hi_f(h1);
+  const unsigned m0 = pack_bf16(r0, r1), m1 = pack_bf16(r2, r3);
+  p[0] = uint2{h0, h1};
+  p[1] = uint2{m0, m1};
+  p[2] = uint2{pack_bf16(r0 - lo_f(m0), r1 - hi_f(m0)), pack_bf16(r2 - lo_f(m1), r3 - hi_f(m1))};
+}
+
+// Weights Bt [rows, ldb] (row = output column, K contiguous) in the order the MFMA lanes read them:
+// P[((slice * ncb + cb) * 3 + part) * 64 + lane] = 8 BF16 of column 16 cb + lane % 16, k = 32 slice +
+// 8 (lane / 16) + 0..7.  Columns at or past `cols` are zero.
+__global__ __launch_bounds__(256) void k_split_pack(const float* __restrict__ Bt, int ldb, int cols, int ncb,
+                                                    int slices, uint4* __restrict__ P) {
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (t >= slices * ncb * 64) return;
+  const int lane = t & 63, cb = (t >> 6) % ncb, sl = (t >> 6) / ncb;
+  const int col = cb * 16 + (lane & 15), k = sl * 32 + (lane >> 4) * 8;
+  v4f a = {0.f, 0.f, 0.f, 0.f}, b = a;
+  if (col < cols) {
+    a = *(const v4f*)(Bt + (long)col * ldb + k);
+    b = *(const v4f*)(Bt + (long)col * ldb + k + 4);
+  }
+  uint2 pa[3], pb[3];
+  split4(a, pa);
+  split4(b, pb);
+#pragma unroll
+  for (int p = 0; p < 3; ++p)
+    P[((long)(sl * ncb + cb) * 3 + p) * 64 + lane] = uint4{pa[p].x, pa[p].y, pb[p].x, pb[p].y};
+}
+
+size_t split_pack_bytes(int cols, int K) { return (size_t)(K / 32) * (dw_pad(cols, 256) / 16) * 3 * 64 * 16; }
+
+void launch_split_pack(const float* Bt, int ldb, int cols, int K, void* out, hipStream_t s) {
+  const int ncb = dw_pad(cols, 256) / 16, slices = K / 32;
+  hipLaunchKernelGGL(k_split_pack, dim3((slices * ncb * 64 + 255) / 256), dim3(256), 0, s, Bt, ldb, cols, ncb, slices,
+                     (uint4*)out);
+}
+
+__device__ __forceinline__ int tile_of(int bid, int total) {
+  // workgroups are dealt round-robin to 8 XCDs; each XCD gets a contiguous range of tiles
+  const int per = (total + 7) / 8;
+  return (bid & 7) * per + (bid >> 3);
+}
+
+// ------------------------------------------------------------------------------------------------
+// Main loop of one 256-thread workgroup: acc = A[row0 .. row0 + 16 RB) B[:, 64 NQ columns], wave w owning
+// the 16 NQ columns from block cb0.  A slices of 32 are split while they are staged into LDS (two buffers,
+// one barrier per slice), in lane order (part, row block, lane), so every LDS access is 16 consecutive bytes
+// per lane; a wave's B parts come from L2 straight into registers, one slice ahead.
+// ------------------------------------------------------------------------------------------------
+template <int RB>
+struct SplitLds {
+  uint4 a[2][3][RB][64];
+};
+
+template <int RB, int NQ>
+__device__ __forceinline__ void split_main(const float* __restrict__ A, long row0, long rows, long lda, int slices,
+                                           const uint4* __restrict__ P, int ncb, int cb0, SplitLds<RB>& lds,
+                                           v4f (&acc)[RB][NQ]) {
+  constexpr int AU = RB * 128;  // (row, quad of 4 k) units of a slice
+  constexpr int AIT = (AU + 255) / 256;
+  const int tid = threadIdx.x, lane = tid & 63;
+
+  // unit u: row u / 128 * 16 + u % 16, quad (u / 16) % 8
+  v4f ra[AIT];
+  const float* ap[AIT];
+#pragma unroll
+  for (int it = 0; it < AIT; ++it) {
+    const int u = tid + 256 * it;
+    long gr = row0 + (u >> 7) * 16 + (u & 15);
+    if (gr > rows - 1) gr = rows - 1;
+    ap[it] = A + gr * lda + ((u >> 4) & 7) * 4;
+  }
+  auto gload = [&](int s) {
+#pragma unroll
+    for (int it = 0; it < AIT; ++it)
+      if (AU % 256 == 0 || tid + 256 * it < AU) ra[it] = *(const v4f*)(ap[it] + s * 32);
+  };
+  auto sstore = [&](int buf) {
+#pragma unroll
+    for (int it = 0; it < AIT; ++it) {
+      const int u = tid + 256 * it;
+      if (AU % 256 == 0 || u < AU) {
+        uint2 p[3];
+        split4(ra[it], p);
+        const int quad = (u >> 4) & 7;
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          *((uint2*)&lds.a[buf][k][u >> 7][(quad >> 1) * 16 + (u & 15)] + (quad & 1)) = p[k];
+      }
+    }
+  };
+  v8s b[NQ][3], bn[NQ][3];
+  auto bload = [&](int s, v8s (&d)[NQ][3]) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) d[q][p] = *(const v8s*)&P[((long)(s * ncb + cb0 + q) * 3 + p) * 64 + lane];
+  };
+
+  gload(0);
+  bload(0, b);
+  sstore(0);
+  if (slices > 1) gload(1);
+  for (int s = 0; s < slices; ++s) {
+    const int buf = s & 1;
+    __syncthreads();  // slice s is in lds.a[buf]; every read of lds.a[buf ^ 1] (slice s - 1) is done
+    if (s + 1 < slices) bload(s + 1, bn);
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+      v8s a[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) a[p] = *(const v8s*)&lds.a[buf][p][i][lane];
+#define DW_SPLIT_MFMA(PA, PB)          \
+  _Pragma("unroll") for (int q = 0; q < NQ; ++q) acc[i][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16( \
+      (v8bf)a[PA], (v8bf)b[q][PB], acc[i][q], 0, 0, 0);
+      DW_SPLIT_MFMA(2, 0)
+      DW_SPLIT_MFMA(0, 2)
+      DW_SPLIT_MFMA(1, 1)
+      DW_SPLIT_MFMA(1, 0)
+      DW_SPLIT_MFMA(0, 1)
+      DW_SPLIT_MFMA(0, 0)
+#undef DW_SPLIT_MFMA
+      if (i == RB / 2 && s + 1 < slices) {  // the next slice, loaded a slice ago
+        sstore(buf ^ 1);
+        if (s + 2 < slices) gload(s + 2);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) b[q][p] = bn[q][p];
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// C[M, N] = A[M, K] B (no epilogue): the orbital GEMMs of the Laplacian pass.  688,128 x 256 x 224: 783 us with
+// FP32 MFMA on 128-row tiles, 480 us here.
+// ------------------------------------------------------------------------------------------------
+template <int RB, int NQ>
+__global__ __launch_bounds__(256, 2) void k_split_gemm(const float* __restrict__ A, int lda,
+                                                       const uint4* __restrict__ P, int ncb, float* __restrict__ Cm,
+                                                       int ldc, int M, int N, int slices, int tilesN, int tilesTotal) {
+  __shared__ SplitLds<RB> lds;
+  const int tile = tile_of(blockIdx.x, tilesTotal);
+  if (tile >= tilesTotal) return;  // uniform over the workgroup, before any barrier
+  const long row0 = (long)(tile / tilesN) * (16 * RB);
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int cb0 = (tile % tilesN) * (4 * NQ) + wv * NQ;
+  v4f acc[RB][NQ];
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) acc[i][q] = v4f{0.f, 0.f, 0.f, 0.f};
+  split_main<RB, NQ>(A, row0, M, lda, slices, P, ncb, cb0, lds, acc);
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int c = (cb0 + q) * 16 + (lane & 15);
+      if (c < N) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const long r = row0 + i * 16 + 4 * (lane >> 4) + j;
+          if (r < M) Cm[r * ldc + c] = acc[i][q][j];
+        }
+      }
+    }
+}
+
+void split_gemm(const float* A, int lda, const void* P, float* C, int ldc, int M, int N, int K, int tile,
+                hipStream_t s) {
+  if (M <= 0 || N <= 0) return;
+  const int ncb = dw_pad(N, 256) / 16;
+  const long big = ((long)(M + 95) / 96) * ((N + 255) / 256);
+  if (tile < 0 ? big >= 512 : tile > 0) {
+    const int tilesN = (N + 255) / 256, total = (M + 95) / 96 * tilesN;
+    hipLaunchKernelGGL((k_split_gemm<6, 4>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, A, lda, (const uint4*)P, ncb,
+                       C, ldc, M, N, K / 32, tilesN, total);
+  } else {
+    const int tilesN = (N + 127) / 128, total = (M + 47) / 48 * tilesN;
+    hipLaunchKernelGGL((k_split_gemm<3, 2>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, A, lda, (const uint4*)P, ncb,
+                       C, ldc, M, N, K / 32, tilesN, total);
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// 1-el embedding GEMM of the Laplacian pass with the tanh forward-Laplacian rule.  A workgroup owns E whole
+// electrons (RBE row blocks of 16 channels each) and 64 NQ columns; `out` already holds the value channel y_0
+// (row 0 of each electron).  Per column: z_ch = (X W)_ch + V[walker, ch], y_k = t' z_k (k = 1 .. 3n),
+// y_lap = t' z_lap + t'' sum_k z_k^2.  The rule runs on the accumulators: a column's
+// channels lie in the four 16-lane groups (4 consecutive channels each), so the sum over the tangents is two
+// lane exchanges and the stores are 64-byte row segments, four rows at a time.  Padding channels are left
+// unwritten: rows are independent and nothing reads those of a padding channel.
+//
+// 1,376,256 rows (2048 walkers of 14 electrons) x 320 x 256: 2000 us with FP32 MFMA, 1240 us here, 16 % of it
+// the tail of the rule and its stores (a 32-wide layer takes 504 us; writing its output alone 340 us at the
+// card's 4.1 TB/s).  Matrix cores are busy for 51 % of the cycles at 2.0 GHz: at this load the card lowers its
+// clock from 2.4.  26 electrons (1.7 M rows): 3600 -> 1960 us; 42 electrons (1.0 M rows): 1930 -> 990 us.
+// ------------------------------------------------------------------------------------------------
+template <int RBE, int E, int NQ>
+__global__ __launch_bounds__(256, 2) void k_split_lap(const float* __restrict__ X, int ldx,
+                                                      const uint4* __restrict__ P, int ncb, int slices,
+                                                      const float* __restrict__ V, int ldv, float* __restrict__ out,
+                                                      int ldo, int permute, Shape sh, int tilesN, int tilesTotal) {
+  constexpr int RB = RBE * E;
+  __shared__ SplitLds<RB> lds;
+  const int tile = tile_of(blockIdx.x, tilesTotal);
+  if (tile >= tilesTotal) return;  // uniform over the workgroup, before any barrier
+  const int n = sh.n, C = sh.C, Cp = sh.Cp;
+  const long n_el = (long)sh.B * n;
+  const long g0 = (long)(tile / tilesN) * E;  // first electron
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, g4 = lane >> 4;
+  const int cb0 = (tile % tilesN) * (4 * NQ) + wv * NQ;
+  const int dn = n - sh.u;
+  const int col = cb0 * 16 + (lane & 15);
+  // the accumulators start from V: its loads run beside the first slice's
+  v4f acc[RB][NQ];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const long g = min(g0 + e, n_el - 1);
+    const float* Vp = V + (g / n * Cp + 4 * g4) * (long)ldv + col;
+#pragma unroll
+    for (int kb = 0; kb < RBE; ++kb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) acc[e * RBE + kb][q][j] = Vp[(long)(kb * 16 + j) * ldv + 16 * q];
+  }
+  split_main<RB, NQ>(X, g0 * Cp, n_el * Cp, ldx, slices, P, ncb, cb0, lds, acc);
+
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const long g = g0 + e;
+    if (g >= n_el) break;  // uniform
+    const long b = g / n;
+    const int i = (int)(g - b * n);
+    long ob = g * Cp;
+    if (permute) ob = (i < sh.u) ? (b * sh.u + i) * Cp : (long)sh.B * sh.u * Cp + (b * dn + (i - sh.u)) * Cp;
+    float* op = out + (ob + 4 * g4) * ldo + col;
+    const float* vp = out + ob * ldo + col;
+    float d1[NQ], d2[NQ], S[NQ], zl[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const float th = vp[16 * q];
+      d1[q] = 1.f - th * th;
+      d2[q] = -2.f * th * d1[q];
+      S[q] = 0.f;
+      zl[q] = 0.f;
+    }
+#pragma unroll
+    for (int kb = 0; kb < RBE; ++kb) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int ch = kb * 16 + 4 * g4 + j;
+        const bool tan = ch >= 1 && ch < C - 1;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+          const float z = acc[e * RBE + kb][q][j];
+          S[q] += tan ? z * z : 0.f;
+          if (ch == C - 1) zl[q] = z;
+          if (tan) op[(long)(kb * 16 + j) * ldo + 16 * q] = d1[q] * z;
+        }
+      }
+    }
+    const int cl = C - 1 - (RBE - 1) * 16;  // the Laplacian's row in the last block
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      float s = S[q] + __shfl_xor(S[q], 16, 64);
+      s += __shfl_xor(s, 32, 64);
+      if (g4 == (cl >> 2)) out[(ob + C - 1) * ldo + col + 16 * q] = d1[q] * zl[q] + d2[q] * s;
+    }
+  }
+}
+
+bool split_lap(const float* X, int ldx, const void* P, int K, const float* V, int ldv, float* out, int ldo,
+               int permute, const Shape& sh, int E_max, int cols, hipStream_t s) {
+  const int RBE = sh.Cp / 16, ncb = dw_pad(sh.W1, 256) / 16;
+  const long n_el = (long)sh.B * sh.n;
+#define DW_SPLIT_LAP(R, EE, Q)                                                                                  \
+  do {                                                                                                          \
+    const int tilesN = sh.W1 / (64 * Q);                                                                        \
+    const long total = (n_el + EE - 1) / EE * tilesN;                                                           \
+    hipLaunchKernelGGL((k_split_lap<R, EE, Q>), dim3((unsigned)((total + 7) / 8 * 8)), dim3(256), 0, s, X, ldx, \
+                       (const uint4*)P, ncb, K / 32, V, ldv, out, ldo, permute, sh, tilesN, (int)total);        \
+    return true;                                                                                                \
+  } while (0)
+  // full tiles (96 rows or one electron, 256 columns: A read and split once) where they give two workgroups to
+  // every CU; otherwise fewer electrons and 128 columns, which fill the chip from half as many rows.  More than
+  // 96 rows per electron take 128 columns so that the accumulators stay in registers.  The choice does not change
+  // results.
+  const int EF = RBE <= 6 ? 6 / RBE : 1;
+  bool big = sh.W1 % 256 == 0 && RBE <= 6 && (n_el + EF - 1) / EF * (sh.W1 / 256) >= 512;
+  if (cols == 128 || (E_max > 0 && E_max < EF)) big = false;
+  if (cols == 256 && sh.W1 % 256 == 0 && RBE <= 6 && E_max <= 0) big = true;
+  switch (RBE * 2 + (big ? 1 : 0)) {
+    case 3: DW_SPLIT_LAP(1, 6, 4);
+    case 5: DW_SPLIT_LAP(2, 3, 4);
+    case 7: DW_SPLIT_LAP(3, 2, 4);
+    case 9: DW_SPLIT_LAP(4, 1, 4);
+    case 11: DW_SPLIT_LAP(5, 1, 4);
+    case 13: DW_SPLIT_LAP(6, 1, 4);
+    case 2: DW_SPLIT_LAP(1, 2, 2);
+    case 4: DW_SPLIT_LAP(2, 1, 2);
+    case 6: DW_SPLIT_LAP(3, 1, 2);
+    case 8: DW_SPLIT_LAP(4, 1, 2);
+    case 10: DW_SPLIT_LAP(5, 1, 2);
+    case 12: DW_SPLIT_LAP(6, 1, 2);
+    case 14: DW_SPLIT_LAP(7, 1, 2);
+    case 16: DW_SPLIT_LAP(8, 1, 2);
+    case 18: DW_SPLIT_LAP(9, 1, 2);
+    case 20: DW_SPLIT_LAP(10, 1, 2);
+    case 22: DW_SPLIT_LAP(11, 1, 2);
+    case 24: DW_SPLIT_LAP(12, 1, 2);
+    default: return false;
+  }
+#undef DW_SPLIT_LAP
+}
+
+}  // namespace dwmi

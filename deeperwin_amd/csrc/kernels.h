@@ -53,6 +53,19 @@ void gemm_lap(GemmPrec prec, const float* X, int ldx, const float* Bt, const uin
               hipStream_t s);
 int lap_electrons_per_tile(int Cp, GemmPrec prec);
 
+// FP32 GEMMs on BF16 MFMA with both operands split into three BF16 parts (gemm_split.hip).  P: weights
+// Bt [rows, K] (row = output column, columns at or past `cols` zero) packed by launch_split_pack into
+// split_pack_bytes(cols, K) bytes; K a multiple of 32.
+size_t split_pack_bytes(int cols, int K);
+void launch_split_pack(const float* Bt, int ldb, int cols, int K, void* out, hipStream_t s);
+// C[M, N] = A[M, K] B.  tile: -1 chosen by size, 0 = 48 x 128, 1 or 2 = 96 x 256 (results do not depend on it).
+void split_gemm(const float* A, int lda, const void* P, float* C, int ldc, int M, int N, int K, int tile,
+                hipStream_t s);
+// 1-el GEMM and tanh forward-Laplacian rule of the derivative channels; `out` holds the value channel already.
+// E_max > 0 / cols = 128 ask for the smaller tiles (results do not depend on them).
+bool split_lap(const float* X, int ldx, const void* P, int K, const float* V, int ldv, float* out, int ldo,
+               int permute, const Shape& sh, int E_max, int cols, hipStream_t s);
+
 // Value-pass 1-el GEMM on the Laplacian GEMM's 16x16 MFMA main loop (FP32): out = tanh(X W + V[walker]),
 // V summed over vsplit parts vstride apart; permute sends rows to spin-major order.
 void gemm_value16(const float* X, int ldx, const float* Bt, int K, const float* V, int ldv, int vsplit, long vstride,

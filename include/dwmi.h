@@ -33,7 +33,8 @@ typedef int dw_status;
 typedef struct dw_model dw_model;
 typedef void* dw_stream; /* a hipStream_t; NULL is the default stream */
 
-/* Precision forms.  DW_FP32: every GEMM in FP32 on MFMA, determinant stage in FP64.  DW_BF16X3:
+/* Precision forms.  DW_FP32: GEMM operands and sums in FP32 (on FP32 MFMA; derivative channels of the Laplacian
+ * pass as dw_model_set_lap_form says), determinant stage in FP64.  DW_BF16X3:
  * embedding and orbital GEMMs on BF16 MFMA with FP32 accumulation, operands split into hi+lo BF16 pairs
  * (three products).  DW_BF16: one BF16 product.  DW_FP64: the whole pass in FP64 (the reference's
  * float_precision="float64" mode, configuration.py:1893).  With fp64_cond_threshold > 0, walkers whose
@@ -251,12 +252,23 @@ typedef struct dw_tuning {
   int32_t fwd_mu_split;   /* K-split (1, 2 or 4) of the spin-mean GEMMs of the value pass (FP32 form) */
   int32_t lap_orb_tile;   /* orbital GEMMs of the Laplacian pass                                     */
   int32_t lap_mu_tile;    /* spin-mean GEMMs of the Laplacian pass                                   */
-  int32_t lap_electrons;  /* electrons per workgroup of the fused Laplacian GEMM (E * Cp <= 192)      */
-  int32_t lap_cols;       /* output columns per workgroup of that GEMM: 0 / 128, or 256 (FP32 form,
-                             E * Cp <= 96; larger tiles fall back to 128)                             */
+  int32_t lap_electrons;  /* electrons per workgroup of the fused Laplacian GEMM (E * Cp <= 192); the
+                             FP32 form takes its small tiles when that is fewer than its full tiles hold */
+  int32_t lap_cols;       /* output columns per workgroup of that GEMM (FP32 form): 0 by size, 128 or 256
+                             (E * Cp <= 96; larger tiles fall back to 128)                            */
 } dw_tuning;
 dw_status dw_model_set_tuning(dw_model* m, const dw_tuning* t);
 dw_status dw_model_get_tuning(const dw_model* m, dw_tuning* out);
+
+/* Derivative channels (tangents, Laplacian) of dw_local_energy's GEMMs in the DW_FP32 form.  SPLIT (default): both
+ * operands split exactly into three BF16 parts, six products on BF16 MFMA with FP32 sums; E_loc as accurate as
+ * with FP32 and 1.2 to 1.3 times faster, equal to it to rounding (small batches take FP32 anyway).  FP32: FP32 MFMA.  The value channel
+ * (log|psi|^2, the determinants) is the same bits in both.  For callers whose FP64 statistics of the energies
+ * (the optimisation's loss and clipping state) have to stay bit-equal from run to run, across releases: the
+ * loss uses FP32. */
+#define DW_LAP_SPLIT 0
+#define DW_LAP_FP32 1
+dw_status dw_model_set_lap_form(dw_model* m, int32_t form);
 
 /* ---- Measurement hooks (no counterpart in the reference; used by the benchmark harness) ----
  * When timing is enabled the library brackets selected launches with HIP events recorded on the

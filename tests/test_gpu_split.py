@@ -1,0 +1,51 @@
+"""The split-operand GEMMs of the Laplacian pass (three BF16 parts per FP32 operand, gemm_split.hip): every
+tile height (1 to 12 row blocks of 16 channels per electron), ragged last tiles, both tile choices.  Sizes just over the 32768 rows from which the split form is taken."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from deeperwin_amd.params import ModelShape, init_params
+from deeperwin_amd.physics import generate_el_ion_mapping, init_walkers_gaussian, random_molecule
+
+pytestmark = pytest.mark.gpu
+U32 = 2.0 ** -24
+
+
+@pytest.mark.parametrize("n,B", [(4, 513), (10, 103), (14, 49), (20, 27), (26, 17), (31, 13), (36, 9), (42, 7),
+                                 (47, 5), (52, 5), (58, 5), (60, 3)])
+def test_split_laplacian_matches_fp64_form_for_every_tile(cuda, n, B):
+    """E_loc of the FP32 form against the FP64 form (per walker, the bound of the parity tests:
+    (1 + |E|)(1e-4 + 4 u kappa), kappa the walker's conditioning), and bit-equal for every tile choice."""
+    from deeperwin_amd._native import NativeModel
+
+    R, Z = random_molecule(np.random.default_rng(n), n)
+    R = R.astype(np.float32)
+    shape = ModelShape(n, (n + 1) // 2, len(Z), 3)
+    params = init_params(shape, n)
+    r0 = init_walkers_gaussian(np.random.default_rng(1), B, R, generate_el_ion_mapping(R, Z, n, shape.n_up))
+    r = torch.as_tensor(r0, dtype=torch.float32, device="cuda").contiguous()
+    Rd = torch.as_tensor(R, dtype=torch.float32, device="cuda")
+    Zd = torch.as_tensor(Z, dtype=torch.float32, device="cuda")
+
+    def eloc(m):
+        e, lp = torch.empty(B, device="cuda"), torch.empty(B, device="cuda")
+        m.local_energy(r, Rd, Zd, e, lp)
+        kappa = m.conditioning(B)
+        torch.cuda.synchronize()
+        return e.cpu().numpy(), lp.cpu().numpy(), kappa.cpu().numpy()
+
+    m64 = NativeModel(shape, "fp64")
+    m64.set_params(params)
+    e64, _, kappa = eloc(m64)
+    m = NativeModel(shape)
+    m.set_params(params)
+    e, lp, _ = eloc(m)
+    assert np.all(np.abs(e - e64) <= (1 + np.abs(e64)) * (1e-4 + 4 * U32 * kappa))
+    for choice in ({"lap_electrons": 1, "lap_cols": 128, "lap_orb_tile": 0},
+                   {"lap_electrons": 0, "lap_cols": 256, "lap_orb_tile": 2}):
+        m.set_tuning(**choice)
+        e1, lp1, _ = eloc(m)
+        np.testing.assert_array_equal(e1, e)
+        np.testing.assert_array_equal(lp1, lp)
