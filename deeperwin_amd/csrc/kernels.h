@@ -34,7 +34,7 @@ enum GemmPrec { GEMM_F32 = 0, GEMM_BF16X3 = 1, GEMM_BF16 = 2, GEMM_F64 = 3 };
 void gemm(GemmPrec prec, const float* A, int lda, const float* Bt, const uint16_t* Bhi, const uint16_t* Blo,
           int ldb, float* C, int ldc, int M, int N, int K, const GemmEpi& ep, hipStream_t s);
 
-// FP64 form (VALU FMA, 64 x 64 tiles).  Same operand conventions; K a multiple of 16.
+// FP64 form (FP64 MFMA, gemm_f64.hip).  Same operand conventions; K a multiple of 16.
 void gemm_f64(const double* A, int lda, const double* Bt, int ldb, double* C, int ldc, int M, int N, int K,
               const GemmEpiD& ep, hipStream_t s);
 
