@@ -115,15 +115,19 @@ struct Weights {
   // FP32 form: the three BF16 parts of Wmain / Wo in MFMA lane order (derivative channels, gemm_split.hip)
   std::vector<DevBuf> WmainS;
   DevBuf WoS[2];
+  // FP32 form: Wmain / Wmu / Wo in MFMA lane order (one-launch value layers, value_layer.hip)
+  std::vector<DevBuf> WmainL, WmuL;
+  DevBuf WoL[2];
   // dpe4: pair-stream sets, el-ion stream, ion maps, ion table; h_map GEMM operands per iteration
   DevBuf Wp, bp, Wei, bei, Whim, bhim, table;
   std::vector<DevBuf> WhmT, WhmT_hi, WhmT_lo, bhm, WhmB;  // WhmB: h_map w [pad128(Kh)][32] (gradient pass)
   void release() {
     for (auto* v : {&Wmain, &Wmu, &bias, &Wmain_hi, &Wmain_lo, &Wmu_hi, &Wmu_lo, &WmainT, &WmuT, &WhmT, &WhmT_hi,
-                    &WhmT_lo, &bhm, &WhmB, &WmainS})
+                    &WhmT_lo, &bhm, &WhmB, &WmainS, &WmainL, &WmuL})
       for (auto& b : *v) b.release();
     for (DevBuf* b : {&W2e, &b2e, &Wo[0], &Wo[1], &Wo_hi[0], &Wo_hi[1], &Wo_lo[0], &Wo_lo[1], &WoT[0], &WoT[1], &kappa,
-                      &wenv, &Wp, &bp, &Wei, &bei, &Whim, &bhim, &table, &WoS[0], &WoS[1]})
+                      &wenv, &Wp, &bp, &Wei, &bei, &Whim, &bhim, &table, &WoS[0], &WoS[1], &WoL[0],
+                      &WoL[1]})
       b->release();
     ready = false;
   }
@@ -340,6 +344,13 @@ dw_status pack_split(DevBuf& out, const DevBuf& Bt, int cols, int K) {
   return DW_OK;
 }
 
+dw_status pack_lanes(DevBuf& out, const DevBuf& Bt, int cols, int K) {
+  HIP_TRY(out.ensure(lane_pack_bytes(cols, K)));
+  launch_lane_pack(Bt.as<float>(), K, cols, K, out.p, nullptr);
+  HIP_TRY(hipGetLastError());
+  return DW_OK;
+}
+
 // Build the device layouts of all weights from the host leaves, in float or double.
 dw_status prepare_weights(dw_model* m, Weights& W, bool dbl) {
   for (auto& e : m->expected)
@@ -348,7 +359,7 @@ dw_status prepare_weights(dw_model* m, Weights& W, bool dbl) {
   const bool split = !dbl && m->prec != GEMM_F32;
   const bool parts3 = !dbl && m->prec == GEMM_F32;
   for (auto* v : {&W.Wmain, &W.Wmu, &W.bias, &W.Wmain_hi, &W.Wmain_lo, &W.Wmu_hi, &W.Wmu_lo, &W.WmainT, &W.WmuT,
-                  &W.WmainS})
+                  &W.WmainS, &W.WmainL, &W.WmuL})
     v->resize(m->L);
   auto up = [&](DevBuf& b, const std::vector<float>& v) { return dbl ? upload_as<double>(b, v) : upload(b, v); };
   for (int l = 0; l < m->L; ++l) {
@@ -378,7 +389,10 @@ dw_status prepare_weights(dw_model* m, Weights& W, bool dbl) {
     if ((st = up(W.WmainT[l], wmT))) return st;
     if ((st = up(W.WmuT[l], wuT))) return st;
     if ((st = up(W.bias[l], b.data))) return st;
-    if (parts3 && (st = pack_split(W.WmainS[l], W.Wmain[l], W1, Kx))) return st;
+    if (parts3 && ((st = pack_split(W.WmainS[l], W.Wmain[l], W1, Kx)) ||
+                   (st = pack_lanes(W.WmainL[l], W.Wmain[l], W1, Kx)) ||
+                   (st = pack_lanes(W.WmuL[l], W.Wmu[l], W1, Km))))
+      return st;
     if (split) {
       if ((st = upload_split(W.Wmain_hi[l], W.Wmain_lo[l], wm))) return st;
       if ((st = upload_split(W.Wmu_hi[l], W.Wmu_lo[l], wu))) return st;
@@ -419,7 +433,8 @@ dw_status prepare_weights(dw_model* m, Weights& W, bool dbl) {
     dw_status st;
     if ((st = up(W.Wo[s], wo))) return st;
     if ((st = up(W.WoT[s], woT))) return st;
-    if (parts3 && (st = pack_split(W.WoS[s], W.Wo[s], m->NOp, W1))) return st;
+    if (parts3 && ((st = pack_split(W.WoS[s], W.Wo[s], m->NOp, W1)) || (st = pack_lanes(W.WoL[s], W.Wo[s], m->NOp, W1))))
+      return st;
     if (split && (st = upload_split(W.Wo_hi[s], W.Wo_lo[s], wo))) return st;
     const Leaf& a = m->leaves[leaf_key("envelope_orbitals", ak[s])];
     const Leaf& we = m->leaves[leaf_key("envelope_orbitals", wk[s])];
@@ -615,14 +630,6 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
       launch_dpe4_tanh<T>(ws.HM, W.bhm[l].as<T>(), sh, s);
       launch_dpe4_conv<T>(ws.WM + l * wm_layer, ws.HM, X[l], m->Kx[l], m->Kt0[l], sh, s);
     }
-    // Laplacian pass, FP32 form: spin means formed inside the per-walker GEMM (same values as below)
-    bool fused_mu = false;
-    if constexpr (!DBL) {
-      if (C > 1 && m->prec == GEMM_F32)
-        fused_mu = gemm_mean_lap(X[l], m->Kx[l], m->Kh[l], W.Wmu[l].as<float>(), m->Km[l], W.bias[l].as<float>(),
-                                 ws.V, m->W1, sh, s);
-    }
-    if (!fused_mu) launch_spin_mean<T>(X[l], m->Kx[l], m->Kh[l], ws.MU, m->Km[l], sh, s);
     // value pass: split K of the per-walker spin-mean GEMM so that it fills the chip (its M is only B)
     int vs = 1;
     if (!DBL && C == 1 && m->prec == GEMM_F32) {
@@ -635,6 +642,23 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
       }
       while (vs > 1 && m->Km[l] % (16 * vs) != 0) vs >>= 1;  // each K slice a multiple of the 16-wide K tile
     }
+    const bool last = (l == m->L - 1);
+    T* outp = last ? ws.H : X[l + 1];
+    const int ldo = last ? m->W1 : m->Kx[l + 1];
+    if constexpr (!DBL) {  // small batches: the whole layer in one launch, bit-equal to what follows
+      if (C == 1 && m->prec == GEMM_F32 && m->tune.fwd_main_tile < 0 &&
+          value_layer(X[l], m->Kx[l], m->Kx[l], m->Kh[l], W.WmainL[l].p, W.WmuL[l].p, m->Km[l], W.bias[l].as<float>(),
+                      vs, outp, ldo, last ? 1 : 0, (int)B, m->n, m->u, m->W1, s))
+        continue;
+    }
+    // Laplacian pass, FP32 form: spin means formed inside the per-walker GEMM (same values as below)
+    bool fused_mu = false;
+    if constexpr (!DBL) {
+      if (C > 1 && m->prec == GEMM_F32)
+        fused_mu = gemm_mean_lap(X[l], m->Kx[l], m->Kh[l], W.Wmu[l].as<float>(), m->Km[l], W.bias[l].as<float>(),
+                                 ws.V, m->W1, sh, s);
+    }
+    if (!fused_mu) launch_spin_mean<T>(X[l], m->Kx[l], m->Kh[l], ws.MU, m->Km[l], sh, s);
     GemmEpiT<T> ev;
     ev.bias = W.bias[l].as<T>();
     ev.C = Cp;
@@ -645,9 +669,6 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
     if (!fused_mu)
       gemm_t(m, ws.MU, m->Km[l], W.Wmu[l].as<T>(), W.Wmu_hi[l], W.Wmu_lo[l], m->Km[l], ws.V, m->W1,
              B * Cp, m->W1, m->Km[l], ev, s);
-    const bool last = (l == m->L - 1);
-    T* outp = last ? ws.H : X[l + 1];
-    const int ldo = last ? m->W1 : m->Kx[l + 1];
     GemmEpiT<T> em;
     em.V = ws.V;
     em.ldv = m->W1;
@@ -685,8 +706,10 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
         e0.ldv = Cp * m->W1;
         e0.act_tanh = 1;
         e0.permute = last ? 1 : 0;
-        gemm(GEMM_F32, X[l], Cp * m->Kx[l], W.Wmain[l].as<float>(), nullptr, nullptr, m->Kx[l], outp, Cp * ldo,
-             (int)(B * m->n), m->W1, m->Kx[l], e0, s);
+        if (!value_layer(X[l], (long)Cp * m->Kx[l], m->Kx[l], m->Kh[l], W.WmainL[l].p, W.WmuL[l].p, m->Km[l],
+                         W.bias[l].as<float>(), 1, outp, (long)Cp * ldo, last ? 1 : 0, (int)B, m->n, m->u, m->W1, s))
+          gemm(GEMM_F32, X[l], Cp * m->Kx[l], W.Wmain[l].as<float>(), nullptr, nullptr, m->Kx[l], outp, Cp * ldo,
+               (int)(B * m->n), m->W1, m->Kx[l], e0, s);
         split_lap(X[l], m->Kx[l], W.WmainS[l].p, m->Kx[l], ws.V, m->W1, outp, ldo, last ? 1 : 0, sh,
                   m->tune.lap_electrons, m->tune.lap_cols, s);
       } else {
@@ -700,19 +723,32 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
   const long up_rows = B * m->u * Cp, dn_rows = B * m->dn * Cp;
   GemmEpiT<T> e0;
   e0.tile = C == 1 ? m->tune.fwd_orb_tile : m->tune.lap_orb_tile;
-  for (int sp = 0; sp < 2; ++sp) {
+  bool orb_done = false;
+  if constexpr (!DBL) {
+    if (C == 1 && m->prec == GEMM_F32 && m->tune.fwd_orb_tile < 0)
+      orb_done = value_orbitals(ws.H, m->W1, m->W1, W.WoL[0].p, W.WoL[1].p, ws.O, m->NO, (int)up_rows, (int)dn_rows,
+                                m->NO, s);
+  }
+  for (int sp = 0; sp < 2 && !orb_done; ++sp) {
     const long rows0 = sp ? up_rows : 0, nr = sp ? dn_rows : up_rows;
     if constexpr (!DBL) {
-      if (split) {  // every channel from the split form, then the value rows in FP32
+      if (split) {  // every channel from the split form; the value rows follow in FP32
         split_gemm(ws.H + rows0 * m->W1, m->W1, W.WoS[sp].p, ws.O + rows0 * m->NO, m->NO, (int)nr, m->NO, m->W1,
                    m->tune.lap_orb_tile, s);
-        gemm(GEMM_F32, ws.H + rows0 * m->W1, Cp * m->W1, W.Wo[sp].as<float>(), nullptr, nullptr, m->W1,
-             ws.O + rows0 * m->NO, Cp * m->NO, (int)(nr / Cp), m->NO, m->W1, GemmEpi{}, s);
         continue;
       }
     }
     gemm_t(m, ws.H + rows0 * m->W1, m->W1, W.Wo[sp].as<T>(), W.Wo_hi[sp], W.Wo_lo[sp], m->W1, ws.O + rows0 * m->NO,
            m->NO, nr, m->NO, m->W1, e0, s);
+  }
+  if constexpr (!DBL) {
+    if (split && !value_orbitals(ws.H, (long)Cp * m->W1, m->W1, W.WoL[0].p, W.WoL[1].p, ws.O, (long)Cp * m->NO,
+                                 (int)(B * m->u), (int)(B * m->dn), m->NO, s))
+      for (int sp = 0; sp < 2; ++sp) {
+        const long rows0 = sp ? up_rows : 0;
+        gemm(GEMM_F32, ws.H + rows0 * m->W1, Cp * m->W1, W.Wo[sp].as<float>(), nullptr, nullptr, m->W1,
+             ws.O + rows0 * m->NO, Cp * m->NO, (int)(B * (sp ? m->dn : m->u)), m->NO, m->W1, GemmEpi{}, s);
+      }
   }
   const OrbSrc<T> src{ws.O, m->NO, r, R, W.kappa.as<T>(), W.wenv.as<T>()};
   if (!det_reads_orbitals(m->n, C))

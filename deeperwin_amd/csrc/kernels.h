@@ -66,6 +66,18 @@ void split_gemm(const float* A, int lda, const void* P, float* C, int ldc, int M
 bool split_lap(const float* X, int ldx, const void* P, int K, const float* V, int ldv, float* out, int ldo,
                int permute, const Shape& sh, int E_max, int cols, hipStream_t s);
 
+// One-launch value layers and orbital GEMMs for small batches (value_layer.hip), bit-equal to the separate kernels.
+// Weights in lane order (launch_lane_pack: Bt [rows >= cols, K] into lane_pack_bytes(cols, K) bytes, K a multiple of
+// 32).  value_layer: out = tanh(X W + V), V = the vs K parts of (spin means of the first Kh columns) W_mu plus bias,
+// added in order; rows of X ldx apart, of out ldo apart.  Both return false, launching nothing, where the batch is too
+// large to gain (the rules stand beside them).
+size_t lane_pack_bytes(int cols, int K);
+void launch_lane_pack(const float* Bt, int ldb, int cols, int K, void* out, hipStream_t s);
+bool value_layer(const float* X, long ldx, int K, int Kh, const void* W, const void* Wmu, int Km, const float* bias,
+                 int vs, float* out, long ldo, int permute, int B, int n, int u, int W1, hipStream_t s);
+bool value_orbitals(const float* H, long ldh, int K, const void* W_up, const void* W_dn, float* O, long ldo,
+                    int up_rows, int dn_rows, int N, hipStream_t s);
+
 // Value-pass 1-el GEMM on the Laplacian GEMM's 16x16 MFMA main loop (FP32): out = tanh(X W + V[walker]),
 // V summed over vsplit parts vstride apart; permute sends rows to spin-major order.
 void gemm_value16(const float* X, int ldx, const float* Bt, int K, const float* V, int ldv, int vsplit, long vstride,
