@@ -34,6 +34,7 @@ Module paths are matched by suffix (``find_leaf``), so dicts whose keys carry ha
 from __future__ import annotations
 
 from dataclasses import dataclass
+from functools import lru_cache
 from typing import Dict, Tuple
 
 import numpy as np
@@ -146,14 +147,18 @@ def is_dpe4(params: Dict) -> bool:
         return False
 
 
+@lru_cache(maxsize=4096)
+def _normalised(path: str) -> str:
+    return "/" + "/".join(s for s in path.split("/") if s != "~")
+
+
 def find_leaf(params: Dict, module_suffix: str, leaf: str):
     """Return params[path][leaf] for the unique path ending in ``module_suffix`` (ignoring ``~`` segments)."""
     hits = []
+    suffix = "/" + module_suffix
     for path, leaves in params.items():
-        norm = "/".join(s for s in path.split("/") if s != "~")
-        if norm == module_suffix or norm.endswith("/" + module_suffix):
-            if leaf in leaves:
-                hits.append(leaves[leaf])
+        if leaf in leaves and _normalised(path).endswith(suffix):
+            hits.append(leaves[leaf])
     if len(hits) != 1:
         raise KeyError(f"expected exactly one parameter '{module_suffix}/{leaf}', found {len(hits)}")
     return hits[0]

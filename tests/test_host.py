@@ -136,3 +136,40 @@ def test_config_validation():
         m.validate()
     for prop in (LocalStepsizeProposalConfig(), MCMCLangevinProposalConfig()):
         MCMCConfig(proposal=prop).validate()
+
+
+def test_unchanged_numpy_leaves_are_not_uploaded_again():
+    """set_params compares numpy leaves byte by byte with what was uploaded: in-place changes (also to NaN and to
+    -0.0, non-contiguous views included) upload again, equal content does not."""
+    from deeperwin_amd._native import NativeModel
+    from deeperwin_amd.params import ModelShape, init_params
+
+    m = NativeModel(ModelShape(4, 2, 2, 1))
+    params = init_params(ModelShape(4, 2, 2, 1), 0)
+    key = next(k for k in params if k.endswith("h_el_1/linear_0"))
+    params[key]["w"] = np.asfortranarray(params[key]["w"])  # a layout whose bytes are not in C order
+    calls = []
+    real = m.lib.dw_model_set_param
+
+    class Spy:
+        def __getattr__(self, name):
+            return getattr(real_lib, name)
+
+        def dw_model_set_param(self, *a):
+            calls.append(a[1])
+            return real(*a)
+
+    real_lib, m.lib = m.lib, Spy()
+    m.set_params(params)
+    n = len(calls)
+    assert n > 0
+    m.set_params(params)
+    assert len(calls) == n
+    for value in (np.nan, 0.0, -0.0, 1.0):
+        params[key]["w"][3, 5] = value
+        m.set_params(params)
+        n, before = len(calls), n
+        assert n > before
+        m.set_params(params)
+        assert len(calls) == n
+    m.lib = real_lib
