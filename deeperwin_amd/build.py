@@ -17,7 +17,7 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 LIB = PKG / "libdwmi.so"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-SOURCES = ["gemm.hip", "gemm_split.hip", "gemm_f64.hip", "value_layer.hip", "wf_kernels.hip", "api.cpp", "observables.hip", "grad.hip", "threefry.hip", "proposals.hip",
+SOURCES = ["gemm.hip", "gemm_split.hip", "gemm_f64.hip", "value_layer.hip", "det_lap.hip", "wf_kernels.hip", "api.cpp", "observables.hip", "grad.hip", "threefry.hip", "proposals.hip",
            "dpe4.hip", "dpe4_grad.hip", "noalloc.hip"]
 COMMON = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Xclang", "-target-feature", "-Xclang",
           "-packed-fp32-ops", f"-I{ROOT / 'include'}", f"-I{CSRC}"]

@@ -141,7 +141,7 @@ struct PassBufs {
   T* X[4] = {nullptr, nullptr, nullptr, nullptr};
   T *MU = nullptr, *V = nullptr, *Z = nullptr, *H = nullptr, *O = nullptr, *A = nullptr;
   T *WM = nullptr, *HM = nullptr, *HIM = nullptr;  // dpe4: mapped pairs, h_map rows, ion maps
-  double *ld = nullptr, *sd = nullptr, *g = nullptr, *lap = nullptr;
+  double *ld = nullptr, *sd = nullptr, *g = nullptr, *lap = nullptr, *minv = nullptr;
   float* dcond = nullptr;
 };
 
@@ -514,6 +514,7 @@ size_t layout_pass(const dw_model* m, long B, int C, char* base, PassBufs<T>* ou
   b.sd = cv.take<double>((size_t)B * m->D);
   b.dcond = cv.take<float>((size_t)B * m->D);
   b.g = cv.take<double>((size_t)std::max<long>(1, C > 1 ? B * m->D * 3 * m->n : 1));
+  b.minv = cv.take<double>(det_inverse_elems(B * m->D, m->n, C));
   b.lap = cv.take<double>((size_t)std::max<long>(1, C > 1 ? B * m->D : 1));
   if (out) *out = b;
   return cv.off;
@@ -757,7 +758,7 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
   {
     Timed t(m, C > 1 ? DW_TIMER_DET_LAP : -1, s);
     const CombineValue cv{out_lp, out_phase, out_flags, out_kappa, cond_thr, 0};
-    combined = launch_det<T>(ws.A, src, ws.ld, ws.sd, ws.g, ws.lap, ws.dcond, sh, s, C == 1 ? &cv : nullptr);
+    combined = launch_det<T>(ws.A, src, ws.minv, ws.ld, ws.sd, ws.g, ws.lap, ws.dcond, sh, s, C == 1 ? &cv : nullptr);
   }
   if (!combined)
     launch_combine(ws.ld, ws.sd, ws.g, ws.lap, ws.dcond, cond_thr, r, R, Z, out_lp, out_phase, out_eloc, out_flags,

@@ -9,6 +9,7 @@
 // The spin means of h (the per-walker part of the symmetric features) are applied through a separate
 // per-(walker, channel) GEMM, so the 1-el GEMM contracts over Kh + 2 Ke instead of 3 Kh + 2 Ke.
 #include "common.h"
+#include "det_common.h"
 #include "kernels.h"
 
 namespace dwmi {
@@ -22,14 +23,6 @@ struct ChainScalars {
   int32_t step_nr;
   int32_t pad;
 };
-
-// Scalar-type generic math (T = float for the FP32/BF16 forms, double for the FP64 form).
-__device__ __forceinline__ float dsqrt(float x) { return sqrtf(x); }
-__device__ __forceinline__ double dsqrt(double x) { return sqrt(x); }
-__device__ __forceinline__ float dtanh(float x) { return tanh_fast(x); }
-__device__ __forceinline__ double dtanh(double x) { return tanh(x); }
-__device__ __forceinline__ float dexp(float x) { return expf(x); }
-__device__ __forceinline__ double dexp(double x) { return exp(x); }
 
 // ------------------------------------------------------------------------------------------------
 // Layer-0 one-electron features: per ion [|r_i - R_I|, r_i - R_I] (utils.py:262-273,
@@ -721,54 +714,16 @@ template void launch_tanh_rule<double>(const double*, double*, int, int, const S
 
 // ------------------------------------------------------------------------------------------------
 // Envelope x backflow (envelope_orbitals.py:91-127): A[b, d, i, k] = env_s[i, c] * bf[i, c], c = d n + k,
-// env_s[i, c] = sum_I w_s[I, c] exp(-kappa_s[I, c] |r_i - R_I|), kappa = softplus(alpha), with the product
-// rule for tangents (env depends on electron i only) and the Laplacian
+// env_s[i, c] = sum_I w_s[I, c] exp(-kappa_s[I, c] |r_i - R_I|), kappa = softplus(alpha); the determinant kernels
+// that read O apply the product rule to tangents (env depends on electron i only) and to the Laplacian themselves:
 //   Lap A = Lap(env) bf + 2 grad_i(env) . grad_i(bf) + env Lap(bf),   Lap e^{-k rho} = (k^2 - 2k/rho) e^{-k rho}.
-// O rows are spin-major (up block then down block, Cp rows per electron); A is [B, D, C, n, n].
+// O rows are spin-major (up block then down block); A is [B, D, n, n] (value pass, n > 32).
 // ------------------------------------------------------------------------------------------------
-// Spin-major row of electron i's first channel in O (up block, then down block, Cp rows per electron).
-__device__ __forceinline__ long orb_row(const Shape& sh, long b, int i) {
-  const int dn = sh.n - sh.u;
-  return (i < sh.u) ? (b * sh.u + i) * sh.Cp : (long)sh.B * sh.u * sh.Cp + (b * dn + (i - sh.u)) * sh.Cp;
-}
-
-// Envelope of electron i of walker b at orbital column col; with GRAD also its gradient in r_i and its
-// Laplacian.  Shared by the envelope kernel and the determinant kernels that apply it while reading O.
-template <typename T, bool GRAD>
-__device__ __forceinline__ void envelope_at(const T* __restrict__ kappa, const T* __restrict__ wenv,
-                                            const float* __restrict__ r, const float* __restrict__ R, const Shape& sh,
-                                            long b, int i, int col, T& env, T& g0, T& g1, T& g2, T& lenv) {
-  const int NO = sh.D * sh.n, s = (i < sh.u) ? 0 : 1;
-  const float* ri = r + (b * sh.n + i) * 3;
-  const T* kap = kappa + (long)s * sh.I * NO;
-  const T* we = wenv + (long)s * sh.I * NO;
-  env = T(0);
-  g0 = T(0);
-  g1 = T(0);
-  g2 = T(0);
-  lenv = T(0);
-#pragma unroll 1
-  for (int I = 0; I < sh.I; ++I) {
-    const T dx = (T)ri[0] - (T)R[I * 3 + 0], dy = (T)ri[1] - (T)R[I * 3 + 1], dz = (T)ri[2] - (T)R[I * 3 + 2];
-    const T rho = dsqrt(dx * dx + dy * dy + dz * dz);
-    const T k = kap[I * NO + col];
-    const T e = we[I * NO + col] * dexp(-k * rho);
-    env += e;
-    if constexpr (GRAD) {
-      const T coef = -k * e / rho;
-      g0 += coef * dx;
-      g1 += coef * dy;
-      g2 += coef * dz;
-      lenv += e * (k * k - T(2) * k / rho);
-    }
-  }
-}
-
 template <typename T>
 __global__ void k_envelope(const T* __restrict__ O, int ldo, const float* __restrict__ r, const float* __restrict__ R,
                            const T* __restrict__ kappa, const T* __restrict__ wenv, T* __restrict__ A, Shape sh) {
   // thread order (b, d, i, k): consecutive threads write consecutive elements of A for every channel
-  const int n = sh.n, NO = sh.D * n, C = sh.C;
+  const int n = sh.n, NO = sh.D * n;
   const long total = (long)sh.B * n * NO;
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= total) return;
@@ -781,38 +736,9 @@ __global__ void k_envelope(const T* __restrict__ O, int ldo, const float* __rest
   const int col = d_ * n + kk_;
   const long orow = orb_row(sh, b, i);
   T env, g0, g1, g2, lenv;
-  if (C > 1)
-    envelope_at<T, true>(kappa, wenv, r, R, sh, b, i, col, env, g0, g1, g2, lenv);
-  else
-    envelope_at<T, false>(kappa, wenv, r, R, sh, b, i, col, env, g0, g1, g2, lenv);
+  envelope_at<T, false>(kappa, wenv, r, R, sh, b, i, col, env, g0, g1, g2, lenv);
   const int d = col / n, k = col % n;
-  const long nn = (long)n * n;
-  T* Ab = A + ((b * sh.D + d) * C) * nn + (long)i * n + k;
-  const T bf0 = O[orow * ldo + col];
-  Ab[0] = env * bf0;
-  if (C > 1) {
-    // tangent channels: loads of 8 channels are issued before their stores
-    const T* Oc = O + (orow + 1) * ldo + col;
-    T* Ac = Ab + nn;
-    const int nt = C - 2;
-    int ch = 0;
-    for (; ch + 8 <= nt; ch += 8) {
-      T v[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) v[q] = env * Oc[(long)(ch + q) * ldo];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) Ac[(long)(ch + q) * nn] = v[q];
-    }
-    for (; ch < nt; ++ch) Ac[(long)ch * nn] = env * Oc[(long)ch * ldo];
-    // electron i's own coordinates also carry the envelope gradient (one rounding: fma with g_c bf0)
-    Ac[(long)(3 * i + 0) * nn] = fma(env, Oc[(long)(3 * i + 0) * ldo], g0 * bf0);
-    Ac[(long)(3 * i + 1) * nn] = fma(env, Oc[(long)(3 * i + 1) * ldo], g1 * bf0);
-    Ac[(long)(3 * i + 2) * nn] = fma(env, Oc[(long)(3 * i + 2) * ldo], g2 * bf0);
-    const T t0 = O[(orow + 1 + 3 * i) * ldo + col];
-    const T t1 = O[(orow + 2 + 3 * i) * ldo + col];
-    const T t2 = O[(orow + 3 + 3 * i) * ldo + col];
-    Ab[(long)(C - 1) * nn] = lenv * bf0 + env * O[(orow + C - 1) * ldo + col] + T(2) * (g0 * t0 + g1 * t1 + g2 * t2);
-  }
+  A[(b * sh.D + d) * (long)nn_i + (long)i * n + k] = env * O[orow * ldo + col];
 }
 
 template <typename T>
@@ -838,99 +764,6 @@ template void launch_envelope<double>(const double*, int, const float*, const fl
 // The 1-norm condition number |M|_1 |M^-1|_1 (Laplacian mode) or the pivot ratio max|U_pp| / min|U_pp|
 // (value mode) is written per matrix to dcond; results are FP64.
 // ------------------------------------------------------------------------------------------------
-__device__ __forceinline__ double readlane_d(double v, int lane) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
-  return __hiloint2double(hi, lo);
-}
-
-__device__ __forceinline__ double wave_max_d(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-  return v;
-}
-__device__ __forceinline__ double wave_min_d(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
-  return v;
-}
-
-// In-register LU of the column-per-lane matrix.  Returns the number of row swaps; perm[] (uniform)
-// records the row order; mydiag receives U_jj in lane j.
-template <int NMAX>
-__device__ __forceinline__ int lu_columns(double (&col)[NMAX], int (&perm)[NMAX], double& mydiag, bool& sing, int n,
-                                          int lane) {
-  int swaps = 0;
-#pragma unroll
-  for (int i = 0; i < NMAX; ++i) perm[i] = i;
-#pragma unroll
-  for (int p = 0; p < NMAX; ++p) {
-    if (p < n) {
-    double best = -1.0;
-    int bidx = p;
-#pragma unroll
-    for (int i = p; i < NMAX; ++i) {
-      if (i < n) {
-        const double a = fabs(col[i]);
-        if (a > best) {
-          best = a;
-          bidx = i;
-        }
-      }
-    }
-    const int piv = __builtin_amdgcn_readlane(bidx, p);
-    const double bval = readlane_d(best, p);
-    if (!(bval > 0.0)) sing = true;
-    if (piv != p) {
-      ++swaps;
-#pragma unroll
-      for (int i = p + 1; i < NMAX; ++i) {
-        if (i == piv) {
-          const double t = col[p];
-          col[p] = col[i];
-          col[i] = t;
-          const int tp = perm[p];
-          perm[p] = perm[i];
-          perm[i] = tp;
-        }
-      }
-    }
-    const double pivot = readlane_d(col[p], p);
-    if (lane == p) {
-      mydiag = col[p];
-      const double rp = 1.0 / pivot;  // multipliers by the reciprocal, as LAPACK's dgetf2 scales
-#pragma unroll
-      for (int i = p + 1; i < NMAX; ++i)
-        if (i < n) col[i] = col[i] * rp;
-    }
-#pragma unroll
-    for (int i = p + 1; i < NMAX; ++i) {
-      if (i < n) {
-        const double li = readlane_d(col[i], p);
-        if (lane > p) col[i] -= li * col[p];
-      }
-    }
-    }
-  }
-  return swaps;
-}
-
-template <int NMAX>
-__device__ __forceinline__ void finish_slogdet(double mydiag, int swaps, bool sing, int n, int lane, double& logabs,
-                                               double& sgn) {
-  const bool act = lane < n;
-  double lg = act ? log(fabs(mydiag)) : 0.0;
-  lg = wave_sum_d(lg);
-  const unsigned long long neg = __ballot(act && mydiag < 0.0);
-  const int nneg = __popcll(neg) + swaps;
-  sgn = (nneg & 1) ? -1.0 : 1.0;
-  logabs = lg;
-  if (sing) {
-    sgn = 0.0;
-    logabs = -INFINITY;
-  }
-}
-
 // Value-pass combine of one walker's D determinants (log|det| l, sign sg, matrix conditioning dc).
 __device__ __forceinline__ void combine_value_walker(const double* l, const double* sg, const float* dc, int D,
                                                      float cond_thr, long b, float* __restrict__ out_lp,
@@ -1086,13 +919,13 @@ __global__ __launch_bounds__(256) void k_det_value(OrbSrc<TA> src, double* __res
   }
 }
 
-// Laplacian mode (n <= 32): WPB matrices per workgroup, one per wavefront; LU and inverse with a lane per
+// Laplacian mode (n <= 16): WPB matrices per workgroup, one per wavefront; LU and inverse with a lane per
 // column, M^-1 through LDS into MFMA operand registers, then the channel passes on FP64 MFMA.
-// ENV: the matrices are read from the orbitals O and the envelope is applied on the way (no stored A);
+// The matrices are read from the orbitals O and the envelope is applied on the way (no stored A);
 // while the value channel is read, each wavefront tabulates in LDS the envelope, the own-electron
 // gradient terms g_c bf0 (channel 3i + c of row i gains them) and the Laplacian channel, [row][column].
-template <int NMAX, int WPB, typename TA, bool ENV>
-__global__ __launch_bounds__(64 * WPB) void k_det_lap(const TA* __restrict__ A, OrbSrc<TA> src, Shape sh,
+template <int NMAX, int WPB, typename TA>
+__global__ __launch_bounds__(64 * WPB) void k_det_lap(OrbSrc<TA> src, Shape sh,
                                                       double* __restrict__ ld, double* __restrict__ sd,
                                                       double* __restrict__ g, double* __restrict__ lapd,
                                                       float* __restrict__ dcond, long nmat, int n, int C) {
@@ -1101,14 +934,12 @@ __global__ __launch_bounds__(64 * WPB) void k_det_lap(const TA* __restrict__ A, 
   long bd = (long)blockIdx.x * WPB + wv;
   const bool valid_mat = bd < nmat;
   if (!valid_mat) bd = nmat - 1;  // keep the wave in the barriers; results are not stored
-  static_assert(NMAX == 16 || NMAX == 32, "channel passes are written for 16 x 16 MFMA blocks");
+  static_assert(NMAX == 16, "larger matrices: det_lap.hip");
   constexpr int NN = NMAX * NMAX;
   double* sMi = dsm + (size_t)wv * NN;
   TA* sE = (TA*)(dsm + (size_t)WPB * NN) + (size_t)wv * 5 * NN;  // ENV tables: [row][column]
   TA* sG = sE + NN;                                               // [c][row][column]
   TA* sL = sE + 4 * NN;
-  const long nn = (long)n * n;
-  const TA* Ab = ENV ? nullptr : A + bd * C * nn;
   const bool act = lane < n;
   const int nd = 3 * n;
   const long b = bd / sh.D;
@@ -1119,7 +950,7 @@ __global__ __launch_bounds__(64 * WPB) void k_det_lap(const TA* __restrict__ A, 
   double csum = 0.0;
 #pragma unroll
   for (int i = 0; i < NMAX; ++i) {
-    if constexpr (ENV) {
+    {
       double v = 0.0;
       TA e0 = TA(0), gb0 = TA(0), gb1 = TA(0), gb2 = TA(0), lp = TA(0);
       if (act && i < n) {
@@ -1146,8 +977,6 @@ __global__ __launch_bounds__(64 * WPB) void k_det_lap(const TA* __restrict__ A, 
         sL[i * NMAX + lane] = lp;
       }
       col[i] = v;
-    } else {
-      col[i] = (act && i < n) ? (double)Ab[i * n + lane] : 0.0;
     }
     csum += fabs(col[i]);
   }
@@ -1201,7 +1030,7 @@ __global__ __launch_bounds__(64 * WPB) void k_det_lap(const TA* __restrict__ A, 
   // grouped reduction (same pairing order as a single wave sum).
   double qacc = 0.0;
   {
-    constexpr int NB = NMAX / 16, G = (NMAX == 16) ? 2 : 1;  // measured: 2 / 1 fastest at n = 14 / 26
+    constexpr int NB = NMAX / 16, G = 2;  // measured fastest at n = 14
     const int ri = lane & 15, kq = lane >> 4;
     double miA[NB][NB][4];
 #pragma unroll
@@ -1210,7 +1039,7 @@ __global__ __launch_bounds__(64 * WPB) void k_det_lap(const TA* __restrict__ A, 
       for (int K = 0; K < NB; ++K)
 #pragma unroll
         for (int q = 0; q < 4; ++q) miA[I][K][q] = sMi[(I * 16 + ri) * NMAX + K * 16 + kq + 4 * q];
-    // ENV: envelope and the O row base of each element this lane holds
+    // envelope and the O row base of each element this lane holds
     TA envq[NB][NB][4];
     const TA* ob[NB][NB][4];
 #pragma unroll
@@ -1220,15 +1049,14 @@ __global__ __launch_bounds__(64 * WPB) void k_det_lap(const TA* __restrict__ A, 
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const int rr = K * 16 + kq + 4 * q, cc = J * 16 + ri;
-          envq[K][J][q] = ENV ? sE[rr * NMAX + cc] : TA(1);
-          ob[K][J][q] = (ENV && rr < n && cc < n) ? src.O + orb_row(sh, b, rr) * src.ldo + dcol + cc : src.O;
+          envq[K][J][q] = sE[rr * NMAX + cc];
+          ob[K][J][q] = (rr < n && cc < n) ? src.O + orb_row(sh, b, rr) * src.ldo + dcol + cc : src.O;
         }
     TA cur[G][NB][NB][4], nxt[G][NB][NB][4];
     auto load = [&](TA (&d)[G][NB][NB][4], int k0) {
 #pragma unroll
       for (int c = 0; c < G; ++c) {
         const int k = k0 + c;
-        const TA* Tg = ENV ? nullptr : Ab + (long)(1 + (k < nd ? k : 0)) * nn;
 #pragma unroll
         for (int K = 0; K < NB; ++K)
 #pragma unroll
@@ -1237,10 +1065,7 @@ __global__ __launch_bounds__(64 * WPB) void k_det_lap(const TA* __restrict__ A, 
             for (int q = 0; q < 4; ++q) {
               const int rr = K * 16 + kq + 4 * q, cc = J * 16 + ri;
               const bool in = k < nd && rr < n && cc < n;
-              if constexpr (ENV)
-                d[c][K][J][q] = in ? ob[K][J][q][(long)(1 + k) * src.ldo] : TA(0);
-              else
-                d[c][K][J][q] = in ? Tg[rr * n + cc] : TA(0);
+              d[c][K][J][q] = in ? ob[K][J][q][(long)(1 + k) * src.ldo] : TA(0);
             }
       }
     };
@@ -1260,13 +1085,9 @@ __global__ __launch_bounds__(64 * WPB) void k_det_lap(const TA* __restrict__ A, 
           for (int J = 0; J < NB; ++J)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-              if constexpr (ENV) {
-                const int rr = K * 16 + kq + 4 * q, cc = J * 16 + ri;
-                const TA own = (rr == kr) ? sG[(kc3 * NMAX + rr) * NMAX + cc] : TA(0);
-                dmB[K][J][q] = (double)fma(envq[K][J][q], cur[c][K][J][q], own);
-              } else {
-                dmB[K][J][q] = (double)cur[c][K][J][q];
-              }
+              const int rr = K * 16 + kq + 4 * q, cc = J * 16 + ri;
+              const TA own = (rr == kr) ? sG[(kc3 * NMAX + rr) * NMAX + cc] : TA(0);
+              dmB[K][J][q] = (double)fma(envq[K][J][q], cur[c][K][J][q], own);
             }
         double t = 0.0;
 #pragma unroll
@@ -1307,12 +1128,11 @@ __global__ __launch_bounds__(64 * WPB) void k_det_lap(const TA* __restrict__ A, 
     qacc = wave_sum_d(qacc);
   }
   // tr(M^-1 Lap M): lane c takes column c of Lap M and row c of M^-1
-  const TA* Tl = ENV ? nullptr : Ab + (long)(C - 1) * nn;
   double tp = 0.0;
   if (act) {
 #pragma unroll
     for (int e = 0; e < NMAX; ++e)
-      if (e < n) tp += sMi[lane * NMAX + e] * (double)(ENV ? sL[e * NMAX + lane] : Tl[e * n + lane]);
+      if (e < n) tp += sMi[lane * NMAX + e] * (double)sL[e * NMAX + lane];
   }
   tp = wave_sum_d(tp);
   if (lane == 0 && valid_mat) {
@@ -1323,226 +1143,6 @@ __global__ __launch_bounds__(64 * WPB) void k_det_lap(const TA* __restrict__ A, 
   }
 }
 
-// Laplacian mode, large matrices (n > 32): one 256-thread workgroup per matrix, FP64 in LDS.
-// Element-parallel partial-pivot LU (wave 0 searches the pivot), inverse by per-column substitution, then
-// the tangent channels on FP64 MFMA blocks (below).
-template <typename TA>
-__global__ __launch_bounds__(256) void k_det_lds(const TA* __restrict__ A, double* __restrict__ ld,
-                                                 double* __restrict__ sd, double* __restrict__ g,
-                                                 double* __restrict__ lapd, float* __restrict__ dcond, int n, int C) {
-  extern __shared__ double sm[];
-  const int P = n + 1;
-  double* T = sm;           // LU factors, then channel matrices
-  double* Mi = T + n * P;   // inverse
-  double* lcol = Mi + n * P;
-  double* red = lcol + 64;
-  int* perm = (int*)(red + 32);
-  __shared__ int piv_sh, sing_sh;
-  const long bd = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const long nn = (long)n * n;
-  const TA* Ab = A + bd * C * nn;
-  double csum_local = 0.0;
-  for (int e = tid; e < n * n; e += 256) T[(e / n) * P + (e % n)] = (double)Ab[e];
-  if (tid < n) perm[tid] = tid;
-  if (tid == 0) sing_sh = 0;
-  __syncthreads();
-  {  // 1-norm of M (max column sum)
-    for (int c = tid; c < n; c += 256) {
-      double cs = 0.0;
-      for (int rr = 0; rr < n; ++rr) cs += fabs(T[rr * P + c]);
-      csum_local = fmax(csum_local, cs);
-    }
-  }
-  int swaps = 0;
-  for (int p = 0; p < n; ++p) {
-    if (wid == 0) {
-      double best = -1.0;
-      int bidx = p;
-      const int rr = p + lane;
-      if (rr < n) {
-        best = fabs(T[rr * P + p]);
-        bidx = rr;
-      }
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        const double ob = __shfl_xor(best, o, 64);
-        const int oi = __shfl_xor(bidx, o, 64);
-        if (ob > best || (ob == best && oi < bidx)) {
-          best = ob;
-          bidx = oi;
-        }
-      }
-      if (lane == 0) {
-        piv_sh = bidx;
-        if (!(best > 0.0)) sing_sh = 1;
-      }
-    }
-    __syncthreads();
-    const int piv = piv_sh;
-    if (piv != p) {
-      for (int j = tid; j < n; j += 256) {
-        const double t = T[p * P + j];
-        T[p * P + j] = T[piv * P + j];
-        T[piv * P + j] = t;
-      }
-      if (tid == 0) {
-        const int tp = perm[p];
-        perm[p] = perm[piv];
-        perm[piv] = tp;
-      }
-      ++swaps;
-    }
-    __syncthreads();
-    const double pivot = T[p * P + p];
-    for (int rr = p + 1 + tid; rr < n; rr += 256) {
-      const double l = T[rr * P + p] / pivot;
-      lcol[rr] = l;
-      T[rr * P + p] = l;
-    }
-    __syncthreads();
-    const int m = n - p - 1;
-    for (int e = tid; e < m * m; e += 256) {
-      const int rr = p + 1 + e / m, cc = p + 1 + e % m;
-      T[rr * P + cc] -= lcol[rr] * T[p * P + cc];
-    }
-    __syncthreads();
-  }
-  double lsum = 0.0;
-  int nneg = 0;
-  double umax = 0.0, umin = 1e300;
-  for (int q = tid; q < n; q += 256) {
-    const double up = T[q * P + q];
-    lsum += log(fabs(up));
-    nneg += up < 0.0 ? 1 : 0;
-    umax = fmax(umax, fabs(up));
-    umin = fmin(umin, fabs(up));
-  }
-  lsum = block_sum_d(lsum, red);
-  const double negs = block_sum_d((double)nneg, red + 8);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    umax = fmax(umax, __shfl_xor(umax, o, 64));
-    umin = fmin(umin, __shfl_xor(umin, o, 64));
-  }
-  __syncthreads();
-  if (lane == 0) {
-    lcol[wid] = umax;
-    lcol[8 + wid] = umin;
-  }
-  __syncthreads();
-  double gmax = 0.0, gmin = 1e300;
-  for (int w = 0; w < 4; ++w) {
-    gmax = fmax(gmax, lcol[w]);
-    gmin = fmin(gmin, lcol[8 + w]);
-  }
-  const bool sing = sing_sh != 0;
-  const double logabs = sing ? -INFINITY : lsum;
-  const double sgn = sing ? 0.0 : ((((int)negs + swaps) & 1) ? -1.0 : 1.0);
-  __syncthreads();
-  // inverse: column j solves L U x = P e_j
-  for (int j = tid; j < n; j += 256) {
-    for (int p = 0; p < n; ++p) {
-      double y = (perm[p] == j) ? 1.0 : 0.0;
-      for (int q = 0; q < p; ++q) y -= T[p * P + q] * Mi[q * P + j];
-      Mi[p * P + j] = y;
-    }
-    for (int p = n - 1; p >= 0; --p) {
-      double x = Mi[p * P + j];
-      for (int q = p + 1; q < n; ++q) x -= T[p * P + q] * Mi[q * P + j];
-      Mi[p * P + j] = x / T[p * P + p];
-    }
-  }
-  __syncthreads();
-  double isum = 0.0;
-  for (int c = tid; c < n; c += 256) {
-    double cs = 0.0;
-    for (int rr = 0; rr < n; ++rr) cs += fabs(Mi[rr * P + c]);
-    isum = fmax(isum, cs);
-  }
-  double nA = 0.0, nI = 0.0;
-  {
-    double a1 = csum_local, a2 = isum;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      a1 = fmax(a1, __shfl_xor(a1, o, 64));
-      a2 = fmax(a2, __shfl_xor(a2, o, 64));
-    }
-    __syncthreads();
-    if (lane == 0) {
-      lcol[wid] = a1;
-      lcol[8 + wid] = a2;
-    }
-    __syncthreads();
-    for (int w = 0; w < 4; ++w) {
-      nA = fmax(nA, lcol[w]);
-      nI = fmax(nI, lcol[8 + w]);
-    }
-  }
-  // Channel passes on FP64 MFMA over 16 x 16 blocks (nb = ceil(n / 16) <= 4): wave J computes the block
-  // column J of Y_k = M^-1 dM_k and the matching blocks of Y_k^T = dM_k^T M^-T, so tr Y_k^2 is the sum of
-  // their elementwise products; lane l holds operand elements [l%16][l/16 + 4s] (A) / [l/16 + 4s][l%16] (B).
-  const int nd = 3 * n;
-  const int nb = (n + 15) >> 4;
-  const int J = wid, ri = lane & 15, kq = lane >> 4;
-  const bool wact = J < nb;
-  auto mi_at = [&](int rr, int cc) -> double { return (rr < n && cc < n) ? Mi[rr * P + cc] : 0.0; };
-  auto dm_at = [&](int rr, int cc) -> double { return (rr < n && cc < n) ? T[rr * P + cc] : 0.0; };
-  double miJ[4][4];  // M^-1[J*16 + ri][K*16 + kq + 4 q]
-#pragma unroll
-  for (int K = 0; K < 4; ++K)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) miJ[K][q] = wact ? mi_at(J * 16 + ri, K * 16 + kq + 4 * q) : 0.0;
-  double qacc = 0.0;
-  for (int ch = 1; ch <= nd; ++ch) {
-    __syncthreads();
-    const TA* Tg = Ab + (long)ch * nn;
-    for (int e = tid; e < n * n; e += 256) T[(e / n) * P + (e % n)] = (double)Tg[e];
-    __syncthreads();
-    double pd = 0.0;
-    if (wact) {
-      double dmJ[4][4];  // dM[K*16 + kq + 4 q][J*16 + ri]
-#pragma unroll
-      for (int K = 0; K < 4; ++K)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          dmJ[K][q] = (K < nb) ? dm_at(K * 16 + kq + 4 * q, J * 16 + ri) : 0.0;
-          pd += miJ[K][q] * dmJ[K][q];
-        }
-      for (int I = 0; I < nb; ++I) {
-        v4d y = {0.0, 0.0, 0.0, 0.0}, yt = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int K = 0; K < 4; ++K) {
-          if (K < nb) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              y = __builtin_amdgcn_mfma_f64_16x16x4f64(mi_at(I * 16 + ri, K * 16 + kq + 4 * q), dmJ[K][q], y, 0, 0, 0);
-              yt = __builtin_amdgcn_mfma_f64_16x16x4f64(dm_at(K * 16 + kq + 4 * q, I * 16 + ri), miJ[K][q], yt, 0, 0, 0);
-            }
-          }
-        }
-        qacc += y[0] * yt[0] + y[1] * yt[1] + y[2] * yt[2] + y[3] * yt[3];
-      }
-    }
-    const double gs = block_sum_d(pd, red);
-    if (tid == 0) g[bd * nd + (ch - 1)] = gs;
-  }
-  qacc = block_sum_d(qacc, red + 8);
-  __syncthreads();
-  const TA* Tl = Ab + (long)(C - 1) * nn;
-  double tp = 0.0;
-  for (int e = tid; e < n * n; e += 256) {
-    const int a = e / n, q = e % n;
-    tp += Mi[a * P + q] * (double)Tl[q * n + a];
-  }
-  const double tr = block_sum_d(tp, red);
-  if (tid == 0) {
-    ld[bd] = logabs;
-    sd[bd] = sgn;
-    lapd[bd] = tr - qacc;
-    dcond[bd] = (float)(nA * nI);
-  }
-}
 
 // Value mode, 32 < n <= 64: one wavefront per matrix, the matrix in LDS (FP64, pitch n + 1), lane j owns
 // column j.  Partial-pivot LU: argmax of the pivot column by shuffles (lowest row on ties), row swap and
@@ -1618,22 +1218,18 @@ __global__ __launch_bounds__(64) void k_det_value_lds(const TA* __restrict__ A, 
 }
 
 template <typename TA>
-bool launch_det(const TA* A, const OrbSrc<TA>& src, double* ld, double* sd, double* g, double* lapd, float* dcond,
+bool launch_det(const TA* A, const OrbSrc<TA>& src, double* minv, double* ld, double* sd, double* g, double* lapd, float* dcond,
                 const Shape& sh, hipStream_t s, const CombineValue* combine) {
   const int n = sh.n;
   const long nmat = (long)sh.B * sh.D;
   const long stride = (long)sh.C * n * n;
+  if (sh.C > 1 && n > 16) {
+    launch_det_lap_large<TA>(src, minv, ld, sd, g, lapd, dcond, sh, s);
+    return false;
+  }
   if (n > 32) {
-    const size_t shm = (size_t)(2 * n * (n + 1) + 64 + 32) * sizeof(double) + 64 * sizeof(int);
-    if (sh.C == 1) {
-      const size_t shv = (size_t)n * (n + 1) * sizeof(double);  // <= 31.5 KB for n <= 63
-      hipLaunchKernelGGL((k_det_value_lds<TA>), dim3((unsigned)nmat), dim3(64), shv, s, A, ld, sd, dcond, n, stride);
-    } else {
-      if (shm > 65536) (void)hipFuncSetAttribute((const void*)k_det_lds<TA>,
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-      hipLaunchKernelGGL((k_det_lds<TA>), dim3((unsigned)nmat), dim3(256), shm, s, A, ld, sd, g, lapd, dcond, n,
-                         sh.C);
-    }
+    const size_t shv = (size_t)n * (n + 1) * sizeof(double);  // <= 31.5 KB for n <= 63
+    hipLaunchKernelGGL((k_det_value_lds<TA>), dim3((unsigned)nmat), dim3(64), shv, s, A, ld, sd, dcond, n, stride);
     return false;
   }
   if (sh.C == 1) {
@@ -1654,23 +1250,16 @@ bool launch_det(const TA* A, const OrbSrc<TA>& src, double* ld, double* sd, doub
       hipLaunchKernelGGL((k_det_value<32, TA>), grid, dim3(256), 0, s, src, ld, sd, dcond, nmat, n, sh, co);
     return co.fuse != 0;
   }
-  if (n <= 16) {
-    // M^-1 (FP64) plus the envelope tables (5 [16][16] arrays of TA) per wavefront
-    constexpr int NM = 16, W = 4;
-    const size_t shm = (size_t)W * (NM * NM) * (sizeof(double) + 5 * sizeof(TA));
-    hipLaunchKernelGGL((k_det_lap<NM, W, TA, true>), dim3((unsigned)((nmat + W - 1) / W)), dim3(64 * W), shm, s, A,
-                       src, sh, ld, sd, g, lapd, dcond, nmat, n, sh.C);
-  } else {
-    constexpr int NM = 32, W = 2;
-    const size_t shm = (size_t)W * (NM * NM) * sizeof(double);
-    hipLaunchKernelGGL((k_det_lap<NM, W, TA, false>), dim3((unsigned)((nmat + W - 1) / W)), dim3(64 * W), shm, s, A,
-                       src, sh, ld, sd, g, lapd, dcond, nmat, n, sh.C);
-  }
+  // M^-1 (FP64) plus the envelope tables (5 [16][16] arrays of TA) per wavefront
+  constexpr int NM = 16, W = 4;
+  const size_t shm = (size_t)W * (NM * NM) * (sizeof(double) + 5 * sizeof(TA));
+  hipLaunchKernelGGL((k_det_lap<NM, W, TA>), dim3((unsigned)((nmat + W - 1) / W)), dim3(64 * W), shm, s, src, sh, ld,
+                     sd, g, lapd, dcond, nmat, n, sh.C);
   return false;
 }
-template bool launch_det<float>(const float*, const OrbSrc<float>&, double*, double*, double*, double*, float*,
+template bool launch_det<float>(const float*, const OrbSrc<float>&, double*, double*, double*, double*, double*, float*,
                                 const Shape&, hipStream_t, const CombineValue*);
-template bool launch_det<double>(const double*, const OrbSrc<double>&, double*, double*, double*, double*, float*,
+template bool launch_det<double>(const double*, const OrbSrc<double>&, double*, double*, double*, double*, double*, float*,
                                  const Shape&, hipStream_t, const CombineValue*);
 
 // ------------------------------------------------------------------------------------------------
