@@ -112,8 +112,8 @@ struct Weights {
   std::vector<DevBuf> Wmain, Wmu, bias, Wmain_hi, Wmain_lo, Wmu_hi, Wmu_lo;
   std::vector<DevBuf> WmainT, WmuT;  // transposed copies for the gradient pass ([pad128(K)][W1])
   DevBuf W2e, b2e, Wo[2], Wo_hi[2], Wo_lo[2], WoT[2], kappa, wenv;
-  // FP32 form: the three BF16 parts of Wmain / Wo in MFMA lane order (derivative channels, gemm_split.hip)
-  std::vector<DevBuf> WmainS;
+  // FP32 form: the three BF16 parts of Wmain / Wmu / Wo in MFMA lane order (derivative channels, gemm_split.hip)
+  std::vector<DevBuf> WmainS, WmuS;
   DevBuf WoS[2];
   // FP32 form: Wmain / Wmu / Wo in MFMA lane order (one-launch value layers, value_layer.hip)
   std::vector<DevBuf> WmainL, WmuL;
@@ -123,7 +123,7 @@ struct Weights {
   std::vector<DevBuf> WhmT, WhmT_hi, WhmT_lo, bhm, WhmB;  // WhmB: h_map w [pad128(Kh)][32] (gradient pass)
   void release() {
     for (auto* v : {&Wmain, &Wmu, &bias, &Wmain_hi, &Wmain_lo, &Wmu_hi, &Wmu_lo, &WmainT, &WmuT, &WhmT, &WhmT_hi,
-                    &WhmT_lo, &bhm, &WhmB, &WmainS, &WmainL, &WmuL})
+                    &WhmT_lo, &bhm, &WhmB, &WmainS, &WmuS, &WmainL, &WmuL})
       for (auto& b : *v) b.release();
     for (DevBuf* b : {&W2e, &b2e, &Wo[0], &Wo[1], &Wo_hi[0], &Wo_hi[1], &Wo_lo[0], &Wo_lo[1], &WoT[0], &WoT[1], &kappa,
                       &wenv, &Wp, &bp, &Wei, &bei, &Whim, &bhim, &table, &WoS[0], &WoS[1], &WoL[0],
@@ -359,7 +359,7 @@ dw_status prepare_weights(dw_model* m, Weights& W, bool dbl) {
   const bool split = !dbl && m->prec != GEMM_F32;
   const bool parts3 = !dbl && m->prec == GEMM_F32;
   for (auto* v : {&W.Wmain, &W.Wmu, &W.bias, &W.Wmain_hi, &W.Wmain_lo, &W.Wmu_hi, &W.Wmu_lo, &W.WmainT, &W.WmuT,
-                  &W.WmainS, &W.WmainL, &W.WmuL})
+                  &W.WmainS, &W.WmuS, &W.WmainL, &W.WmuL})
     v->resize(m->L);
   auto up = [&](DevBuf& b, const std::vector<float>& v) { return dbl ? upload_as<double>(b, v) : upload(b, v); };
   for (int l = 0; l < m->L; ++l) {
@@ -390,6 +390,7 @@ dw_status prepare_weights(dw_model* m, Weights& W, bool dbl) {
     if ((st = up(W.WmuT[l], wuT))) return st;
     if ((st = up(W.bias[l], b.data))) return st;
     if (parts3 && ((st = pack_split(W.WmainS[l], W.Wmain[l], W1, Kx)) ||
+                   (st = pack_split(W.WmuS[l], W.Wmu[l], W1, Km)) ||
                    (st = pack_lanes(W.WmainL[l], W.Wmain[l], W1, Kx)) ||
                    (st = pack_lanes(W.WmuL[l], W.Wmu[l], W1, Km))))
       return st;
@@ -602,9 +603,7 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
   const int Cp = rows_per_electron(C);
   Shape sh{(int)B, m->n, m->u, m->I, m->D, C, Cp, m->W1, m->W2, m->L};
   const long rows = B * m->n * Cp;
-  // below 32768 rows a pass is launches and latency, and the value channel's own launches cost more than the
-  // split saves (16,384 rows of 256 LiH walkers: 760 us a call against 741)
-  const bool split = !DBL && C > 1 && m->prec == GEMM_F32 && m->lap_form == DW_LAP_SPLIT && rows >= 32768;
+  const bool split = !DBL && C > 1 && m->prec == GEMM_F32 && m->lap_form == DW_LAP_SPLIT;
   Timed pass_timer(m, C > 1 ? DW_TIMER_LOCAL_ENERGY : DW_TIMER_FORWARD, s);
   T* const* X = ws.X;
   if (prop) {  // the pass runs on the Gaussian proposal, formed and stored by the features kernel
@@ -651,6 +650,40 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
           value_layer(X[l], m->Kx[l], m->Kx[l], m->Kh[l], W.WmainL[l].p, W.WmuL[l].p, m->Km[l], W.bias[l].as<float>(),
                       vs, outp, ldo, last ? 1 : 0, (int)B, m->n, m->u, m->W1, s))
         continue;
+    }
+    if constexpr (!DBL) {
+      if (split) {
+        // derivative channels of V, then the value channel (row 0 of each electron) with the value pass's
+        // arithmetic, then the derivative channels of the layer
+        split_mean(X[l], m->Kx[l], m->Kh[l], W.WmuS[l].p, m->Km[l], ws.V, m->W1, sh, s);
+        const int ldx = Cp * m->Kx[l], Km = m->Km[l];
+        if (!value_layer(X[l], ldx, m->Kx[l], m->Kh[l], W.WmainL[l].p, W.WmuL[l].p, Km, W.bias[l].as<float>(), 1, outp,
+                         (long)Cp * ldo, last ? 1 : 0, (int)B, m->n, m->u, m->W1, s)) {
+          Shape s1 = sh;
+          s1.C = 1;
+          s1.Cp = 1;
+          launch_spin_mean<float>(X[l], ldx, m->Kh[l], ws.MU, Km, s1, s);
+          GemmEpi ev;
+          ev.bias = W.bias[l].as<float>();
+          ev.nC = m->n;
+          gemm(GEMM_F32, ws.MU, Km, W.Wmu[l].as<float>(), nullptr, nullptr, Km, ws.V, Cp * m->W1, (int)B, m->W1, Km, ev,
+               s);  // over the value rows of V
+          GemmEpi em;
+          em.V = ws.V;
+          em.ldv = Cp * m->W1;
+          em.nC = em.n = m->n;
+          em.u = m->u;
+          em.B = (int)B;
+          em.act_tanh = 1;
+          em.permute = last ? 1 : 0;
+          gemm(GEMM_F32, X[l], ldx, W.Wmain[l].as<float>(), nullptr, nullptr, m->Kx[l], outp, Cp * ldo,
+               (int)(B * m->n), m->W1, m->Kx[l], em, s);
+        }
+        Timed t(m, l >= 1 ? DW_TIMER_GEMM_1EL_LAP : -1, s);
+        split_lap(X[l], m->Kx[l], W.WmainS[l].p, m->Kx[l], ws.V, m->W1, outp, ldo, last ? 1 : 0, sh,
+                  m->tune.lap_electrons, m->tune.lap_cols, s);
+        continue;
+      }
     }
     // Laplacian pass, FP32 form: spin means formed inside the per-walker GEMM (same values as below)
     bool fused_mu = false;
@@ -699,20 +732,6 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
         gemm_t(m, X[l], m->Kx[l], W.Wmain[l].as<T>(), W.Wmain_hi[l], W.Wmain_lo[l], m->Kx[l], ws.Z, m->W1,
                rows, m->W1, m->Kx[l], em, s);
         launch_tanh_rule<T>(ws.Z, outp, ldo, last ? 1 : 0, sh, s);
-      } else if (split) {
-        // value channel (row 0 of each electron) as in the value pass, then the derivative channels
-        GemmEpi e0 = em;
-        e0.C = 1;
-        e0.nC = m->n;
-        e0.ldv = Cp * m->W1;
-        e0.act_tanh = 1;
-        e0.permute = last ? 1 : 0;
-        if (!value_layer(X[l], (long)Cp * m->Kx[l], m->Kx[l], m->Kh[l], W.WmainL[l].p, W.WmuL[l].p, m->Km[l],
-                         W.bias[l].as<float>(), 1, outp, (long)Cp * ldo, last ? 1 : 0, (int)B, m->n, m->u, m->W1, s))
-          gemm(GEMM_F32, X[l], Cp * m->Kx[l], W.Wmain[l].as<float>(), nullptr, nullptr, m->Kx[l], outp, Cp * ldo,
-               (int)(B * m->n), m->W1, m->Kx[l], e0, s);
-        split_lap(X[l], m->Kx[l], W.WmainS[l].p, m->Kx[l], ws.V, m->W1, outp, ldo, last ? 1 : 0, sh,
-                  m->tune.lap_electrons, m->tune.lap_cols, s);
       } else {
         gemm_lap(m->prec, X[l], m->Kx[l], W.Wmain[l].as<float>(), W.Wmain_hi[l].as<uint16_t>(),
                  W.Wmain_lo[l].as<uint16_t>(), m->Kx[l], ws.V, m->W1, outp, ldo, last ? 1 : 0, sh,

@@ -87,6 +87,11 @@ struct SplitLds {
   uint4 a[2][3][RB][64];
 };
 
+// One product of row block i with the NQ column blocks (parts PA of a, PB of b).
+#define DW_SPLIT_MFMA(PA, PB) \
+  _Pragma("unroll") for (int q = 0; q < NQ; ++q) acc[i][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16( \
+      (v8bf)a[PA], (v8bf)b[q][PB], acc[i][q], 0, 0, 0);
+
 template <int RB, int NQ>
 __device__ __forceinline__ void split_main(const float* __restrict__ A, long row0, long rows, long lda, int slices,
                                            const uint4* __restrict__ P, int ncb, int cb0, SplitLds<RB>& lds,
@@ -145,16 +150,12 @@ __device__ __forceinline__ void split_main(const float* __restrict__ A, long row
       v8s a[3];
 #pragma unroll
       for (int p = 0; p < 3; ++p) a[p] = *(const v8s*)&lds.a[buf][p][i][lane];
-#define DW_SPLIT_MFMA(PA, PB)          \
-  _Pragma("unroll") for (int q = 0; q < NQ; ++q) acc[i][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16( \
-      (v8bf)a[PA], (v8bf)b[q][PB], acc[i][q], 0, 0, 0);
       DW_SPLIT_MFMA(2, 0)
       DW_SPLIT_MFMA(0, 2)
       DW_SPLIT_MFMA(1, 1)
       DW_SPLIT_MFMA(1, 0)
       DW_SPLIT_MFMA(0, 1)
       DW_SPLIT_MFMA(0, 0)
-#undef DW_SPLIT_MFMA
       if (i == RB / 2 && s + 1 < slices) {  // the next slice, loaded a slice ago
         sstore(buf ^ 1);
         if (s + 2 < slices) gload(s + 2);
@@ -349,6 +350,118 @@ bool split_lap(const float* X, int ldx, const void* P, int K, const float* V, in
     default: return false;
   }
 #undef DW_SPLIT_LAP
+}
+
+// ------------------------------------------------------------------------------------------------
+// Per-walker term of a 1-el layer for the derivative channels, spin means fused in:
+//   V[r, o] = sum_k MU[r, k] Wmu[o, k],  r = b Cp + ch,
+//   MU[r, k] = mean over the electrons of spin s(k) of X[(b n + i) Cp + ch, k - s Kh]   (electrons in order, FP32).
+// A workgroup forms the means of 48 rows x 128 k at a time and splits them straight into LDS (37 KB: four workgroups
+// per CU, whose load and MFMA phases overlap); the weights' parts come from L2.  Bound by the read of X's h columns
+(1.41 GB for 2048 walkers of 14 electrons: 364 us = 3.9 TB/s against 471 us with FP32 MFMA; 26 electrons, 1024
+walkers: 575 -> 461 us; 256 LiH walkers: 67 -> 28 us with 64 columns per workgroup).
+// ------------------------------------------------------------------------------------------------
+template <int NQ>
+__global__ __launch_bounds__(256) void k_split_mean(const float* __restrict__ X, int Kx, int Kh,
+                                                    const uint4* __restrict__ P, int ncb, int Km,
+                                                    float* __restrict__ V, int ldv, Shape sh, int tilesN, int total) {
+  constexpr int RB = 3, CS = 4;  // row blocks, 32-wide slices per chunk
+  __shared__ uint4 lds[CS][3][RB][64];
+  const int tile = tile_of(blockIdx.x, total);
+  if (tile >= total) return;  // uniform over the workgroup, before any barrier
+  const long rows = (long)sh.B * sh.Cp, r0 = (long)(tile / tilesN) * (16 * RB);
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int cb0 = (tile % tilesN) * (4 * NQ) + wv * NQ;
+  const int n = sh.n, u = sh.u, Cp = sh.Cp;
+  const long xstride = (long)Cp * Kx;  // one electron further
+  v4f acc[RB][NQ];
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) acc[i][q] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int kc = 0; kc < Km; kc += 32 * CS) {
+    const int ns = min(CS, (Km - kc) >> 5);
+    __syncthreads();  // the previous chunk's reads are done
+    // consecutive lanes take consecutive quads of a row (coalesced); 4 quads a slice-row group
+    for (int t = tid; t < 16 * RB * 8 * ns; t += 256) {
+      const int rr = t / (8 * ns), qd = t - rr * (8 * ns);
+      const long r = r0 + rr;
+      const int k = kc + 4 * qd;
+      v4f v = {0.f, 0.f, 0.f, 0.f};
+      if (r < rows && k < 2 * Kh) {
+        const long b = div_idx(r, Cp);
+        const int ch = (int)(r - b * Cp);
+        const int s = k >= Kh ? 1 : 0;
+        const int i0 = s ? u : 0, i1 = s ? n : u;
+        const float* xp = X + ((b * n + i0) * Cp + ch) * (long)Kx + (k - s * Kh);
+#pragma unroll 8
+        for (int i = i0; i < i1; ++i, xp += xstride) {
+          const v4f x = *(const v4f*)xp;
+          v[0] += x[0];
+          v[1] += x[1];
+          v[2] += x[2];
+          v[3] += x[3];
+        }
+        const float inv = 1.f / (float)(i1 - i0);
+        v[0] *= inv;
+        v[1] *= inv;
+        v[2] *= inv;
+        v[3] *= inv;
+      }
+      uint2 p[3];
+      split4(v, p);
+      const int quad = qd & 7;
+#pragma unroll
+      for (int m = 0; m < 3; ++m)
+        *((uint2*)&lds[qd >> 3][m][rr >> 4][(quad >> 1) * 16 + (rr & 15)] + (quad & 1)) = p[m];
+    }
+    __syncthreads();
+    for (int s = 0; s < ns; ++s) {
+      v8s b[NQ][3];
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+          b[q][m] = *(const v8s*)&P[((long)(((kc >> 5) + s) * ncb + cb0 + q) * 3 + m) * 64 + lane];
+#pragma unroll
+      for (int i = 0; i < RB; ++i) {
+        v8s a[3];
+#pragma unroll
+        for (int m = 0; m < 3; ++m) a[m] = *(const v8s*)&lds[s][m][i][lane];
+        DW_SPLIT_MFMA(2, 0)
+        DW_SPLIT_MFMA(0, 2)
+        DW_SPLIT_MFMA(1, 1)
+        DW_SPLIT_MFMA(1, 0)
+        DW_SPLIT_MFMA(0, 1)
+        DW_SPLIT_MFMA(0, 0)
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const long r = r0 + i * 16 + 4 * (lane >> 4) + j;
+        if (r < rows) V[r * ldv + (cb0 + q) * 16 + (lane & 15)] = acc[i][q][j];
+      }
+}
+
+void split_mean(const float* X, int Kx, int Kh, const void* P, int Km, float* V, int ldv, const Shape& sh,
+                hipStream_t s) {
+  const int ncb = dw_pad(sh.W1, 256) / 16;
+  const long tilesM = ((long)sh.B * sh.Cp + 47) / 48;
+  // 256 columns (X read once) where that gives two workgroups to every CU
+  if (sh.W1 % 256 == 0 && tilesM * (sh.W1 / 256) >= 512) {
+    const int tilesN = sh.W1 / 256, total = (int)(tilesM * tilesN);
+    hipLaunchKernelGGL((k_split_mean<4>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh, (const uint4*)P, ncb,
+                       Km, V, ldv, sh, tilesN, total);
+  } else {
+    const int tilesN = sh.W1 / 64, total = (int)(tilesM * tilesN);
+    hipLaunchKernelGGL((k_split_mean<1>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh, (const uint4*)P, ncb,
+                       Km, V, ldv, sh, tilesN, total);
+  }
 }
 
 }  // namespace dwmi

@@ -61,6 +61,9 @@ void launch_split_pack(const float* Bt, int ldb, int cols, int K, void* out, hip
 // C[M, N] = A[M, K] B.  tile: -1 chosen by size, 0 = 48 x 128, 1 or 2 = 96 x 256 (results do not depend on it).
 void split_gemm(const float* A, int lda, const void* P, float* C, int ldc, int M, int N, int K, int tile,
                 hipStream_t s);
+// V[(b Cp + ch), o] of the derivative channels: spin means of X's first Kh columns times W_mu (no bias).
+void split_mean(const float* X, int Kx, int Kh, const void* P, int Km, float* V, int ldv, const Shape& sh,
+                hipStream_t s);
 // 1-el GEMM and tanh forward-Laplacian rule of the derivative channels; `out` holds the value channel already.
 // E_max > 0 / cols = 128 ask for the smaller tiles (results do not depend on them).
 bool split_lap(const float* X, int ldx, const void* P, int K, const float* V, int ldv, float* out, int ldo,

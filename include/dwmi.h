@@ -262,7 +262,7 @@ dw_status dw_model_get_tuning(const dw_model* m, dw_tuning* out);
 
 /* Derivative channels (tangents, Laplacian) of dw_local_energy's GEMMs in the DW_FP32 form.  SPLIT (default): both
  * operands split exactly into three BF16 parts, six products on BF16 MFMA with FP32 sums; E_loc as accurate as
- * with FP32 and 1.2 to 1.3 times faster, equal to it to rounding (small batches take FP32 anyway).  FP32: FP32 MFMA.  The value channel
+ * with FP32 and 1.2 to 1.5 times faster, equal to it to rounding.  FP32: FP32 MFMA.  The value channel
  * (log|psi|^2, the determinants) is the same bits in both.  For callers whose FP64 statistics of the energies
  * (the optimisation's loss and clipping state) have to stay bit-equal from run to run, across releases: the
  * loss uses FP32. */

@@ -1,5 +1,5 @@
 """The split-operand GEMMs of the Laplacian pass (three BF16 parts per FP32 operand, gemm_split.hip): every
-tile height (1 to 12 row blocks of 16 channels per electron), ragged last tiles, both tile choices.  Sizes just over the 32768 rows from which the split form is taken."""
+tile height (1 to 12 row blocks of 16 channels per electron), ragged last tiles, both tile choices."""
 from __future__ import annotations
 
 import numpy as np
