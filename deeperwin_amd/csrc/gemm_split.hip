@@ -358,8 +358,8 @@ bool split_lap(const float* X, int ldx, const void* P, int K, const float* V, in
 //   MU[r, k] = mean over the electrons of spin s(k) of X[(b n + i) Cp + ch, k - s Kh]   (electrons in order, FP32).
 // A workgroup forms the means of 48 rows x 128 k at a time and splits them straight into LDS (37 KB: four workgroups
 // per CU, whose load and MFMA phases overlap); the weights' parts come from L2.  Bound by the read of X's h columns
-(1.41 GB for 2048 walkers of 14 electrons: 364 us = 3.9 TB/s against 471 us with FP32 MFMA; 26 electrons, 1024
-walkers: 575 -> 461 us; 256 LiH walkers: 67 -> 28 us with 64 columns per workgroup).
+// (1.41 GB for 2048 walkers of 14 electrons: 364 us = 3.9 TB/s against 471 us with FP32 MFMA; 26 electrons, 1024
+// walkers: 575 -> 461 us; 256 LiH walkers: 67 -> 28 us with 64 columns per workgroup).
 // ------------------------------------------------------------------------------------------------
 template <int NQ>
 __global__ __launch_bounds__(256) void k_split_mean(const float* __restrict__ X, int Kx, int Kh,
