@@ -114,7 +114,11 @@ struct Weights {
   DevBuf W2e, b2e, Wo[2], Wo_hi[2], Wo_lo[2], WoT[2], kappa, wenv;
   // FP32 form: the three BF16 parts of Wmain / Wmu / Wo in MFMA lane order (derivative channels, gemm_split.hip)
   std::vector<DevBuf> WmainS, WmuS;
-  DevBuf WoS[2];
+  // and the two FP16 parts of 2^shift Wmain (layers >= 1) / Wo; shift kNoHalf: magnitudes outside FP16's reach
+  std::vector<DevBuf> WmainH;
+  std::vector<int> shiftH;
+  DevBuf WoH[2];
+  int shiftO[2] = {0, 0};
   // FP32 form: Wmain / Wmu / Wo in MFMA lane order (one-launch value layers, value_layer.hip)
   std::vector<DevBuf> WmainL, WmuL;
   DevBuf WoL[2];
@@ -123,10 +127,10 @@ struct Weights {
   std::vector<DevBuf> WhmT, WhmT_hi, WhmT_lo, bhm, WhmB;  // WhmB: h_map w [pad128(Kh)][32] (gradient pass)
   void release() {
     for (auto* v : {&Wmain, &Wmu, &bias, &Wmain_hi, &Wmain_lo, &Wmu_hi, &Wmu_lo, &WmainT, &WmuT, &WhmT, &WhmT_hi,
-                    &WhmT_lo, &bhm, &WhmB, &WmainS, &WmuS, &WmainL, &WmuL})
+                    &WhmT_lo, &bhm, &WhmB, &WmainS, &WmuS, &WmainH, &WmainL, &WmuL})
       for (auto& b : *v) b.release();
     for (DevBuf* b : {&W2e, &b2e, &Wo[0], &Wo[1], &Wo_hi[0], &Wo_hi[1], &Wo_lo[0], &Wo_lo[1], &WoT[0], &WoT[1], &kappa,
-                      &wenv, &Wp, &bp, &Wei, &bei, &Whim, &bhim, &table, &WoS[0], &WoS[1], &WoL[0],
+                      &wenv, &Wp, &bp, &Wei, &bei, &Whim, &bhim, &table, &WoH[0], &WoH[1], &WoL[0],
                       &WoL[1]})
       b->release();
     ready = false;
@@ -140,6 +144,7 @@ template <typename T>
 struct PassBufs {
   T* X[4] = {nullptr, nullptr, nullptr, nullptr};
   T *MU = nullptr, *V = nullptr, *Z = nullptr, *H = nullptr, *O = nullptr, *A = nullptr;
+  float* amax[2] = {nullptr, nullptr};  // per-electron maxima of a layer's derivative channels (split form)
   T *WM = nullptr, *HM = nullptr, *HIM = nullptr;  // dpe4: mapped pairs, h_map rows, ion maps
   double *ld = nullptr, *sd = nullptr, *g = nullptr, *lap = nullptr, *minv = nullptr;
   float* dcond = nullptr;
@@ -344,6 +349,24 @@ dw_status pack_split(DevBuf& out, const DevBuf& Bt, int cols, int K) {
   return DW_OK;
 }
 
+constexpr int kNoHalf = INT32_MIN;
+
+// Power of two that brings weights of this layout under 2^15 (gemm_split.hip bounds it), or kNoHalf.
+int half_shift(const std::vector<float>& w) {
+  float m = 0.f;
+  for (float x : w) m = std::fabs(x) > m || std::isnan(x) ? std::fabs(x) : m;
+  if (!(m < 1.7e10f)) return kNoHalf;  // 2^34 and above, NaN
+  return m > 0.f ? std::min(40, 14 - std::ilogb(m)) : 0;
+}
+
+dw_status pack_half(DevBuf& out, int shift, const DevBuf& Bt, int cols, int K) {
+  if (shift == kNoHalf) return DW_OK;
+  HIP_TRY(out.ensure(split_pack16_bytes(cols, K)));
+  launch_split_pack16(Bt.as<float>(), K, cols, K, shift, out.p, nullptr);
+  HIP_TRY(hipGetLastError());
+  return DW_OK;
+}
+
 dw_status pack_lanes(DevBuf& out, const DevBuf& Bt, int cols, int K) {
   HIP_TRY(out.ensure(lane_pack_bytes(cols, K)));
   launch_lane_pack(Bt.as<float>(), K, cols, K, out.p, nullptr);
@@ -359,8 +382,9 @@ dw_status prepare_weights(dw_model* m, Weights& W, bool dbl) {
   const bool split = !dbl && m->prec != GEMM_F32;
   const bool parts3 = !dbl && m->prec == GEMM_F32;
   for (auto* v : {&W.Wmain, &W.Wmu, &W.bias, &W.Wmain_hi, &W.Wmain_lo, &W.Wmu_hi, &W.Wmu_lo, &W.WmainT, &W.WmuT,
-                  &W.WmainS, &W.WmuS, &W.WmainL, &W.WmuL})
+                  &W.WmainS, &W.WmuS, &W.WmainH, &W.WmainL, &W.WmuL})
     v->resize(m->L);
+  W.shiftH.assign(m->L, kNoHalf);
   auto up = [&](DevBuf& b, const std::vector<float>& v) { return dbl ? upload_as<double>(b, v) : upload(b, v); };
   for (int l = 0; l < m->L; ++l) {
     char buf[64];
@@ -389,7 +413,9 @@ dw_status prepare_weights(dw_model* m, Weights& W, bool dbl) {
     if ((st = up(W.WmainT[l], wmT))) return st;
     if ((st = up(W.WmuT[l], wuT))) return st;
     if ((st = up(W.bias[l], b.data))) return st;
+    if (parts3) W.shiftH[l] = l > 0 && Kx % 64 == 0 && Kx - Kt0 <= 64 ? half_shift(wm) : kNoHalf;
     if (parts3 && ((st = pack_split(W.WmainS[l], W.Wmain[l], W1, Kx)) ||
+                   (st = pack_half(W.WmainH[l], W.shiftH[l], W.Wmain[l], W1, Kx)) ||
                    (st = pack_split(W.WmuS[l], W.Wmu[l], W1, Km)) ||
                    (st = pack_lanes(W.WmainL[l], W.Wmain[l], W1, Kx)) ||
                    (st = pack_lanes(W.WmuL[l], W.Wmu[l], W1, Km))))
@@ -434,7 +460,9 @@ dw_status prepare_weights(dw_model* m, Weights& W, bool dbl) {
     dw_status st;
     if ((st = up(W.Wo[s], wo))) return st;
     if ((st = up(W.WoT[s], woT))) return st;
-    if (parts3 && ((st = pack_split(W.WoS[s], W.Wo[s], m->NOp, W1)) || (st = pack_lanes(W.WoL[s], W.Wo[s], m->NOp, W1))))
+    if (parts3) W.shiftO[s] = half_shift(wo);
+    if (parts3 && ((st = pack_half(W.WoH[s], W.shiftO[s], W.Wo[s], m->NOp, W1)) ||
+                   (st = pack_lanes(W.WoL[s], W.Wo[s], m->NOp, W1))))
       return st;
     if (split && (st = upload_split(W.Wo_hi[s], W.Wo_lo[s], wo))) return st;
     const Leaf& a = m->leaves[leaf_key("envelope_orbitals", ak[s])];
@@ -503,6 +531,8 @@ size_t layout_pass(const dw_model* m, long B, int C, char* base, PassBufs<T>* ou
   b.MU = cv.take<T>((size_t)B * Cp * kmmax);
   b.V = cv.take<T>((size_t)B * Cp * m->W1 * (C == 1 ? 4 : 1));  // value pass: up to 4 K-split parts
   if (sizeof(T) == 8 && C > 1) b.Z = cv.take<T>((size_t)rows * m->W1);  // unfused pre-activations (FP64 form)
+  if (sizeof(T) == 4 && C > 1)
+    for (auto& a : b.amax) a = cv.take<float>((size_t)B * m->n * (m->W1 / 32));
   b.H = cv.take<T>((size_t)rows * m->W1);
   b.O = cv.take<T>((size_t)rows * m->NO);
   if (!det_reads_orbitals(m->n, C)) b.A = cv.take<T>((size_t)B * m->D * C * m->n * m->n);  // envelope x orbitals
@@ -621,6 +651,7 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
   }
   const long vstride = B * Cp * (long)m->W1;
   const long wm_layer = B * (long)m->n * m->n * (C > 1 ? 5 : 1) * 32;
+  int amax_np = 0;  // maxima per electron of the last split layer, in ws.amax[l & 1]
   for (int l = 0; l < m->L; ++l) {
     if (m->dpe4) {  // e_ee of this iteration: hm = tanh rule of (X_l[:, h] W_map), then the convolution
       GemmEpiT<T> eh;
@@ -680,8 +711,10 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
                (int)(B * m->n), m->W1, m->Kx[l], em, s);
         }
         Timed t(m, l >= 1 ? DW_TIMER_GEMM_1EL_LAP : -1, s);
-        split_lap(X[l], m->Kx[l], W.WmainS[l].p, m->Kx[l], ws.V, m->W1, outp, ldo, last ? 1 : 0, sh,
-                  m->tune.lap_electrons, m->tune.lap_cols, s);
+        const bool half = W.shiftH[l] != kNoHalf;
+        amax_np = split_lap(X[l], m->Kx[l], half ? W.WmainH[l].p : W.WmainS[l].p, W.shiftH[l], m->Kx[l],
+                            half ? ws.amax[(l + 1) & 1] : nullptr, amax_np, (m->Kx[l] - m->Kt0[l]) / 32, ws.V, m->W1, outp,
+                            ldo, ws.amax[l & 1], last ? 1 : 0, sh, m->tune.lap_electrons, m->tune.lap_cols, s);
         continue;
       }
     }
@@ -752,9 +785,11 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
   for (int sp = 0; sp < 2 && !orb_done; ++sp) {
     const long rows0 = sp ? up_rows : 0, nr = sp ? dn_rows : up_rows;
     if constexpr (!DBL) {
-      if (split) {  // every channel from the split form; the value rows follow in FP32
-        split_gemm(ws.H + rows0 * m->W1, m->W1, W.WoS[sp].p, ws.O + rows0 * m->NO, m->NO, (int)nr, m->NO, m->W1,
-                   m->tune.lap_orb_tile, s);
+      if (split && W.shiftO[sp] != kNoHalf) {  // every channel from the split form; the value rows follow in FP32
+        const int ms = m->W1 / 32;
+        split_gemm(ws.H + rows0 * m->W1, m->W1, W.WoH[sp].p, W.shiftO[sp],
+                   ws.amax[(m->L - 1) & 1] + (sp ? B * m->u * ms : 0), amax_np, ms, Cp / 16, ws.O + rows0 * m->NO, m->NO,
+                   (int)nr, m->NO, m->W1, m->tune.lap_orb_tile, s);
         continue;
       }
     }

@@ -1,18 +1,27 @@
-// FP32 GEMMs of the Laplacian pass's derivative channels on BF16 MFMA.
+// FP32 GEMMs of the Laplacian pass's derivative channels on 16-bit MFMA with FP32 sums.
 //
-// Every FP32 operand is the exact sum of three BF16 numbers (x = h + m + l: h = bf16(x), m = bf16(x - h),
-// l = x - h - m; 8 + 8 + 8 significant bits), so a product a b is the sum of nine BF16 products.  The three
-// below 2^-26 |a b| (m l, l m, l l) are left out, the other six accumulate in FP32, smallest first:
-//   l h + h l + m m + m h + h m + h h.
-// What is left out is under the rounding of one FP32 multiply-add, and a 32-wide K slice rounds the
-// accumulator six times where the FP32 MFMA (16x16x4) rounds it at least eight times.
-// v_mfma_f32_16x16x32_bf16 runs at 16 times the FP32 rate, so six products cost 6 / 16 of the FP32 form.
+// Two forms.  BF16 parts: an FP32 operand is the exact sum of three BF16 numbers (x = h + m + l: h = bf16(x),
+// m = bf16(x - h), l = x - h - m; 8 + 8 + 8 significant bits), so a product is the sum of nine BF16 products; the three
+// below 2^-26 |a b| (m l, l m, l l) are left out.  FP16 parts: x = h + m with 11 + 11 bits and a rest below 2^-23 |x|,
+// three products (m m, below 2^-24 |a b|, left out); it needs operands near the top of FP16's range, so a row block (one
+// electron's channels) and the weights are scaled by powers of two, and an element keeps those bits down to 2^-17 of its
+// block's largest (below that its absolute error is 2^-40 of the largest).  In both a 32-wide K slice rounds the
+// accumulator six or three times, where the FP32 MFMA (16x16x4) rounds it at least eight times; over 320 products of
+// random operands that leaves 1.3e-7 (BF16) and 1.2e-7 (FP16) of the norm against 1.6e-7 for FP32.
+// The 16-bit MFMA runs at 16 times the FP32 rate: 6 / 16 and 3 / 16 of the FP32 form's time.
+//
+// FP16 parts are taken where the largest magnitudes are known: the layer's kernel leaves the maxima of what it writes,
+// and the columns of other kernels (pair features, the last slices) are looked at while they wait in registers.
+// Layer 0 (K of a few features) and the mean product, bound by memory, use BF16 parts.
+//
 // Measured against 64 bits (E_loc of 256 to 2048 walkers, 4 to 42 electrons, both models): the same relative
 // error as the FP32 form to two digits (4e-6 to 6e-5, set by the value channel), 2e-7 to 6e-7 between the two.
 //
 // Only derivative channels (tangents, Laplacian) come from here.  The value channel of the pass (the first row
 // of an electron) keeps the FP32 MFMA of the value pass: log|psi|, the orbital matrices and their inverses
 // amplify its rounding by the walker's conditioning, the derivative channels enter E_loc linearly.
+#include <type_traits>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -38,6 +47,17 @@ __device__ __forceinline__ void split4(v4f x, uint2 (&p)[3]) {
   p[0] = uint2{h0, h1};
   p[1] = uint2{m0, m1};
   p[2] = uint2{pack_bf16(r0 - lo_f(m0), r1 - hi_f(m0)), pack_bf16(r2 - lo_f(m1), r3 - hi_f(m1))};
+}
+
+// Four floats -> two FP16 parts of each (x = h + m + rest, |rest| below 2^-23 of |x| for |x| >= 2^-2).
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void split4h(v4f x, uint2 (&p)[2]) {
+  const v2h h0 = __builtin_convertvector(v2f{x[0], x[1]}, v2h), h1 = __builtin_convertvector(v2f{x[2], x[3]}, v2h);
+  const v2h m0 = __builtin_convertvector(v2f{x[0] - (float)h0[0], x[1] - (float)h0[1]}, v2h);
+  const v2h m1 = __builtin_convertvector(v2f{x[2] - (float)h1[0], x[3] - (float)h1[1]}, v2h);
+  p[0] = uint2{__builtin_bit_cast(unsigned, h0), __builtin_bit_cast(unsigned, h1)};
+  p[1] = uint2{__builtin_bit_cast(unsigned, m0), __builtin_bit_cast(unsigned, m1)};
 }
 
 // Weights Bt [rows, ldb] (row = output column, K contiguous) in the order the MFMA lanes read them:
@@ -70,6 +90,46 @@ void launch_split_pack(const float* Bt, int ldb, int cols, int K, void* out, hip
                      (uint4*)out);
 }
 
+// The same order with two FP16 parts of 2^shift W: P16[((slice * ncb + cb) * 2 + part) * 64 + lane].
+__global__ __launch_bounds__(256) void k_split_pack16(const float* __restrict__ Bt, int ldb, int cols, int ncb,
+                                                      int slices, float scale, uint4* __restrict__ P) {
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (t >= slices * ncb * 64) return;
+  const int lane = t & 63, cb = (t >> 6) % ncb, sl = (t >> 6) / ncb;
+  const int col = cb * 16 + (lane & 15), k = sl * 32 + (lane >> 4) * 8;
+  v4f a = {0.f, 0.f, 0.f, 0.f}, b = a;
+  if (col < cols) {
+    a = *(const v4f*)(Bt + (long)col * ldb + k);
+    b = *(const v4f*)(Bt + (long)col * ldb + k + 4);
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    a[j] *= scale;
+    b[j] *= scale;
+  }
+  uint2 pa[2], pb[2];
+  split4h(a, pa);
+  split4h(b, pb);
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+    P[((long)(sl * ncb + cb) * 2 + p) * 64 + lane] = uint4{pa[p].x, pa[p].y, pb[p].x, pb[p].y};
+}
+
+size_t split_pack16_bytes(int cols, int K) { return (size_t)(K / 32) * (dw_pad(cols, 256) / 16) * 2 * 64 * 16; }
+
+void launch_split_pack16(const float* Bt, int ldb, int cols, int K, int shift, void* out, hipStream_t s) {
+  const int ncb = dw_pad(cols, 256) / 16, slices = K / 32;
+  hipLaunchKernelGGL(k_split_pack16, dim3((slices * ncb * 64 + 255) / 256), dim3(256), 0, s, Bt, ldb, cols, ncb, slices,
+                     ldexpf(1.f, shift), (uint4*)out);
+}
+
+// Power of two that brings a block of largest magnitude `m` under 2^15.  Bounded so that the units of the accumulators
+// (this plus the weights' shift of -20 .. 40) and their inverse stay in range.
+__device__ __forceinline__ int split_shift(float m) {
+  const int e = (int)((__float_as_uint(m) >> 23) & 255u) - 127;
+  return min(40, max(-100, 14 - e));
+}
+
 __device__ __forceinline__ int tile_of(int bid, int total) {
   // workgroups are dealt round-robin to 8 XCDs; each XCD gets a contiguous range of tiles
   const int per = (total + 7) / 8;
@@ -82,69 +142,80 @@ __device__ __forceinline__ int tile_of(int bid, int total) {
 // one barrier per slice), in lane order (part, row block, lane), so every LDS access is 16 consecutive bytes
 // per lane; a wave's B parts come from L2 straight into registers, one slice ahead.
 // ------------------------------------------------------------------------------------------------
-template <int RB>
-struct SplitLds {
-  uint4 a[2][3][RB][64];
-};
-
 // One product of row block i with the NQ column blocks (parts PA of a, PB of b).
 #define DW_SPLIT_MFMA(PA, PB) \
   _Pragma("unroll") for (int q = 0; q < NQ; ++q) acc[i][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16( \
       (v8bf)a[PA], (v8bf)b[q][PB], acc[i][q], 0, 0, 0);
+#define DW_SPLIT_MFMA16(PA, PB) \
+  _Pragma("unroll") for (int q = 0; q < NQ; ++q) acc[i][q] = __builtin_amdgcn_mfma_f32_16x16x32_f16( \
+      __builtin_bit_cast(v8h, a[PA]), __builtin_bit_cast(v8h, b[q][PB]), acc[i][q], 0, 0, 0);
 
-template <int RB, int NQ>
-__device__ __forceinline__ void split_main(const float* __restrict__ A, long row0, long rows, long lda, int slices,
-                                           const uint4* __restrict__ P, int ncb, int cb0, SplitLds<RB>& lds,
-                                           v4f (&acc)[RB][NQ]) {
-  constexpr int AU = RB * 128;  // (row, quad of 4 k) units of a slice
-  constexpr int AIT = (AU + 255) / 256;
-  const int tid = threadIdx.x, lane = tid & 63;
+template <int RB, int PARTS>
+struct SplitLds {
+  uint4 a[2][PARTS][RB][64];
+};
 
-  // unit u: row u / 128 * 16 + u % 16, quad (u / 16) % 8
-  v4f ra[AIT];
+// Weights of a split GEMM in lane order: three BF16 parts of W, or two FP16 parts of 2^shift W.
+struct SplitB {
+  const uint4* P;
+  int ncb, slices, shift;
+};
+
+// Unit u of a slice: row u / 128 * 16 + u % 16 (row block u / 128), quad of 4 k (u / 16) % 8.
+template <int RB>
+struct SplitUnits {
+  static constexpr int AU = RB * 128, AIT = (AU + 255) / 256;
   const float* ap[AIT];
-#pragma unroll
-  for (int it = 0; it < AIT; ++it) {
-    const int u = tid + 256 * it;
-    long gr = row0 + (u >> 7) * 16 + (u & 15);
-    if (gr > rows - 1) gr = rows - 1;
-    ap[it] = A + gr * lda + ((u >> 4) & 7) * 4;
-  }
-  auto gload = [&](int s) {
-#pragma unroll
-    for (int it = 0; it < AIT; ++it)
-      if (AU % 256 == 0 || tid + 256 * it < AU) ra[it] = *(const v4f*)(ap[it] + s * 32);
-  };
-  auto sstore = [&](int buf) {
+  __device__ __forceinline__ SplitUnits(const float* A, long row0, long rows, long lda) {
 #pragma unroll
     for (int it = 0; it < AIT; ++it) {
-      const int u = tid + 256 * it;
-      if (AU % 256 == 0 || u < AU) {
+      const int u = threadIdx.x + 256 * it;
+      long gr = row0 + (u >> 7) * 16 + (u & 15);
+      if (gr > rows - 1) gr = rows - 1;
+      ap[it] = A + gr * lda + ((u >> 4) & 7) * 4;
+    }
+  }
+  __device__ __forceinline__ bool in(int it) const { return AU % 256 == 0 || (int)threadIdx.x + 256 * it < AU; }
+  __device__ __forceinline__ void load(int s, v4f (&ra)[AIT]) const {
+#pragma unroll
+    for (int it = 0; it < AIT; ++it)
+      if (in(it)) ra[it] = *(const v4f*)(ap[it] + s * 32);
+  }
+  static __device__ __forceinline__ int block(int it) { return ((int)threadIdx.x + 256 * it) >> 7; }
+};
+
+template <int NQ, int PARTS>
+__device__ __forceinline__ void split_bload(const SplitB& W, int s, int cb0, v8s (&d)[NQ][PARTS]) {
+#pragma unroll
+  for (int q = 0; q < NQ; ++q)
+#pragma unroll
+    for (int p = 0; p < PARTS; ++p)
+      d[q][p] = *(const v8s*)&W.P[((long)(s * W.ncb + cb0 + q) * PARTS + p) * 64 + (threadIdx.x & 63)];
+}
+
+// BF16 parts: any K.
+template <int RB, int NQ>
+__device__ __forceinline__ void split_main(const SplitUnits<RB>& U, const SplitB& W, int cb0, SplitLds<RB, 3>& lds,
+                                           v4f (&acc)[RB][NQ]) {
+  constexpr int AIT = SplitUnits<RB>::AIT;
+  const int tid = threadIdx.x, lane = tid & 63, slices = W.slices;
+  v4f ra[AIT];
+  auto sstore = [&](int buf) {
+#pragma unroll
+    for (int it = 0; it < AIT; ++it)
+      if (U.in(it)) {
+        const int u = tid + 256 * it, quad = (u >> 4) & 7;
         uint2 p[3];
         split4(ra[it], p);
-        const int quad = (u >> 4) & 7;
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-          *((uint2*)&lds.a[buf][k][u >> 7][(quad >> 1) * 16 + (u & 15)] + (quad & 1)) = p[k];
+        for (int k = 0; k < 3; ++k) *((uint2*)&lds.a[buf][k][u >> 7][(quad >> 1) * 16 + (u & 15)] + (quad & 1)) = p[k];
       }
-    }
   };
   v8s b[NQ][3], bn[NQ][3];
-  auto bload = [&](int s, v8s (&d)[NQ][3]) {
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-#pragma unroll
-      for (int p = 0; p < 3; ++p) d[q][p] = *(const v8s*)&P[((long)(s * ncb + cb0 + q) * 3 + p) * 64 + lane];
-  };
-
-  gload(0);
-  bload(0, b);
-  sstore(0);
-  if (slices > 1) gload(1);
-  for (int s = 0; s < slices; ++s) {
+  auto slice = [&](int s, v8s (&b)[NQ][3], v8s (&bn)[NQ][3]) {
     const int buf = s & 1;
     __syncthreads();  // slice s is in lds.a[buf]; every read of lds.a[buf ^ 1] (slice s - 1) is done
-    if (s + 1 < slices) bload(s + 1, bn);
+    if (s + 1 < slices) split_bload<NQ, 3>(W, s + 1, cb0, bn);
 #pragma unroll
     for (int i = 0; i < RB; ++i) {
       v8s a[3];
@@ -158,38 +229,154 @@ __device__ __forceinline__ void split_main(const float* __restrict__ A, long row
       DW_SPLIT_MFMA(0, 0)
       if (i == RB / 2 && s + 1 < slices) {  // the next slice, loaded a slice ago
         sstore(buf ^ 1);
-        if (s + 2 < slices) gload(s + 2);
+        if (s + 2 < slices) U.load(s + 2, ra);
       }
     }
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-#pragma unroll
-      for (int p = 0; p < 3; ++p) b[q][p] = bn[q][p];
+  };
+  U.load(0, ra);
+  split_bload<NQ, 3>(W, 0, cb0, b);
+  sstore(0);
+  if (slices > 1) U.load(1, ra);
+  int s = 0;
+  for (; s + 1 < slices; s += 2) {
+    slice(s, b, bn);
+    slice(s + 1, bn, b);
   }
+  if (s < slices) slice(s, b, bn);
+}
+
+// FP16 parts of rows scaled by sc[] (a power of two per row block): an even number of slices, taken in the order
+// slices - tail, .., slices - 1, 0, 1, ..; the first two are already in ra0 and ra1.  Rows are loaded two slices ahead.
+template <int RB, int NQ>
+__device__ __forceinline__ void split_main16(const SplitUnits<RB>& U, const SplitB& W, int tail,
+                                             v4f (&ra0)[SplitUnits<RB>::AIT], v4f (&ra1)[SplitUnits<RB>::AIT],
+                                             const float (&sc)[SplitUnits<RB>::AIT], int cb0, SplitLds<RB, 2>& lds,
+                                             v4f (&acc)[RB][NQ]) {
+  constexpr int AIT = SplitUnits<RB>::AIT;
+  const int tid = threadIdx.x, lane = tid & 63, slices = W.slices;
+  auto at = [&](int t) { return t < tail ? slices - tail + t : t - tail; };
+  auto sstore = [&](int buf, v4f (&ra)[AIT]) {
+#pragma unroll
+    for (int it = 0; it < AIT; ++it)
+      if (U.in(it)) {
+        const int u = tid + 256 * it, quad = (u >> 4) & 7;
+        v4f x = ra[it];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] *= sc[it];
+        uint2 p[2];
+        split4h(x, p);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) *((uint2*)&lds.a[buf][k][u >> 7][(quad >> 1) * 16 + (u & 15)] + (quad & 1)) = p[k];
+      }
+  };
+  v8s b[NQ][2], bn[NQ][2];
+  auto slice = [&](int t, v8s (&b)[NQ][2], v8s (&bn)[NQ][2], v4f (&ra)[AIT]) {
+    const int buf = t & 1;
+    __syncthreads();  // slice t is in lds.a[buf]; every read of lds.a[buf ^ 1] (slice t - 1) is done
+    if (t + 1 < slices) split_bload<NQ, 2>(W, at(t + 1), cb0, bn);
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+      v8s a[2];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) a[p] = *(const v8s*)&lds.a[buf][p][i][lane];
+      DW_SPLIT_MFMA16(1, 0)
+      DW_SPLIT_MFMA16(0, 1)
+      DW_SPLIT_MFMA16(0, 0)
+      if (i == RB / 2 && t + 1 < slices) {  // slice t + 1, loaded two slices ago
+        sstore(buf ^ 1, ra);
+        if (t + 3 < slices) U.load(at(t + 3), ra);
+      }
+    }
+  };
+  split_bload<NQ, 2>(W, at(0), cb0, b);
+  sstore(0, ra0);
+  if (slices > 2) U.load(at(2), ra0);
+  for (int t = 0; t < slices; t += 2) {
+    slice(t, b, bn, ra1);
+    slice(t + 1, bn, b, ra0);
+  }
+}
+
+// Scales of a tile's row blocks (16 rows of one electron each, rbe blocks an electron): from the per-wave maxima that
+// the producer of A left (np per electron, ms apart) and, for the `tail` slices it did not write, from the rows
+// themselves (the first slices read; C channels an electron).  sM: RB words; eA gets the shifts; returns with sc[] set and the LDS words
+// readable by all.
+template <int RB>
+__device__ __forceinline__ void tile_scales(const SplitUnits<RB>& U, const float* __restrict__ amax, int np, int ms, int tail,
+                                            const v4f (&ra0)[SplitUnits<RB>::AIT],
+                                            const v4f (&ra1)[SplitUnits<RB>::AIT], long block0, long blocks, int rbe, int C,
+                                            unsigned* sM, int* eA, float (&sc)[SplitUnits<RB>::AIT]) {
+  constexpr int AIT = SplitUnits<RB>::AIT;
+  const int tid = threadIdx.x;
+  if (tid < RB) {
+    const long el = min(block0 + tid, blocks - 1) / rbe;
+    float m = 0.f;
+    for (int p = 0; p < np; ++p) m = fmaxf(m, amax[el * ms + p]);
+    sM[tid] = __float_as_uint(m);
+  }
+  __syncthreads();
+  if (tail > 0) {  // uniform
+#pragma unroll
+    for (int it = 0; it < AIT; ++it) {
+      float m = 0.f;
+      const int ch = (int)((block0 + U.block(it)) % rbe) * 16 + (tid & 15);
+      if (U.in(it) && ch > 0 && ch < C) {  // derivative channels only: the rows of padding channels hold anything
+#pragma unroll
+        for (int j = 0; j < 4; ++j) m = fmaxf(m, fabsf(ra0[it][j]));
+        if (tail > 1) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) m = fmaxf(m, fabsf(ra1[it][j]));
+        }
+      }
+      // a wave's 64 units of one step lie in one row block; blocks of an electron share the scale
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+      if ((tid & 63) == 0 && U.in(it)) {
+        const int e0 = (int)((block0 + U.block(it)) / rbe * rbe - block0);
+        for (int k = max(e0, 0); k < min(e0 + rbe, RB); ++k) atomicMax(&sM[k], __float_as_uint(m));
+      }
+    }
+    __syncthreads();
+  }
+  if (tid < RB) eA[tid] = split_shift(__uint_as_float(sM[tid]));
+#pragma unroll
+  for (int it = 0; it < AIT; ++it)
+    sc[it] = ldexpf(1.f, split_shift(__uint_as_float(sM[min(U.block(it), RB - 1)])));
 }
 
 // ------------------------------------------------------------------------------------------------
 // C[M, N] = A[M, K] B (no epilogue): the orbital GEMMs of the Laplacian pass.  688,128 x 256 x 224: 783 us with
-// FP32 MFMA on 128-row tiles, 480 us here.
+// FP32 MFMA on 128-row tiles, 480 us with BF16 parts, 349 us here.
 // ------------------------------------------------------------------------------------------------
 template <int RB, int NQ>
-__global__ __launch_bounds__(256, 2) void k_split_gemm(const float* __restrict__ A, int lda,
-                                                       const uint4* __restrict__ P, int ncb, float* __restrict__ Cm,
-                                                       int ldc, int M, int N, int slices, int tilesN, int tilesTotal) {
-  __shared__ SplitLds<RB> lds;
+__global__ __launch_bounds__(256, 2) void k_split_gemm(const float* __restrict__ A, int lda, SplitB W,
+                                                       const float* __restrict__ amax, int np, int ms, int rbe,
+                                                       float* __restrict__ Cm, int ldc, int M, int N, int tilesN,
+                                                       int tilesTotal) {
+  constexpr int AIT = SplitUnits<RB>::AIT;
+  __shared__ SplitLds<RB, 2> lds;
+  __shared__ unsigned sM[RB];
+  __shared__ int eA[RB];
   const int tile = tile_of(blockIdx.x, tilesTotal);
   if (tile >= tilesTotal) return;  // uniform over the workgroup, before any barrier
   const long row0 = (long)(tile / tilesN) * (16 * RB);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int cb0 = (tile % tilesN) * (4 * NQ) + wv * NQ;
+  const SplitUnits<RB> U(A, row0, M, lda);
+  v4f ra0[AIT], ra1[AIT];
+  float sc[AIT];
+  U.load(0, ra0);
+  U.load(1, ra1);
+  tile_scales<RB>(U, amax, np, ms, 0, ra0, ra1, row0 >> 4, M >> 4, rbe, 0, sM, eA, sc);
   v4f acc[RB][NQ];
 #pragma unroll
   for (int i = 0; i < RB; ++i)
 #pragma unroll
     for (int q = 0; q < NQ; ++q) acc[i][q] = v4f{0.f, 0.f, 0.f, 0.f};
-  split_main<RB, NQ>(A, row0, M, lda, slices, P, ncb, cb0, lds, acc);
+  split_main16<RB, NQ>(U, W, 0, ra0, ra1, sc, cb0, lds, acc);
 #pragma unroll
-  for (int i = 0; i < RB; ++i)
+  for (int i = 0; i < RB; ++i) {
+    const float inv = ldexpf(1.f, -(eA[i] + W.shift));
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       const int c = (cb0 + q) * 16 + (lane & 15);
@@ -197,25 +384,26 @@ __global__ __launch_bounds__(256, 2) void k_split_gemm(const float* __restrict__
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const long r = row0 + i * 16 + 4 * (lane >> 4) + j;
-          if (r < M) Cm[r * ldc + c] = acc[i][q][j];
+          if (r < M) Cm[r * ldc + c] = acc[i][q][j] * inv;
         }
       }
     }
+  }
 }
 
-void split_gemm(const float* A, int lda, const void* P, float* C, int ldc, int M, int N, int K, int tile,
-                hipStream_t s) {
+void split_gemm(const float* A, int lda, const void* P16, int shift, const float* amax, int np, int ms, int rbe, float* C,
+                int ldc, int M, int N, int K, int tile, hipStream_t s) {
   if (M <= 0 || N <= 0) return;
-  const int ncb = dw_pad(N, 256) / 16;
+  const SplitB W{(const uint4*)P16, dw_pad(N, 256) / 16, K / 32, shift};
   const long big = ((long)(M + 95) / 96) * ((N + 255) / 256);
   if (tile < 0 ? big >= 512 : tile > 0) {
     const int tilesN = (N + 255) / 256, total = (M + 95) / 96 * tilesN;
-    hipLaunchKernelGGL((k_split_gemm<6, 4>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, A, lda, (const uint4*)P, ncb,
-                       C, ldc, M, N, K / 32, tilesN, total);
+    hipLaunchKernelGGL((k_split_gemm<6, 4>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, A, lda, W, amax, np, ms, rbe, C,
+                       ldc, M, N, tilesN, total);
   } else {
     const int tilesN = (N + 127) / 128, total = (M + 47) / 48 * tilesN;
-    hipLaunchKernelGGL((k_split_gemm<3, 2>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, A, lda, (const uint4*)P, ncb,
-                       C, ldc, M, N, K / 32, tilesN, total);
+    hipLaunchKernelGGL((k_split_gemm<3, 2>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, A, lda, W, amax, np, ms, rbe, C,
+                       ldc, M, N, tilesN, total);
   }
 }
 
@@ -228,18 +416,22 @@ void split_gemm(const float* A, int lda, const void* P, float* C, int ldc, int M
 // lane exchanges and the stores are 64-byte row segments, four rows at a time.  Padding channels are left
 // unwritten: rows are independent and nothing reads those of a padding channel.
 //
-// 1,376,256 rows (2048 walkers of 14 electrons) x 320 x 256: 2000 us with FP32 MFMA, 1240 us here, 16 % of it
-// the tail of the rule and its stores (a 32-wide layer takes 504 us; writing its output alone 340 us at the
-// card's 4.1 TB/s).  Matrix cores are busy for 51 % of the cycles at 2.0 GHz: at this load the card lowers its
-// clock from 2.4.  26 electrons (1.7 M rows): 3600 -> 1960 us; 42 electrons (1.0 M rows): 1930 -> 990 us.
+// 1,376,256 rows (2048 walkers of 14 electrons) x 320 x 256: 2000 us with FP32 MFMA, 1240 us with BF16 parts, 980 us
+// with FP16 parts and rows loaded two slices ahead (1050 us with one slice).  Reading X and writing the output take 610
+// us at the card's rates (6.4 TB/s reads alone, 4.1 TB/s writes alone); matrix cores are busy for a third of the cycles
+// (with BF16 parts for half of them, at 2.0 GHz: the card lowers its clock from 2.4).  26 electrons (1.7 M rows): 3600,
+// 1960, 1540 us; 42 electrons (1.0 M rows): 1930, 990, 905 us.
 // ------------------------------------------------------------------------------------------------
-template <int RBE, int E, int NQ>
-__global__ __launch_bounds__(256, 2) void k_split_lap(const float* __restrict__ X, int ldx,
-                                                      const uint4* __restrict__ P, int ncb, int slices,
+template <int RBE, int E, int NQ, bool HALF>
+__global__ __launch_bounds__(256, 2) void k_split_lap(const float* __restrict__ X, int ldx, SplitB W,
+                                                      const float* __restrict__ amax, int np, int tail,
                                                       const float* __restrict__ V, int ldv, float* __restrict__ out,
-                                                      int ldo, int permute, Shape sh, int tilesN, int tilesTotal) {
-  constexpr int RB = RBE * E;
-  __shared__ SplitLds<RB> lds;
+                                                      int ldo, float* __restrict__ omax, int permute, Shape sh,
+                                                      int tilesN, int tilesTotal) {
+  constexpr int RB = RBE * E, AIT = SplitUnits<RB>::AIT;
+  __shared__ SplitLds<RB, HALF ? 2 : 3> lds;
+  __shared__ unsigned sM[HALF ? RB : 1];
+  __shared__ int eA[HALF ? RB : 1];
   const int tile = tile_of(blockIdx.x, tilesTotal);
   if (tile >= tilesTotal) return;  // uniform over the workgroup, before any barrier
   const int n = sh.n, C = sh.C, Cp = sh.Cp;
@@ -249,7 +441,15 @@ __global__ __launch_bounds__(256, 2) void k_split_lap(const float* __restrict__ 
   const int cb0 = (tile % tilesN) * (4 * NQ) + wv * NQ;
   const int dn = n - sh.u;
   const int col = cb0 * 16 + (lane & 15);
-  // the accumulators start from V: its loads run beside the first slice's
+  const SplitUnits<RB> U(X, g0 * Cp, n_el * Cp, ldx);
+  v4f ra0[HALF ? AIT : 1], ra1[HALF ? AIT : 1];
+  float sc[HALF ? AIT : 1];
+  if constexpr (HALF) {
+    const int first = tail > 0 ? W.slices - tail : 0;
+    U.load(first, ra0);
+    U.load(tail == 1 ? 0 : first + 1, ra1);
+  }
+  // the accumulators start from V (in their units): its loads run beside the first slices'
   v4f acc[RB][NQ];
 #pragma unroll
   for (int e = 0; e < E; ++e) {
@@ -262,7 +462,21 @@ __global__ __launch_bounds__(256, 2) void k_split_lap(const float* __restrict__ 
 #pragma unroll
         for (int q = 0; q < NQ; ++q) acc[e * RBE + kb][q][j] = Vp[(long)(kb * 16 + j) * ldv + 16 * q];
   }
-  split_main<RB, NQ>(X, g0 * Cp, n_el * Cp, ldx, slices, P, ncb, cb0, lds, acc);
+  if constexpr (HALF) {
+    tile_scales<RB>(U, amax, np, sh.W1 >> 5, tail, ra0, ra1, g0 * RBE, n_el * RBE, RBE, C, sM, eA, sc);
+    __syncthreads();  // eA
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+      const float unit = ldexpf(1.f, eA[i] + W.shift);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][q][j] *= unit;
+    }
+    split_main16<RB, NQ>(U, W, tail, ra0, ra1, sc, cb0, lds, acc);
+  } else {
+    split_main<RB, NQ>(U, W, cb0, lds, acc);
+  }
 
 #pragma unroll
   for (int e = 0; e < E; ++e) {
@@ -274,7 +488,8 @@ __global__ __launch_bounds__(256, 2) void k_split_lap(const float* __restrict__ 
     if (permute) ob = (i < sh.u) ? (b * sh.u + i) * Cp : (long)sh.B * sh.u * Cp + (b * dn + (i - sh.u)) * Cp;
     float* op = out + (ob + 4 * g4) * ldo + col;
     const float* vp = out + ob * ldo + col;
-    float d1[NQ], d2[NQ], S[NQ], zl[NQ];
+    const float inv = HALF ? ldexpf(1.f, -(eA[HALF ? e * RBE : 0] + W.shift)) : 1.f;
+    float d1[NQ], d2[NQ], S[NQ], zl[NQ], mx = 0.f;  // mx: largest |y| of the derivative channels
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       const float th = vp[16 * q];
@@ -291,10 +506,14 @@ __global__ __launch_bounds__(256, 2) void k_split_lap(const float* __restrict__ 
         const bool tan = ch >= 1 && ch < C - 1;
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
-          const float z = acc[e * RBE + kb][q][j];
+          const float z = acc[e * RBE + kb][q][j] * inv;
           S[q] += tan ? z * z : 0.f;
           if (ch == C - 1) zl[q] = z;
-          if (tan) op[(long)(kb * 16 + j) * ldo + 16 * q] = d1[q] * z;
+          if (tan) {
+            const float y = d1[q] * z;
+            mx = fmaxf(mx, fabsf(y));
+            op[(long)(kb * 16 + j) * ldo + 16 * q] = y;
+          }
         }
       }
     }
@@ -303,22 +522,36 @@ __global__ __launch_bounds__(256, 2) void k_split_lap(const float* __restrict__ 
     for (int q = 0; q < NQ; ++q) {
       float s = S[q] + __shfl_xor(S[q], 16, 64);
       s += __shfl_xor(s, 32, 64);
-      if (g4 == (cl >> 2)) out[(ob + C - 1) * ldo + col + 16 * q] = d1[q] * zl[q] + d2[q] * s;
+      if (g4 == (cl >> 2)) {
+        const float y = d1[q] * zl[q] + d2[q] * s;
+        mx = fmaxf(mx, fabsf(y));
+        out[(ob + C - 1) * ldo + col + 16 * q] = y;
+      }
     }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    if (lane == 0) omax[ob / Cp * (sh.W1 >> 5) + cb0 / NQ] = mx;
   }
 }
 
-bool split_lap(const float* X, int ldx, const void* P, int K, const float* V, int ldv, float* out, int ldo,
-               int permute, const Shape& sh, int E_max, int cols, hipStream_t s) {
-  const int RBE = sh.Cp / 16, ncb = dw_pad(sh.W1, 256) / 16;
+int split_lap(const float* X, int ldx, const void* P, int shift, int K, const float* amax, int np, int tail,
+              const float* V, int ldv, float* out, int ldo, float* omax, int permute, const Shape& sh, int E_max,
+              int cols, hipStream_t s) {
+  const int RBE = sh.Cp / 16;
+  const SplitB W{(const uint4*)P, dw_pad(sh.W1, 256) / 16, K / 32, amax ? shift : 0};
   const long n_el = (long)sh.B * sh.n;
-#define DW_SPLIT_LAP(R, EE, Q)                                                                                  \
-  do {                                                                                                          \
-    const int tilesN = sh.W1 / (64 * Q);                                                                        \
-    const long total = (n_el + EE - 1) / EE * tilesN;                                                           \
-    hipLaunchKernelGGL((k_split_lap<R, EE, Q>), dim3((unsigned)((total + 7) / 8 * 8)), dim3(256), 0, s, X, ldx, \
-                       (const uint4*)P, ncb, K / 32, V, ldv, out, ldo, permute, sh, tilesN, (int)total);        \
-    return true;                                                                                                \
+#define DW_SPLIT_LAP(R, EE, Q)                                                                                        \
+  do {                                                                                                                \
+    const int tilesN = sh.W1 / (64 * Q);                                                                              \
+    const long total = (n_el + EE - 1) / EE * tilesN;                                                                 \
+    const dim3 grid((unsigned)((total + 7) / 8 * 8));                                                                 \
+    if (amax)                                                                                                         \
+      hipLaunchKernelGGL((k_split_lap<R, EE, Q, true>), grid, dim3(256), 0, s, X, ldx, W, amax, np, tail, V, ldv, out, \
+                         ldo, omax, permute, sh, tilesN, (int)total);                                                 \
+    else                                                                                                              \
+      hipLaunchKernelGGL((k_split_lap<R, EE, Q, false>), grid, dim3(256), 0, s, X, ldx, W, amax, np, tail, V, ldv,     \
+                         out, ldo, omax, permute, sh, tilesN, (int)total);                                            \
+    return sh.W1 / (16 * Q);                                                                                          \
   } while (0)
   // full tiles (96 rows or one electron, 256 columns: A read and split once) where they give two workgroups to
   // every CU; otherwise fewer electrons and 128 columns, which fill the chip from half as many rows.  More than
@@ -347,7 +580,7 @@ bool split_lap(const float* X, int ldx, const void* P, int K, const float* V, in
     case 20: DW_SPLIT_LAP(10, 1, 2);
     case 22: DW_SPLIT_LAP(11, 1, 2);
     case 24: DW_SPLIT_LAP(12, 1, 2);
-    default: return false;
+    default: return 0;
   }
 #undef DW_SPLIT_LAP
 }

@@ -53,21 +53,30 @@ void gemm_lap(GemmPrec prec, const float* X, int ldx, const float* Bt, const uin
               hipStream_t s);
 int lap_electrons_per_tile(int Cp, GemmPrec prec);
 
-// FP32 GEMMs on BF16 MFMA with both operands split into three BF16 parts (gemm_split.hip).  P: weights
+// FP32 GEMMs on 16-bit MFMA with both operands split into three BF16 or two FP16 parts (gemm_split.hip).  P: weights
 // Bt [rows, K] (row = output column, columns at or past `cols` zero) packed by launch_split_pack into
 // split_pack_bytes(cols, K) bytes; K a multiple of 32.
 size_t split_pack_bytes(int cols, int K);
 void launch_split_pack(const float* Bt, int ldb, int cols, int K, void* out, hipStream_t s);
-// C[M, N] = A[M, K] B.  tile: -1 chosen by size, 0 = 48 x 128, 1 or 2 = 96 x 256 (results do not depend on it).
-void split_gemm(const float* A, int lda, const void* P, float* C, int ldc, int M, int N, int K, int tile,
-                hipStream_t s);
+// The same weights as two FP16 parts of 2^shift W (K columns from Bt, split_pack16_bytes(cols, K) bytes).
+size_t split_pack16_bytes(int cols, int K);
+void launch_split_pack16(const float* Bt, int ldb, int cols, int K, int shift, void* out, hipStream_t s);
+// C[M, N] = A[M, K] B for rows of electrons (16 rbe rows each), K a multiple of 64, B in FP16 parts.  amax: np per-wave
+// maxima of each electron's A rows, ms apart.  tile: -1 chosen by size, 0 = 48 x 128, 1 or 2 = 96 x 256 (results do not
+// depend on it).
+void split_gemm(const float* A, int lda, const void* P16, int shift, const float* amax, int np, int ms, int rbe, float* C,
+                int ldc, int M, int N, int K, int tile, hipStream_t s);
 // V[(b Cp + ch), o] of the derivative channels: spin means of X's first Kh columns times W_mu (no bias).
 void split_mean(const float* X, int Kx, int Kh, const void* P, int Km, float* V, int ldv, const Shape& sh,
                 hipStream_t s);
-// 1-el GEMM and tanh forward-Laplacian rule of the derivative channels; `out` holds the value channel already.
-// E_max > 0 / cols = 128 ask for the smaller tiles (results do not depend on them).
-bool split_lap(const float* X, int ldx, const void* P, int K, const float* V, int ldv, float* out, int ldo,
-               int permute, const Shape& sh, int E_max, int cols, hipStream_t s);
+// 1-el GEMM and tanh forward-Laplacian rule of the derivative channels; `out` holds the value channel already.  With
+// amax (np maxima per electron, W1 / 32 apart, covering all but the last `tail` <= 2 slices of 32 columns; K a multiple of 64)
+// P is in FP16 parts, without it in BF16 parts.  omax (W1 / 32 places per electron, in the order of out's rows) receives the maxima
+// of the derivative channels written, one per wave: returns their number per electron (0: shape not supported).  E_max
+// > 0 / cols = 128 ask for the smaller tiles (results do not depend on them).
+int split_lap(const float* X, int ldx, const void* P, int shift, int K, const float* amax, int np, int tail,
+              const float* V, int ldv, float* out, int ldo, float* omax, int permute, const Shape& sh, int E_max,
+              int cols, hipStream_t s);
 
 // One-launch value layers and orbital GEMMs for small batches (value_layer.hip), bit-equal to the separate kernels.
 // Weights in lane order (launch_lane_pack: Bt [rows >= cols, K] into lane_pack_bytes(cols, K) bytes, K a multiple of

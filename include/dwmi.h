@@ -261,11 +261,11 @@ dw_status dw_model_set_tuning(dw_model* m, const dw_tuning* t);
 dw_status dw_model_get_tuning(const dw_model* m, dw_tuning* out);
 
 /* Derivative channels (tangents, Laplacian) of dw_local_energy's GEMMs in the DW_FP32 form.  SPLIT (default): both
- * operands split exactly into three BF16 parts, six products on BF16 MFMA with FP32 sums; E_loc as accurate as
- * with FP32 and 1.2 to 1.5 times faster, equal to it to rounding.  FP32: FP32 MFMA.  The value channel
- * (log|psi|^2, the determinants) is the same bits in both.  For callers whose FP64 statistics of the energies
- * (the optimisation's loss and clipping state) have to stay bit-equal from run to run, across releases: the
- * loss uses FP32. */
+ * operands split into 16-bit parts (three BF16, or two FP16 scaled by powers of two) whose products are summed in FP32
+ * on 16-bit MFMA; E_loc as accurate as with FP32 and 1.3 to 1.9 times faster, equal to it to rounding.  FP32: FP32
+ * MFMA.  The value channel (log|psi|^2, the determinants) is the same bits in both.  For callers whose FP64 statistics
+ * of the energies (the optimisation's loss and clipping state) have to stay bit-equal from run to run, across releases:
+ * the loss uses FP32. */
 #define DW_LAP_SPLIT 0
 #define DW_LAP_FP32 1
 dw_status dw_model_set_lap_form(dw_model* m, int32_t form);

@@ -49,3 +49,41 @@ def test_split_laplacian_matches_fp64_form_for_every_tile(cuda, n, B):
         e1, lp1, _ = eloc(m)
         np.testing.assert_array_equal(e1, e)
         np.testing.assert_array_equal(lp1, lp)
+    # what the scratch held before (rows of padding channels stay as they were) does not reach the results
+    for byte in (0x7E, 0xFF, 0x00):  # 8.5e37, NaN, 0
+        ws = torch.full((m.workspace_bytes(B, 1),), byte, dtype=torch.uint8, device="cuda")
+        m.set_workspace(ws)
+        e1, lp1, _ = eloc(m)
+        np.testing.assert_array_equal(e1, e)
+        np.testing.assert_array_equal(lp1, lp)
+    m.set_workspace(None)
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -20, 1.0, 2.0 ** 12])
+def test_split_operands_of_any_magnitude(cuda, scale):
+    """Orbital weights scaled by a power of two (E_loc does not change): the power-of-two scales of the FP16 parts
+    follow the operands (bound as above)."""
+    from deeperwin_amd._native import NativeModel
+
+    n, B = 14, 21
+    R, Z = random_molecule(np.random.default_rng(n), n)
+    R = R.astype(np.float32)
+    shape = ModelShape(n, 7, len(Z), 2)
+    params = init_params(shape, 3)
+    for path, leaves in params.items():
+        if path.endswith("bf_up/linear_0") or path.endswith("bf_dn/linear_0"):
+            leaves["w"] = (leaves["w"] * np.float32(scale)).astype(np.float32)  # every orbital by one factor
+    r0 = init_walkers_gaussian(np.random.default_rng(1), B, R, generate_el_ion_mapping(R, Z, n, 7))
+    r = torch.as_tensor(r0, dtype=torch.float32, device="cuda").contiguous()
+    Rd = torch.as_tensor(R, dtype=torch.float32, device="cuda")
+    Zd = torch.as_tensor(Z, dtype=torch.float32, device="cuda")
+    out = []
+    for prec in ("fp64", "fp32"):
+        m = NativeModel(shape, prec)
+        m.set_params(params)
+        e = torch.empty(B, device="cuda")
+        m.local_energy(r, Rd, Zd, e)
+        kappa = m.conditioning(B).cpu().numpy() if prec == "fp64" else kappa
+        torch.cuda.synchronize()
+        out.append(e.cpu().numpy())
+    assert np.all(np.abs(out[1] - out[0]) <= (1 + np.abs(out[0])) * (1e-4 + 4 * U32 * kappa))
