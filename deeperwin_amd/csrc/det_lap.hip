@@ -1,12 +1,15 @@
-// Laplacian-mode determinants of more than 16 electrons (FP64), in two launches: log|det|, sign and M^-1 per matrix,
+// Laplacian-mode determinants (FP64), in two launches: log|det|, sign and M^-1 per matrix,
 // then the channel passes
 //   Y_k = M^-1 dM_k,  g_k = tr Y_k,  q_k = tr(Y_k^2),  Lap log|det| = tr(M^-1 Lap M) - sum_k q_k.
 // Both read the orbitals O and apply the envelope themselves, so the product envelope x orbitals (3 n + 2 matrices per
 // determinant) is never stored.
 //
 // 16,384 matrices of 26 (1024 walkers): 4.17 ms for the determinants and 1.99 ms for the stored product before, 0.84 ms
-// (inverses) + 2.08 ms (channels) here; 1,536 matrices of 42: 4.06 + 0.75 ms before, 0.55 + 1.04 ms here.  The channel
+// (inverses) + 2.08 ms (channels) here; 1,536 matrices of 42: 4.06 + 0.75 ms before, 0.55 + 1.04 ms here; 32,768
+// matrices of 14: 1.14 ms (one wavefront per matrix) before, 0.08 + 0.43 ms here.  Above 16 electrons the channel
 // passes run at half the FP64 matrix rate, padding to 16 x 16 blocks counted (1.06 and 0.54 ms at 78 TFLOP/s).
+#include <utility>
+
 #include "common.h"
 #include "det_common.h"
 #include "kernels.h"
@@ -21,7 +24,136 @@ __device__ __forceinline__ double value_at(const OrbSrc<TA>& src, const Shape& s
   return (double)(env * src.O[orb_row(sh, b, i) * src.ldo + oc]);
 }
 
-// n <= 32: one matrix per wavefront, a lane per column, LU and inverse in registers.  Minv [matrix][n][n].
+// Lane P of every 16-lane row to all lanes of that row (DPP row_newbcast).
+template <int P>
+__device__ __forceinline__ int row_bcast(int v) {
+  return __builtin_amdgcn_mov_dpp(v, 0x150 + P, 0xF, 0xF, true);
+}
+template <int P>
+__device__ __forceinline__ double row_bcast(double v) {
+  return __hiloint2double(row_bcast<P>(__double2hiint(v)), row_bcast<P>(__double2loint(v)));
+}
+template <typename F, int... I>
+__device__ __forceinline__ void unroll_seq(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
+// n <= 16: four matrices per wavefront, one per 16-lane row, a lane per column; entries are broadcast inside a row by
+// DPP, so all four eliminate at once (a matrix per wavefront kept 14 of 64 lanes busy: 32,768 matrices of 14 took 358
+// us, 83 us here).  The operations and their order are lu_columns'.
+template <typename TA>
+__global__ __launch_bounds__(256) void k_det_inv16(OrbSrc<TA> src, Shape sh, double* __restrict__ Minv,
+                                                   double* __restrict__ ld, double* __restrict__ sd,
+                                                   float* __restrict__ dcond, long nmat) {
+  constexpr int N = 16;
+  const int lane = threadIdx.x & 63, c = lane & 15, n = sh.n;
+  long bd = (long)blockIdx.x * 16 + (threadIdx.x >> 4);
+  const bool valid = bd < nmat;
+  if (!valid) bd = nmat - 1;  // whole waves stay in the lane exchanges; results are not stored
+  const long b = bd / sh.D;
+  const int dcol = (int)(bd - b * sh.D) * n;
+  const bool act = c < n;
+  double col[N];
+  int perm[N];
+  double csum = 0.0;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    col[i] = (act && i < n) ? value_at<TA>(src, sh, b, i, dcol + c) : 0.0;
+    csum += fabs(col[i]);
+    perm[i] = i;
+  }
+  auto row_max = [](double v) {
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+    return v;
+  };
+  const double normA = row_max(csum);
+  double mydiag = 1.0;
+  bool sing = false;
+  int swaps = 0;
+  unroll_seq(
+      [&](auto PP) {
+        constexpr int p = PP;
+        if (p < n) {  // uniform
+          double best = -1.0;
+          int bidx = p;
+#pragma unroll
+          for (int i = p; i < N; ++i) {
+            const double a = fabs(col[i]);
+            const bool take = i < n && a > best;
+            best = take ? a : best;
+            bidx = take ? i : bidx;
+          }
+          const int piv = row_bcast<p>(bidx);
+          if (!(row_bcast<p>(best) > 0.0)) sing = true;
+          swaps += piv != p ? 1 : 0;
+          const double old = col[p];
+          const int oldp = perm[p];
+#pragma unroll
+          for (int i = p + 1; i < N; ++i) {
+            const bool sw = i == piv;
+            col[p] = sw ? col[i] : col[p];
+            perm[p] = sw ? perm[i] : perm[p];
+            col[i] = sw ? old : col[i];
+            perm[i] = sw ? oldp : perm[i];
+          }
+          if (c == p) mydiag = col[p];
+          const double rp = 1.0 / row_bcast<p>(col[p]);
+#pragma unroll
+          for (int i = p + 1; i < N; ++i) {
+            const double l = col[i] * rp;
+            if (c == p) col[i] = l;
+            const double li = row_bcast<p>(col[i]);
+            if (c > p) col[i] -= li * col[p];
+          }
+        }
+      },
+      std::make_integer_sequence<int, N>{});
+  double lg = act ? log(fabs(mydiag)) : 0.0;
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) lg += __shfl_xor(lg, o, 64);
+  const unsigned long long neg = __ballot(act && mydiag < 0.0);
+  const int nneg = __popc((unsigned)(neg >> (lane & 48)) & 0xFFFFu) + swaps;
+  double x[N];  // column c of the inverse: L y = P e_c, then U x = y
+  unroll_seq(
+      [&](auto PP) {
+        constexpr int p = PP;
+        double y = (p < n && perm[p] == c) ? 1.0 : 0.0;
+        if (p < n)
+          unroll_seq([&](auto QQ) { y -= row_bcast<int(QQ)>(col[p]) * x[int(QQ)]; }, std::make_integer_sequence<int, p>{});
+        x[p] = y;
+      },
+      std::make_integer_sequence<int, N>{});
+  unroll_seq(
+      [&](auto PP) {
+        constexpr int p = N - 1 - int(PP);
+        if (p < n) {
+          double y = x[p];
+          unroll_seq(
+              [&](auto QQ) {
+                constexpr int q = p + 1 + int(QQ);
+                if (q < n) y -= row_bcast<q>(col[p]) * x[q];
+              },
+              std::make_integer_sequence<int, N - 1 - p>{});
+          x[p] = y / row_bcast<p>(col[p]);
+        }
+      },
+      std::make_integer_sequence<int, N>{});
+  double isum = 0.0;
+#pragma unroll
+  for (int a = 0; a < N; ++a) {
+    isum += act ? fabs(x[a]) : 0.0;
+    if (act && a < n && valid) Minv[bd * n * n + a * n + c] = x[a];
+  }
+  const double normMi = row_max(isum);
+  if (c == 0 && valid) {
+    ld[bd] = sing ? -INFINITY : lg;
+    sd[bd] = sing ? 0.0 : ((nneg & 1) ? -1.0 : 1.0);
+    dcond[bd] = (float)(normA * normMi);
+  }
+}
+
+// 16 < n <= 32: one matrix per wavefront, a lane per column, LU and inverse in registers.  Minv [matrix][n][n].
 template <int NMAX, typename TA>
 __global__ __launch_bounds__(256) void k_det_inv(OrbSrc<TA> src, Shape sh, double* __restrict__ Minv,
                                                  double* __restrict__ ld, double* __restrict__ sd,
@@ -203,7 +335,7 @@ __global__ __launch_bounds__(64) void k_det_inv_lds(OrbSrc<TA> src, Shape sh, do
 // products take; tr Y comes from the diagonal the same tile holds.
 // ------------------------------------------------------------------------------------------------
 template <int NB, typename TA>
-__global__ __launch_bounds__(256, NB == 4 ? 1 : (NB == 2 && sizeof(TA) == 4 ? 3 : 2)) void k_det_chan(OrbSrc<TA> src, Shape sh,
+__global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof(TA) == 4 ? 3 : 2)) void k_det_chan(OrbSrc<TA> src, Shape sh,
                                                                                const double* __restrict__ Minv,
                                                                                double* __restrict__ g,
                                                                                double* __restrict__ lapd, int nmat) {
@@ -377,11 +509,14 @@ static void launch_chan(const OrbSrc<TA>& src, const Shape& sh, const double* Mi
 }
 
 template <typename TA>
-void launch_det_lap_large(const OrbSrc<TA>& src, double* Minv, double* ld, double* sd, double* g, double* lapd,
+void launch_det_lap(const OrbSrc<TA>& src, double* Minv, double* ld, double* sd, double* g, double* lapd,
                           float* dcond, const Shape& sh, hipStream_t s) {
   const int n = sh.n;
   const long nmat = (long)sh.B * sh.D;
-  if (n <= 32) {
+  if (n <= 16) {
+    hipLaunchKernelGGL((k_det_inv16<TA>), dim3((unsigned)((nmat + 15) / 16)), dim3(256), 0, s, src, sh, Minv, ld, sd,
+                       dcond, nmat);
+  } else if (n <= 32) {
     hipLaunchKernelGGL((k_det_inv<32, TA>), dim3((unsigned)((nmat + 3) / 4)), dim3(256), 0, s, src, sh, Minv, ld, sd,
                        dcond, nmat);
   } else {
@@ -391,14 +526,15 @@ void launch_det_lap_large(const OrbSrc<TA>& src, double* Minv, double* ld, doubl
     hipLaunchKernelGGL((k_det_inv_lds<TA>), dim3((unsigned)nmat), dim3(64), shm, s, src, sh, Minv, ld, sd, dcond);
   }
   switch ((n + 15) / 16) {
+    case 1: launch_chan<1, TA>(src, sh, Minv, g, lapd, s); break;
     case 2: launch_chan<2, TA>(src, sh, Minv, g, lapd, s); break;
     case 3: launch_chan<3, TA>(src, sh, Minv, g, lapd, s); break;
     default: launch_chan<4, TA>(src, sh, Minv, g, lapd, s); break;
   }
 }
-template void launch_det_lap_large<float>(const OrbSrc<float>&, double*, double*, double*, double*, double*, float*,
+template void launch_det_lap<float>(const OrbSrc<float>&, double*, double*, double*, double*, double*, float*,
                                           const Shape&, hipStream_t);
-template void launch_det_lap_large<double>(const OrbSrc<double>&, double*, double*, double*, double*, double*, float*,
+template void launch_det_lap<double>(const OrbSrc<double>&, double*, double*, double*, double*, double*, float*,
                                            const Shape&, hipStream_t);
 
 }  // namespace dwmi

@@ -134,9 +134,9 @@ struct OrbSrc {
 // True when the determinant kernels for n electrons and C channels apply the envelope while reading O
 // (no envelope launch, no stored product); otherwise launch_envelope fills A first.
 inline bool det_reads_orbitals(int n, int C) { return C > 1 || n <= 32; }
-// Doubles of inverse matrices that launch_det needs as scratch (`minv`): the Laplacian pass of more than 16 electrons.
+// Doubles of inverse matrices that launch_det needs as scratch (`minv`): the Laplacian pass.
 inline size_t det_inverse_elems(long matrices, int n, int C) {
-  return C > 1 && n > 16 ? (size_t)matrices * n * n : 0;
+  return C > 1 ? (size_t)matrices * n * n : 0;
 }
 // Outputs of the value-pass combine (launch_combine's, C == 1) when launch_det runs it itself.
 struct CombineValue {
@@ -152,9 +152,9 @@ struct CombineValue {
 template <typename TA>
 bool launch_det(const TA* A, const OrbSrc<TA>& src, double* minv, double* ld, double* sd, double* g, double* lapd, float* dcond,
                 const Shape& sh, hipStream_t s, const CombineValue* combine = nullptr);
-// Its part for the Laplacian pass of more than 16 electrons (det_lap.hip).
+// Its part for the Laplacian pass (det_lap.hip).
 template <typename TA>
-void launch_det_lap_large(const OrbSrc<TA>& src, double* minv, double* ld, double* sd, double* g, double* lapd,
+void launch_det_lap(const OrbSrc<TA>& src, double* minv, double* ld, double* sd, double* g, double* lapd,
                           float* dcond, const Shape& sh, hipStream_t s);
 void launch_combine(const double* ld, const double* sd, const double* g, const double* lapd, const float* dcond,
                     float cond_thr, const float* r, const float* R, const float* Z, float* out_lp, float* out_phase,

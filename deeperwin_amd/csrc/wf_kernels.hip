@@ -919,231 +919,6 @@ __global__ __launch_bounds__(256) void k_det_value(OrbSrc<TA> src, double* __res
   }
 }
 
-// Laplacian mode (n <= 16): WPB matrices per workgroup, one per wavefront; LU and inverse with a lane per
-// column, M^-1 through LDS into MFMA operand registers, then the channel passes on FP64 MFMA.
-// The matrices are read from the orbitals O and the envelope is applied on the way (no stored A);
-// while the value channel is read, each wavefront tabulates in LDS the envelope, the own-electron
-// gradient terms g_c bf0 (channel 3i + c of row i gains them) and the Laplacian channel, [row][column].
-template <int NMAX, int WPB, typename TA>
-__global__ __launch_bounds__(64 * WPB) void k_det_lap(OrbSrc<TA> src, Shape sh,
-                                                      double* __restrict__ ld, double* __restrict__ sd,
-                                                      double* __restrict__ g, double* __restrict__ lapd,
-                                                      float* __restrict__ dcond, long nmat, int n, int C) {
-  extern __shared__ double dsm[];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  long bd = (long)blockIdx.x * WPB + wv;
-  const bool valid_mat = bd < nmat;
-  if (!valid_mat) bd = nmat - 1;  // keep the wave in the barriers; results are not stored
-  static_assert(NMAX == 16, "larger matrices: det_lap.hip");
-  constexpr int NN = NMAX * NMAX;
-  double* sMi = dsm + (size_t)wv * NN;
-  TA* sE = (TA*)(dsm + (size_t)WPB * NN) + (size_t)wv * 5 * NN;  // ENV tables: [row][column]
-  TA* sG = sE + NN;                                               // [c][row][column]
-  TA* sL = sE + 4 * NN;
-  const bool act = lane < n;
-  const int nd = 3 * n;
-  const long b = bd / sh.D;
-  const int dcol = (int)(bd - b * sh.D) * n;  // first orbital column of this determinant
-
-  double col[NMAX];
-  int perm[NMAX];
-  double csum = 0.0;
-#pragma unroll
-  for (int i = 0; i < NMAX; ++i) {
-    {
-      double v = 0.0;
-      TA e0 = TA(0), gb0 = TA(0), gb1 = TA(0), gb2 = TA(0), lp = TA(0);
-      if (act && i < n) {
-        const int oc = dcol + lane;
-        TA env, g0, g1, g2, lv;
-        envelope_at<TA, true>(src.kappa, src.wenv, src.r, src.R, sh, b, i, oc, env, g0, g1, g2, lv);
-        const TA* Oi = src.O + orb_row(sh, b, i) * src.ldo + oc;
-        const TA bf0 = Oi[0];
-        const TA t0 = Oi[(long)(1 + 3 * i) * src.ldo];
-        const TA t1 = Oi[(long)(2 + 3 * i) * src.ldo];
-        const TA t2 = Oi[(long)(3 + 3 * i) * src.ldo];
-        v = (double)(env * bf0);
-        e0 = env;
-        gb0 = g0 * bf0;
-        gb1 = g1 * bf0;
-        gb2 = g2 * bf0;
-        lp = lv * bf0 + env * Oi[(long)(C - 1) * src.ldo] + TA(2) * (g0 * t0 + g1 * t1 + g2 * t2);
-      }
-      if (lane < NMAX) {  // zero outside n x n
-        sE[i * NMAX + lane] = e0;
-        sG[(0 * NMAX + i) * NMAX + lane] = gb0;
-        sG[(1 * NMAX + i) * NMAX + lane] = gb1;
-        sG[(2 * NMAX + i) * NMAX + lane] = gb2;
-        sL[i * NMAX + lane] = lp;
-      }
-      col[i] = v;
-    }
-    csum += fabs(col[i]);
-  }
-  const double normA = wave_max_d(csum);
-  double mydiag = 1.0;
-  bool sing = false;
-  const int swaps = lu_columns<NMAX>(col, perm, mydiag, sing, n, lane);
-  double logabs, sgn;
-  finish_slogdet<NMAX>(mydiag, swaps, sing, n, lane, logabs, sgn);
-
-  // inverse, column `lane`: solve L y = P e_lane, then U x = y
-  double x[NMAX];
-#pragma unroll
-  for (int p = 0; p < NMAX; ++p) {
-    if (p < n) {
-      double y = (perm[p] == lane) ? 1.0 : 0.0;
-#pragma unroll
-      for (int q = 0; q < p; ++q) y -= readlane_d(col[p], q) * x[q];
-      x[p] = y;
-    } else {
-      x[p] = 0.0;
-    }
-  }
-#pragma unroll
-  for (int p = NMAX - 1; p >= 0; --p) {
-    if (p < n) {
-      double y = x[p];
-#pragma unroll
-      for (int q = p + 1; q < NMAX; ++q)
-        if (q < n) y -= readlane_d(col[p], q) * x[q];
-      x[p] = y / readlane_d(col[p], p);
-    }
-  }
-  double isum = 0.0;
-#pragma unroll
-  for (int a = 0; a < NMAX; ++a) isum += act ? fabs(x[a]) : 0.0;
-  const double normMi = wave_max_d(isum);
-  // M^-1 to LDS, row-major [a][e]
-  if (lane < NMAX) {
-#pragma unroll
-    for (int a = 0; a < NMAX; ++a) sMi[a * NMAX + lane] = act ? x[a] : 0.0;
-  }
-  __syncthreads();
-
-  // Channel passes on FP64 MFMA (v_mfma_f64_16x16x4f64) over NB x NB blocks of 16.  Lane l holds
-  // M^-1[I*16 + l%16][K*16 + l/16 + 4s] (A operand of Y_k = M^-1 dM_k) and dM_k[K*16 + l/16 + 4s][J*16 + l%16]
-  // (its B operand); the same registers are the B and A operands of (Y_k^T)_IJ = sum_K (dM_k)_KI^T (M^-1)_JK^T.
-  // Both products come out in one layout, so tr Y_k^2 is the sum of their elementwise product, and tr Y_k
-  // is the sum of the operand products.  Channels run in groups of G: the loads of the next group are
-  // issued before the current group is multiplied, and the G traces tr Y_k leave the wavefront in one
-  // grouped reduction (same pairing order as a single wave sum).
-  double qacc = 0.0;
-  {
-    constexpr int NB = NMAX / 16, G = 2;  // measured fastest at n = 14
-    const int ri = lane & 15, kq = lane >> 4;
-    double miA[NB][NB][4];
-#pragma unroll
-    for (int I = 0; I < NB; ++I)
-#pragma unroll
-      for (int K = 0; K < NB; ++K)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) miA[I][K][q] = sMi[(I * 16 + ri) * NMAX + K * 16 + kq + 4 * q];
-    // envelope and the O row base of each element this lane holds
-    TA envq[NB][NB][4];
-    const TA* ob[NB][NB][4];
-#pragma unroll
-    for (int K = 0; K < NB; ++K)
-#pragma unroll
-      for (int J = 0; J < NB; ++J)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int rr = K * 16 + kq + 4 * q, cc = J * 16 + ri;
-          envq[K][J][q] = sE[rr * NMAX + cc];
-          ob[K][J][q] = (rr < n && cc < n) ? src.O + orb_row(sh, b, rr) * src.ldo + dcol + cc : src.O;
-        }
-    TA cur[G][NB][NB][4], nxt[G][NB][NB][4];
-    auto load = [&](TA (&d)[G][NB][NB][4], int k0) {
-#pragma unroll
-      for (int c = 0; c < G; ++c) {
-        const int k = k0 + c;
-#pragma unroll
-        for (int K = 0; K < NB; ++K)
-#pragma unroll
-          for (int J = 0; J < NB; ++J)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const int rr = K * 16 + kq + 4 * q, cc = J * 16 + ri;
-              const bool in = k < nd && rr < n && cc < n;
-              d[c][K][J][q] = in ? ob[K][J][q][(long)(1 + k) * src.ldo] : TA(0);
-            }
-      }
-    };
-    load(cur, 0);
-    for (int k0 = 0; k0 < nd; k0 += G) {
-      load(nxt, k0 + G);
-      // one channel at a time: only the loads of the next group overlap the products (register budget)
-      __builtin_amdgcn_sched_barrier(0);
-      double gp[G];
-#pragma unroll
-      for (int c = 0; c < G; ++c) {
-        double dmB[NB][NB][4];
-        const int kr = (k0 + c) / 3, kc3 = (k0 + c) - 3 * kr;  // the channel's electron and component
-#pragma unroll
-        for (int K = 0; K < NB; ++K)
-#pragma unroll
-          for (int J = 0; J < NB; ++J)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const int rr = K * 16 + kq + 4 * q, cc = J * 16 + ri;
-              const TA own = (rr == kr) ? sG[(kc3 * NMAX + rr) * NMAX + cc] : TA(0);
-              dmB[K][J][q] = (double)fma(envq[K][J][q], cur[c][K][J][q], own);
-            }
-        double t = 0.0;
-#pragma unroll
-        for (int I = 0; I < NB; ++I)
-#pragma unroll
-          for (int K = 0; K < NB; ++K)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) t += miA[I][K][q] * dmB[K][I][q];
-        gp[c] = t;
-#pragma unroll
-        for (int I = 0; I < NB; ++I)
-#pragma unroll
-          for (int J = 0; J < NB; ++J) {
-            v4d y = {0.0, 0.0, 0.0, 0.0}, yt = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int K = 0; K < NB; ++K)
-#pragma unroll
-              for (int q = 0; q < 4; ++q) {
-                y = __builtin_amdgcn_mfma_f64_16x16x4f64(miA[I][K][q], dmB[K][J][q], y, 0, 0, 0);
-                yt = __builtin_amdgcn_mfma_f64_16x16x4f64(dmB[K][I][q], miA[J][K][q], yt, 0, 0, 0);
-              }
-            qacc += y[0] * yt[0] + y[1] * yt[1] + y[2] * yt[2] + y[3] * yt[3];
-          }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      const double s = wave_sum_group<G>(gp, lane);
-      const int kc = k0 + lane / (64 / G);
-      if (lane % (64 / G) == 0 && kc < nd && valid_mat) g[bd * nd + kc] = s;
-#pragma unroll
-      for (int c = 0; c < G; ++c)
-#pragma unroll
-        for (int K = 0; K < NB; ++K)
-#pragma unroll
-          for (int J = 0; J < NB; ++J)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) cur[c][K][J][q] = nxt[c][K][J][q];
-    }
-    qacc = wave_sum_d(qacc);
-  }
-  // tr(M^-1 Lap M): lane c takes column c of Lap M and row c of M^-1
-  double tp = 0.0;
-  if (act) {
-#pragma unroll
-    for (int e = 0; e < NMAX; ++e)
-      if (e < n) tp += sMi[lane * NMAX + e] * (double)sL[e * NMAX + lane];
-  }
-  tp = wave_sum_d(tp);
-  if (lane == 0 && valid_mat) {
-    ld[bd] = logabs;
-    sd[bd] = sgn;
-    lapd[bd] = tp - qacc;
-    dcond[bd] = (float)(normA * normMi);
-  }
-}
-
-
 // Value mode, 32 < n <= 64: one wavefront per matrix, the matrix in LDS (FP64, pitch n + 1), lane j owns
 // column j.  Partial-pivot LU: argmax of the pivot column by shuffles (lowest row on ties), row swap and
 // rank-1 update column-parallel; a single-wavefront workgroup, so each barrier only orders the LDS
@@ -1223,8 +998,8 @@ bool launch_det(const TA* A, const OrbSrc<TA>& src, double* minv, double* ld, do
   const int n = sh.n;
   const long nmat = (long)sh.B * sh.D;
   const long stride = (long)sh.C * n * n;
-  if (sh.C > 1 && n > 16) {
-    launch_det_lap_large<TA>(src, minv, ld, sd, g, lapd, dcond, sh, s);
+  if (sh.C > 1) {
+    launch_det_lap<TA>(src, minv, ld, sd, g, lapd, dcond, sh, s);
     return false;
   }
   if (n > 32) {
@@ -1250,12 +1025,6 @@ bool launch_det(const TA* A, const OrbSrc<TA>& src, double* minv, double* ld, do
       hipLaunchKernelGGL((k_det_value<32, TA>), grid, dim3(256), 0, s, src, ld, sd, dcond, nmat, n, sh, co);
     return co.fuse != 0;
   }
-  // M^-1 (FP64) plus the envelope tables (5 [16][16] arrays of TA) per wavefront
-  constexpr int NM = 16, W = 4;
-  const size_t shm = (size_t)W * (NM * NM) * (sizeof(double) + 5 * sizeof(TA));
-  hipLaunchKernelGGL((k_det_lap<NM, W, TA>), dim3((unsigned)((nmat + W - 1) / W)), dim3(64 * W), shm, s, src, sh, ld,
-                     sd, g, lapd, dcond, nmat, n, sh.C);
-  return false;
 }
 template bool launch_det<float>(const float*, const OrbSrc<float>&, double*, double*, double*, double*, double*, float*,
                                 const Shape&, hipStream_t, const CombineValue*);

@@ -1,4 +1,4 @@
-"""Laplacian-mode determinants of more than 16 electrons (det_lap.hip) at the edges of their 16 x 16 blocks."""
+"""Laplacian-mode determinants (det_lap.hip) at the edges of their 16 x 16 blocks."""
 from __future__ import annotations
 
 import numpy as np
@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 U32 = 2.0 ** -24
 
 
-@pytest.mark.parametrize("n,D", [(17, 1), (31, 3), (32, 2), (33, 1), (48, 2), (49, 1), (63, 1)])
+@pytest.mark.parametrize("n,D", [(2, 1), (7, 5), (8, 1), (15, 3), (16, 7), (17, 1), (31, 3), (32, 2), (33, 1), (48, 2), (49, 1), (63, 1)])
 def test_large_determinants_at_block_edges(cuda, n, D):
     """log|psi|^2 of the Laplacian pass against the FP64 oracle (FP64 form: float32 rounding of the output plus 1e-13
     kappa; FP32 form: the parity tests' bound); E_loc of a walker bit-equal in a batch (which fills the workgroups
