@@ -2,8 +2,19 @@
 #pragma once
 #include "common.h"
 #include "kernels.h"
+#include <utility>
 
 namespace dwmi {
+
+// Calls f with 0 .. N-1 as compile-time constants (register arrays keep constant indices whatever the body's size).
+template <typename F, int... I>
+__device__ __forceinline__ void unroll_seq(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void unroll_seq(F&& f) {
+  unroll_seq(f, std::make_integer_sequence<int, N>{});
+}
 
 // Scalar-type generic math (T = float for the FP32/BF16 forms, double for the FP64 form).
 __device__ __forceinline__ float dsqrt(float x) { return sqrtf(x); }

@@ -33,11 +33,6 @@ template <int P>
 __device__ __forceinline__ double row_bcast(double v) {
   return __hiloint2double(row_bcast<P>(__double2hiint(v)), row_bcast<P>(__double2loint(v)));
 }
-template <typename F, int... I>
-__device__ __forceinline__ void unroll_seq(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-
 // n <= 16: four matrices per wavefront, one per 16-lane row, a lane per column; entries are broadcast inside a row by
 // DPP, so all four eliminate at once (a matrix per wavefront kept 14 of 64 lanes busy: 32,768 matrices of 14 took 358
 // us, 83 us here).  The operations and their order are lu_columns'.

@@ -764,17 +764,21 @@ template void launch_envelope<double>(const double*, int, const float*, const fl
 // The 1-norm condition number |M|_1 |M^-1|_1 (Laplacian mode) or the pivot ratio max|U_pp| / min|U_pp|
 // (value mode) is written per matrix to dcond; results are FP64.
 // ------------------------------------------------------------------------------------------------
-// Value-pass combine of one walker's D determinants (log|det| l, sign sg, matrix conditioning dc).
-__device__ __forceinline__ void combine_value_walker(const double* l, const double* sg, const float* dc, int D,
-                                                     float cond_thr, long b, float* __restrict__ out_lp,
-                                                     float* __restrict__ out_phase, uint32_t* __restrict__ out_flags,
-                                                     float* __restrict__ out_kappa) {
+// Value-pass combine of one walker's D determinants (log|det| l, sign sg, matrix conditioning dc): the maximum, then
+// the sum of the terms e_d = sg_d exp(l_d - m) (formed by the caller's `term`, in any lane) in the order of d.
+__device__ __forceinline__ double walker_max(const double* l, int D) {
   double m = -INFINITY;
   for (int d = 0; d < D; ++d) m = fmax(m, (double)l[d]);
+  return m;
+}
+template <typename Term>
+__device__ __forceinline__ void combine_value_walker(Term term, double m, const float* dc, int D, float cond_thr, long b,
+                                                     float* __restrict__ out_lp, float* __restrict__ out_phase,
+                                                     uint32_t* __restrict__ out_flags, float* __restrict__ out_kappa) {
   double S = 0.0, Sabs = 0.0, cmax = 0.0;
   uint32_t fl = 0;
   for (int d = 0; d < D; ++d) {
-    const double e = sg[d] * exp(l[d] - m);
+    const double e = term(d);
     S += e;
     Sabs += fabs(e);
     cmax = fmax(cmax, (double)dc[d]);
@@ -793,102 +797,160 @@ __device__ __forceinline__ void combine_value_walker(const double* l, const doub
   if (out_flags) out_flags[b] = fl;
 }
 
+// Maximum over a group of NMAX lanes, in every lane of it.  DPP moves (VALU) up to 16 lanes, one lane exchange above.
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+template <int NMAX>
+__device__ __forceinline__ double group_max(double v) {
+  v = fmax(v, dpp_d<0xB1>(v));   // quad_perm [1, 0, 3, 2]
+  v = fmax(v, dpp_d<0x4E>(v));   // quad_perm [2, 3, 0, 1]
+  v = fmax(v, dpp_d<0x141>(v));  // row_half_mirror: the other quad of the 8
+  if constexpr (NMAX >= 16) v = fmax(v, dpp_d<0x140>(v));  // row_mirror: the other 8 of the row
+  if constexpr (NMAX >= 32) v = fmax(v, __shfl_xor(v, 16, 32));
+  return v;
+}
+
+// Orders one wavefront's LDS traffic (its LDS operations complete in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Value mode: 64 / NMAX matrices per wavefront (lane group g holds matrix g), 4 wavefronts per workgroup.
-// The matrix is formed with a lane per column (coalesced reads of O), staged in wave-private LDS, and
-// factorised with a lane per row: a row interchange is then a relabelling (no data moves), the pivot is a
-// butterfly arg-max over the group's lanes (largest |a|, lowest row on ties), and each remaining row takes
-// the pivot row's entries by shuffle.  Multipliers a[i][p] * (1 / pivot) (the reciprocal, as LAPACK's
-// dgetf2 scales) and updates a[i][c] -= l a[piv][c] are the same operations as a column-oriented
-// elimination, so U, log|det| (summed over U's diagonal in a fixed lane order) and the conditioning are
-// too; the sign counts the negative pivots and the parity of the pivot order.
+// The matrix is formed with a lane per column (coalesced reads of O, all rows in flight; lane t computes electron
+// t's distance to a nucleus once for the group), transposed through wave-private LDS, and factorised with a lane per
+// row: a row interchange is then a relabelling (no data moves).  The pivot is the group's largest |a| (lowest row on
+// ties): a DPP maximum, then the first set bit of a ballot.  The pivot lane writes its row to LDS and the others read
+// it 16 bytes at a time.  Multipliers a[i][p] * (1 / pivot) (the reciprocal, as LAPACK's dgetf2 scales) and updates
+// a[i][c] -= l a[piv][c] are the same operations as a column-oriented elimination, so U, log|det| (summed over U's
+// diagonal in a fixed lane order) and the conditioning are too; the sign counts the negative pivots and the parity of
+// the pivot order (unused rows below each pivot row).  Rows that were a pivot row keep being updated: nothing reads
+// them again.
+// What bounds it: VALU issue of the FP64 chain and the envelope's exponentials.  With the arg-max and the pivot row
+// by lane shuffles (ds_bpermute: 400 a wavefront at 14 electrons), the LDS pipe bound it: 32,768 matrices of 14 took
+// 63.5 us, 34.6 here (8 waves per SIMD would spill: 72); 16,000 of 17: 98 -> 70; 16,384 of 30: 246 -> 118; 4,096 of 4:
+// 10.0 -> 6.5.
 template <int NMAX, typename TA>
-__global__ __launch_bounds__(256) void k_det_value(OrbSrc<TA> src, double* __restrict__ ld, double* __restrict__ sd,
+__global__ __launch_bounds__(256, sizeof(TA) == 8 ? 2 : (NMAX <= 16 ? 6 : 4)) void k_det_value(OrbSrc<TA> src, double* __restrict__ ld, double* __restrict__ sd,
                                                    float* __restrict__ dcond, long nmat, int n, Shape sh,
                                                    CombineValue co) {
-  constexpr int G = 64 / NMAX;
+  constexpr int G = 64 / NMAX, BT = 4;
   const int lane = threadIdx.x & 63;
+  const int wv = threadIdx.x >> 6;
   const int g = lane / NMAX, t = lane % NMAX, base = g * NMAX;
-  const long bd = ((long)blockIdx.x * 4 + (threadIdx.x >> 6)) * G + g;
+  const long bd = ((long)blockIdx.x * 4 + wv) * G + g;
   const bool valid = bd < nmat;
   const long bdl = valid ? bd : nmat - 1;  // out-of-range groups factor a copy, never stored
   const long b = bdl / sh.D;
   const int oc = (int)(bdl - b * sh.D) * n + t;  // orbital column of matrix column t
   const bool act = t < n;                         // column t (forming), row t (factorising) exists
-  // element (r, c) = env(r_r, column c) * O[electron r, column c]: the envelope is applied as O is read.
-  // Lane t forms column t in a rolled loop (the element phase stays out of the unrolled factorisation);
-  // element (r, c) of group g sits at slot base + (c ^ r) of LDS row r, so both this write (fixed r) and
+  // element (r, c) of group g sits at slot base + (c ^ r) of LDS row r, so both the write (fixed r) and
   // the row read below (fixed c, lanes over r) touch distinct banks.
   __shared__ TA sA[4][NMAX][64];
-  TA (*mine)[64] = sA[threadIdx.x >> 6];
-#pragma unroll 1
-  for (int r = 0; r < n; ++r) {
-    TA v = TA(0);
-    if (act) {
-      TA env, g0, g1, g2, lv;
-      envelope_at<TA, false>(src.kappa, src.wenv, src.r, src.R, sh, b, r, oc, env, g0, g1, g2, lv);
-      v = env * src.O[orb_row(sh, b, r) * src.ldo + oc];
+  __shared__ __align__(16) double sP[4][64];  // the pivot row of each group
+  TA (*mine)[64] = sA[wv];
+  double* prow = &sP[wv][base];
+  {
+    TA env[NMAX], o[NMAX];
+#pragma unroll
+    for (int r = 0; r < NMAX; ++r) {
+      env[r] = TA(0);
+      o[r] = (act && r < n) ? src.O[orb_row(sh, b, r) * src.ldo + oc] : TA(0);
     }
-    mine[r][base + (t ^ r)] = v;
+    TA* rho = reinterpret_cast<TA*>(prow);
+    const float* ri = src.r + (b * n + (act ? t : 0)) * 3;
+    const TA r0 = (TA)ri[0], r1 = (TA)ri[1], r2 = (TA)ri[2];
+    const int NO = sh.D * n, oa = act ? oc : 0;
+#pragma unroll 1
+    for (int I = 0; I < sh.I; ++I) {
+      const TA dx = r0 - (TA)src.R[I * 3 + 0], dy = r1 - (TA)src.R[I * 3 + 1], dz = r2 - (TA)src.R[I * 3 + 2];
+      rho[t] = dsqrt(dx * dx + dy * dy + dz * dz);
+      const TA ku = src.kappa[I * NO + oa], wu = src.wenv[I * NO + oa];
+      const TA kd = src.kappa[(sh.I + I) * NO + oa], wd = src.wenv[(sh.I + I) * NO + oa];
+      wave_lds_order();
+      unroll_seq<NMAX / 4>([&](auto r4) {  // four rows at a time: their exponentials overlap
+        if (r4.value * 4 < n) {
+#pragma unroll
+          for (int r = r4.value * 4; r < r4.value * 4 + 4; ++r) {
+            const TA k = r < sh.u ? ku : kd;
+            const TA e = (r < sh.u ? wu : wd) * dexp(-k * rho[r]);
+            env[r] += e;
+          }
+        }
+      });
+      wave_lds_order();
+    }
+#pragma unroll
+    for (int r = 0; r < NMAX; ++r)
+      if (r < n) mine[r][base + (t ^ r)] = act ? env[r] * o[r] : TA(0);
   }
-  __syncthreads();  // every wavefront runs the same iterations: no early exit above
+  wave_lds_order();
   double a[NMAX];  // row t
 #pragma unroll
   for (int c = 0; c < NMAX; ++c) a[c] = (act && c < n) ? (double)mine[t][base + (c ^ t)] : 0.0;
-  bool used = !act;  // padding rows never pivot
-  int step_of = 0;   // elimination step at which this row became the pivot row
+  bool used = !act;                                      // padding rows never pivot
+  unsigned left = n < 32 ? (1u << n) - 1u : 0xffffffffu;  // rows of the group that have not been the pivot row
+  int inv = 0;                                           // inversions of the pivot order
   bool sing = false;
   double mydiag = 1.0;  // lane p: U[p][p]
-#pragma unroll
-  for (int p = 0; p < NMAX; ++p) {
+  unroll_seq<NMAX>([&](auto step) {
+    constexpr int p = step.value;
     if (p < n) {
       const double ap = fabs(a[p]);
-      double v = (used || !(ap >= 0.0)) ? -1.0 : ap;
-      int idx = t;
-#pragma unroll
-      for (int o = NMAX / 2; o > 0; o >>= 1) {
-        const double v2 = __shfl_xor(v, o, NMAX);
-        const int i2 = __shfl_xor(idx, o, NMAX);
-        if (v2 > v || (v2 == v && i2 < idx)) {
-          v = v2;
-          idx = i2;
-        }
-      }
-      if (!(v > 0.0)) sing = true;
-      const double pivot = __shfl(a[p], base + idx, 64);
-      if (t == p) mydiag = pivot;
+      const double v = (used || !(ap >= 0.0)) ? -1.0 : ap;
+      const double vm = group_max<NMAX>(v);
+      const unsigned long long hit = __ballot(v == vm);
+      const int idx = __ffs((unsigned)(hit >> base)) - 1;
+      if (!(vm > 0.0)) sing = true;
       if (t == idx) {
         used = true;
-        step_of = p;
-      }
-      const double rp = 1.0 / pivot;
-      const double l = a[p] * rp;
 #pragma unroll
-      for (int c = p + 1; c < NMAX; ++c) {
-        if (c < n) {
-          const double pc = __shfl(a[c], base + idx, 64);
-          if (!used) a[c] -= l * pc;
+        for (int c = p & ~1; c < NMAX; c += 2) {
+          const double2 q = {a[c], a[c + 1]};
+          *reinterpret_cast<double2*>(prow + c) = q;
         }
       }
+      inv += __popc(left & ((1u << idx) - 1u));
+      left &= ~(1u << idx);
+      wave_lds_order();
+      const double pivot = prow[p];
+      if (t == p) mydiag = pivot;
+      const double rp = 1.0 / pivot;
+      const double l = a[p] * rp;
+      // BT columns a batch: loads of a batch together, no work past the last batch that holds a column
+      unroll_seq<(NMAX - ((p + 1) & ~(BT - 1))) / BT>([&](auto batch) {
+        constexpr int c0 = ((p + 1) & ~(BT - 1)) + batch.value * BT;
+        if (c0 < n) {
+          double pc[BT];
+#pragma unroll
+          for (int c = 0; c < BT; c += 2) {
+            if (c0 + c + 1 > p) {
+              const double2 q = *reinterpret_cast<const double2*>(prow + c0 + c);
+              pc[c] = q.x;
+              pc[c + 1] = q.y;
+            }
+          }
+#pragma unroll
+          for (int c = 0; c < BT; ++c)
+            if (c0 + c > p) a[c0 + c] -= l * pc[c];
+        }
+      });
+      wave_lds_order();
     }
-  }
-  // parity of the pivot order: inversions of step_of over the rows
-  int inv = 0;
-#pragma unroll
-  for (int c = 0; c < NMAX; ++c) {
-    const int sc = __shfl(step_of, base + c, 64);
-    if (act && c > t && c < n && sc < step_of) ++inv;
-  }
+  });
   double lg = act ? log(fabs(mydiag)) : 0.0;
-  int neg = (act && mydiag < 0.0) ? 1 : 0;
-  double umax = act ? fabs(mydiag) : 0.0, umin = act ? fabs(mydiag) : 1e300;
+  const double umax = group_max<NMAX>(act ? fabs(mydiag) : 0.0);
+  const double umin = -group_max<NMAX>(act ? -fabs(mydiag) : -1e300);
 #pragma unroll
-  for (int o = NMAX / 2; o > 0; o >>= 1) {
-    lg += __shfl_xor(lg, o, NMAX);
-    neg += __shfl_xor(neg, o, NMAX);
-    inv += __shfl_xor(inv, o, NMAX);
-    umax = fmax(umax, __shfl_xor(umax, o, NMAX));
-    umin = fmin(umin, __shfl_xor(umin, o, NMAX));
-  }
+  for (int o = NMAX / 2; o > 0; o >>= 1) lg += __shfl_xor(lg, o, NMAX);
+  const unsigned long long negs = __ballot(act && mydiag < 0.0);
+  const unsigned gm = NMAX < 32 ? (1u << (NMAX & 31)) - 1u : 0xffffffffu;
+  const int neg = __popc((unsigned)(negs >> base) & gm);
   const double ldv = sing ? -INFINITY : lg, sdv = sing ? 0.0 : (((neg + inv) & 1) ? -1.0 : 1.0);
   const float dcv = (float)(umax / umin);
   if (t == 0 && valid) {
@@ -899,9 +961,10 @@ __global__ __launch_bounds__(256) void k_det_value(OrbSrc<TA> src, double* __res
   if (co.fuse) {
     // the workgroup's 256 / NMAX matrices are whole walkers (D divides that number): combine them here
     constexpr int MPW = 256 / NMAX;
+    // (one wavefront: a lane per matrix forms its term, a lane per walker sums)
     __shared__ double c_ld[MPW], c_sd[MPW];
     __shared__ float c_dc[MPW];
-    const int mi = (int)(threadIdx.x >> 6) * G + g;
+    const int mi = wv * G + g;
     if (t == 0) {
       c_ld[mi] = ldv;
       c_sd[mi] = sdv;
@@ -909,12 +972,21 @@ __global__ __launch_bounds__(256) void k_det_value(OrbSrc<TA> src, double* __res
     }
     __syncthreads();
     const int D = sh.D, wpw = MPW / D;
-    if ((int)threadIdx.x < wpw) {
-      const long b = (long)blockIdx.x * wpw + threadIdx.x;
-      const int o = (int)threadIdx.x * D;
-      if (b < sh.B)
-        combine_value_walker(c_ld + o, c_sd + o, c_dc + o, D, co.cond_thr, b, co.out_lp, co.out_phase, co.out_flags,
-                             co.out_kappa);
+    if (wv == 0) {
+      const int w = lane / D, o = w * D;  // lanes at or past MPW: no matrix
+      double m = 0.0;
+      if (lane < MPW) {
+        m = walker_max(c_ld + o, D);
+        c_sd[lane] *= exp(c_ld[lane] - m);
+      }
+      wave_lds_order();
+      m = __shfl(m, lane < wpw ? lane * D : 0, 64);
+      const long b = (long)blockIdx.x * wpw + lane;
+      if (lane < wpw && b < sh.B) {
+        const double* e = c_sd + lane * D;
+        combine_value_walker([&](int d) { return e[d]; }, m, c_dc + lane * D, D, co.cond_thr, b, co.out_lp,
+                             co.out_phase, co.out_flags, co.out_kappa);
+      }
     }
   }
 }
@@ -1050,7 +1122,10 @@ __global__ void k_combine_value(const double* __restrict__ ld, const double* __r
   const long b = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= sh.B) return;
   const int D = sh.D;
-  combine_value_walker(ld + b * D, sd + b * D, dcond + b * D, D, cond_thr, b, out_lp, out_phase, out_flags, out_kappa);
+  const double *l = ld + b * D, *sg = sd + b * D;
+  const double m = walker_max(l, D);
+  combine_value_walker([&](int d) { return sg[d] * exp(l[d] - m); }, m, dcond + b * D, D, cond_thr, b, out_lp, out_phase,
+                       out_flags, out_kappa);
 }
 
 // Laplacian pass: one wavefront per walker; the formulas above.  Lanes split the 3n gradient components
