@@ -624,10 +624,11 @@ struct Proposal {
 
 // One pass of the wavefunction over B walkers with C channels (C == 1: value; C == 3n+2: Laplacian).
 // `ws` is the pass's scratch (layout_pass); out_kappa (may be null) receives the per-walker conditioning.
+// keep_layers: every layer's activations are left in ws.X (a value pass that the gradient continues).
 template <typename T>
 dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, const float* R, const float* Z, int C,
                    hipStream_t s, float* out_lp, float* out_phase, float* out_eloc, uint32_t* out_flags,
-                   float* out_kappa, float cond_thr, const Proposal* prop = nullptr) {
+                   float* out_kappa, float cond_thr, const Proposal* prop = nullptr, bool keep_layers = false) {
   constexpr bool DBL = sizeof(T) == 8;
   Weights& W = DBL ? m->wd : m->wf;
   const int Cp = rows_per_electron(C);
@@ -652,6 +653,29 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
   const long vstride = B * Cp * (long)m->W1;
   const long wm_layer = B * (long)m->n * m->n * (C > 1 ? 5 : 1) * 32;
   int amax_np = 0;  // maxima per electron of the last split layer, in ws.amax[l & 1]
+  // Value channel of layers l .. (all that follow, or l alone in the dpe4 model, whose next layer needs the
+  // convolution first) in one launch; returns how many it took (0: none).
+  auto value_layers = [&](int l, int vs, int stride, bool keep) -> int {
+    if constexpr (DBL) {
+      return 0;
+    } else {
+      const int cnt = m->dpe4 ? 1 : m->L - l;
+      if (cnt > DW_MAX_LAYERS) return 0;
+      ValueNetLayer a[DW_MAX_LAYERS];
+      for (int k = 0; k < cnt; ++k) {
+        const int j = l + k;
+        const bool fin = j == m->L - 1;
+        const long ldo = fin ? m->W1 : m->Kx[j + 1];
+        int parts = vs;
+        while (parts > 1 && m->Km[j] % (16 * parts) != 0) parts >>= 1;
+        a[k] = ValueNetLayer{X[j], (long)stride * m->Kx[j], W.WmainL[j].p, W.WmuL[j].p, W.bias[j].template as<float>(),
+                             fin ? ws.H : (keep || k + 1 == cnt ? X[j + 1] : nullptr), stride * ldo, m->Kx[j], m->Km[j],
+                             m->Kh[j], m->Kt0[j], parts};
+      }
+      return value_net(a, cnt, l + cnt == m->L ? 1 : 0, (int)B, m->n, m->u, m->W1, s) ? cnt : 0;
+    }
+  };
+  int value_done = 0;  // layers whose value channel is complete
   for (int l = 0; l < m->L; ++l) {
     if (m->dpe4) {  // e_ee of this iteration: hm = tanh rule of (X_l[:, h] W_map), then the convolution
       GemmEpiT<T> eh;
@@ -662,7 +686,7 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
       launch_dpe4_conv<T>(ws.WM + l * wm_layer, ws.HM, X[l], m->Kx[l], m->Kt0[l], sh, s);
     }
     // value pass: split K of the per-walker spin-mean GEMM so that it fills the chip (its M is only B)
-    int vs = 1;
+    int vs = 1, vs0 = 1;
     if (!DBL && C == 1 && m->prec == GEMM_F32) {
       if (m->tune.fwd_mu_split > 0) {
         vs = m->tune.fwd_mu_split;
@@ -671,6 +695,7 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
         const long tiles64 = ((B * Cp + 63) / 64) * ((m->W1 + 63) / 64);
         vs = tiles64 >= 512 ? 1 : (tiles64 >= 128 ? 2 : 4);
       }
+      vs0 = vs;
       while (vs > 1 && m->Km[l] % (16 * vs) != 0) vs >>= 1;  // each K slice a multiple of the 16-wide K tile
     }
     const bool last = (l == m->L - 1);
@@ -681,6 +706,12 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
           value_layer(X[l], m->Kx[l], m->Kx[l], m->Kh[l], W.WmainL[l].p, W.WmuL[l].p, m->Km[l], W.bias[l].as<float>(),
                       vs, outp, ldo, last ? 1 : 0, (int)B, m->n, m->u, m->W1, s))
         continue;
+      if (C == 1 && m->prec == GEMM_F32 && m->tune.fwd_main_tile < 0) {
+        if (const int took = value_layers(l, vs0, 1, keep_layers)) {
+          l += took - 1;
+          continue;
+        }
+      }
     }
     if constexpr (!DBL) {
       if (split) {
@@ -688,8 +719,12 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
         // arithmetic, then the derivative channels of the layer
         split_mean(X[l], m->Kx[l], m->Kh[l], W.WmuS[l].p, m->Km[l], ws.V, m->W1, sh, s);
         const int ldx = Cp * m->Kx[l], Km = m->Km[l];
-        if (!value_layer(X[l], ldx, m->Kx[l], m->Kh[l], W.WmainL[l].p, W.WmuL[l].p, Km, W.bias[l].as<float>(), 1, outp,
-                         (long)Cp * ldo, last ? 1 : 0, (int)B, m->n, m->u, m->W1, s)) {
+        if (value_done <= l &&
+            value_layer(X[l], ldx, m->Kx[l], m->Kh[l], W.WmainL[l].p, W.WmuL[l].p, Km, W.bias[l].as<float>(), 1, outp,
+                        (long)Cp * ldo, last ? 1 : 0, (int)B, m->n, m->u, m->W1, s))
+          value_done = l + 1;
+        if (value_done <= l) value_done = l + value_layers(l, 1, Cp, true);
+        if (value_done <= l) {
           Shape s1 = sh;
           s1.C = 1;
           s1.Cp = 1;
@@ -920,7 +955,7 @@ dw_status run_grad(dw_model* m, const float* r, long B, const float* R, const fl
   PassBufs<T> pb;
   dw_status st = pass_scratch(m, B, 1, &pb);
   if (st) return st;
-  st = run_pass<T>(m, pb, r, B, R, Z, 1, s, out_lp, nullptr, nullptr, nullptr, nullptr, 0.f);
+  st = run_pass<T>(m, pb, r, B, R, Z, 1, s, out_lp, nullptr, nullptr, nullptr, nullptr, 0.f, nullptr, true);
   if (st) return st;
   HIP_TRY(m->grad_arena.ensure(layout_grad<T>(m, B, nullptr, nullptr)));
   GradBufs<T> g;

@@ -81,12 +81,26 @@ int split_lap(const float* X, int ldx, const void* P, int shift, int K, const fl
 // One-launch value layers and orbital GEMMs for small batches (value_layer.hip), bit-equal to the separate kernels.
 // Weights in lane order (launch_lane_pack: Bt [rows >= cols, K] into lane_pack_bytes(cols, K) bytes, K a multiple of
 // 32).  value_layer: out = tanh(X W + V), V = the vs K parts of (spin means of the first Kh columns) W_mu plus bias,
-// added in order; rows of X ldx apart, of out ldo apart.  Both return false, launching nothing, where the batch is too
+// added in order; rows of X ldx apart, of out ldo apart.  All return false, launching nothing, where the batch is too
 // large to gain (the rules stand beside them).
 size_t lane_pack_bytes(int cols, int K);
 void launch_lane_pack(const float* Bt, int ldb, int cols, int K, void* out, hipStream_t s);
 bool value_layer(const float* X, long ldx, int K, int Kh, const void* W, const void* Wmu, int Km, const float* bias,
                  int vs, float* out, long ldo, int permute, int B, int n, int u, int W1, hipStream_t s);
+// value_net: L consecutive value layers in one launch (W1 = 256; layers after the first take their first Kt = 256
+// columns from the one before and the rest from X); out may be null for all but the last layer, the only one that
+// `permute` applies to.
+struct ValueNetLayer {
+  const float* X;
+  long ldx;
+  const void *W, *Wmu;
+  const float* bias;
+  float* out;
+  long ldo;
+  int K, Km, Kh, Kt, vs;
+};
+constexpr int DW_MAX_LAYERS = 8;
+bool value_net(const ValueNetLayer* layers, int L, int permute, int B, int n, int u, int W1, hipStream_t s);
 bool value_orbitals(const float* H, long ldh, int K, const void* W_up, const void* W_dn, float* O, long ldo,
                     int up_rows, int dn_rows, int N, hipStream_t s);
 

@@ -9,9 +9,11 @@
 //
 // Small batches were bound by latency: three launches a layer, 20 short K slices with two barriers each and a load
 // to wait for.  256 LiH walkers (1,024 rows x 320 x 256): 30 us a layer in three launches, 10 us here; both orbital
-// GEMMs 17 us in two launches, 4.2 us in one.
+// GEMMs 17 us in two launches, 4.2 us in one.  Larger batches take all layers in one launch, whole walkers and all
+// columns per workgroup (k_value_net below).
 #include "common.h"
 #include "kernels.h"
+#include <algorithm>
 
 namespace dwmi {
 
@@ -282,6 +284,236 @@ __global__ __launch_bounds__(256) void k_value_orb(const float* __restrict__ H, 
         if (r < M) O[(base + r) * ldo + c] = acc[i][e];
       }
   }
+}
+
+// ------------------------------------------------------------------------------------------------
+// Whole layers of 256 columns for rw walkers (rw n <= 16 RB rows) per workgroup of 16 waves, wave w owning columns
+// [16 w, 16 w + 16) of the per-electron GEMM and of the mean product.  The activations stay in LDS from layer to
+// layer; the mean product's slices run between the per-electron GEMM's, so both weights stream from L2 at an even rate
+// two slices ahead; a layer has three barriers.
+// What bounds it: FP32 MFMA (28,672 rows x 320 x 256 with 2,048 x 512 x 256: 37 us at the matrix rate), then the phases
+// without products (means, tanh, barriers: about 12 us).  28,672 rows (2,048 N2 walkers), per layer of three: 72 us in
+// three launches (means, mean product, per-electron GEMM), 55 here.
+// ------------------------------------------------------------------------------------------------
+struct NetLayer {
+  const float* X;  // row (b n + i): [h (Kt, filled here for l > 0) | pair columns]
+  long ldx;
+  const v4f *W, *Wmu;
+  const float* bias;
+  float* out;  // may be null for l < L - 1
+  long ldo;
+  int K, Km, Kh, vs;
+  FastDiv fm;  // by Km / 4
+};
+struct ValueNet {
+  NetLayer l[DW_MAX_LAYERS];
+  int L, permute, B, n, u, rw, mu_off;  // mu_off: floats of the row area
+  FastDiv fq, fn;                       // by K / 4 of the first layer, n
+};
+
+template <int RB>
+__global__ __launch_bounds__(1024) void k_value_net(ValueNet p) {
+  extern __shared__ __align__(16) float smem[];
+  constexpr int NT = 1024, TL = (RB * 16 * 16 + NT - 1) / NT;
+  v4f* const As = (v4f*)smem;
+  float* const Ms = smem + p.mu_off;  // spin means, rw x (Km + 4); after the products each wave's V, rw x 16
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, g = lane >> 4, cl = lane & 15;
+  const int b0 = blockIdx.x * p.rw;
+  const int rw = min(p.rw, p.B - b0), n = p.n, rows = rw * n, dn = n - p.u;
+  const int c = wv * 16 + cl;
+  {
+    const float* Xb = p.l[0].X + (long)b0 * n * p.l[0].ldx;
+    const long ldx = p.l[0].ldx;
+    stage_rows<RB, NT>(As, p.l[0].K >> 2, p.fq, [&](int r) { return Xb + min(r, rows - 1) * ldx; });
+  }
+#pragma unroll 1
+  for (int l = 0; l < p.L; ++l) {
+    const NetLayer& q = p.l[l];
+    const int S = q.K >> 4, SV = q.Km >> 4, Sp = SV / q.vs, pitch = q.Km + 4;
+    const v4f* bp = q.W + (long)wv * S * 64 + lane;
+    const v4f* mp = q.Wmu + (long)wv * SV * 64 + lane;
+    v4f b0v = bp[0], b1v = bp[64 * min(1, S - 1)];
+    v4f m0 = mp[0], m1 = mp[64 * min(1, SV - 1)];
+    // the next layer's pair columns, written to LDS when this layer's products are done
+    v4f tl[TL];
+    const bool more = l + 1 < p.L;
+    if (more) {
+      const NetLayer& nx = p.l[l + 1];
+      const int tq = (nx.K - 256) >> 2;  // quads of pair columns (at most 16)
+#pragma unroll
+      for (int t = 0; t < TL; ++t) {
+        const int idx = tid + t * NT, row = idx >> 4, quad = idx & 15;
+        if (quad < tq && row < RB * 16)
+          tl[t] = *(const v4f*)(nx.X + ((long)b0 * n + min(row, rows - 1)) * nx.ldx + 256 + quad * 4);
+      }
+    }
+    const float bias = q.bias[c];
+    __syncthreads();  // rows of this layer complete
+    const int Kh4 = q.Kh >> 2, Km4 = q.Km >> 2;
+    for (int t = tid; t < rw * Km4; t += NT) {  // spin means: electrons in order, then 1 / n_s
+      const int w = t / q.fm, f = t - w * Km4;
+      v4f v = {0.f, 0.f, 0.f, 0.f};
+      if (f < 2 * Kh4) {
+        const int sp = f >= Kh4 ? 1 : 0;
+        const int quad = f - sp * Kh4, i0 = sp ? p.u : 0, i1 = sp ? n : p.u;
+#pragma unroll 4
+        for (int i = i0; i < i1; ++i) {
+          const v4f x = As[slot<RB>(w * n + i, quad)];
+          v[0] += x[0];
+          v[1] += x[1];
+          v[2] += x[2];
+          v[3] += x[3];
+        }
+        const float inv = 1.f / (float)(i1 - i0);
+        v[0] *= inv;
+        v[1] *= inv;
+        v[2] *= inv;
+        v[3] *= inv;
+      }
+      *(v4f*)(Ms + w * pitch + 4 * f) = v;
+    }
+    __syncthreads();
+    v4f acc[RB], va = {0.f, 0.f, 0.f, 0.f}, vsum = va;
+#pragma unroll
+    for (int i = 0; i < RB; ++i) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
+    const float* ap = Ms + min(cl, rw - 1) * pitch + 4 * g;
+    int j = 0, jp = 0;  // mean product: next slice, its number inside its part
+    bool first = true;
+    auto mean_slice = [&](const v4f& b) {
+      const v4f a = *(const v4f*)(ap + 16 * j);
+#pragma unroll
+      for (int st = 0; st < 4; ++st) va = __builtin_amdgcn_mfma_f32_16x16x4f32(a[st], b[st], va, 0, 0, 0);
+      ++j;
+      if (++jp == Sp) {  // uniform: parts added in order, the bias on the first
+#pragma unroll
+        for (int e = 0; e < 4; ++e) vsum[e] = first ? va[e] + bias : vsum[e] + va[e];
+        va = v4f{0.f, 0.f, 0.f, 0.f};
+        first = false;
+        jp = 0;
+      }
+    };
+#pragma unroll 1
+    for (int s = 0; s < S; ++s) {
+      v4f a[RB];
+#pragma unroll
+      for (int i = 0; i < RB; ++i) a[i] = As[((s * RB + i) * 4 + g) * 16 + ((cl + 4 * s + g) & 15)];
+      const v4f bc = b0v;
+      b0v = b1v;
+      b1v = bp[64 * min(s + 2, S - 1)];
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
+#pragma unroll
+        for (int i = 0; i < RB; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][st], bc[st], acc[i], 0, 0, 0);
+      if (j < SV) {  // two slices of the mean product (uniform)
+        const v4f c0 = m0, c1 = m1;
+        m0 = mp[64 * min(j + 2, SV - 1)];
+        m1 = mp[64 * min(j + 3, SV - 1)];
+        mean_slice(c0);
+        if (j < SV) mean_slice(c1);
+      }
+    }
+    while (j < SV) {
+      const v4f c0 = m0;
+      m0 = m1;
+      m1 = mp[64 * min(j + 2, SV - 1)];
+      mean_slice(c0);
+    }
+    __syncthreads();  // every wave is done with the rows and the means
+    float* const Vs = Ms + wv * rw * 16;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (4 * g + e < rw) Vs[(4 * g + e) * 16 + cl] = vsum[e];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    float* const out = q.out;
+    const bool perm = p.permute && !more;
+    int g4 = 4 * g;  // opaque: the outputs' addresses are formed here, not kept in registers over the layers
+    asm volatile("" : "+v"(g4));
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = i * 16 + g4 + e;
+        const int w = min(r / p.fn, rw - 1);
+        const float y = tanh_fast(acc[i][e] + Vs[w * 16 + cl]);
+        if (more) smem[slot<RB>(r, c >> 2) * 4 + (c & 3)] = y;
+        if (out && r < rows) {
+          const int el = r - w * n;
+          const long bb = b0 + w;
+          long orow = bb * n + el;
+          if (perm) orow = (el < p.u) ? bb * p.u + el : (long)p.B * p.u + bb * dn + (el - p.u);
+          out[orow * q.ldo + c] = y;
+        }
+      }
+    if (more) {
+      const int tq = (p.l[l + 1].K - 256) >> 2;
+#pragma unroll
+      for (int t = 0; t < TL; ++t) {
+        const int idx = tid + t * NT, row = idx >> 4, quad = idx & 15;
+        if (quad < tq && row < RB * 16) As[slot<RB>(row, 64 + quad)] = tl[t];
+      }
+    }
+  }
+}
+
+template <int RB>
+static void launch_net(const ValueNet& p, size_t shm, hipStream_t s) {
+  if (shm > 65536)
+    (void)hipFuncSetAttribute((const void*)k_value_net<RB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
+  hipLaunchKernelGGL((k_value_net<RB>), dim3((unsigned)((p.B + p.rw - 1) / p.rw)), dim3(1024), shm, s, p);
+}
+
+// A layer of RB row blocks takes about 5.5 RB + 15 us a round of 256 workgroups, at any batch; the separate kernels about
+// 18 + 0.0025 us a row.  Measured per layer of three, separate / here: 14 electrons 37.6 / 27 (512 walkers), 54 / 38
+// (1,000), 72 / 55 (2,048), 121 / 97 (3,000); 4 electrons 101 / 75 (8,192); 42 electrons 38 / 31 (192), 66 / 50 (512);
+// 60 electrons 47 / 37 (200) but 105 / 111 (600: one walker a workgroup, whose mean product fills one MFMA row of 16).
+bool value_net(const ValueNetLayer* layers, int L, int permute, int B, int n, int u, int W1, hipStream_t s) {
+  if (W1 != 256 || L < 1 || L > DW_MAX_LAYERS || B < 1) return false;
+  ValueNet p{};
+  int Kmax = 0, Kmm = 256;
+  for (int l = 0; l < L; ++l) {
+    const ValueNetLayer& a = layers[l];
+    if (a.K % 16 || a.K < 16 || a.K > 16 * MAXS || a.Km % (16 * a.vs) || a.Km < 16 || a.Kh % 4 || a.ldx % 4) return false;
+    if (l > 0 && (a.Kh != 256 || a.Kt != 256 || a.K < 256 || a.K > 320)) return false;
+    Kmax = a.K > Kmax ? a.K : Kmax;
+    Kmm = a.Km > Kmm ? a.Km : Kmm;
+    p.l[l] = NetLayer{a.X, a.ldx, (const v4f*)a.W, (const v4f*)a.Wmu, a.bias, a.out, a.ldo, a.K, a.Km, a.Kh, a.vs,
+                      fast_div(a.Km / 4)};
+  }
+  p.L = L;
+  p.permute = permute;
+  p.B = B;
+  p.n = n;
+  p.u = u;
+  p.fq = fast_div(layers[0].K / 4);
+  p.fn = fast_div(n);
+  double cost = 18.0 + 0.0025 * (double)B * n;
+  int best = 0, best_rw = 0;
+  for (int RB = 1; RB <= 7; ++RB) {
+    const int rw = std::min(std::min(16 * RB / n, 16), B);
+    if (rw < 1 || ((size_t)16 * RB * Kmax + (size_t)rw * (Kmm + 4)) * 4 > 160 * 1024) continue;
+    const double t = (((B + rw - 1) / rw + 255) / 256) * (5.5 * RB + 15.0);
+    if (t < cost) {
+      cost = t;
+      best = RB;
+      best_rw = rw;
+    }
+  }
+  if (!best) return false;
+  p.rw = best_rw;
+  p.mu_off = 16 * best * Kmax;
+  const size_t shm = ((size_t)p.mu_off + (size_t)p.rw * (Kmm + 4)) * 4;
+  switch (best) {
+    case 1: launch_net<1>(p, shm, s); break;
+    case 2: launch_net<2>(p, shm, s); break;
+    case 3: launch_net<3>(p, shm, s); break;
+    case 4: launch_net<4>(p, shm, s); break;
+    case 5: launch_net<5>(p, shm, s); break;
+    case 6: launch_net<6>(p, shm, s); break;
+    default: launch_net<7>(p, shm, s); break;
+  }
+  return true;
 }
 
 template <int RB>
