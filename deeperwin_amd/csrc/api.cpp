@@ -678,11 +678,17 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
   int value_done = 0;  // layers whose value channel is complete
   for (int l = 0; l < m->L; ++l) {
     if (m->dpe4) {  // e_ee of this iteration: hm = tanh rule of (X_l[:, h] W_map), then the convolution
-      GemmEpiT<T> eh;
-      eh.tile = 0;  // 64 x 64 tiles: the output is only 32 wide
-      gemm_t(m, X[l], m->Kx[l], W.WhmT[l].as<T>(), W.WhmT_hi[l], W.WhmT_lo[l], m->Kt0[l], ws.HM, 32, rows, 32,
-             m->Kt0[l], eh, s);
-      launch_dpe4_tanh<T>(ws.HM, W.bhm[l].as<T>(), sh, s);
+      bool mapped = false;
+      if constexpr (!DBL)
+        mapped = m->prec == GEMM_F32 && launch_dpe4_hmap(X[l], m->Kx[l], W.WhmT[l].template as<float>(), m->Kt0[l],
+                                                         W.bhm[l].template as<float>(), ws.HM, sh, s);
+      if (!mapped) {
+        GemmEpiT<T> eh;
+        eh.tile = 0;  // 64 x 64 tiles: the output is only 32 wide
+        gemm_t(m, X[l], m->Kx[l], W.WhmT[l].as<T>(), W.WhmT_hi[l], W.WhmT_lo[l], m->Kt0[l], ws.HM, 32, rows, 32,
+               m->Kt0[l], eh, s);
+        launch_dpe4_tanh<T>(ws.HM, W.bhm[l].as<T>(), sh, s);
+      }
       launch_dpe4_conv<T>(ws.WM + l * wm_layer, ws.HM, X[l], m->Kx[l], m->Kt0[l], sh, s);
     }
     // value pass: split K of the per-walker spin-mean GEMM so that it fills the chip (its M is only B)

@@ -200,6 +200,10 @@ void launch_dpe4_elion(const float* r, const float* R, const float* Z, const T* 
                        const T* bhim, const T* table, int n_types, int z_min, T* him, T* const* X, const int* Kx,
                        const int* tail, const Shape& sh, hipStream_t s);
 // hm [B n Cp][32] = tanh rule of (hm + bias) over each electron's channel rows, in place.
+// h_map with its tanh rule in one launch (FP32; Wt [32, K], rows = output columns); false, launching nothing, for shapes
+// it does not take (K a multiple of 16 up to 512, Cp <= 192).
+bool launch_dpe4_hmap(const float* X, int ldx, const float* Wt, int K, const float* bias, float* hm, const Shape& sh,
+                      hipStream_t s);
 template <typename T>
 void launch_dpe4_tanh(T* hm, const T* bias, const Shape& sh, hipStream_t s);
 // e_ee of one iteration from wm (that iteration's slice) and hm into X columns col0 .. col0 + 31.
