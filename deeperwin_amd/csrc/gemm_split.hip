@@ -592,14 +592,16 @@ int split_lap(const float* X, int ldx, const void* P, int shift, int K, const fl
 // A workgroup forms the means of 48 rows x 128 k at a time and splits them straight into LDS (37 KB: four workgroups
 // per CU, whose load and MFMA phases overlap); the weights' parts come from L2.  Bound by the read of X's h columns
 // (1.41 GB for 2048 walkers of 14 electrons: 364 us = 3.9 TB/s against 471 us with FP32 MFMA; 26 electrons, 1024
-// walkers: 575 -> 461 us; 256 LiH walkers: 67 -> 28 us with 64 columns per workgroup).
+// walkers: 575 -> 461 us; 256 LiH walkers: 67 -> 28 us with 64 columns per workgroup).  NP = 2 keeps the first two parts
+// and three products, the BF16x3 form's arithmetic (1,000 walkers of 14: 206 us a layer in two launches, 159 + 15 for the
+// value rows here).
 // ------------------------------------------------------------------------------------------------
-template <int NQ>
+template <int NQ, int NP>
 __global__ __launch_bounds__(256) void k_split_mean(const float* __restrict__ X, int Kx, int Kh,
                                                     const uint4* __restrict__ P, int ncb, int Km,
                                                     float* __restrict__ V, int ldv, Shape sh, int tilesN, int total) {
   constexpr int RB = 3, CS = 4;  // row blocks, 32-wide slices per chunk
-  __shared__ uint4 lds[CS][3][RB][64];
+  __shared__ uint4 lds[CS][NP][RB][64];
   const int tile = tile_of(blockIdx.x, total);
   if (tile >= total) return;  // uniform over the workgroup, before any barrier
   const long rows = (long)sh.B * sh.Cp, r0 = (long)(tile / tilesN) * (16 * RB);
@@ -645,25 +647,27 @@ __global__ __launch_bounds__(256) void k_split_mean(const float* __restrict__ X,
       split4(v, p);
       const int quad = qd & 7;
 #pragma unroll
-      for (int m = 0; m < 3; ++m)
+      for (int m = 0; m < NP; ++m)
         *((uint2*)&lds[qd >> 3][m][rr >> 4][(quad >> 1) * 16 + (rr & 15)] + (quad & 1)) = p[m];
     }
     __syncthreads();
     for (int s = 0; s < ns; ++s) {
-      v8s b[NQ][3];
+      v8s b[NQ][NP];
 #pragma unroll
       for (int q = 0; q < NQ; ++q)
 #pragma unroll
-        for (int m = 0; m < 3; ++m)
+        for (int m = 0; m < NP; ++m)
           b[q][m] = *(const v8s*)&P[((long)(((kc >> 5) + s) * ncb + cb0 + q) * 3 + m) * 64 + lane];
 #pragma unroll
       for (int i = 0; i < RB; ++i) {
-        v8s a[3];
+        v8s a[NP];
 #pragma unroll
-        for (int m = 0; m < 3; ++m) a[m] = *(const v8s*)&lds[s][m][i][lane];
-        DW_SPLIT_MFMA(2, 0)
-        DW_SPLIT_MFMA(0, 2)
-        DW_SPLIT_MFMA(1, 1)
+        for (int m = 0; m < NP; ++m) a[m] = *(const v8s*)&lds[s][m][i][lane];
+        if constexpr (NP == 3) {
+          DW_SPLIT_MFMA(2, 0)
+          DW_SPLIT_MFMA(0, 2)
+          DW_SPLIT_MFMA(1, 1)
+        }
         DW_SPLIT_MFMA(1, 0)
         DW_SPLIT_MFMA(0, 1)
         DW_SPLIT_MFMA(0, 0)
@@ -681,20 +685,29 @@ __global__ __launch_bounds__(256) void k_split_mean(const float* __restrict__ X,
       }
 }
 
-void split_mean(const float* X, int Kx, int Kh, const void* P, int Km, float* V, int ldv, const Shape& sh,
-                hipStream_t s) {
+template <int NP>
+static void launch_mean(const float* X, int Kx, int Kh, const void* P, int Km, float* V, int ldv, const Shape& sh,
+                        hipStream_t s) {
   const int ncb = dw_pad(sh.W1, 256) / 16;
   const long tilesM = ((long)sh.B * sh.Cp + 47) / 48;
   // 256 columns (X read once) where that gives two workgroups to every CU
   if (sh.W1 % 256 == 0 && tilesM * (sh.W1 / 256) >= 512) {
     const int tilesN = sh.W1 / 256, total = (int)(tilesM * tilesN);
-    hipLaunchKernelGGL((k_split_mean<4>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh, (const uint4*)P, ncb,
-                       Km, V, ldv, sh, tilesN, total);
+    hipLaunchKernelGGL((k_split_mean<4, NP>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh, (const uint4*)P,
+                       ncb, Km, V, ldv, sh, tilesN, total);
   } else {
     const int tilesN = sh.W1 / 64, total = (int)(tilesM * tilesN);
-    hipLaunchKernelGGL((k_split_mean<1>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh, (const uint4*)P, ncb,
-                       Km, V, ldv, sh, tilesN, total);
+    hipLaunchKernelGGL((k_split_mean<1, NP>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh, (const uint4*)P,
+                       ncb, Km, V, ldv, sh, tilesN, total);
   }
+}
+
+void split_mean(const float* X, int Kx, int Kh, const void* P, int Km, int parts, float* V, int ldv, const Shape& sh,
+                hipStream_t s) {
+  if (parts == 3)
+    launch_mean<3>(X, Kx, Kh, P, Km, V, ldv, sh, s);
+  else
+    launch_mean<2>(X, Kx, Kh, P, Km, V, ldv, sh, s);
 }
 
 }  // namespace dwmi

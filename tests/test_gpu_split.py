@@ -87,3 +87,32 @@ def test_split_operands_of_any_magnitude(cuda, scale):
         torch.cuda.synchronize()
         out.append(e.cpu().numpy())
     assert np.all(np.abs(out[1] - out[0]) <= (1 + np.abs(out[0])) * (1e-4 + 4 * U32 * kappa))
+
+
+@pytest.mark.parametrize("n,B", [(3, 5), (4, 700), (14, 33), (14, 601), (26, 18), (45, 4)])
+def test_bf16x3_mean_product_with_the_means_formed_in_it(cuda, n, B):
+    """BF16x3 form: log|psi|^2 the same bits whichever kernels form the mean product (the value rows keep theirs), E_loc
+    within the form's own accuracy of the other (the parity tests' bound, u = 2^-17), at both tile widths."""
+    from deeperwin_amd._native import LAP_FP32, LAP_SPLIT, NativeModel
+
+    R, Z = random_molecule(np.random.default_rng(n), n)
+    R = R.astype(np.float32)
+    shape = ModelShape(n, (n + 1) // 2, len(Z), 2)
+    params = init_params(shape, n)
+    r0 = init_walkers_gaussian(np.random.default_rng(1), B, R, generate_el_ion_mapping(R, Z, n, shape.n_up))
+    r = torch.as_tensor(r0, dtype=torch.float32, device="cuda").contiguous()
+    Rd = torch.as_tensor(R, dtype=torch.float32, device="cuda")
+    Zd = torch.as_tensor(Z, dtype=torch.float32, device="cuda")
+    m = NativeModel(shape, "bf16x3")
+    m.set_params(params)
+    out = []
+    for form in (LAP_FP32, LAP_SPLIT):
+        m.set_lap_form(form)
+        e, lp = torch.empty(B, device="cuda"), torch.empty(B, device="cuda")
+        m.local_energy(r, Rd, Zd, e, lp)
+        kappa = m.conditioning(B)
+        torch.cuda.synchronize()
+        out.append((e.cpu().numpy(), lp.cpu().numpy(), kappa.cpu().numpy()))
+    (e0, lp0, kappa), (e1, lp1, _) = out
+    np.testing.assert_array_equal(lp1, lp0)
+    assert np.all(np.abs(e1 - e0) <= (1 + np.abs(e0)) * (1e-4 + 4 * 2.0 ** -17 * kappa))
