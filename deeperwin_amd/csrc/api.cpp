@@ -810,7 +810,7 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
       em.permute = last ? 1 : 0;
       if constexpr (!DBL) {
         if (m->prec == GEMM_F32 && m->tune.fwd_main_tile == 3) {  // 16x16-MFMA tiles of 96 electrons
-          gemm_value16(X[l], m->Kx[l], W.Wmain[l].as<float>(), m->Kx[l], ws.V, m->W1, vs, vstride, outp,
+          gemm_value16(X[l], m->Kx[l], W.WmainL[l].as<float>(), m->Kx[l], ws.V, m->W1, vs, vstride, outp,
                        ldo, last ? 1 : 0, sh, s);
           continue;
         }
@@ -824,7 +824,7 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
                rows, m->W1, m->Kx[l], em, s);
         launch_tanh_rule<T>(ws.Z, outp, ldo, last ? 1 : 0, sh, s);
       } else {
-        gemm_lap(m->prec, X[l], m->Kx[l], W.Wmain[l].as<float>(), W.Wmain_hi[l].as<uint16_t>(),
+        gemm_lap(m->prec, X[l], m->Kx[l], W.WmainL[l].as<float>(), W.Wmain_hi[l].as<uint16_t>(),
                  W.Wmain_lo[l].as<uint16_t>(), m->Kx[l], ws.V, m->W1, outp, ldo, last ? 1 : 0, sh,
                  m->tune.lap_electrons, m->tune.lap_cols, s);
       }

@@ -516,9 +516,12 @@ namespace dwmi {
 //   z_ch = (X W)_ch + V[walker, ch]                     (V: spin-mean part + bias, per walker & channel)
 //   y_0 = tanh z_0,  y_k = t' z_k (k = 1..3n),  y_lap = t' z_lap + t'' sum_k z_k^2,  padded channels 0.
 // MFMA: v_mfma_f32_16x16x4_f32 (FP32) or v_mfma_f32_16x16x32_bf16 (BF16 forms, A split hi/lo in LDS).
+// FP32: bound by the matrix rate (1,376,256 rows x 320 x 256: 1.46 ms) plus the rule's phase, which three workgroups per
+// CU overlap in part.  Weights from L2 in lane order instead of LDS, rows in LDS 16 bytes a read with one barrier per 32 k
+// instead of two per 16, and registers held to three workgroups per CU: 2.19 -> 2.09 ms.
 // ------------------------------------------------------------------------------------------------
 template <int RB, int PREC, int BN, bool VAL = false>
-__global__ __launch_bounds__(256) void k_gemm_lap(const float* __restrict__ X, int ldx,
+__global__ __launch_bounds__(256, PREC == 0 ? 3 : 1) void k_gemm_lap(const float* __restrict__ X, int ldx,
                                                   const float* __restrict__ Bt, const uint16_t* __restrict__ Bhi,
                                                   const uint16_t* __restrict__ Blo, int K,
                                                   const float* __restrict__ V, int ldv, float* __restrict__ out,
@@ -529,13 +532,13 @@ __global__ __launch_bounds__(256) void k_gemm_lap(const float* __restrict__ X, i
   constexpr int ROWS = RB * 16;
   constexpr int WN = BN / 4;    // columns per wave
   constexpr int NQ = WN / 16;   // 16-column MFMA blocks per wave
-  constexpr int BK = (PREC == 0) ? 16 : 32;  // FP32: 16 measured faster than 32 (2.05 vs 2.10 ms at N2)
+  constexpr int BK = 32;
   constexpr int LDK = BK + 8;  // bf16 row pitch (elements)
   // epilogue window: all 128 columns at once when the tile fits in 60 KB of LDS, else two passes of 64
   constexpr int NC = ((size_t)RB * 16 * (128 + 4) * 4 <= 60 * 1024) ? 128 : 64;
   constexpr int EP = NC + 4;   // epilogue pitch (floats)
   constexpr size_t LOAD_BYTES = (PREC == 0)
-                                    ? (size_t)BK * (ROWS + 4) * 4 + (size_t)BK * (BN + 4) * 4
+                                    ? (size_t)2 * ROWS * BK * 4
                                     : (size_t)(ROWS + BN) * LDK * 2 * (PREC == 1 ? 2 : 1);
   constexpr size_t EPI_BYTES = (size_t)ROWS * EP * 4;
   constexpr size_t SMEM = LOAD_BYTES > EPI_BYTES ? LOAD_BYTES : EPI_BYTES;
@@ -562,72 +565,70 @@ __global__ __launch_bounds__(256) void k_gemm_lap(const float* __restrict__ X, i
     for (int b = 0; b < NQ; ++b) acc[a][b] = v4f{0.f, 0.f, 0.f, 0.f};
 
   if constexpr (PREC == 0) {
-    float(*As)[ROWS + 4] = (float(*)[ROWS + 4])smem;
-    float(*Bs)[BN + 4] = (float(*)[BN + 4])(smem + (size_t)BK * (ROWS + 4) * 4);
-    constexpr int KV = BK / 4;         // float4 per row of a K-slice
-    constexpr int AV = ROWS * KV;      // float4 per A tile
+    // Rows of 32 k in LDS, 16 bytes per (row, quad of 4 k): slice, row block, lane group, row, the 16 rows of a quad
+    // rotated by its number (the loads' walk along a row and the fragment reads both cover all banks); two buffers, one
+    // barrier per 32 k.  Weights come from L2 in lane order, one slice ahead.  Slices of 16 in order, step st of lane
+    // group g taking k = 4 g + st: the order of k_gemm_f32.
+    v4f* const As = (v4f*)smem;
+    constexpr int AV = ROWS * 8;  // quads per 32 k
     constexpr int AIT = (AV + 255) / 256;
-    constexpr int BIT = BN * KV / 256;
-    float4 ra[AIT], rb[BIT];
+    const int g = lane >> 4, cl = lane & 15, S = K >> 4;
+    const v4f* bp[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+      bp[q] = (const v4f*)Bt + (long)(col0 / 16 + wv * NQ + q) * S * 64 + lane;
+    v4f ra[AIT], b[NQ], bn[NQ];
+    auto slot = [](int row, int quad) { return (((quad >> 2) * RB + (row >> 4)) * 4 + (quad & 3)) * 16 + ((row + quad) & 15); };
     auto gload = [&](int k0) {
 #pragma unroll
       for (int it = 0; it < AIT; ++it) {
         const int idx = tid + 256 * it;
         if (idx < AV) {
-          const int m = idx / KV, kq = (idx % KV) * 4;
-          long gr = row0 + m;
+          long gr = row0 + (idx >> 3);
           if (gr > rows_total - 1) gr = rows_total - 1;
-          ra[it] = *(const float4*)(X + gr * ldx + k0 + kq);
+          ra[it] = *(const v4f*)(X + gr * ldx + k0 + (idx & 7) * 4);
         }
       }
-#pragma unroll
-      for (int it = 0; it < BIT; ++it) {
-        const int idx = tid + 256 * it, m = idx / KV, kq = (idx % KV) * 4;
-        rb[it] = *(const float4*)(Bt + (long)(col0 + m) * K + k0 + kq);
-      }
     };
-    auto sstore = [&]() {
+    auto sstore = [&](int buf) {
 #pragma unroll
       for (int it = 0; it < AIT; ++it) {
         const int idx = tid + 256 * it;
-        if (idx < AV) {
-          const int m = idx / KV, kq = (idx % KV) * 4;
-          As[kq + 0][m] = ra[it].x;
-          As[kq + 1][m] = ra[it].y;
-          As[kq + 2][m] = ra[it].z;
-          As[kq + 3][m] = ra[it].w;
-        }
-      }
-#pragma unroll
-      for (int it = 0; it < BIT; ++it) {
-        const int idx = tid + 256 * it, m = idx / KV, kq = (idx % KV) * 4;
-        Bs[kq + 0][m] = rb[it].x;
-        Bs[kq + 1][m] = rb[it].y;
-        Bs[kq + 2][m] = rb[it].z;
-        Bs[kq + 3][m] = rb[it].w;
+        if (idx < AV) As[buf * AV + slot(idx >> 3, idx & 7)] = ra[it];
       }
     };
     gload(0);
-    for (int k0 = 0; k0 < K; k0 += BK) {
-      __syncthreads();
-      sstore();
-      __syncthreads();
-      if (k0 + BK < K) gload(k0 + BK);
 #pragma unroll
-      for (int kk = 0; kk < BK; kk += 4) {
-        // MFMA step kk / 4 of lane group g = lane / 16 takes k = kk / 4 + 4 g (A and B alike): the four rows
-        // one read touches lie 4 k apart, so with the pitch of 4 (mod 64) floats they start 16 banks apart
-        const int kr = (kk >> 2) + 4 * (lane >> 4);
-        float bq[NQ];
+    for (int q = 0; q < NQ; ++q) bn[q] = bp[q][0];
+    sstore(0);
+    if (K > 32) gload(32);
+    __syncthreads();
+    for (int k0 = 0; k0 < K; k0 += 32) {
+      const int buf = (k0 >> 5) & 1;
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) bq[q] = Bs[kr][wv * WN + q * 16 + (lane & 15)];
+      for (int h = 0; h < 2; ++h) {
+        const int sl = (k0 >> 4) + h;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+          b[q] = bn[q];
+          bn[q] = bp[q][64 * min(sl + 1, S - 1)];
+        }
+        const v4f* ap = As + buf * AV + h * RB * 64 + g * 16 + ((cl + 4 * h + g) & 15);
 #pragma unroll
         for (int rb2 = 0; rb2 < RB; ++rb2) {
-          const float a = As[kr][rb2 * 16 + (lane & 15)];
+          const v4f a = ap[rb2 * 64];
 #pragma unroll
-          for (int q = 0; q < NQ; ++q)
-            acc[rb2][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bq[q], acc[rb2][q], 0, 0, 0);
+          for (int st = 0; st < 4; ++st)
+#pragma unroll
+            for (int q = 0; q < NQ; ++q)
+              acc[rb2][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[st], b[q][st], acc[rb2][q], 0, 0, 0);
         }
+      }
+      // the other buffer was last read before the previous barrier
+      if (k0 + 32 < K) {
+        sstore(buf ^ 1);
+        if (k0 + 64 < K) gload(k0 + 64);
+        __syncthreads();
       }
     }
   } else {
