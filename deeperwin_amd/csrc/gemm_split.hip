@@ -592,11 +592,11 @@ int split_lap(const float* X, int ldx, const void* P, int shift, int K, const fl
 // A workgroup forms the means of 48 rows x 128 k at a time and splits them straight into LDS (37 KB: four workgroups
 // per CU, whose load and MFMA phases overlap); the weights' parts come from L2.  Bound by the read of X's h columns
 // (1.41 GB for 2048 walkers of 14 electrons: 364 us = 3.9 TB/s against 471 us with FP32 MFMA; 26 electrons, 1024
-// walkers: 575 -> 461 us; 256 LiH walkers: 67 -> 28 us with 64 columns per workgroup).  NP = 2 keeps the first two parts
+// walkers: 575 -> 461 us; 256 LiH walkers: 67 -> 28 us a layer with 64 columns per workgroup).  NP = 2 keeps the first two parts
 // and three products, the BF16x3 form's arithmetic (1,000 walkers of 14: 206 us a layer in two launches, 159 + 15 for the
 // value rows here).
 // ------------------------------------------------------------------------------------------------
-template <int NQ, int NP>
+template <int NQ, int NP, bool FEW>
 __global__ __launch_bounds__(256) void k_split_mean(const float* __restrict__ X, int Kx, int Kh,
                                                     const uint4* __restrict__ P, int ncb, int Km,
                                                     float* __restrict__ V, int ldv, Shape sh, int tilesN, int total) {
@@ -618,37 +618,85 @@ __global__ __launch_bounds__(256) void k_split_mean(const float* __restrict__ X,
     const int ns = min(CS, (Km - kc) >> 5);
     __syncthreads();  // the previous chunk's reads are done
     // consecutive lanes take consecutive quads of a row (coalesced); 4 quads a slice-row group
-    for (int t = tid; t < 16 * RB * 8 * ns; t += 256) {
-      const int rr = t / (8 * ns), qd = t - rr * (8 * ns);
-      const long r = r0 + rr;
-      const int k = kc + 4 * qd;
-      v4f v = {0.f, 0.f, 0.f, 0.f};
-      if (r < rows && k < 2 * Kh) {
-        const long b = div_idx(r, Cp);
-        const int ch = (int)(r - b * Cp);
-        const int s = k >= Kh ? 1 : 0;
-        const int i0 = s ? u : 0, i1 = s ? n : u;
-        const float* xp = X + ((b * n + i0) * Cp + ch) * (long)Kx + (k - s * Kh);
-#pragma unroll 8
-        for (int i = i0; i < i1; ++i, xp += xstride) {
-          const v4f x = *(const v4f*)xp;
-          v[0] += x[0];
-          v[1] += x[1];
-          v[2] += x[2];
-          v[3] += x[3];
-        }
-        const float inv = 1.f / (float)(i1 - i0);
-        v[0] *= inv;
-        v[1] *= inv;
-        v[2] *= inv;
-        v[3] *= inv;
-      }
+    auto put = [&](int rr, int qd, v4f v, float inv) {
+      v[0] *= inv;
+      v[1] *= inv;
+      v[2] *= inv;
+      v[3] *= inv;
       uint2 p[3];
       split4(v, p);
       const int quad = qd & 7;
 #pragma unroll
       for (int m = 0; m < NP; ++m)
         *((uint2*)&lds[qd >> 3][m][rr >> 4][(quad >> 1) * 16 + (rr & 15)] + (quad & 1)) = p[m];
+    };
+    const int units = 16 * RB * 8 * ns;
+    if constexpr (FEW) {
+      // up to four electrons of a spin: all of a thread's means together (one after another they wait for their few
+      // loads: 37 us a layer for 256 walkers of 4 electrons, 28 so; where there are workgroups enough to
+      // hide the wait, the registers cost more: 316 -> 450 us at 2,048 walkers of 14)
+      constexpr int TT = RB * 2;
+      const float* xp[TT];
+      v4f v[TT];
+      int cnt[TT], rr[TT], qd[TT];
+#pragma unroll
+      for (int a = 0; a < TT; ++a) {
+        const int t = tid + a * 256;
+        rr[a] = t / (8 * ns);
+        qd[a] = t - rr[a] * (8 * ns);
+        const long r = r0 + rr[a];
+        const int k = kc + 4 * qd[a];
+        v[a] = v4f{0.f, 0.f, 0.f, 0.f};
+        cnt[a] = 0;
+        xp[a] = X;
+        if (t < units && r < rows && k < 2 * Kh) {
+          const long b = div_idx(r, Cp);
+          const int s = k >= Kh ? 1 : 0;
+          cnt[a] = s ? n - u : u;
+          xp[a] = X + ((b * n + (s ? u : 0)) * Cp + (r - b * Cp)) * (long)Kx + (k - s * Kh);
+        }
+      }
+#pragma unroll 2
+      for (int i = 0; i < 4; ++i) {
+        v4f x[TT];
+#pragma unroll
+        for (int a = 0; a < TT; ++a) x[a] = i < cnt[a] ? *(const v4f*)(xp[a] + i * xstride) : v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int a = 0; a < TT; ++a) {
+          v[a][0] += x[a][0];
+          v[a][1] += x[a][1];
+          v[a][2] += x[a][2];
+          v[a][3] += x[a][3];
+        }
+      }
+#pragma unroll
+      for (int a = 0; a < TT; ++a)
+        if (tid + a * 256 < units) put(rr[a], qd[a], v[a], cnt[a] ? 1.f / (float)cnt[a] : 0.f);
+    } else {
+      for (int t = tid; t < units; t += 256) {
+        const int rr = t / (8 * ns), qd = t - rr * (8 * ns);
+        const long r = r0 + rr;
+        const int k = kc + 4 * qd;
+        v4f v = {0.f, 0.f, 0.f, 0.f};
+        float inv = 0.f;
+        if (r < rows && k < 2 * Kh) {
+          const long b = div_idx(r, Cp);
+          const int ch = (int)(r - b * Cp);
+          const int s = k >= Kh ? 1 : 0;
+          const int i0 = s ? u : 0, i1 = s ? n : u;
+          const float* xp = X + ((b * n + i0) * Cp + ch) * (long)Kx + (k - s * Kh);
+#pragma unroll 8
+          for (int i = i0; i < i1; ++i, xp += xstride) {
+            const v4f x = *(const v4f*)xp;
+            v[0] += x[0];
+            v[1] += x[1];
+            v[2] += x[2];
+            v[3] += x[3];
+          }
+          inv = 1.f / (float)(i1 - i0);
+        }
+        put(rr, qd, v, inv);
+      }
     }
     __syncthreads();
     for (int s = 0; s < ns; ++s) {
@@ -693,12 +741,16 @@ static void launch_mean(const float* X, int Kx, int Kh, const void* P, int Km, f
   // 256 columns (X read once) where that gives two workgroups to every CU
   if (sh.W1 % 256 == 0 && tilesM * (sh.W1 / 256) >= 512) {
     const int tilesN = sh.W1 / 256, total = (int)(tilesM * tilesN);
-    hipLaunchKernelGGL((k_split_mean<4, NP>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh, (const uint4*)P,
+    hipLaunchKernelGGL((k_split_mean<4, NP, false>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh, (const uint4*)P,
                        ncb, Km, V, ldv, sh, tilesN, total);
   } else {
     const int tilesN = sh.W1 / 64, total = (int)(tilesM * tilesN);
-    hipLaunchKernelGGL((k_split_mean<1, NP>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh, (const uint4*)P,
-                       ncb, Km, V, ldv, sh, tilesN, total);
+    if (sh.u <= 4 && sh.n - sh.u <= 4)
+      hipLaunchKernelGGL((k_split_mean<1, NP, true>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh,
+                         (const uint4*)P, ncb, Km, V, ldv, sh, tilesN, total);
+    else
+      hipLaunchKernelGGL((k_split_mean<1, NP, false>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh,
+                         (const uint4*)P, ncb, Km, V, ldv, sh, tilesN, total);
   }
 }
 

@@ -116,3 +116,32 @@ def test_bf16x3_mean_product_with_the_means_formed_in_it(cuda, n, B):
     (e0, lp0, kappa), (e1, lp1, _) = out
     np.testing.assert_array_equal(lp1, lp0)
     assert np.all(np.abs(e1 - e0) <= (1 + np.abs(e0)) * (1e-4 + 4 * 2.0 ** -17 * kappa))
+
+
+@pytest.mark.parametrize("n,B", [(2, 3), (4, 50), (5, 19), (7, 33), (8, 21), (9, 21)])
+def test_mean_product_of_small_batches(cuda, n, B):
+    """Up to four electrons of a spin and 64-column workgroups: the means of a thread formed together.  E_loc bit-equal to
+    the batch repeated until it takes the 256-column workgroups (the same sums)."""
+    from deeperwin_amd._native import NativeModel
+
+    R, Z = random_molecule(np.random.default_rng(n), n)
+    R = R.astype(np.float32)
+    shape = ModelShape(n, (n + 1) // 2, len(Z), 2)
+    params = init_params(shape, n)
+    r0 = init_walkers_gaussian(np.random.default_rng(1), B, R, generate_el_ion_mapping(R, Z, n, shape.n_up))
+    r = torch.as_tensor(r0, dtype=torch.float32, device="cuda").contiguous()
+    Rd = torch.as_tensor(R, dtype=torch.float32, device="cuda")
+    Zd = torch.as_tensor(Z, dtype=torch.float32, device="cuda")
+    m = NativeModel(shape)
+    m.set_params(params)
+
+    def eloc(y):
+        e = torch.empty(len(y), device="cuda")
+        m.local_energy(y, Rd, Zd, e)
+        return e
+
+    rows = B * ((3 * n + 2 + 15) // 16 * 16)  # channel rows; the wide workgroups take over at 512 tiles of 48
+    big = r.repeat(512 * 48 // rows + 2, 1, 1).contiguous()
+    e = eloc(r)
+    assert torch.isfinite(e).all()
+    assert torch.equal(eloc(big)[:B], e)
