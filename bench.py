@@ -65,17 +65,6 @@ def parse():
     return ap.parse_args()
 
 
-def traffic_from_profiles():
-    """HBM bytes per launch of the dominant kernel from the committed rocprofv3 --pmc summary, if any."""
-    f = ROOT / "profiles" / "gemm_1el_lap_n2_traffic.txt"
-    if not f.exists():
-        return None
-    for line in f.read_text().splitlines():
-        if line.startswith("bytes_per_launch:"):
-            return float(line.split(":", 1)[1])
-    return None
-
-
 def precision_study(args):
     """C4H2-like molecule (4 C on a 2.6 bohr rhombus + 2 H), 26 electrons, 16 dets, 4096 walkers: E_loc of
     every walker in each precision form, timed, and compared with the FP64 form on the SAME walkers (the
@@ -764,12 +753,23 @@ def main():
     K = shape.width1 + 2 * shape.width2
     flops = 2.0 * M * K * shape.width1
     avg_s = (gemm_ms / max(gemm_n, 1)) / 1e3
-    achieved = flops / avg_s / 1e12
     peak = PEAK_TFLOPS[args.precision]
-    roofline = {"bound": "mfma", "achieved": round(achieved, 2), "peak": peak, "unit": "TFLOP/s",
-                "frac": round(achieved / peak, 4), "traffic": traffic_from_profiles(),
-                "kernel": "1-el embedding GEMM, Laplacian mode (k_gemm_lap)",
-                "flops_per_launch": flops, "avg_launch_ms": round(avg_s * 1e3, 4), "launches": gemm_n}
+    if args.precision == "fp32":
+        # two FP16 parts per operand, three products each, on 16-bit MFMA: bound by X read, V read, layer written
+        nbytes = 4.0 * (M * (K + shape.width1) + B * C * shape.width1)
+        gbs, tf = nbytes / avg_s / 1e9, 3 * flops / avg_s / 1e12
+        roofline = {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                    "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None,
+                    "kernel": "1-el embedding GEMM, Laplacian mode (k_split_lap, three FP16 products)",
+                    "bytes_per_launch": nbytes, "flops_per_launch": flops, "mfma_tflops": round(tf, 1),
+                    "mfma_frac": round(tf / PEAK_TFLOPS["bf16"], 4), "avg_launch_ms": round(avg_s * 1e3, 4),
+                    "launches": gemm_n}
+    else:
+        achieved = flops / avg_s / 1e12
+        roofline = {"bound": "mfma", "achieved": round(achieved, 2), "peak": peak, "unit": "TFLOP/s",
+                    "frac": round(achieved / peak, 4), "traffic": None,
+                    "kernel": "1-el embedding GEMM, Laplacian mode (k_gemm_lap)",
+                    "flops_per_launch": flops, "avg_launch_ms": round(avg_s * 1e3, 4), "launches": gemm_n}
 
     out = {
         "metric": METRIC, "value": round(value, 1), "unit": "walker local-energies/s", "n_gpus": 1,

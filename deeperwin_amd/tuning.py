@@ -42,15 +42,18 @@ def lap_electron_choices(n_el: int) -> List[int]:
 
 
 def search_space(n_el: int) -> List[Tuple[str, Sequence[int], str]]:
-    """(field, candidates, pass it affects) in the order the sweep visits them."""
+    """(field, candidates, pass it affects) in the order the sweep visits them.  -1 leaves the choice to the library:
+    a fixed tile keeps the separate kernels, which for the value layers, the orbital GEMMs of a value pass and the
+    mean product are slower at most sizes than what the library picks (8 electrons, 512 walkers: value pass 150 us with
+    64 x 64 tiles, 108 us with the library's choice)."""
     return [
-        ("fwd_main_tile", TILE_CHOICES + (3, 4), "value"),
+        ("fwd_main_tile", (-1,) + TILE_CHOICES + (3, 4), "value"),
         ("fwd_mu_split", SPLIT_CHOICES, "value"),
-        ("fwd_orb_tile", TILE_CHOICES, "value"),
+        ("fwd_orb_tile", (-1,) + TILE_CHOICES, "value"),
         ("lap_cols", (128, 256), "lap"),
         ("lap_electrons", lap_electron_choices(n_el), "lap"),
-        ("lap_mu_tile", TILE_CHOICES, "lap"),
-        ("lap_orb_tile", TILE_CHOICES, "lap"),
+        ("lap_mu_tile", (-1,) + TILE_CHOICES, "lap"),
+        ("lap_orb_tile", (-1,) + TILE_CHOICES, "lap"),
     ]
 
 
