@@ -113,7 +113,7 @@ struct Weights {
   std::vector<DevBuf> WmainT, WmuT;  // transposed copies for the gradient pass ([pad128(K)][W1])
   DevBuf W2e, b2e, Wo[2], Wo_hi[2], Wo_lo[2], WoT[2], kappa, wenv;
   // FP32 form: the three BF16 parts of Wmain / Wmu / Wo in MFMA lane order (derivative channels, gemm_split.hip); of
-  // Wmu in the BF16 forms too
+  // Wmain and Wmu in the BF16 forms too
   std::vector<DevBuf> WmainS, WmuS;
   // and the two FP16 parts of 2^shift Wmain (layers >= 1) / Wo; shift kNoHalf: magnitudes outside FP16's reach
   std::vector<DevBuf> WmainH;
@@ -422,7 +422,7 @@ dw_status prepare_weights(dw_model* m, Weights& W, bool dbl) {
                    (st = pack_lanes(W.WmuL[l], W.Wmu[l], W1, Km))))
       return st;
     if (split) {
-      if ((st = pack_split(W.WmuS[l], W.Wmu[l], W1, Km))) return st;
+      if ((st = pack_split(W.WmainS[l], W.Wmain[l], W1, Kx)) || (st = pack_split(W.WmuS[l], W.Wmu[l], W1, Km))) return st;
       if ((st = upload_split(W.Wmain_hi[l], W.Wmain_lo[l], wm))) return st;
       if ((st = upload_split(W.Wmu_hi[l], W.Wmu_lo[l], wu))) return st;
     }
@@ -824,9 +824,8 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
                rows, m->W1, m->Kx[l], em, s);
         launch_tanh_rule<T>(ws.Z, outp, ldo, last ? 1 : 0, sh, s);
       } else {
-        gemm_lap(m->prec, X[l], m->Kx[l], W.WmainL[l].as<float>(), W.Wmain_hi[l].as<uint16_t>(),
-                 W.Wmain_lo[l].as<uint16_t>(), m->Kx[l], ws.V, m->W1, outp, ldo, last ? 1 : 0, sh,
-                 m->tune.lap_electrons, m->tune.lap_cols, s);
+        gemm_lap(m->prec, X[l], m->Kx[l], (m->prec == GEMM_F32 ? W.WmainL[l] : W.WmainS[l]).template as<float>(),
+                 m->Kx[l], ws.V, m->W1, outp, ldo, last ? 1 : 0, sh, m->tune.lap_electrons, m->tune.lap_cols, s);
       }
     }
   }

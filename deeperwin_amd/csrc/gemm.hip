@@ -518,12 +518,13 @@ namespace dwmi {
 // MFMA: v_mfma_f32_16x16x4_f32 (FP32) or v_mfma_f32_16x16x32_bf16 (BF16 forms, A split hi/lo in LDS).
 // FP32: bound by the matrix rate (1,376,256 rows x 320 x 256: 1.46 ms) plus the rule's phase, which three workgroups per
 // CU overlap in part.  Weights from L2 in lane order instead of LDS, rows in LDS 16 bytes a read with one barrier per 32 k
-// instead of two per 16, and registers held to three workgroups per CU: 2.19 -> 2.09 ms.
+// instead of two per 16, and registers held to three workgroups per CU: 2.19 -> 2.09 ms.  BF16x3: the weights' parts from L2
+// in the split kernels' order and two row buffers in the same way: E_loc of 1,000 walkers of 14 (8 determinants) 3.57 ->
+// 3.35 ms, of 500 walkers of 26 6.21 -> 5.91.
 // ------------------------------------------------------------------------------------------------
 template <int RB, int PREC, int BN, bool VAL = false>
 __global__ __launch_bounds__(256, PREC == 0 ? 3 : 1) void k_gemm_lap(const float* __restrict__ X, int ldx,
-                                                  const float* __restrict__ Bt, const uint16_t* __restrict__ Bhi,
-                                                  const uint16_t* __restrict__ Blo, int K,
+                                                  const float* __restrict__ Bt, int K,
                                                   const float* __restrict__ V, int ldv, float* __restrict__ out,
                                                   int ldo, int permute, int E, Shape sh, int tilesN, int vsplit = 1,
                                                   long vstride = 0) {
@@ -539,7 +540,7 @@ __global__ __launch_bounds__(256, PREC == 0 ? 3 : 1) void k_gemm_lap(const float
   constexpr int EP = NC + 4;   // epilogue pitch (floats)
   constexpr size_t LOAD_BYTES = (PREC == 0)
                                     ? (size_t)2 * ROWS * BK * 4
-                                    : (size_t)(ROWS + BN) * LDK * 2 * (PREC == 1 ? 2 : 1);
+                                    : (size_t)2 * ROWS * LDK * 2 * (PREC == 1 ? 2 : 1);
   constexpr size_t EPI_BYTES = (size_t)ROWS * EP * 4;
   constexpr size_t SMEM = LOAD_BYTES > EPI_BYTES ? LOAD_BYTES : EPI_BYTES;
   __shared__ __align__(16) unsigned char smem[SMEM];
@@ -632,15 +633,15 @@ __global__ __launch_bounds__(256, PREC == 0 ? 3 : 1) void k_gemm_lap(const float
       }
     }
   } else {
-    constexpr bool X3 = (PREC == 1);
-    uint16_t(*Ah)[LDK] = (uint16_t(*)[LDK])smem;
-    uint16_t(*Bh)[LDK] = (uint16_t(*)[LDK])(smem + (size_t)ROWS * LDK * 2);
-    uint16_t(*Al)[LDK] = (uint16_t(*)[LDK])(smem + (size_t)(ROWS + BN) * LDK * 2);
-    uint16_t(*Bl)[LDK] = (uint16_t(*)[LDK])(smem + (size_t)(2 * ROWS + BN) * LDK * 2);
+    // Rows split into BF16 parts while staged, two buffers, one barrier per 32 k; the weights' parts come from L2 in lane
+    // order, a slice ahead.
+    constexpr int NP = (PREC == 1) ? 2 : 1;
+    constexpr bool X3 = NP == 2;
+    constexpr int PART = ROWS * LDK;  // elements of one part of a buffer
+    uint16_t* const Ab = (uint16_t*)smem;
     constexpr int AV = ROWS * BK / 4;
     constexpr int AIT = (AV + 255) / 256;
-    float4 ra[AIT];
-    uint2 rbh[4], rbl[4];
+    v4f ra[AIT];
     auto gload = [&](int k0) {
 #pragma unroll
       for (int it = 0; it < AIT; ++it) {
@@ -649,71 +650,74 @@ __global__ __launch_bounds__(256, PREC == 0 ? 3 : 1) void k_gemm_lap(const float
           const int m = idx >> 3, kq = (idx & 7) * 4;
           long gr = row0 + m;
           if (gr > rows_total - 1) gr = rows_total - 1;
-          ra[it] = *(const float4*)(X + gr * ldx + k0 + kq);
+          ra[it] = *(const v4f*)(X + gr * ldx + k0 + kq);
         }
       }
-#pragma unroll
-      for (int it = 0; it < 4; ++it) {
-        const int idx = tid + 256 * it, m = idx >> 3, kq = (idx & 7) * 4;
-        rbh[it] = *(const uint2*)(Bhi + (long)(col0 + m) * K + k0 + kq);
-        if (X3) rbl[it] = *(const uint2*)(Blo + (long)(col0 + m) * K + k0 + kq);
-      }
     };
-    auto sstore = [&]() {
+    auto sstore = [&](int buf) {
+      uint16_t* const Ah = Ab + buf * NP * PART;
 #pragma unroll
       for (int it = 0; it < AIT; ++it) {
         const int idx = tid + 256 * it;
         if (idx < AV) {
           const int m = idx >> 3, kq = (idx & 7) * 4;
-          const float f[4] = {ra[it].x, ra[it].y, ra[it].z, ra[it].w};
           unsigned short h[4], l[4];
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            h[q] = f2bf_bits(f[q]);
-            l[q] = f2bf_bits(f[q] - bf_bits2f(h[q]));
+            h[q] = f2bf_bits(ra[it][q]);
+            l[q] = f2bf_bits(ra[it][q] - bf_bits2f(h[q]));
           }
           uint2 hv, lv;
           hv.x = h[0] | ((unsigned)h[1] << 16);
           hv.y = h[2] | ((unsigned)h[3] << 16);
           lv.x = l[0] | ((unsigned)l[1] << 16);
           lv.y = l[2] | ((unsigned)l[3] << 16);
-          *(uint2*)&Ah[m][kq] = hv;
-          if (X3) *(uint2*)&Al[m][kq] = lv;
+          *(uint2*)(Ah + m * LDK + kq) = hv;
+          if (X3) *(uint2*)(Ah + PART + m * LDK + kq) = lv;
         }
-      }
-#pragma unroll
-      for (int it = 0; it < 4; ++it) {
-        const int idx = tid + 256 * it, m = idx >> 3, kq = (idx & 7) * 4;
-        *(uint2*)&Bh[m][kq] = rbh[it];
-        if (X3) *(uint2*)&Bl[m][kq] = rbl[it];
       }
     };
-    gload(0);
-    for (int k0 = 0; k0 < K; k0 += BK) {
-      __syncthreads();
-      sstore();
-      __syncthreads();
-      if (k0 + BK < K) gload(k0 + BK);
-      const int kc = 8 * (lane >> 4);
-      v8s bh[2], bl[2];
+    const int ncb = (sh.W1 + 255) / 256 * 16;
+    const uint4* bp = (const uint4*)Bt + (long)(col0 / 16 + wv * 2) * 3 * 64 + lane;
+    v8s b[2][NP], bn[2][NP];
+    auto bload = [&](int sl) {
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        bh[q] = *(const v8s*)&Bh[wv * 32 + q * 16 + (lane & 15)][kc];
-        if (X3) bl[q] = *(const v8s*)&Bl[wv * 32 + q * 16 + (lane & 15)][kc];
-      }
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int m = 0; m < NP; ++m) bn[q][m] = *(const v8s*)&bp[((long)sl * ncb + q) * 192 + m * 64];
+    };
+    gload(0);
+    bload(0);
+    sstore(0);
+    if (K > BK) gload(BK);
+    __syncthreads();
+    for (int k0 = 0; k0 < K; k0 += BK) {
+      const int buf = (k0 / BK) & 1;
+      const uint16_t* Ah = Ab + buf * NP * PART + (lane & 15) * LDK + 8 * (lane >> 4);
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int m = 0; m < NP; ++m) b[q][m] = bn[q][m];
+      bload(min(k0 / BK + 1, K / BK - 1));
 #pragma unroll
       for (int rb2 = 0; rb2 < RB; ++rb2) {
-        const v8s ah = *(const v8s*)&Ah[rb2 * 16 + (lane & 15)][kc];
+        const v8s ah = *(const v8s*)(Ah + rb2 * 16 * LDK);
         v8s al;
-        if (X3) al = *(const v8s*)&Al[rb2 * 16 + (lane & 15)][kc];
+        if (X3) al = *(const v8s*)(Ah + PART + rb2 * 16 * LDK);
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-          if (X3) {
-            acc[rb2][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16((v8bf)al, (v8bf)bh[q], acc[rb2][q], 0, 0, 0);
-            acc[rb2][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16((v8bf)ah, (v8bf)bl[q], acc[rb2][q], 0, 0, 0);
+          if constexpr (X3) {
+            acc[rb2][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16((v8bf)al, (v8bf)b[q][0], acc[rb2][q], 0, 0, 0);
+            acc[rb2][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16((v8bf)ah, (v8bf)b[q][NP - 1], acc[rb2][q], 0, 0, 0);
           }
-          acc[rb2][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16((v8bf)ah, (v8bf)bh[q], acc[rb2][q], 0, 0, 0);
+          acc[rb2][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16((v8bf)ah, (v8bf)b[q][0], acc[rb2][q], 0, 0, 0);
         }
+      }
+      // the other buffer was last read before the previous barrier
+      if (k0 + BK < K) {
+        sstore(buf ^ 1);
+        if (k0 + 2 * BK < K) gload(k0 + 2 * BK);
+        __syncthreads();
       }
     }
   }
@@ -826,8 +830,7 @@ __global__ __launch_bounds__(256, PREC == 0 ? 3 : 1) void k_gemm_lap(const float
 }
 
 template <int PREC>
-static void gemm_lap_rb(int RB, const float* X, int ldx, const float* Bt, const uint16_t* Bhi, const uint16_t* Blo,
-                        int K, const float* V, int ldv, float* out, int ldo, int permute, int E, const Shape& sh,
+static void gemm_lap_rb(int RB, const float* X, int ldx, const float* Bt, int K, const float* V, int ldv, float* out, int ldo, int permute, int E, const Shape& sh,
                         int cols, hipStream_t s) {
   const long tilesM = ((long)sh.B * sh.n + E - 1) / E;
   if constexpr (PREC == 0) {
@@ -837,7 +840,7 @@ static void gemm_lap_rb(int RB, const float* X, int ldx, const float* Bt, const 
       const dim3 grid((unsigned)((tilesM * tilesN + 7) / 8 * 8));
 #define DW_LAP_CASE256(R)                                                                                            \
   case R:                                                                                                            \
-    hipLaunchKernelGGL((k_gemm_lap<R, 0, 256>), grid, dim3(256), 0, s, X, ldx, Bt, Bhi, Blo, K, V, ldv, out, ldo, \
+    hipLaunchKernelGGL((k_gemm_lap<R, 0, 256>), grid, dim3(256), 0, s, X, ldx, Bt, K, V, ldv, out, ldo, \
                        permute, E, sh, tilesN);                                                                      \
     return;
       switch (RB) {
@@ -856,7 +859,7 @@ static void gemm_lap_rb(int RB, const float* X, int ldx, const float* Bt, const 
   const dim3 grid((unsigned)((tilesM * tilesN + 7) / 8 * 8));
 #define DW_LAP_CASE(R)                                                                                                  \
   case R:                                                                                                               \
-    hipLaunchKernelGGL((k_gemm_lap<R, PREC, 128>), grid, dim3(256), 0, s, X, ldx, Bt, Bhi, Blo, K, V, ldv, out, ldo, \
+    hipLaunchKernelGGL((k_gemm_lap<R, PREC, 128>), grid, dim3(256), 0, s, X, ldx, Bt, K, V, ldv, out, ldo, \
                        permute, E, sh, tilesN);                                                                         \
     break;
   switch (RB) {
@@ -887,8 +890,7 @@ void gemm_value16(const float* X, int ldx, const float* Bt, int K, const float* 
   const int tilesN = sh.W1 / 128;
   const long tilesM = ((long)sh.B * sh.n + E - 1) / E;
   const dim3 grid((unsigned)((tilesM * tilesN + 7) / 8 * 8));
-  hipLaunchKernelGGL((k_gemm_lap<6, 0, 128, true>), grid, dim3(256), 0, s, X, ldx, Bt,
-                     nullptr, nullptr, K, V, ldv, out, ldo, permute, E, v, tilesN, vsplit, vstride);
+  hipLaunchKernelGGL((k_gemm_lap<6, 0, 128, true>), grid, dim3(256), 0, s, X, ldx, Bt, K, V, ldv, out, ldo, permute, E, v, tilesN, vsplit, vstride);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1005,17 +1007,17 @@ int lap_electrons_per_tile(int Cp, GemmPrec prec) {
   return E < 1 ? 1 : E;
 }
 
-void gemm_lap(GemmPrec prec, const float* X, int ldx, const float* Bt, const uint16_t* Bhi, const uint16_t* Blo, int K,
+void gemm_lap(GemmPrec prec, const float* X, int ldx, const float* Bt, int K,
               const float* V, int ldv, float* out, int ldo, int permute, const Shape& sh, int E_override, int cols,
               hipStream_t s) {
   const int E = E_override > 0 ? E_override : lap_electrons_per_tile(sh.Cp, prec);
   const int RB = E * sh.Cp / 16;
   if (prec == GEMM_F32)
-    gemm_lap_rb<0>(RB, X, ldx, Bt, Bhi, Blo, K, V, ldv, out, ldo, permute, E, sh, cols, s);
+    gemm_lap_rb<0>(RB, X, ldx, Bt, K, V, ldv, out, ldo, permute, E, sh, cols, s);
   else if (prec == GEMM_BF16X3)
-    gemm_lap_rb<1>(RB, X, ldx, Bt, Bhi, Blo, K, V, ldv, out, ldo, permute, E, sh, cols, s);
+    gemm_lap_rb<1>(RB, X, ldx, Bt, K, V, ldv, out, ldo, permute, E, sh, cols, s);
   else
-    gemm_lap_rb<2>(RB, X, ldx, Bt, Bhi, Blo, K, V, ldv, out, ldo, permute, E, sh, cols, s);
+    gemm_lap_rb<2>(RB, X, ldx, Bt, K, V, ldv, out, ldo, permute, E, sh, cols, s);
 }
 
 }  // namespace dwmi

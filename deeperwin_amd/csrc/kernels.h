@@ -47,9 +47,9 @@ struct Shape {
 // Fused 1-el GEMM + tanh forward-Laplacian rule of the Laplacian pass (rows: Cp per electron).
 // E_override > 0 sets the electrons per workgroup (E * Cp / 16 <= 12); 0 picks lap_electrons_per_tile:
 // FP32 min(4, 192 / Cp), BF16 forms 96 / Cp (at least 1).
-// cols = 256 asks for 256-column tiles (FP32 form, E * Cp <= 96); otherwise 128.  FP32 (and gemm_value16): Bt is in lane
-// order (launch_lane_pack), K a multiple of 32.
-void gemm_lap(GemmPrec prec, const float* X, int ldx, const float* Bt, const uint16_t* Bhi, const uint16_t* Blo, int K,
+// cols = 256 asks for 256-column tiles (FP32 form, E * Cp <= 96); otherwise 128.  Bt: FP32 (and gemm_value16) in lane
+// order (launch_lane_pack), BF16 forms the parts of launch_split_pack; K a multiple of 32.
+void gemm_lap(GemmPrec prec, const float* X, int ldx, const float* Bt, int K,
               const float* V, int ldv, float* out, int ldo, int permute, const Shape& sh, int E_override, int cols,
               hipStream_t s);
 int lap_electrons_per_tile(int Cp, GemmPrec prec);
