@@ -608,12 +608,20 @@ __global__ __launch_bounds__(256) void k_dpe4_pairs_value(const float* __restric
 // takes k = 4 t + g; a stream layer's output rows are ordered so that group g holds features 4 t + g, register t: the
 // next product's B operand, with no exchange.  A map's rows keep their order (16 nb + 4 g + e): 16-byte stores.
 // v_mfma_f32_16x16x4_f32 adds its four products to C as fmaf in order of k, so every sum is the chain
-// z = b; z = fmaf(x_k, w_k, z), k ascending, of a kernel without MFMA.
+// z = b; z = fmaf(x_k, w_k, z), k ascending, of a kernel without MFMA; the residual's sum is rounded by itself
+// (residual() below), so the rest is too.
 // Pairs of a relation are enumerated walker by walker (same: up-up then down-down; diff: up-down then down-up).
 // What bounds it: stores and tanh.  200,704 pairs (1,024 walkers of 14), 4 iterations, Laplacian: 762 us with a
 // thread per (electron, feature) reading x from LDS, 166 us here; value, 144,500 pairs (500 walkers of 17): 69 us
 // with a lane per pair, 31 us here.
 // ------------------------------------------------------------------------------------------------------
+// (x + y) / sqrt 2.  y is the product t' z for a tangent: the compiler would fuse it into the sum, and every energy (and
+// with it the FP64 loss) would change by a rounding against the kernels that keep x and y apart.
+__device__ __forceinline__ float residual(float x, float y) {
+#pragma clang fp contract(off)
+  return (x + y) * (float)0.70710678118654752440;
+}
+
 template <int NCH>
 __global__ __launch_bounds__(256, 4) void k_dpe4_pairs_mfma(const float* __restrict__ r, const float* __restrict__ Wp,
                                                          const float* __restrict__ bp, float* __restrict__ wm, Shape sh,
@@ -647,7 +655,6 @@ __global__ __launch_bounds__(256, 4) void k_dpe4_pairs_mfma(const float* __restr
   const int P = s == 0 ? u * u + d * d : 2 * u * d;  // pairs of this relation per walker
   const long total = (long)sh.B * P;
   const long per_l = (long)sh.B * n * n * NCH * EMB;
-  const float rs2 = (float)0.70710678118654752440;
   for (long t0 = ((long)blk * 4 + (threadIdx.x >> 6)) * 16; t0 < total; t0 += (long)nblk * 64) {
     const bool ok = t0 + cl < total;
     const long t = ok ? t0 + cl : total - 1;
@@ -753,7 +760,7 @@ __global__ __launch_bounds__(256, 4) void k_dpe4_pairs_mfma(const float* __restr
           for (int c = 0; c < NCH; ++c) zz[c] = z[c][nb][e];
           tanh_channels<NCH, float>(zz, y, 2.f);
 #pragma unroll
-          for (int c = 0; c < NCH; ++c) x[c][4 * nb + e] = l == 0 ? y[c] : (x[c][4 * nb + e] + y[c]) * rs2;
+          for (int c = 0; c < NCH; ++c) x[c][4 * nb + e] = l == 0 ? y[c] : residual(x[c][4 * nb + e], y[c]);
         }
     }
   }
