@@ -4,10 +4,11 @@
 // Both read the orbitals O and apply the envelope themselves, so the product envelope x orbitals (3 n + 2 matrices per
 // determinant) is never stored.
 //
-// 16,384 matrices of 26 (1024 walkers): 4.17 ms for the determinants and 1.99 ms for the stored product before, 0.84 ms
-// (inverses) + 2.08 ms (channels) here; 1,536 matrices of 42: 4.06 + 0.75 ms before, 0.55 + 1.04 ms here; 32,768
-// matrices of 14: 1.14 ms (one wavefront per matrix) before, 0.08 + 0.43 ms here.  Above 16 electrons the channel
-// passes run at half the FP64 matrix rate, padding to 16 x 16 blocks counted (1.06 and 0.54 ms at 78 TFLOP/s).
+// 16,384 matrices of 26 (1024 walkers): 4.17 ms for the determinants and 1.99 ms for the stored product before, 0.73 ms
+// (inverses) + 2.30 ms (channels) here; 3,072 matrices of 42: 0.70 + 2.13 ms; 32,768 matrices of 14: 1.14 ms (one
+// wavefront per matrix) before, 0.13 + 0.60 ms here.  The fixed order of the channels' sums takes 0.24, 0.19 and 0.10 ms of
+// that, against each wave adding up its own channels.  Above 16 electrons the channel passes run at half the FP64 matrix
+// rate, padding to 16 x 16 blocks counted.
 #include <utility>
 
 #include "common.h"
@@ -32,6 +33,40 @@ __device__ __forceinline__ int row_bcast(int v) {
 template <int P>
 __device__ __forceinline__ double row_bcast(double v) {
   return __hiloint2double(row_bcast<P>(__double2hiint(v)), row_bcast<P>(__double2loint(v)));
+}
+// Sums over the wavefront's lanes, in every lane; lanes paired as in wave_sum_d (xor 32, 16, 8, 4, 2, 1), without LDS.
+// After xor 8 the 16 lanes of a row hold 8 values twice, so a rotation by 4 meets the lane that xor 4 does; and so on.
+template <int CTRL>
+__device__ __forceinline__ double row_ror(double v) {
+  return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), 0x120 + CTRL, 0xF, 0xF, true),
+                          __builtin_amdgcn_mov_dpp(__double2loint(v), 0x120 + CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ double row_sum_dpp(double v) {
+  v += row_ror<8>(v);
+  v += row_ror<4>(v);
+  v += row_ror<2>(v);
+  v += row_ror<1>(v);
+  return v;
+}
+// v_permlane32_swap(a, b): the low halves of a and b, and their high halves; the sum of the two holds a's sum over xor 32
+// in the low half and b's in the high one.  v_permlane16_swap does the same for neighbouring rows of 16.
+__device__ __forceinline__ double fold32(double a, double b) {
+  const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+  return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+__device__ __forceinline__ double fold16(double a, double b) {
+  const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+  return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+__device__ __forceinline__ double wave_sum_dpp(double v) {
+  v = fold32(v, v);
+  return row_sum_dpp(fold16(v, v));
+}
+// Four sums at once: rows of 16 lanes get v0's, v2's, v1's and v3's.
+__device__ __forceinline__ double wave_sums_dpp(double v0, double v1, double v2, double v3) {
+  return row_sum_dpp(fold16(fold32(v0, v1), fold32(v2, v3)));
 }
 // n <= 16: four matrices per wavefront, one per 16-lane row, a lane per column; entries are broadcast inside a row by
 // DPP, so all four eliminate at once (a matrix per wavefront kept 14 of 64 lanes busy: 32,768 matrices of 14 took 358
@@ -210,9 +245,10 @@ __global__ __launch_bounds__(256) void k_det_inv(OrbSrc<TA> src, Shape sh, doubl
 }
 
 // 32 < n <= 63: one matrix per 64-thread workgroup, a lane per column, matrix and inverse in LDS (pitch n + 1).
-// Column-parallel elimination and substitution: a step reads one broadcast and one own element and four partial sums
-// run side by side, so a matrix is about n^2 pipelined LDS steps (a workgroup of 256 threads with barriers per
-// elimination step and 42 busy lanes in the substitution took most of 4.1 ms per 1536 matrices of 42).
+// Column-parallel elimination and substitution: a step reads one broadcast and one own element (eight steps' reads in
+// flight) and every element is one chain, in the order of a row-by-row elimination, so a matrix is about n^2 pipelined LDS
+// steps.  3,072 matrices of 42: 0.70 ms (a workgroup of 256 threads, with barriers per elimination step and 42 busy lanes in
+// the substitution, took several times that).
 template <typename TA>
 __global__ __launch_bounds__(64) void k_det_inv_lds(OrbSrc<TA> src, Shape sh, double* __restrict__ Minv,
                                                     double* __restrict__ ld, double* __restrict__ sd,
@@ -267,8 +303,7 @@ __global__ __launch_bounds__(64) void k_det_inv_lds(OrbSrc<TA> src, Shape sh, do
       }
     }
     __syncthreads();
-    const double rp = 1.0 / T[p * P + p];
-    if (act && j > p) T[j * P + p] *= rp;  // multiplier of row j
+    if (act && j > p) T[j * P + p] /= T[p * P + p];  // multiplier of row j
     __syncthreads();
     if (act && j > p) {
       const double u = T[p * P + j];
@@ -283,31 +318,20 @@ __global__ __launch_bounds__(64) void k_det_inv_lds(OrbSrc<TA> src, Shape sh, do
   double isum = 0.0;
   if (act) {
     for (int p = 0; p < n; ++p) {
-      double y0 = (perm[p] == j) ? 1.0 : 0.0, y1 = 0.0, y2 = 0.0, y3 = 0.0;
-      int q = 0;
-#pragma unroll 2
-      for (; q + 4 <= p; q += 4) {
-        y0 -= T[p * P + q] * X[q * P + j];
-        y1 -= T[p * P + q + 1] * X[(q + 1) * P + j];
-        y2 -= T[p * P + q + 2] * X[(q + 2) * P + j];
-        y3 -= T[p * P + q + 3] * X[(q + 3) * P + j];
-      }
-      for (; q < p; ++q) y0 -= T[p * P + q] * X[q * P + j];
-      X[p * P + j] = (y0 + y1) + (y2 + y3);
+      double y = (perm[p] == j) ? 1.0 : 0.0;
+#pragma unroll 8
+      for (int q = 0; q < p; ++q) y -= T[p * P + q] * X[q * P + j];
+      X[p * P + j] = y;
     }
     for (int p = n - 1; p >= 0; --p) {
-      double y0 = X[p * P + j], y1 = 0.0, y2 = 0.0, y3 = 0.0;
-      int q = p + 1;
-#pragma unroll 2
-      for (; q + 4 <= n; q += 4) {
-        y0 -= T[p * P + q] * X[q * P + j];
-        y1 -= T[p * P + q + 1] * X[(q + 1) * P + j];
-        y2 -= T[p * P + q + 2] * X[(q + 2) * P + j];
-        y3 -= T[p * P + q + 3] * X[(q + 3) * P + j];
-      }
-      for (; q < n; ++q) y0 -= T[p * P + q] * X[q * P + j];
-      const double x = ((y0 + y1) + (y2 + y3)) / T[p * P + p];
-      X[p * P + j] = x;
+      double y = X[p * P + j];
+#pragma unroll 8
+      for (int q = p + 1; q < n; ++q) y -= T[p * P + q] * X[q * P + j];
+      X[p * P + j] = y / T[p * P + p];
+    }
+#pragma unroll 4
+    for (int p = 0; p < n; ++p) {
+      const double x = X[p * P + j];
       isum += fabs(x);
       Minv[bd * n * n + p * n + j] = x;
     }
@@ -323,24 +347,35 @@ __global__ __launch_bounds__(64) void k_det_inv_lds(OrbSrc<TA> src, Shape sh, do
 // ------------------------------------------------------------------------------------------------
 // Channel passes, one matrix per workgroup of 4 waves, wave w taking channels w, w + 4, ...  NB = ceil(n / 16)
 // blocks of 16 per side on v_mfma_f64_16x16x4f64: lane l (g = l / 16, c = l % 16) holds M^-1[16 I + c][16 K + g + 4 q]
-// as A operand (registers for NB = 2) and dM_k[16 K + g + 4 q][16 J + c] as B operand, read from O with the envelope
+// as A operand (registers for NB <= 2) and dM_k[16 K + g + 4 q][16 J + c] as B operand, read from O with the envelope
 // applied (tables of the envelope and of the own-electron terms in LDS); the next channel's O is loaded before this
-// channel's products.  tr(Y^2) = sum_IJ Y_IJ o (Y_JI)^T: a block is transposed through a wave-private LDS tile instead
+// channel's products.  tr(Y^2) = sum_IJ Y_IJ o (Y_JI)^T: blocks are transposed through wave-private LDS tiles instead
 // of being computed a second time as (dM^T M^-T), so a channel is NB^3 x 4 MFMAs of 64 cycles, half of what two
-// products take; tr Y comes from the diagonal the same tile holds.
+// products take.
+//
+// Order of the sums (fixed: an ill-conditioned walker's E_loc, and with it the FP64 loss, turns a rounding here into a
+// last bit): lane l of block (I, J) forms s_IJ = sum_e Y_IJ[4 e + g][c] Y_JI[c][4 e + g]; a chain per lane (NB <= 2) or
+// per lane and J (NB > 2) adds them channel by channel, (I, J) in order, then the lanes meet.  The channels of a round
+// lie in different waves, so they leave their s_IJ in LDS and every wave continues a part of the chains: a barrier or two
+// a round of 4 channels (16 for NB = 1, whose channels are short).  tr Y is one chain of the operands' products per lane.
 // ------------------------------------------------------------------------------------------------
+template <int NB>
+constexpr int chan_region() {  // doubles of LDS per wave: transposition tiles, behind or over them the s_IJ of a round
+  return NB == 1 ? 16 * 17 + 4 * 64 : NB == 2 ? 16 * 17 + 2 * 4 * 64 : NB * NB * 64;
+}
+
 template <int NB, typename TA>
 __global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof(TA) == 4 ? 3 : 2)) void k_det_chan(OrbSrc<TA> src, Shape sh,
                                                                                const double* __restrict__ Minv,
                                                                                double* __restrict__ g,
                                                                                double* __restrict__ lapd, int nmat) {
   extern __shared__ double sm[];
-  constexpr int NP = 16 * NB, PM = NP + 1;
+  constexpr int NP = 16 * NB, PM = NP + 1, REGION = chan_region<NB>(), RC = NB == 1 ? 4 : 1, NT = NB * NB;
+  constexpr bool TWO = NB == 2;  // two buffers of s_IJ: one barrier a round
   const int n = sh.n, nd = 3 * n, C = sh.C;
   double* sM = sm;                        // M^-1, NP x PM, zero outside n x n
-  double* sT = sM + NP * PM;              // transposition tiles, 4 x 16 x 17
-  double* sD = sT + 4 * 16 * 17;          // diagonals of Y_k, nd x 16
-  double* red = sD + nd * 16;             // 32
+  double* sT = sM + NP * PM;              // 4 x REGION; before the rounds the Laplacian channel, n rows of NP
+  double* red = sT + 4 * REGION;          // 32
   TA* sE = (TA*)(red + 32);               // envelope, NP x NP, zero outside
   // own-electron terms g_c bf0, 3 x NP x NP; FP64 orbitals of more than 48 electrons have no room for them and form
   // the channel's row again (4 x NP)
@@ -353,14 +388,10 @@ __global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof
   const int dcol = (int)(bd - b * sh.D) * n;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, gq = lane >> 4, cl = lane & 15;
 
+  TA* const sL = (TA*)sT;
   for (int e = tid; e < NP * NP; e += 256) {
     const int i = e / NP, c = e - (e / NP) * NP;
     sM[i * PM + c] = (i < n && c < n) ? Minv[(long)bd * n * n + i * n + c] : 0.0;
-  }
-  __syncthreads();
-  double tp = 0.0;  // tr(M^-1 Lap M)
-  for (int e = tid; e < NP * NP; e += 256) {
-    const int i = e / NP, c = e - (e / NP) * NP;
     TA env = TA(0), b0 = TA(0), b1 = TA(0), b2 = TA(0);
     if (i < n && c < n) {
       TA g0, g1, g2, le;
@@ -373,8 +404,7 @@ __global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof
       b0 = g0 * bf0;
       b1 = g1 * bf0;
       b2 = g2 * bf0;
-      const TA lp = le * bf0 + env * Oi[(long)(C - 1) * src.ldo] + TA(2) * (g0 * t0 + g1 * t1 + g2 * t2);
-      tp += sM[c * PM + i] * (double)lp;
+      sL[e] = le * bf0 + env * Oi[(long)(C - 1) * src.ldo] + TA(2) * (g0 * t0 + g1 * t1 + g2 * t2);
     }
     sE[e] = env;
     if constexpr (TABLE) {
@@ -384,6 +414,17 @@ __global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof
     }
   }
   __syncthreads();
+  double tp = 0.0;  // tr(M^-1 Lap M): a row of M^-1 per lane, or elements 256 apart per thread
+  if constexpr (NB <= 2) {
+    if (tid < n)
+      for (int e = 0; e < n; ++e) tp += sM[tid * PM + e] * (double)sL[e * NP + tid];
+  } else {
+    for (int e = tid; e < n * n; e += 256) {
+      const int a = e / n, q = e - (e / n) * n;
+      tp += sM[a * PM + q] * (double)sL[q * NP + a];
+    }
+  }
+  __syncthreads();  // sL has been read
 
   constexpr bool REG = NB <= 2;
   double mi[REG ? NB : 1][REG ? NB : 1][4];
@@ -421,81 +462,133 @@ __global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof
         }
       }
   };
-  double* T = sT + wv * 16 * 17;
-  double qacc = 0.0;
+  double* const T = sT + wv * REGION;
+  // s_IJ of channel c of a wave's round: 64 lanes at this place in its region
+  constexpr int S0 = NB <= 2 ? 16 * 17 : 0;
+  int buf = 0;
   constexpr bool AHEAD = sizeof(TA) == 4;  // FP64 orbitals: no registers for a second channel
+  double qacc = 0.0;  // NB <= 2: chain of lane 16 wv + lane (lanes 0 to 15); NB > 2: chain of (J = wv, lane)
   if (AHEAD && wv < nd) load(wv);
-  for (int k = wv; k < nd; k += 4) {
-    const int kr = k / 3, kc = k - 3 * kr;  // the channel's electron and axis
-    double dm[NB][NB][4];
-    if (!AHEAD) load(k);
-    if constexpr (!TABLE) {
-      TA own = TA(0);
-      if (lane < n) {
-        TA env, g0, g1, g2, le;
-        envelope_at<TA, true>(src.kappa, src.wenv, src.r, src.R, sh, b, kr, dcol + lane, env, g0, g1, g2, le);
-        own = (kc == 0 ? g0 : kc == 1 ? g1 : g2) * src.O[orb_row(sh, b, kr) * src.ldo + dcol + lane];
-      }
-      sG[wv * NP + lane] = own;  // NP == 64; read by this wave only, in order
-    }
+  for (int k0 = 0; k0 < nd; k0 += 4 * RC) {  // every wave takes every round (barriers)
+    double gp[4];  // NB > 2: tr Y's chains
+    gp[3] = 0.0;
 #pragma unroll
-    for (int K = 0; K < NB; ++K)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int rr = K * 16 + gq + 4 * q;
-        const TA* er = sE + rr * NP + cl;
-        const TA* gr = (TABLE ? sG + (kc * NP + rr) * NP : sG + wv * NP) + cl;
-#pragma unroll
-        for (int J = 0; J < NB; ++J) {
-          const TA own = rr == kr ? gr[16 * J] : TA(0);
-          dm[K][J][q] = (double)fma(er[16 * J], nxt[K][J][q], own);
+    for (int rc = 0; rc < RC; ++rc) {
+      const int k = k0 + 4 * rc + wv;
+      if (k >= nd) break;  // uniform over the wave
+      const int kr = k / 3, kc = k - 3 * kr;  // the channel's electron and axis
+      double dm[NB][NB][4];
+      if (!AHEAD) load(k);
+      if constexpr (!TABLE) {
+        TA own = TA(0);
+        if (lane < n) {
+          TA env, g0, g1, g2, le;
+          envelope_at<TA, true>(src.kappa, src.wenv, src.r, src.R, sh, b, kr, dcol + lane, env, g0, g1, g2, le);
+          own = (kc == 0 ? g0 : kc == 1 ? g1 : g2) * src.O[orb_row(sh, b, kr) * src.ldo + dcol + lane];
         }
+        sG[wv * NP + lane] = own;  // NP == 64; read by this wave only, in order
       }
-    if (AHEAD && k + 4 < nd) load(k + 4);
-    __builtin_amdgcn_sched_barrier(0);  // the products follow one block pair at a time (register budget)
-    double gp = 0.0;
 #pragma unroll
-    for (int I = 0; I < NB; ++I)
+      for (int K = 0; K < NB; ++K)
 #pragma unroll
-      for (int J = I; J < NB; ++J) {
-        v4d y = {0.0, 0.0, 0.0, 0.0}, z = y;
+        for (int q = 0; q < 4; ++q) {
+          const int rr = K * 16 + gq + 4 * q;
+          const TA* er = sE + rr * NP + cl;
+          const TA* gr = (TABLE ? sG + (kc * NP + rr) * NP : sG + wv * NP) + cl;
 #pragma unroll
-        for (int K = 0; K < NB; ++K)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            y = __builtin_amdgcn_mfma_f64_16x16x4f64(mia(I, K, q), dm[K][J][q], y, 0, 0, 0);
-            if (J > I) z = __builtin_amdgcn_mfma_f64_16x16x4f64(mia(J, K, q), dm[K][I][q], z, 0, 0, 0);
+          for (int J = 0; J < NB; ++J) {
+            const TA own = rr == kr ? gr[16 * J] : TA(0);
+            dm[K][J][q] = (double)fma(er[16 * J], nxt[K][J][q], own);
           }
-        if (J == I) z = y;
-        // lane l, element e: row 4 e + g, column c of the block (LDS accesses of one wave stay in order)
+        }
+      if (AHEAD && k + 4 < nd) load(k + 4);
+      __builtin_amdgcn_sched_barrier(0);  // the products follow one block pair at a time (register budget)
+      double st[NT], t = 0.0;  // t: tr Y, the operands' products over (I, K, q); above 32 electrons a chain for each I
 #pragma unroll
-        for (int e = 0; e < 4; ++e) T[(4 * e + gq) * 17 + cl] = z[e];
-        double s = 0.0;
+      for (int I = 0; I < NB; ++I)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s += y[e] * T[cl * 17 + 4 * e + gq];
-        qacc += J > I ? 2.0 * s : s;
-        if (J == I) gp += T[cl * 18];
-        __builtin_amdgcn_sched_barrier(0);
+        for (int J = I; J < NB; ++J) {
+          v4d y = {0.0, 0.0, 0.0, 0.0}, z = y;
+          if (NB > 2 && J == I) t = 0.0;
+#pragma unroll
+          for (int K = 0; K < NB; ++K)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              y = __builtin_amdgcn_mfma_f64_16x16x4f64(mia(I, K, q), dm[K][J][q], y, 0, 0, 0);
+              if (J > I) z = __builtin_amdgcn_mfma_f64_16x16x4f64(mia(J, K, q), dm[K][I][q], z, 0, 0, 0);
+              if (J == I) t += mia(I, K, q) * dm[K][I][q];
+            }
+          if constexpr (NB > 2)
+            if (J == I) gp[I] = t;
+          // lane l, element e: row 4 e + g, column c of the block (LDS accesses of one wave stay in order)
+          auto against = [&](double* tile, const v4d& a, const v4d& other) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) tile[(4 * e + gq) * 17 + cl] = other[e];
+            v4d w;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = tile[cl * 17 + 4 * e + gq];
+            return a[0] * w[0] + a[1] * w[1] + a[2] * w[2] + a[3] * w[3];
+          };
+          if (J == I) {
+            st[I * NB + I] = against(T, y, y);
+          } else {
+            st[I * NB + J] = against(T, y, z);
+            st[J * NB + I] = against(T + (NB > 2 ? 16 * 17 : 0), z, y);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+      for (int x = 0; x < NT; ++x) T[S0 + buf + (rc * NT + x) * 64 + lane] = st[x];  // over the tiles (NB > 2), now read
+      if constexpr (NB <= 2) {
+        const double s = wave_sum_dpp(t);
+        if (lane == 0) g[(long)bd * nd + k] = s;
+      } else {
+        const double s = wave_sums_dpp(gp[0], gp[1], gp[2], gp[3]);
+        const double s0 = readlane_d(s, 0), s1 = readlane_d(s, 32), s2 = readlane_d(s, 16), s3 = readlane_d(s, 48);
+        if (lane == 0) g[(long)bd * nd + k] = ((s0 + s1) + s2) + s3;
       }
-    if (lane < 16) sD[k * 16 + lane] = gp;
-  }
-  qacc = block_sum_d(qacc, red);
-  tp = block_sum_d(tp, red + 16);
-  __syncthreads();
-  for (int k = tid; k < nd; k += 256) {
-    double s = 0.0;
+    }
+    __syncthreads();  // every wave's s_IJ of the round are in LDS
+    const int nc = min(4 * RC, nd - k0);
+    if constexpr (NB <= 2) {
+      if (lane < 16)
+        for (int c = 0; c < nc; ++c) {
+          const double* p = sT + (c & 3) * REGION + S0 + buf + (c >> 2) * NT * 64 + 16 * wv + lane;
 #pragma unroll
-    for (int c = 0; c < 16; ++c) s += sD[k * 16 + c];
-    g[(long)bd * nd + k] = s;
+          for (int x = 0; x < NT; ++x) qacc += p[64 * x];
+        }
+    } else if (wv < NB) {
+      for (int c = 0; c < nc; ++c) {
+        const double* p = sT + c * REGION + wv * 64 + lane;
+#pragma unroll
+        for (int I = 0; I < NB; ++I) qacc += p[I * NB * 64];
+      }
+    }
+    if constexpr (TWO)
+      buf ^= NT * 64;
+    else
+      __syncthreads();  // and have been read
   }
-  if (tid == 0) lapd[bd] = tp - qacc;
+  if constexpr (NB <= 2) {  // the 64 chains to the lanes of wave 0
+    if (lane < 16) sT[16 * wv + lane] = qacc;
+    __syncthreads();
+    if (wv == 0) {
+      const double q = wave_sum_d(sT[lane]);
+      tp = wave_sum_d(tp);
+      if (lane == 0) lapd[bd] = tp - q;
+    }
+  } else {
+    qacc = block_sum_d(qacc, red);
+    tp = block_sum_d(tp, red + 16);
+    if (tid == 0) lapd[bd] = tp - qacc;
+  }
 }
 
 template <int NB, typename TA>
 static void launch_chan(const OrbSrc<TA>& src, const Shape& sh, const double* Minv, double* g, double* lapd,
                         hipStream_t s) {
   constexpr int NP = 16 * NB;
-  const size_t shm = (size_t)(NP * (NP + 1) + 4 * 16 * 17 + 3 * sh.n * 16 + 32) * sizeof(double) +
+  const size_t shm = (size_t)(NP * (NP + 1) + 4 * chan_region<NB>() + 32) * sizeof(double) +
                      ((size_t)NP * NP + (NB < 4 || sizeof(TA) == 4 ? 3 * NP * NP : 4 * NP)) * sizeof(TA);
   if (shm > 65536)
     (void)hipFuncSetAttribute((const void*)k_det_chan<NB, TA>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);

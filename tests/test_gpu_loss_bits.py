@@ -1,5 +1,5 @@
-"""The loss's FP64 statistics bit for bit (dpe4 model): loss, clipping state and local energies against values stored in
-``golden/loss_bits.npz``.
+"""The loss's FP64 statistics bit for bit: loss, clipping state and local energies (dpe4 model) against values stored in
+``golden/loss_bits.npz``, local energies of ill-conditioned walkers (FermiNet) against ``golden/energy_bits.npz``.
 
 The stored values are the library's own, from commit 9ab37b9 (``golden/make_loss_bits.py``): these quantities leave in FP64
 or feed a clipping state that is carried from run to run, so kernels may be replaced but their roundings may not.
@@ -22,9 +22,17 @@ FILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "loss_
 CASES = [("dpe4", 2, 16, 30), ("dpe4", 5, 32, 19), ("dpe4", 9, 8, 13), ("dpe4", 14, 16, 12), ("dpe4", 16, 8, 9),
          ("dpe4", 17, 32, 8), ("dpe4", 26, 8, 7), ("dpe4", 33, 8, 6), ("dpe4", 42, 16, 5)]
 
+ENERGY_FILE = os.path.join(os.path.dirname(FILE), "energy_bits.npz")
+
+# (precision, electrons, determinants, seeded walkers, those taken): walkers whose last bit shows the order of FP64 sums
+ENERGIES = [("fp32", 16, 8, 8000, (1055,)), ("fp32", 17, 8, 8000, (5569, 7831)), ("fp32", 26, 8, 4000, (3225,)),
+            ("fp32", 32, 8, 2000, (1069, 1805)), ("fp32", 33, 8, 4000, (645, 925, 962, 2560, 2699)),
+            ("fp32", 42, 8, 3000, (952, 2970)), ("fp32", 52, 4, 2000, (2, 54, 119, 1555)),
+            ("fp32", 63, 4, 1000, (131, 257, 305, 570, 887, 968))]
+
 
 def key(case) -> str:
-    return "%s_%d_%d_%d" % case
+    return "_".join(str(x) for x in case[:4])
 
 
 def statistics(case):
@@ -60,3 +68,29 @@ def test_loss_statistics_keep_their_bits(cuda, case):
     for got, ref in zip(statistics(case), want):
         assert got.dtype == ref.dtype
         np.testing.assert_array_equal(got, ref)
+
+
+def energies(case):
+    """E_loc of the case's walkers, in the form that the loss takes."""
+    import torch
+
+    from deeperwin_amd._native import LAP_FP32, NativeModel
+
+    precision, n, D, B, rows = case
+    R, Z = random_molecule(np.random.default_rng(n), n)
+    R = R.astype(np.float32)
+    shape = ModelShape(n, (n + 1) // 2, len(Z), D)
+    m = NativeModel(shape, precision)
+    m.set_params(init_params(shape, n))
+    m.set_lap_form(LAP_FP32)
+    r = init_walkers_gaussian(np.random.default_rng(1), B, R, generate_el_ion_mapping(R, Z, n, shape.n_up))
+    r = torch.as_tensor(r[list(rows)], dtype=torch.float32, device="cuda").contiguous()
+    e = torch.empty(len(r), device="cuda")
+    m.local_energy(r, torch.as_tensor(R, device="cuda"), torch.as_tensor(np.asarray(Z), dtype=torch.float32, device="cuda"), e)
+    return e.cpu().numpy()
+
+
+@pytest.mark.parametrize("case", ENERGIES, ids=key)
+def test_energies_of_ill_conditioned_walkers_keep_their_bits(cuda, case):
+    with np.load(ENERGY_FILE) as g:
+        np.testing.assert_array_equal(energies(case), g[key(case)])
