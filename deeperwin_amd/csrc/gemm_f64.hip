@@ -7,9 +7,11 @@ namespace dwmi {
 
 // ------------------------------------------------------------------------------------------------
 // Tile (32 WM) x (32 WN) per 256-thread workgroup; 4 waves in 2 x 2, each wave owns WM x WN blocks of 16 x 16.
-// Both operand slices (16 k) are staged untransposed in LDS, two buffers and one barrier per slice; MFMA step s
-// of lane group g = lane / 16 takes k = 4 g + s, so a lane reads its operands of a slice as two 16-byte vectors
-// per block (row pitch 18 doubles: the 16 rows of a read start 4 banks apart).  A block's step takes the matrix
+// Both operand slices (16 k) are staged in LDS, two buffers and one barrier per slice; MFMA step s of lane group
+// g = lane / 16 takes k = 4 s + g, so that an element is one chain over k ascending, as a VALU kernel forms it (in another
+// order ill-conditioned walkers' E_loc differ in the last bit, 1 of 500 at 42 electrons).  Element k of a row lies at
+// 4 (k % 4) + k / 4: a lane reads its operands of a slice as two 16-byte vectors per block (row pitch 18 doubles: the 16
+// rows of a read start 4 banks apart).  A block's step takes the matrix
 // core 64 cycles and needs 16 bytes per lane from LDS for WM + WN blocks of operands, so the matrix core bounds
 // it (a VALU tile of 4 x 4 per thread waited on LDS: 64 bytes per 16 multiply-adds).  172,032 x 320 x 256 (256
 // walkers of 14 electrons, Laplacian pass): 1160 us with the VALU tile, 533 us with this (53 TFLOP/s; 60 without
@@ -52,11 +54,18 @@ __global__ __launch_bounds__(256) void k_gemm_f64(const double* __restrict__ A, 
       rb[it] = *(const v2d*)(Bt + (long)(col0 + (idx >> 3)) * ldb + k0 + (idx & 7) * 2);
     }
   };
+  const int at = 8 * (tid & 1) + ((tid & 7) >> 1);  // place of k = 2 (tid % 8); k + 1 lies 4 further
   auto sstore = [&](int buf) {
 #pragma unroll
-    for (int it = 0; it < AIT; ++it) *(v2d*)&As[buf][(tid + 256 * it) >> 3][(tid & 7) * 2] = ra[it];
+    for (int it = 0; it < AIT; ++it) {
+      As[buf][(tid + 256 * it) >> 3][at] = ra[it][0];
+      As[buf][(tid + 256 * it) >> 3][at + 4] = ra[it][1];
+    }
 #pragma unroll
-    for (int it = 0; it < BIT; ++it) *(v2d*)&Bs[buf][(tid + 256 * it) >> 3][(tid & 7) * 2] = rb[it];
+    for (int it = 0; it < BIT; ++it) {
+      Bs[buf][(tid + 256 * it) >> 3][at] = rb[it][0];
+      Bs[buf][(tid + 256 * it) >> 3][at + 4] = rb[it][1];
+    }
   };
 
   const int S = K / BK;

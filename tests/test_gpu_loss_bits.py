@@ -28,7 +28,10 @@ ENERGY_FILE = os.path.join(os.path.dirname(FILE), "energy_bits.npz")
 ENERGIES = [("fp32", 16, 8, 8000, (1055,)), ("fp32", 17, 8, 8000, (5569, 7831)), ("fp32", 26, 8, 4000, (3225,)),
             ("fp32", 32, 8, 2000, (1069, 1805)), ("fp32", 33, 8, 4000, (645, 925, 962, 2560, 2699)),
             ("fp32", 42, 8, 3000, (952, 2970)), ("fp32", 52, 4, 2000, (2, 54, 119, 1555)),
-            ("fp32", 63, 4, 1000, (131, 257, 305, 570, 887, 968))]
+            ("fp32", 63, 4, 1000, (131, 257, 305, 570, 887, 968)),
+            ("fp64", 14, 8, 15000, (3158, 6227)), ("fp64", 16, 8, 10000, (5816,)), ("fp64", 17, 8, 7500, (975, 1496)),
+            ("fp64", 26, 8, 4000, (887, 988, 1230, 1314, 2039)), ("fp64", 33, 8, 2500, (20, 950, 1594, 2383)),
+            ("fp64", 42, 8, 1500, (176,)), ("fp64", 52, 4, 1000, (54, 119, 284)), ("fp64", 63, 4, 500, (131, 257))]
 
 
 def key(case) -> str:
