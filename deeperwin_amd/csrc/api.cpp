@@ -725,7 +725,7 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
       if (split) {
         // derivative channels of V, then the value channel (row 0 of each electron) with the value pass's
         // arithmetic, then the derivative channels of the layer
-        split_mean(X[l], m->Kx[l], m->Kh[l], W.WmuS[l].p, m->Km[l], 3, ws.V, m->W1, sh, s);
+        split_mean(X[l], m->Kx[l], m->Kh[l], W.WmuS[l].p, m->Km[l], ws.V, m->W1, sh, s);
         const int ldx = Cp * m->Kx[l], Km = m->Km[l];
         if (value_done <= l &&
             value_layer(X[l], ldx, m->Kx[l], m->Kh[l], W.WmainL[l].p, W.WmuL[l].p, Km, W.bias[l].as<float>(), 1, outp,
@@ -761,27 +761,14 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
         continue;
       }
     }
-    // Laplacian pass: spin means formed inside the per-walker GEMM (FP32 form: same values as below; BF16x3 form: the
-    // same three products, added over 32 k at a time)
+    // Laplacian pass: spin means formed inside the per-walker GEMM (same values as below)
     bool fused_mu = false;
     if constexpr (!DBL) {
       if (C > 1 && m->prec == GEMM_F32)
         fused_mu = gemm_mean_lap(X[l], m->Kx[l], m->Kh[l], W.Wmu[l].as<float>(), m->Km[l], W.bias[l].as<float>(),
                                  ws.V, m->W1, sh, s);
-      if (C > 1 && m->prec == GEMM_BF16X3 && m->lap_form == DW_LAP_SPLIT && m->tune.lap_mu_tile < 0 && m->W1 % 64 == 0) {
-        split_mean(X[l], m->Kx[l], m->Kh[l], W.WmuS[l].p, m->Km[l], 2, ws.V, m->W1, sh, s);
-        // the value rows with the value pass's arithmetic: a rounding there moves the BF16 parts of all that follows
-        Shape s1 = sh;
-        s1.C = 1;
-        s1.Cp = 1;
-        launch_spin_mean<float>(X[l], Cp * m->Kx[l], m->Kh[l], ws.MU, m->Km[l], s1, s);
-        GemmEpi e1;
-        e1.bias = W.bias[l].as<float>();
-        e1.nC = m->n;
-        gemm_t(m, ws.MU, m->Km[l], W.Wmu[l].as<T>(), W.Wmu_hi[l], W.Wmu_lo[l], m->Km[l], ws.V, Cp * m->W1, (int)B, m->W1,
-               m->Km[l], e1, s);
-        fused_mu = true;
-      }
+      if (C > 1 && m->prec == GEMM_BF16X3 && m->tune.lap_mu_tile < 0)
+        fused_mu = mean_bf16x3(X[l], m->Kx[l], m->Kh[l], W.WmuS[l].p, m->Km[l], W.bias[l].as<float>(), ws.V, m->W1, sh, s);
     }
     if (!fused_mu) launch_spin_mean<T>(X[l], m->Kx[l], m->Kh[l], ws.MU, m->Km[l], sh, s);
     GemmEpiT<T> ev;

@@ -39,6 +39,12 @@ __device__ __forceinline__ unsigned pack_bf16(float a, float b) {  // v_cvt_pk_b
 __device__ __forceinline__ float lo_f(unsigned u) { return __uint_as_float(u << 16); }
 __device__ __forceinline__ float hi_f(unsigned u) { return __uint_as_float(u & 0xFFFF0000u); }
 
+// v * f, rounded: a part's rest is not fused with it.
+__device__ __forceinline__ v4f scaled(v4f v, float f) {
+#pragma clang fp contract(off)
+  return v4f{v[0] * f, v[1] * f, v[2] * f, v[3] * f};
+}
+
 // Four floats -> the three parts of each, packed in 8 bytes per part.
 __device__ __forceinline__ void split4(v4f x, uint2 (&p)[3]) {
   const unsigned h0 = pack_bf16(x[0], x[1]), h1 = pack_bf16(x[2], x[3]);
@@ -592,15 +598,19 @@ int split_lap(const float* X, int ldx, const void* P, int shift, int K, const fl
 // A workgroup forms the means of 48 rows x 128 k at a time and splits them straight into LDS (37 KB: four workgroups
 // per CU, whose load and MFMA phases overlap); the weights' parts come from L2.  Bound by the read of X's h columns
 // (1.41 GB for 2048 walkers of 14 electrons: 364 us = 3.9 TB/s against 471 us with FP32 MFMA; 26 electrons, 1024
-// walkers: 575 -> 461 us; 256 LiH walkers: 67 -> 28 us a layer with 64 columns per workgroup).  NP = 2 keeps the first two parts
-// and three products, the BF16x3 form's arithmetic (1,000 walkers of 14: 206 us a layer in two launches, 159 + 15 for the
-// value rows here).
+// walkers: 575 -> 461 us; 256 LiH walkers: 67 -> 28 us a layer with 64 columns per workgroup).
+//
+// NP = 2 is the BF16x3 form: the first two parts and three products, every row (the value channel and its bias too), 64
+// rows.  Its sums are k_gemm_bf16's (v_mfma_f32_32x32x16_bf16 over 16 k at a time, low x high, high x low, high x high), so
+// results are bit-equal to the separate kernels (k_spin_mean and that GEMM), which small batches keep (launch_mean).
 // ------------------------------------------------------------------------------------------------
 template <int NQ, int NP, bool FEW>
-__global__ __launch_bounds__(256) void k_split_mean(const float* __restrict__ X, int Kx, int Kh,
+__global__ __launch_bounds__(256, NP == 2 ? 4 : 1) void k_split_mean(const float* __restrict__ X, int Kx, int Kh,
                                                     const uint4* __restrict__ P, int ncb, int Km,
-                                                    float* __restrict__ V, int ldv, Shape sh, int tilesN, int total) {
-  constexpr int RB = 3, CS = 4;  // row blocks, 32-wide slices per chunk
+                                                    const float* __restrict__ bias, float* __restrict__ V, int ldv,
+                                                    Shape sh, int tilesN, int total) {
+  constexpr int RB = NP == 2 ? 4 : 3, CS = 4;  // row blocks, 32-wide slices per chunk
+  static_assert(NP == 3 || (NQ == 4 && !FEW), "the BF16x3 form takes 64 columns a wave");
   __shared__ uint4 lds[CS][NP][RB][64];
   const int tile = tile_of(blockIdx.x, total);
   if (tile >= total) return;  // uniform over the workgroup, before any barrier
@@ -609,20 +619,34 @@ __global__ __launch_bounds__(256) void k_split_mean(const float* __restrict__ X,
   const int cb0 = (tile % tilesN) * (4 * NQ) + wv * NQ;
   const int n = sh.n, u = sh.u, Cp = sh.Cp;
   const long xstride = (long)Cp * Kx;  // one electron further
-  v4f acc[RB][NQ];
+  v4f acc[NP == 3 ? RB : 1][NQ];
+  v16f acc2[NP == 2 ? 2 : 1][NP == 2 ? 2 : 1];  // 32 x 32 blocks
+  if constexpr (NP == 3) {
 #pragma unroll
-  for (int i = 0; i < RB; ++i)
+    for (int i = 0; i < RB; ++i)
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) acc[i][q] = v4f{0.f, 0.f, 0.f, 0.f};
+      for (int q = 0; q < NQ; ++q) acc[i][q] = v4f{0.f, 0.f, 0.f, 0.f};
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc2[i][q][j] = 0.f;
+  }
   for (int kc = 0; kc < Km; kc += 32 * CS) {
     const int ns = min(CS, (Km - kc) >> 5);
     __syncthreads();  // the previous chunk's reads are done
     // consecutive lanes take consecutive quads of a row (coalesced); 4 quads a slice-row group
     auto put = [&](int rr, int qd, v4f v, float inv) {
-      v[0] *= inv;
-      v[1] *= inv;
-      v[2] *= inv;
-      v[3] *= inv;
+      if constexpr (NP == 2) {
+        v = scaled(v, inv);
+      } else {
+        v[0] *= inv;
+        v[1] *= inv;
+        v[2] *= inv;
+        v[3] *= inv;
+      }
       uint2 p[3];
       split4(v, p);
       const int quad = qd & 7;
@@ -700,66 +724,112 @@ __global__ __launch_bounds__(256) void k_split_mean(const float* __restrict__ X,
     }
     __syncthreads();
     for (int s = 0; s < ns; ++s) {
-      v8s b[NQ][NP];
+      if constexpr (NP == 3) {
+        v8s b[NQ][NP];
 #pragma unroll
-      for (int q = 0; q < NQ; ++q)
+        for (int q = 0; q < NQ; ++q)
 #pragma unroll
-        for (int m = 0; m < NP; ++m)
-          b[q][m] = *(const v8s*)&P[((long)(((kc >> 5) + s) * ncb + cb0 + q) * 3 + m) * 64 + lane];
+          for (int m = 0; m < NP; ++m)
+            b[q][m] = *(const v8s*)&P[((long)(((kc >> 5) + s) * ncb + cb0 + q) * 3 + m) * 64 + lane];
 #pragma unroll
-      for (int i = 0; i < RB; ++i) {
-        v8s a[NP];
+        for (int i = 0; i < RB; ++i) {
+          v8s a[NP];
 #pragma unroll
-        for (int m = 0; m < NP; ++m) a[m] = *(const v8s*)&lds[s][m][i][lane];
-        if constexpr (NP == 3) {
+          for (int m = 0; m < NP; ++m) a[m] = *(const v8s*)&lds[s][m][i][lane];
           DW_SPLIT_MFMA(2, 0)
           DW_SPLIT_MFMA(0, 2)
           DW_SPLIT_MFMA(1, 1)
+          DW_SPLIT_MFMA(1, 0)
+          DW_SPLIT_MFMA(0, 1)
+          DW_SPLIT_MFMA(0, 0)
         }
-        DW_SPLIT_MFMA(1, 0)
-        DW_SPLIT_MFMA(0, 1)
-        DW_SPLIT_MFMA(0, 0)
+      } else {
+        // lane l of a 32 x 32 x 16 block: row or column l % 32 (of two 16-blocks), k = 16 h + 8 (l / 32) + 0..7
+        const int blk = (lane >> 4) & 1;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int at = (lane & 15) + 16 * (2 * h + (lane >> 5));
+          v8s a[2][2], b[2][2];
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+              a[q][m] = *(const v8s*)&lds[s][m][2 * q + blk][at];
+              b[q][m] = *(const v8s*)&P[((long)(((kc >> 5) + s) * ncb + cb0 + 2 * q + blk) * 3 + m) * 64 + at];
+            }
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+              acc2[i][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16((v8bf)a[i][1], (v8bf)b[q][0], acc2[i][q], 0, 0, 0);
+              acc2[i][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16((v8bf)a[i][0], (v8bf)b[q][1], acc2[i][q], 0, 0, 0);
+              acc2[i][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16((v8bf)a[i][0], (v8bf)b[q][0], acc2[i][q], 0, 0, 0);
+            }
+        }
       }
     }
   }
+  if constexpr (NP == 3) {
 #pragma unroll
-  for (int i = 0; i < RB; ++i)
+    for (int i = 0; i < RB; ++i)
 #pragma unroll
-    for (int q = 0; q < NQ; ++q)
+      for (int q = 0; q < NQ; ++q)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const long r = r0 + i * 16 + 4 * (lane >> 4) + j;
-        if (r < rows) V[r * ldv + (cb0 + q) * 16 + (lane & 15)] = acc[i][q][j];
-      }
-}
-
-template <int NP>
-static void launch_mean(const float* X, int Kx, int Kh, const void* P, int Km, float* V, int ldv, const Shape& sh,
-                        hipStream_t s) {
-  const int ncb = dw_pad(sh.W1, 256) / 16;
-  const long tilesM = ((long)sh.B * sh.Cp + 47) / 48;
-  // 256 columns (X read once) where that gives two workgroups to every CU
-  if (sh.W1 % 256 == 0 && tilesM * (sh.W1 / 256) >= 512) {
-    const int tilesN = sh.W1 / 256, total = (int)(tilesM * tilesN);
-    hipLaunchKernelGGL((k_split_mean<4, NP, false>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh, (const uint4*)P,
-                       ncb, Km, V, ldv, sh, tilesN, total);
+        for (int j = 0; j < 4; ++j) {
+          const long r = r0 + i * 16 + 4 * (lane >> 4) + j;
+          if (r < rows) V[r * ldv + (cb0 + q) * 16 + (lane & 15)] = acc[i][q][j];
+        }
   } else {
-    const int tilesN = sh.W1 / 64, total = (int)(tilesM * tilesN);
-    if (sh.u <= 4 && sh.n - sh.u <= 4)
-      hipLaunchKernelGGL((k_split_mean<1, NP, true>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh,
-                         (const uint4*)P, ncb, Km, V, ldv, sh, tilesN, total);
-    else
-      hipLaunchKernelGGL((k_split_mean<1, NP, false>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh,
-                         (const uint4*)P, ncb, Km, V, ldv, sh, tilesN, total);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int c = cb0 * 16 + 32 * q + (lane & 31);
+      const float bc = bias[c];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const long r = r0 + 32 * i + 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3);
+          if (r < rows) {
+            float v = acc2[i][q][j];
+            if ((unsigned)r % (unsigned)Cp == 0) v += bc;
+            V[r * ldv + c] = v;
+          }
+        }
+    }
   }
 }
 
-void split_mean(const float* X, int Kx, int Kh, const void* P, int Km, int parts, float* V, int ldv, const Shape& sh,
-                hipStream_t s) {
-  if (parts == 3)
-    launch_mean<3>(X, Kx, Kh, P, Km, V, ldv, sh, s);
+template <int NQ, bool FEW>
+static void mean_launch3(const float* X, int Kx, int Kh, const void* P, int ncb, int Km, float* V, int ldv, const Shape& sh,
+                         hipStream_t s) {
+  const int tilesN = sh.W1 / (64 * NQ), total = (int)(((long)sh.B * sh.Cp + 47) / 48 * tilesN);
+  hipLaunchKernelGGL((k_split_mean<NQ, 3, FEW>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh, (const uint4*)P, ncb,
+                     Km, (const float*)nullptr, V, ldv, sh, tilesN, total);
+}
+
+void split_mean(const float* X, int Kx, int Kh, const void* P, int Km, float* V, int ldv, const Shape& sh, hipStream_t s) {
+  const int ncb = dw_pad(sh.W1, 256) / 16;
+  // 256 columns (X read once) where that gives two workgroups to every CU
+  if (sh.W1 % 256 == 0 && ((long)sh.B * sh.Cp + 47) / 48 * (sh.W1 / 256) >= 512)
+    mean_launch3<4, false>(X, Kx, Kh, P, ncb, Km, V, ldv, sh, s);
+  else if (sh.u <= 4 && sh.n - sh.u <= 4)
+    mean_launch3<1, true>(X, Kx, Kh, P, ncb, Km, V, ldv, sh, s);
   else
-    launch_mean<2>(X, Kx, Kh, P, Km, V, ldv, sh, s);
+    mean_launch3<1, false>(X, Kx, Kh, P, ncb, Km, V, ldv, sh, s);
+}
+
+// From 600 tiles of 64 rows up, where the fused kernel keeps every CU busy; below, its few workgroups form their means one
+// after another and the two separate kernels win.  E_loc, separate / fused: 14 electrons 510 / 702 us (85 walkers, 64
+// tiles), 1,939 / 2,052 (583, 438), 2,794 / 2,766 (833, 625), 3,306 / 3,236 (1,000, 750), 4,384 / 4,225 (1,365, 1,024); 8
+// electrons 1,184 / 1,262 (438 tiles), 1,739 / 1,705 (625); 26 electrons 1,287 / 1,460 (128), 5,350 / 5,189 (625).
+bool mean_bf16x3(const float* X, int Kx, int Kh, const void* P, int Km, const float* bias, float* V, int ldv, const Shape& sh,
+                 hipStream_t s) {
+  const long tilesM = ((long)sh.B * sh.Cp + 63) / 64;
+  if (sh.W1 % 256 != 0 || tilesM * (sh.W1 / 256) < 600) return false;
+  const int tilesN = sh.W1 / 256, total = (int)(tilesM * tilesN);
+  hipLaunchKernelGGL((k_split_mean<4, 2, false>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh, (const uint4*)P,
+                     dw_pad(sh.W1, 256) / 16, Km, bias, V, ldv, sh, tilesN, total);
+  return true;
 }
 
 }  // namespace dwmi

@@ -67,10 +67,13 @@ void launch_split_pack16(const float* Bt, int ldb, int cols, int K, int shift, v
 // depend on it).
 void split_gemm(const float* A, int lda, const void* P16, int shift, const float* amax, int np, int ms, int rbe, float* C,
                 int ldc, int M, int N, int K, int tile, hipStream_t s);
-// V[(b Cp + ch), o] of the derivative channels: spin means of X's first Kh columns times W_mu (no bias), from `parts`
-// BF16 parts of each (3: FP32 accuracy; 2: the BF16x3 form's products).
-void split_mean(const float* X, int Kx, int Kh, const void* P, int Km, int parts, float* V, int ldv, const Shape& sh,
-                hipStream_t s);
+// V[(b Cp + ch), o] of the derivative channels: spin means of X's first Kh columns times W_mu (no bias), from three BF16 parts
+// of each (FP32 accuracy).
+void split_mean(const float* X, int Kx, int Kh, const void* P, int Km, float* V, int ldv, const Shape& sh, hipStream_t s);
+// The same for the BF16x3 form, all channels and the bias, bit-equal to launch_spin_mean and its GEMM; false, launching
+// nothing, where the batch is too small to gain.
+bool mean_bf16x3(const float* X, int Kx, int Kh, const void* P, int Km, const float* bias, float* V, int ldv, const Shape& sh,
+                 hipStream_t s);
 // 1-el GEMM and tanh forward-Laplacian rule of the derivative channels; `out` holds the value channel already.  With
 // amax (np maxima per electron, W1 / 32 apart, covering all but the last `tail` <= 2 slices of 32 columns; K a multiple of 64)
 // P is in FP16 parts, without it in BF16 parts.  omax (W1 / 32 places per electron, in the order of out's rows) receives the maxima

@@ -265,8 +265,7 @@ dw_status dw_model_get_tuning(const dw_model* m, dw_tuning* out);
  * on 16-bit MFMA; E_loc as accurate as with FP32 and 1.3 to 1.9 times faster, equal to it to rounding.  FP32: FP32
  * MFMA.  The value channel (log|psi|^2, the determinants) is the same bits in both.  For callers whose FP64 statistics
  * of the energies (the optimisation's loss and clipping state) have to stay bit-equal from run to run, across releases:
- * the loss uses FP32.  In the DW_BF16X3 form the same switch chooses between forming the spin means inside their product
- * (SPLIT) and in a pass before it; the same BF16 products either way. */
+ * the loss uses FP32.  The other precision forms have one form only. */
 #define DW_LAP_SPLIT 0
 #define DW_LAP_FP32 1
 dw_status dw_model_set_lap_form(dw_model* m, int32_t form);
