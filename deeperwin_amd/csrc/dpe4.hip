@@ -18,6 +18,7 @@
 // k_dpe4_conv and k_dpe4_conv_lap (e_ee into X_l).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 
@@ -432,32 +433,37 @@ __global__ __launch_bounds__(256) void k_dpe4_conv(const T* __restrict__ wm, con
 // Laplacian pass: e_ee[i][ch][f] = sum_j w[i, j][f] hm[j][ch][f] plus the pair derivatives:
 //   tangent row (e, c):  + (delta_{e j} - delta_{e i}) g_c[i, j] hm[j][0]
 //   Laplacian row:       + L_w[i, j] hm[j][0] + 2 sum_c g_c[i, j] (hm[j][(j, c)] - hm[j][(i, c)])
-// (g = d w / d d, L_w the pair's total Laplacian; the self pair's w is constant).  One workgroup per walker, its w in
-// LDS for NI electrons i at a time; a thread owns (channel row, f) and NI electrons i, so every element of hm is read
-// once per NI and the row's own e is fixed: its derivative terms are NI products at j = e, and one chain of its own
-// for i = e.  The Laplacian row takes a group of 32 lanes per electron i.  Terms are added in order of j.
+// (g = d w / d d, L_w the pair's total Laplacian; the self pair's w is constant).  A workgroup takes a walker,
+// w of NI electrons i at a time in LDS (all blocks of NI in turn, or one) and a part of the channel rows (conv_launch says
+// how many); a thread owns (channel row, f) and NI electrons i, so every element of hm is read once per NI and the row's own
+// e is fixed: its derivative terms are NI products at j = e, and one chain of its own for i = e.  The Laplacian row takes a
+// group of 32 lanes per electron i.  Terms are added in order of j, whatever the split.
 // What bounds it: memory, w and hm read two to three times (the derivative terms' rows no longer in L2), e_ee written.
 // 1,024 walkers of 14 (48 rows): 269 us with a thread per (i, f) and 16
 // channel rows testing each row against (i, j), 196 us here.
 // ------------------------------------------------------------------------------------------------------
 template <int NI, typename T>
 __global__ __launch_bounds__(512) void k_dpe4_conv_lap(const T* __restrict__ wm, const T* __restrict__ hm,
-                                                       T* __restrict__ X, int Kx, int col0, Shape sh) {
+                                                       T* __restrict__ X, int Kx, int col0, Shape sh, int iblocks,
+                                                       int parts) {
   extern __shared__ unsigned char smem_raw[];
   T* ws = (T*)smem_raw;  // [NI][n][32]: w of electrons i0 .. i0 + NI - 1
   const int n = sh.n, C = sh.C, Cp = sh.Cp;
-  const long b = blockIdx.x;
+  // workgroup: walker, block of electrons (iblocks = 1: all of them in turn), part of the channel rows
+  const int part = (int)(blockIdx.x % (unsigned)parts), rest = (int)(blockIdx.x / (unsigned)parts);
+  const int ib = rest % iblocks;
+  const long b = rest / iblocks;
   const int grp = threadIdx.x >> 5, f = threadIdx.x & 31;
   const T* hb = hm + b * n * Cp * EMB + f;
   const T* wb = wm + b * n * n * 5 * EMB + f;
   const long hj = (long)Cp * EMB;
-  for (int i0 = 0; i0 < n; i0 += NI) {
-    if (i0) __syncthreads();
+  for (int i0 = ib * NI; i0 < n; i0 += iblocks * NI) {
+    if (i0 > ib * NI) __syncthreads();
     for (int p = grp; p < NI * n; p += 16)
       ws[p * EMB + f] = i0 * n + p < n * n ? wb[(long)(i0 * n + p) * 5 * EMB] : T(0);
     __syncthreads();
     const T* wf = ws + f;
-    for (int ch = grp; ch < Cp; ch += 16) {
+    for (int ch = part * 16 + grp; ch < Cp; ch += parts * 16) {
       if (ch == C - 1) continue;
       T acc[NI], own = T(0);
 #pragma unroll
@@ -489,7 +495,7 @@ __global__ __launch_bounds__(512) void k_dpe4_conv_lap(const T* __restrict__ wm,
         if (i0 + k < n) out[(long)k * Cp * Kx] = i0 + k == e ? own : acc[k];
     }
     const int i = i0 + grp;
-    if (grp < NI && i < n) {
+    if (part == parts - 1 && grp < NI && i < n) {
       T acc = T(0);
 #pragma unroll 2
       for (int j = 0; j < n; ++j) {
@@ -845,8 +851,18 @@ bool launch_dpe4_hmap(const float* X, int ldx, const float* Wt, int K, const flo
 
 template <typename T, int NI>
 static void conv_launch(const T* wm, const T* hm, T* X, int Kx, int col0, const Shape& sh, hipStream_t s) {
-  hipLaunchKernelGGL((k_dpe4_conv_lap<NI, T>), dim3((unsigned)sh.B), dim3(512), (size_t)NI * sh.n * EMB * sizeof(T), s,
-                     wm, hm, X, Kx, col0, sh);
+  // Up to 512 workgroups are made of a small batch, whose threads otherwise walk the blocks of electrons and their channel
+  // rows one after another, waiting for memory at every j; more than two blocks are separate at any batch (hm stays in L2).
+  // E_loc (1 determinant) with a workgroup per walker / as chosen, us: 42 electrons 3,968 / 1,255 (1 walker), 7,424 / 3,552
+  // (64), 14,061 / 11,231 (256); 26 electrons 1,723 / 889 (16), 7,777 / 7,465 (512); 20 electrons 1,528 / 1,125 (64), 4,903
+  // (512; 5,038 with two blocks); 14 electrons 741 / 654 (16), 1,611 / 1,527 (256), 2,630 (512; 2,747 with two parts); FP64, 42
+  // electrons 9,536 / 4,015 (16).
+  const int blocks = (sh.n + NI - 1) / NI;
+  const long most = 512;
+  const int ib = blocks > 2 || (long)sh.B * blocks <= most ? blocks : 1;
+  const int parts = (int)std::max<long>(1, std::min<long>((sh.Cp + 15) / 16, most / ((long)sh.B * ib)));
+  hipLaunchKernelGGL((k_dpe4_conv_lap<NI, T>), dim3((unsigned)(sh.B * ib * parts)), dim3(512),
+                     (size_t)NI * sh.n * EMB * sizeof(T), s, wm, hm, X, Kx, col0, sh, ib, parts);
 }
 
 template <typename T>
