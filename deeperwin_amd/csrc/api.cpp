@@ -112,14 +112,14 @@ struct Weights {
   std::vector<DevBuf> Wmain, Wmu, bias, Wmain_hi, Wmain_lo, Wmu_hi, Wmu_lo;
   std::vector<DevBuf> WmainT, WmuT;  // transposed copies for the gradient pass ([pad128(K)][W1])
   DevBuf W2e, b2e, Wo[2], Wo_hi[2], Wo_lo[2], WoT[2], kappa, wenv;
-  // FP32 form: the three BF16 parts of Wmain / Wmu / Wo in MFMA lane order (derivative channels, gemm_split.hip); of
-  // Wmain and Wmu in the BF16 forms too
+  // FP32 form, derivative channels (gemm_split.hip): the three BF16 parts of Wmu, and of Wmain where it has no FP16 parts, in
+  // MFMA lane order; of Wmain and Wmu in the BF16 forms too
   std::vector<DevBuf> WmainS, WmuS;
-  // and the two FP16 parts of 2^shift Wmain (layers >= 1) / Wo; shift kNoHalf: magnitudes outside FP16's reach
+  // and the two FP16 parts of Wmain's (layers >= 1) and Wo's scaled columns; halfH / halfO false: half_shifts refused
   std::vector<DevBuf> WmainH;
-  std::vector<int> shiftH;
+  std::vector<char> halfH;
   DevBuf WoH[2];
-  int shiftO[2] = {0, 0};
+  bool halfO[2] = {false, false};
   // FP32 form: Wmain / Wmu / Wo in MFMA lane order (one-launch value layers, value_layer.hip)
   std::vector<DevBuf> WmainL, WmuL;
   DevBuf WoL[2];
@@ -350,20 +350,53 @@ dw_status pack_split(DevBuf& out, const DevBuf& Bt, int cols, int K) {
   return DW_OK;
 }
 
-constexpr int kNoHalf = INT32_MIN;
-
-// Power of two that brings weights of this layout under 2^15 (gemm_split.hip bounds it), or kNoHalf.
-int half_shift(const std::vector<float>& w) {
-  float m = 0.f;
-  for (float x : w) m = std::fabs(x) > m || std::isnan(x) ? std::fabs(x) : m;
-  if (!(m < 1.7e10f)) return kNoHalf;  // 2^34 and above, NaN
-  return m > 0.f ? std::min(40, 14 - std::ilogb(m)) : 0;
+// Per output column of weights Bt [cols, K] the power of two that brings the column under 2^15, for the FP16 parts of
+// gemm_split.hip; empty where those are not enough:
+// - a column's largest weight outside [least, 2^34) (the units of the accumulators have to stay in range), or NaN;
+// - an input whose scaled weights are all below 2^-12 of another's: the rest of a row's element is up to 2^-39 of the row
+//   block's largest, and meets weights up to 2^12 times those of the input that has that largest: 2^-27 of its term, below
+//   FP32's rounding of it; with more it would not be.
+std::vector<int> half_shifts(const std::vector<float>& w, int cols, int K, float least) {
+  std::vector<int> shift(pad_to(cols, 256), 0);
+  std::vector<float> unit(K, 0.f);
+  for (int c = 0; c < cols; ++c) {
+    const float* row = w.data() + (size_t)c * K;
+    int32_t bits = 0;  // of the largest magnitude (NaN above all)
+    for (int k = 0; k < K; ++k) {
+      int32_t x;
+      std::memcpy(&x, row + k, 4);
+      x &= 0x7fffffff;
+      bits = x > bits ? x : bits;
+    }
+    if (bits == 0) continue;
+    float m;
+    std::memcpy(&m, &bits, 4);
+    if (!(m >= least && m < 0x1p34f)) return {};
+    shift[c] = 14 - std::ilogb(m);
+    const float scale = std::ldexp(1.f, shift[c]);
+    for (int k = 0; k < K; ++k) {
+      const float x = std::fabs(row[k]) * scale;
+      unit[k] = x > unit[k] ? x : unit[k];
+    }
+  }
+  float lo = 0x1p15f, hi = 0.f;
+  for (float x : unit) {
+    if (x > 0.f && x < lo) lo = x;
+    if (x > hi) hi = x;
+  }
+  if (hi > 4096.f * lo) return {};
+  return shift;
 }
 
-dw_status pack_half(DevBuf& out, int shift, const DevBuf& Bt, int cols, int K) {
-  if (shift == kNoHalf) return DW_OK;
+// The FP16 parts of the columns of w = Bt (host and device); `ok` says whether they can be taken.
+template <typename Flag>
+dw_status pack_half(DevBuf& out, Flag& ok, const std::vector<float>& w, const DevBuf& Bt, int cols, int K, float least) {
+  const std::vector<int> shift = half_shifts(w, cols, K, least);
+  ok = !shift.empty();
+  if (!ok) return DW_OK;
   HIP_TRY(out.ensure(split_pack16_bytes(cols, K)));
-  launch_split_pack16(Bt.as<float>(), K, cols, K, shift, out.p, nullptr);
+  HIP_TRY(hipMemcpy(split_pack16_shifts(out.p, cols, K), shift.data(), shift.size() * sizeof(int), hipMemcpyHostToDevice));
+  launch_split_pack16(Bt.as<float>(), K, cols, K, out.p, nullptr);
   HIP_TRY(hipGetLastError());
   return DW_OK;
 }
@@ -385,7 +418,7 @@ dw_status prepare_weights(dw_model* m, Weights& W, bool dbl) {
   for (auto* v : {&W.Wmain, &W.Wmu, &W.bias, &W.Wmain_hi, &W.Wmain_lo, &W.Wmu_hi, &W.Wmu_lo, &W.WmainT, &W.WmuT,
                   &W.WmainS, &W.WmuS, &W.WmainH, &W.WmainL, &W.WmuL})
     v->resize(m->L);
-  W.shiftH.assign(m->L, kNoHalf);
+  W.halfH.assign(m->L, 0);
   auto up = [&](DevBuf& b, const std::vector<float>& v) { return dbl ? upload_as<double>(b, v) : upload(b, v); };
   for (int l = 0; l < m->L; ++l) {
     char buf[64];
@@ -414,9 +447,10 @@ dw_status prepare_weights(dw_model* m, Weights& W, bool dbl) {
     if ((st = up(W.WmainT[l], wmT))) return st;
     if ((st = up(W.WmuT[l], wuT))) return st;
     if ((st = up(W.bias[l], b.data))) return st;
-    if (parts3) W.shiftH[l] = l > 0 && Kx % 64 == 0 && Kx - Kt0 <= 64 ? half_shift(wm) : kNoHalf;
-    if (parts3 && ((st = pack_split(W.WmainS[l], W.Wmain[l], W1, Kx)) ||
-                   (st = pack_half(W.WmainH[l], W.shiftH[l], W.Wmain[l], W1, Kx)) ||
+    if (parts3 && l > 0 && Kx % 64 == 0 && Kx - Kt0 <= 64 &&
+        (st = pack_half(W.WmainH[l], W.halfH[l], wm, W.Wmain[l], W1, Kx, 0x1p-46f)))
+      return st;
+    if (parts3 && ((!W.halfH[l] && (st = pack_split(W.WmainS[l], W.Wmain[l], W1, Kx))) ||
                    (st = pack_split(W.WmuS[l], W.Wmu[l], W1, Km)) ||
                    (st = pack_lanes(W.WmainL[l], W.Wmain[l], W1, Kx)) ||
                    (st = pack_lanes(W.WmuL[l], W.Wmu[l], W1, Km))))
@@ -462,8 +496,7 @@ dw_status prepare_weights(dw_model* m, Weights& W, bool dbl) {
     dw_status st;
     if ((st = up(W.Wo[s], wo))) return st;
     if ((st = up(W.WoT[s], woT))) return st;
-    if (parts3) W.shiftO[s] = half_shift(wo);
-    if (parts3 && ((st = pack_half(W.WoH[s], W.shiftO[s], W.Wo[s], m->NOp, W1)) ||
+    if (parts3 && ((st = pack_half(W.WoH[s], W.halfO[s], wo, W.Wo[s], m->NOp, W1, 0x1p-60f)) ||
                    (st = pack_lanes(W.WoL[s], W.Wo[s], m->NOp, W1))))
       return st;
     if (split && (st = upload_split(W.Wo_hi[s], W.Wo_lo[s], wo))) return st;
@@ -754,8 +787,8 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
                (int)(B * m->n), m->W1, m->Kx[l], em, s);
         }
         Timed t(m, l >= 1 ? DW_TIMER_GEMM_1EL_LAP : -1, s);
-        const bool half = W.shiftH[l] != kNoHalf;
-        amax_np = split_lap(X[l], m->Kx[l], half ? W.WmainH[l].p : W.WmainS[l].p, W.shiftH[l], m->Kx[l],
+        const bool half = W.halfH[l];
+        amax_np = split_lap(X[l], m->Kx[l], half ? W.WmainH[l].p : W.WmainS[l].p, m->Kx[l],
                             half ? ws.amax[(l + 1) & 1] : nullptr, amax_np, (m->Kx[l] - m->Kt0[l]) / 32, ws.V, m->W1, outp,
                             ldo, ws.amax[l & 1], last ? 1 : 0, sh, m->tune.lap_electrons, m->tune.lap_cols, s);
         continue;
@@ -829,9 +862,9 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
   for (int sp = 0; sp < 2 && !orb_done; ++sp) {
     const long rows0 = sp ? up_rows : 0, nr = sp ? dn_rows : up_rows;
     if constexpr (!DBL) {
-      if (split && W.shiftO[sp] != kNoHalf) {  // every channel from the split form; the value rows follow in FP32
+      if (split && W.halfO[sp]) {  // every channel from the split form; the value rows follow in FP32
         const int ms = m->W1 / 32;
-        split_gemm(ws.H + rows0 * m->W1, m->W1, W.WoH[sp].p, W.shiftO[sp],
+        split_gemm(ws.H + rows0 * m->W1, m->W1, W.WoH[sp].p,
                    ws.amax[(m->L - 1) & 1] + (sp ? B * m->u * ms : 0), amax_np, ms, Cp / 16, ws.O + rows0 * m->NO, m->NO,
                    (int)nr, m->NO, m->W1, m->tune.lap_orb_tile, s);
         continue;

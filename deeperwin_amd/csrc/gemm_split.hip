@@ -4,8 +4,8 @@
 // m = bf16(x - h), l = x - h - m; 8 + 8 + 8 significant bits), so a product is the sum of nine BF16 products; the three
 // below 2^-26 |a b| (m l, l m, l l) are left out.  FP16 parts: x = h + m with 11 + 11 bits and a rest below 2^-23 |x|,
 // three products (m m, below 2^-24 |a b|, left out); it needs operands near the top of FP16's range, so a row block (one
-// electron's channels) and the weights are scaled by powers of two, and an element keeps those bits down to 2^-17 of its
-// block's largest (below that its absolute error is 2^-40 of the largest).  In both a 32-wide K slice rounds the
+// electron's channels) and each column of the weights are scaled by powers of two, and an element keeps those bits down to
+// 2^-17 of its block's or column's largest (below that its absolute error is 2^-39 of the largest).  In both a 32-wide K slice rounds the
 // accumulator six or three times, where the FP32 MFMA (16x16x4) rounds it at least eight times; over 320 products of
 // random operands that leaves 1.3e-7 (BF16) and 1.2e-7 (FP16) of the norm against 1.6e-7 for FP32.
 // The 16-bit MFMA runs at 16 times the FP32 rate: 6 / 16 and 3 / 16 of the FP32 form's time.
@@ -96,9 +96,10 @@ void launch_split_pack(const float* Bt, int ldb, int cols, int K, void* out, hip
                      (uint4*)out);
 }
 
-// The same order with two FP16 parts of 2^shift W: P16[((slice * ncb + cb) * 2 + part) * 64 + lane].
+// The same order with two FP16 parts of W times a power of two per output column: P16[((slice * ncb + cb) * 2 + part) * 64 +
+// lane], then the columns' shifts (16 ncb of them).
 __global__ __launch_bounds__(256) void k_split_pack16(const float* __restrict__ Bt, int ldb, int cols, int ncb,
-                                                      int slices, float scale, uint4* __restrict__ P) {
+                                                      int slices, uint4* __restrict__ P) {
   const int t = blockIdx.x * 256 + threadIdx.x;
   if (t >= slices * ncb * 64) return;
   const int lane = t & 63, cb = (t >> 6) % ncb, sl = (t >> 6) / ncb;
@@ -108,6 +109,7 @@ __global__ __launch_bounds__(256) void k_split_pack16(const float* __restrict__ 
     a = *(const v4f*)(Bt + (long)col * ldb + k);
     b = *(const v4f*)(Bt + (long)col * ldb + k + 4);
   }
+  const float scale = ldexpf(1.f, ((const int*)(P + (long)slices * ncb * 128))[col]);
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     a[j] *= scale;
@@ -121,16 +123,21 @@ __global__ __launch_bounds__(256) void k_split_pack16(const float* __restrict__ 
     P[((long)(sl * ncb + cb) * 2 + p) * 64 + lane] = uint4{pa[p].x, pa[p].y, pb[p].x, pb[p].y};
 }
 
-size_t split_pack16_bytes(int cols, int K) { return (size_t)(K / 32) * (dw_pad(cols, 256) / 16) * 2 * 64 * 16; }
+size_t split_pack16_bytes(int cols, int K) {
+  return (size_t)(K / 32) * (dw_pad(cols, 256) / 16) * 2 * 64 * 16 + (size_t)dw_pad(cols, 256) * sizeof(int);
+}
+int* split_pack16_shifts(void* P16, int cols, int K) {
+  return (int*)((uint4*)P16 + (size_t)(K / 32) * (dw_pad(cols, 256) / 16) * 128);
+}
 
-void launch_split_pack16(const float* Bt, int ldb, int cols, int K, int shift, void* out, hipStream_t s) {
+void launch_split_pack16(const float* Bt, int ldb, int cols, int K, void* out, hipStream_t s) {
   const int ncb = dw_pad(cols, 256) / 16, slices = K / 32;
   hipLaunchKernelGGL(k_split_pack16, dim3((slices * ncb * 64 + 255) / 256), dim3(256), 0, s, Bt, ldb, cols, ncb, slices,
-                     ldexpf(1.f, shift), (uint4*)out);
+                     (uint4*)out);
 }
 
 // Power of two that brings a block of largest magnitude `m` under 2^15.  Bounded so that the units of the accumulators
-// (this plus the weights' shift of -20 .. 40) and their inverse stay in range.
+// (this plus a weight column's shift of -19 .. 60, orbitals 74) and their inverse stay in range.
 __device__ __forceinline__ int split_shift(float m) {
   const int e = (int)((__float_as_uint(m) >> 23) & 255u) - 127;
   return min(40, max(-100, 14 - e));
@@ -161,10 +168,11 @@ struct SplitLds {
   uint4 a[2][PARTS][RB][64];
 };
 
-// Weights of a split GEMM in lane order: three BF16 parts of W, or two FP16 parts of 2^shift W.
+// Weights of a split GEMM in lane order: three BF16 parts of W, or two FP16 parts of its scaled columns (and their shifts).
 struct SplitB {
   const uint4* P;
-  int ncb, slices, shift;
+  int ncb, slices;
+  __device__ __forceinline__ int shift(int col) const { return ((const int*)(P + (long)slices * ncb * 128))[col]; }
 };
 
 // Unit u of a slice: row u / 128 * 16 + u % 16 (row block u / 128), quad of 4 k (u / 16) % 8.
@@ -352,7 +360,8 @@ __device__ __forceinline__ void tile_scales(const SplitUnits<RB>& U, const float
 
 // ------------------------------------------------------------------------------------------------
 // C[M, N] = A[M, K] B (no epilogue): the orbital GEMMs of the Laplacian pass.  688,128 x 256 x 224: 783 us with
-// FP32 MFMA on 128-row tiles, 480 us with BF16 parts, 349 us here.
+// FP32 MFMA on 128-row tiles, 480 us with BF16 parts, 349 us here with one scale for all weights; a scale per column takes
+// 1 to 2 % more (365 -> 371 us there, 1,064,960 x 256 x 416 1,090 -> 1,117; with its loads before the main loop 1,181).
 // ------------------------------------------------------------------------------------------------
 template <int RB, int NQ>
 __global__ __launch_bounds__(256, 2) void k_split_gemm(const float* __restrict__ A, int lda, SplitB W,
@@ -380,12 +389,16 @@ __global__ __launch_bounds__(256, 2) void k_split_gemm(const float* __restrict__
 #pragma unroll
     for (int q = 0; q < NQ; ++q) acc[i][q] = v4f{0.f, 0.f, 0.f, 0.f};
   split_main16<RB, NQ>(U, W, 0, ra0, ra1, sc, cb0, lds, acc);
+  float wi[NQ];  // 2^-shift of this lane's columns
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) wi[q] = ldexpf(1.f, -W.shift((cb0 + q) * 16 + (lane & 15)));
 #pragma unroll
   for (int i = 0; i < RB; ++i) {
-    const float inv = ldexpf(1.f, -(eA[i] + W.shift));
+    const float ai = ldexpf(1.f, -eA[i]);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       const int c = (cb0 + q) * 16 + (lane & 15);
+      const float inv = ai * wi[q];
       if (c < N) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -397,10 +410,10 @@ __global__ __launch_bounds__(256, 2) void k_split_gemm(const float* __restrict__
   }
 }
 
-void split_gemm(const float* A, int lda, const void* P16, int shift, const float* amax, int np, int ms, int rbe, float* C,
+void split_gemm(const float* A, int lda, const void* P16, const float* amax, int np, int ms, int rbe, float* C,
                 int ldc, int M, int N, int K, int tile, hipStream_t s) {
   if (M <= 0 || N <= 0) return;
-  const SplitB W{(const uint4*)P16, dw_pad(N, 256) / 16, K / 32, shift};
+  const SplitB W{(const uint4*)P16, dw_pad(N, 256) / 16, K / 32};
   const long big = ((long)(M + 95) / 96) * ((N + 255) / 256);
   if (tile < 0 ? big >= 512 : tile > 0) {
     const int tilesN = (N + 255) / 256, total = (M + 95) / 96 * tilesN;
@@ -450,7 +463,10 @@ __global__ __launch_bounds__(256, 2) void k_split_lap(const float* __restrict__ 
   const SplitUnits<RB> U(X, g0 * Cp, n_el * Cp, ldx);
   v4f ra0[HALF ? AIT : 1], ra1[HALF ? AIT : 1];
   float sc[HALF ? AIT : 1];
+  int shifts[NQ];  // of this lane's columns
   if constexpr (HALF) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) shifts[q] = W.shift(col + 16 * q);
     const int first = tail > 0 ? W.slices - tail : 0;
     U.load(first, ra0);
     U.load(tail == 1 ? 0 : first + 1, ra1);
@@ -473,11 +489,13 @@ __global__ __launch_bounds__(256, 2) void k_split_lap(const float* __restrict__ 
     __syncthreads();  // eA
 #pragma unroll
     for (int i = 0; i < RB; ++i) {
-      const float unit = ldexpf(1.f, eA[i] + W.shift);
+      const float unit = ldexpf(1.f, eA[i]);
 #pragma unroll
-      for (int q = 0; q < NQ; ++q)
+      for (int q = 0; q < NQ; ++q) {
+        const float u = unit * ldexpf(1.f, shifts[q]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][q][j] *= unit;
+        for (int j = 0; j < 4; ++j) acc[i][q][j] *= u;
+      }
     }
     split_main16<RB, NQ>(U, W, tail, ra0, ra1, sc, cb0, lds, acc);
   } else {
@@ -494,7 +512,10 @@ __global__ __launch_bounds__(256, 2) void k_split_lap(const float* __restrict__ 
     if (permute) ob = (i < sh.u) ? (b * sh.u + i) * Cp : (long)sh.B * sh.u * Cp + (b * dn + (i - sh.u)) * Cp;
     float* op = out + (ob + 4 * g4) * ldo + col;
     const float* vp = out + ob * ldo + col;
-    const float inv = HALF ? ldexpf(1.f, -(eA[HALF ? e * RBE : 0] + W.shift)) : 1.f;
+    float inv[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+      inv[q] = HALF ? ldexpf(1.f, -eA[HALF ? e * RBE : 0]) * ldexpf(1.f, -shifts[q]) : 1.f;
     float d1[NQ], d2[NQ], S[NQ], zl[NQ], mx = 0.f;  // mx: largest |y| of the derivative channels
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
@@ -512,7 +533,7 @@ __global__ __launch_bounds__(256, 2) void k_split_lap(const float* __restrict__ 
         const bool tan = ch >= 1 && ch < C - 1;
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
-          const float z = acc[e * RBE + kb][q][j] * inv;
+          const float z = acc[e * RBE + kb][q][j] * inv[q];
           S[q] += tan ? z * z : 0.f;
           if (ch == C - 1) zl[q] = z;
           if (tan) {
@@ -540,11 +561,11 @@ __global__ __launch_bounds__(256, 2) void k_split_lap(const float* __restrict__ 
   }
 }
 
-int split_lap(const float* X, int ldx, const void* P, int shift, int K, const float* amax, int np, int tail,
+int split_lap(const float* X, int ldx, const void* P, int K, const float* amax, int np, int tail,
               const float* V, int ldv, float* out, int ldo, float* omax, int permute, const Shape& sh, int E_max,
               int cols, hipStream_t s) {
   const int RBE = sh.Cp / 16;
-  const SplitB W{(const uint4*)P, dw_pad(sh.W1, 256) / 16, K / 32, amax ? shift : 0};
+  const SplitB W{(const uint4*)P, dw_pad(sh.W1, 256) / 16, K / 32};
   const long n_el = (long)sh.B * sh.n;
 #define DW_SPLIT_LAP(R, EE, Q)                                                                                        \
   do {                                                                                                                \

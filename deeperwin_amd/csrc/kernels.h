@@ -59,13 +59,15 @@ int lap_electrons_per_tile(int Cp, GemmPrec prec);
 // split_pack_bytes(cols, K) bytes; K a multiple of 32.
 size_t split_pack_bytes(int cols, int K);
 void launch_split_pack(const float* Bt, int ldb, int cols, int K, void* out, hipStream_t s);
-// The same weights as two FP16 parts of 2^shift W (K columns from Bt, split_pack16_bytes(cols, K) bytes).
+// The same weights as two FP16 parts of each column times 2^shift (K columns from Bt, split_pack16_bytes(cols, K) bytes); the
+// columns' shifts are put at split_pack16_shifts before.
 size_t split_pack16_bytes(int cols, int K);
-void launch_split_pack16(const float* Bt, int ldb, int cols, int K, int shift, void* out, hipStream_t s);
+int* split_pack16_shifts(void* P16, int cols, int K);
+void launch_split_pack16(const float* Bt, int ldb, int cols, int K, void* out, hipStream_t s);
 // C[M, N] = A[M, K] B for rows of electrons (16 rbe rows each), K a multiple of 64, B in FP16 parts.  amax: np per-wave
 // maxima of each electron's A rows, ms apart.  tile: -1 chosen by size, 0 = 48 x 128, 1 or 2 = 96 x 256 (results do not
 // depend on it).
-void split_gemm(const float* A, int lda, const void* P16, int shift, const float* amax, int np, int ms, int rbe, float* C,
+void split_gemm(const float* A, int lda, const void* P16, const float* amax, int np, int ms, int rbe, float* C,
                 int ldc, int M, int N, int K, int tile, hipStream_t s);
 // V[(b Cp + ch), o] of the derivative channels: spin means of X's first Kh columns times W_mu (no bias), from three BF16 parts
 // of each (FP32 accuracy).
@@ -79,7 +81,7 @@ bool mean_bf16x3(const float* X, int Kx, int Kh, const void* P, int Km, const fl
 // P is in FP16 parts, without it in BF16 parts.  omax (W1 / 32 places per electron, in the order of out's rows) receives the maxima
 // of the derivative channels written, one per wave: returns their number per electron (0: shape not supported).  E_max
 // > 0 / cols = 128 ask for the smaller tiles (results do not depend on them).
-int split_lap(const float* X, int ldx, const void* P, int shift, int K, const float* amax, int np, int tail,
+int split_lap(const float* X, int ldx, const void* P, int K, const float* amax, int np, int tail,
               const float* V, int ldv, float* out, int ldo, float* omax, int permute, const Shape& sh, int E_max,
               int cols, hipStream_t s);
 
