@@ -8,6 +8,8 @@ from __future__ import annotations
 
 import ctypes
 import os
+from contextlib import contextmanager
+from contextvars import ContextVar
 from pathlib import Path
 from typing import Dict, Optional
 
@@ -76,6 +78,7 @@ SIGNATURES = {
     "dw_workspace_size": ([_vp, _i32, _i32], ctypes.c_size_t),
     "dw_model_set_chunk": ([_vp, _i32], ctypes.c_int),
     "dw_model_set_lap_form": ([_vp, _i32], ctypes.c_int),
+    "dw_local_energy_form": ([_vp, _i32, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp], ctypes.c_int),
     "dw_model_set_workspace": ([_vp, _vp, ctypes.c_size_t], ctypes.c_int),
     "dw_model_set_tuning": ([_vp, ctypes.POINTER(Tuning)], ctypes.c_int),
     "dw_model_get_tuning": ([_vp, ctypes.POINTER(Tuning)], ctypes.c_int),
@@ -88,8 +91,20 @@ SIGNATURES = {
 }
 
 _lib: Optional[ctypes.CDLL] = None
+_lap_form: ContextVar[Optional[int]] = ContextVar("dwmi_lap_form", default=None)
 _memcmp = ctypes.CDLL(None).memcmp
 _memcmp.argtypes, _memcmp.restype = [_vp, _vp, ctypes.c_size_t], ctypes.c_int
+
+
+@contextmanager
+def lap_form(form: int):
+    """The form (LAP_SPLIT or LAP_FP32) of every local energy that this thread takes inside the block, whichever model or
+    function object computes it; other threads and the models' own settings are not affected."""
+    token = _lap_form.set(int(form))
+    try:
+        yield
+    finally:
+        _lap_form.reset(token)
 
 
 def load_library() -> ctypes.CDLL:
@@ -143,7 +158,7 @@ class NativeModel:
         _check(self.lib.dw_model_create(ctypes.byref(desc), ctypes.byref(h)))
         self.handle = h
         self._param_token = None
-        self._lap_form = LAP_SPLIT
+        self._model_lap_form = LAP_SPLIT
         if chunk:
             _check(self.lib.dw_model_set_chunk(self.handle, int(chunk)))
 
@@ -229,7 +244,7 @@ class NativeModel:
     def set_lap_form(self, form: int) -> int:
         """dw_model_set_lap_form: LAP_SPLIT (default) or LAP_FP32.  Returns the form before."""
         _check(self.lib.dw_model_set_lap_form(self.handle, int(form)))
-        old, self._lap_form = self._lap_form, int(form)
+        old, self._model_lap_form = self._model_lap_form, int(form)
         return old
 
     def set_chunk(self, walkers: int) -> None:
@@ -302,8 +317,12 @@ class NativeModel:
                                   _ptr(out_phase), _stream()))
 
     def local_energy(self, r, R, Z, out_eloc, out_lp=None, out_flags=None) -> None:
-        _check(self.lib.dw_local_energy(self.handle, _ptr(r), r.shape[0], _ptr(R), _ptr(Z), _ptr(out_eloc),
-                                        _ptr(out_lp), _ptr(out_flags), _stream()))
+        args = (_ptr(r), r.shape[0], _ptr(R), _ptr(Z), _ptr(out_eloc), _ptr(out_lp), _ptr(out_flags), _stream())
+        form = _lap_form.get()
+        if form is None:
+            _check(self.lib.dw_local_energy(self.handle, *args))
+        else:
+            _check(self.lib.dw_local_energy_form(self.handle, form, *args))
 
     def set_proposal(self, name: str = "normal", r_min: float = 0.1, r_max: float = 1.0,
                      langevin_scale: float = 1.0) -> None:

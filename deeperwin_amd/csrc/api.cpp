@@ -659,17 +659,19 @@ struct Proposal {
 
 // One pass of the wavefunction over B walkers with C channels (C == 1: value; C == 3n+2: Laplacian).
 // `ws` is the pass's scratch (layout_pass); out_kappa (may be null) receives the per-walker conditioning.
-// keep_layers: every layer's activations are left in ws.X (a value pass that the gradient continues).
+// keep_layers: every layer's activations are left in ws.X (a value pass that the gradient continues).  lap_form: derivative
+// channels of a Laplacian pass in the FP32 form.
 template <typename T>
 dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, const float* R, const float* Z, int C,
                    hipStream_t s, float* out_lp, float* out_phase, float* out_eloc, uint32_t* out_flags,
-                   float* out_kappa, float cond_thr, const Proposal* prop = nullptr, bool keep_layers = false) {
+                   float* out_kappa, float cond_thr, const Proposal* prop = nullptr, bool keep_layers = false,
+                   int lap_form = DW_LAP_SPLIT) {
   constexpr bool DBL = sizeof(T) == 8;
   Weights& W = DBL ? m->wd : m->wf;
   const int Cp = rows_per_electron(C);
   Shape sh{(int)B, m->n, m->u, m->I, m->D, C, Cp, m->W1, m->W2, m->L};
   const long rows = B * m->n * Cp;
-  const bool split = !DBL && C > 1 && m->prec == GEMM_F32 && m->lap_form == DW_LAP_SPLIT;
+  const bool split = !DBL && C > 1 && m->prec == GEMM_F32 && lap_form == DW_LAP_SPLIT;
   Timed pass_timer(m, C > 1 ? DW_TIMER_LOCAL_ENERGY : DW_TIMER_FORWARD, s);
   T* const* X = ws.X;
   if (prop) {  // the pass runs on the Gaussian proposal, formed and stored by the features kernel
@@ -1133,7 +1135,7 @@ dw_status run_grad(dw_model* m, const float* r, long B, const float* R, const fl
 // One pass in the model's precision, its scratch from the model (arena or caller-owned workspace).
 dw_status pass(dw_model* m, const float* r, long B, const float* R, const float* Z, int C, hipStream_t s,
                float* out_lp, float* out_phase, float* out_eloc, uint32_t* out_flags, float* out_kappa,
-               float cond_thr) {
+               float cond_thr, int lap_form = DW_LAP_SPLIT) {
   if (m->prec == GEMM_F64) {
     PassBufs<double> pb;
     dw_status st = pass_scratch(m, B, C, &pb);
@@ -1143,7 +1145,8 @@ dw_status pass(dw_model* m, const float* r, long B, const float* R, const float*
   PassBufs<float> pb;
   dw_status st = pass_scratch(m, B, C, &pb);
   if (st) return st;
-  return run_pass<float>(m, pb, r, B, R, Z, C, s, out_lp, out_phase, out_eloc, out_flags, out_kappa, cond_thr);
+  return run_pass<float>(m, pb, r, B, R, Z, C, s, out_lp, out_phase, out_eloc, out_flags, out_kappa, cond_thr, nullptr, false,
+                         lap_form);
 }
 
 }  // namespace
@@ -1484,7 +1487,15 @@ dw_status dw_logpsi(dw_model* m, const float* r, int32_t n_walkers, const float*
 
 dw_status dw_local_energy(dw_model* m, const float* r, int32_t n_walkers, const float* R, const float* Z,
                           float* out_eloc, float* out_log_psi_sqr, uint32_t* out_flags, dw_stream stream) {
+  return dw_local_energy_form(m, m ? m->lap_form : DW_LAP_SPLIT, r, n_walkers, R, Z, out_eloc, out_log_psi_sqr, out_flags,
+                              stream);
+}
+
+dw_status dw_local_energy_form(dw_model* m, int32_t lap_form, const float* r, int32_t n_walkers, const float* R,
+                               const float* Z, float* out_eloc, float* out_log_psi_sqr, uint32_t* out_flags,
+                               dw_stream stream) {
   if (!m || !r || !R || !Z || !out_eloc) return fail(DW_ERR_INVALID, "null argument");
+  if (lap_form != DW_LAP_SPLIT && lap_form != DW_LAP_FP32) return fail(DW_ERR_INVALID, "unknown Laplacian form");
   if (n_walkers <= 0) return fail(DW_ERR_INVALID, "n_walkers must be positive");
   const bool recompute = m->prec != GEMM_F64 && m->d.fp64_cond_threshold > 0.f;
   hipStream_t s = (hipStream_t)stream;
@@ -1503,7 +1514,7 @@ dw_status dw_local_energy(dw_model* m, const float* r, int32_t n_walkers, const 
   for (long b0 = 0; b0 < n_walkers; b0 += chunk) {
     const long nb = std::min<long>(chunk, n_walkers - b0);
     st = pass(m, r + b0 * m->n * 3, nb, R, Z, C, s, out_log_psi_sqr ? out_log_psi_sqr + b0 : nullptr, nullptr,
-              out_eloc + b0, flags ? flags + b0 : nullptr, m->kappa_w.as<float>() + b0, m->d.fp64_cond_threshold);
+              out_eloc + b0, flags ? flags + b0 : nullptr, m->kappa_w.as<float>() + b0, m->d.fp64_cond_threshold, lap_form);
     if (st) return st;
   }
   if (!recompute) return DW_OK;

@@ -7,17 +7,22 @@ reference computes it); the potential is the non-periodic Coulomb sum (hamiltoni
 """
 from __future__ import annotations
 
+from contextlib import nullcontext
 from typing import Dict, Optional
 
 import torch
 
-from ._native import FLAG_NONFINITE
+from ._native import FLAG_NONFINITE, LAP_FP32, LAP_SPLIT
+from ._native import lap_form as lap_form_of_calls
 from .wavefunction import NativeLogPsiSquared, _as_device
 
 
 def build_local_energy(log_psi_squared, is_complex: bool = False, is_periodic: bool = False,
                        include_heg_background: bool = False, forward_lap: bool = False, max_batch_size: int = 64,
-                       native_chunk: int = 0):
+                       native_chunk: int = 0, lap_form: Optional[str] = None):
+    """``lap_form``: derivative channels of the FP32 form on 16-bit MFMA with split operands (``"split"``) or on FP32 MFMA
+    (``"fp32"``); None takes split, and FP32 where the loss asks for it (dw_local_energy_form in include/dwmi.h)."""
+    form = None if lap_form is None else {"split": LAP_SPLIT, "fp32": LAP_FP32}[lap_form]
     if not isinstance(log_psi_squared, NativeLogPsiSquared):
         raise TypeError("build_local_energy expects the native log_psi_squared from build_log_psi_squared")
     if is_complex:
@@ -35,7 +40,8 @@ def build_local_energy(log_psi_squared, is_complex: bool = False, is_periodic: b
         Rt, Zt = _as_device(R), _as_device(Z)
         e = torch.empty(rt.shape[0], device="cuda", dtype=torch.float32)
         flags = torch.empty(rt.shape[0], device="cuda", dtype=torch.int32)
-        model.local_energy(rt, Rt, Zt, e, None, flags)
+        with nullcontext() if form is None else lap_form_of_calls(form):
+            model.local_energy(rt, Rt, Zt, e, None, flags)
         if return_flags:
             return e, flags
         return e

@@ -14,7 +14,7 @@ from typing import Dict
 
 import torch
 
-from ._native import LAP_FP32, clip_energies
+from ._native import LAP_FP32, clip_energies, lap_form
 from .config import ClippingConfig
 from .wavefunction import NativeLogPsiSquared, _as_device
 
@@ -41,12 +41,9 @@ def build_value_and_grad_func(log_psi_sqr_func, get_local_energy, clipping_confi
         model = log_psi_sqr_func.model_for(params, n_up, n_dn)
         rt = _as_device(r).reshape(-1, n_up + n_dn, 3)
         Rt, Zt = _as_device(R), _as_device(Z)
-        # the loss and the clipping state leave in FP64 and are carried from run to run: bit-stable energies
-        form = model.set_lap_form(LAP_FP32)
-        try:
+        # the loss and the clipping state leave in FP64 and are carried along: energies whose sums keep their order
+        with lap_form(LAP_FP32):
             e_loc = get_local_energy(params, spin_state, rt, Rt, Zt, fixed_params)
-        finally:
-            model.set_lap_form(form)
         st = None if state is None else torch.as_tensor(state, dtype=torch.float64, device="cuda").reshape(2)
         weights, e_clip, stats = clip_energies(e_loc, st, cc.name, cc.center, cc.width_metric, cc.clip_by,
                                                cc.from_previous_step)

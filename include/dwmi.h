@@ -261,14 +261,21 @@ dw_status dw_model_set_tuning(dw_model* m, const dw_tuning* t);
 dw_status dw_model_get_tuning(const dw_model* m, dw_tuning* out);
 
 /* Derivative channels (tangents, Laplacian) of dw_local_energy's GEMMs in the DW_FP32 form.  SPLIT (default): both
- * operands split into 16-bit parts (three BF16, or two FP16 scaled by powers of two) whose products are summed in FP32
- * on 16-bit MFMA; E_loc as accurate as with FP32 and 1.3 to 1.9 times faster, equal to it to rounding.  FP32: FP32
- * MFMA.  The value channel (log|psi|^2, the determinants) is the same bits in both.  For callers whose FP64 statistics
- * of the energies (the optimisation's loss and clipping state) have to stay bit-equal from run to run, across releases:
- * the loss uses FP32.  The other precision forms have one form only. */
+ * operands split into 16-bit parts (three BF16, or two FP16 scaled by powers of two, which carry 22 to 24 significant bits)
+ * whose products are summed in FP32 on 16-bit MFMA; 1.3 to 1.9 times faster.  E_loc is as far from 64 bits as with FP32
+ * (the value channel sets that error); between the two forms it differs by less than a quarter of it, 5e-7 of 1 + |E_loc|
+ * for the median walker of up to 20 electrons.  FP32: FP32 MFMA.  The value channel (log|psi|^2, the
+ * determinants) is the same bits in both.  In either form a walker's E_loc is the same bits from run to run and in any
+ * batch.  For callers whose FP64 statistics of the energies are carried along (the optimisation's loss and clipping state):
+ * FP32 also keeps the order of every sum that the kernels had before the split form came; the loss uses it.  The other
+ * precision forms have one form only.  dw_model_set_lap_form sets what dw_local_energy takes; dw_local_energy_form takes
+ * the form of one call and leaves the model's setting alone. */
 #define DW_LAP_SPLIT 0
 #define DW_LAP_FP32 1
 dw_status dw_model_set_lap_form(dw_model* m, int32_t form);
+dw_status dw_local_energy_form(dw_model* m, int32_t lap_form, const float* r, int32_t n_walkers, const float* R,
+                               const float* Z, float* out_eloc, float* out_log_psi_sqr, uint32_t* out_flags,
+                               dw_stream stream);
 
 /* ---- Measurement hooks (no counterpart in the reference; used by the benchmark harness) ----
  * When timing is enabled the library brackets selected launches with HIP events recorded on the
