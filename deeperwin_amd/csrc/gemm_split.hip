@@ -587,7 +587,7 @@ int split_lap(const float* X, int ldx, const void* P, int K, const float* amax, 
   const int EF = RBE <= 6 ? 6 / RBE : 1;
   bool big = sh.W1 % 256 == 0 && RBE <= 6 && (n_el + EF - 1) / EF * (sh.W1 / 256) >= 512;
   if (cols == 128 || (E_max > 0 && E_max < EF)) big = false;
-  if (cols == 256 && sh.W1 % 256 == 0 && RBE <= 6 && E_max <= 0) big = true;
+  if (cols == 256 && sh.W1 % 256 == 0 && RBE <= 6 && (E_max <= 0 || E_max >= EF)) big = true;
   switch (RBE * 2 + (big ? 1 : 0)) {
     case 3: DW_SPLIT_LAP(1, 6, 4);
     case 5: DW_SPLIT_LAP(2, 3, 4);

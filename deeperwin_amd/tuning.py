@@ -41,20 +41,25 @@ def lap_electron_choices(n_el: int) -> List[int]:
     return [e for e in range(1, 7) if e * cp <= 192]
 
 
-def search_space(n_el: int) -> List[Tuple[str, Sequence[int], str]]:
-    """(field, candidates, pass it affects) in the order the sweep visits them.  -1 leaves the choice to the library:
-    a fixed tile keeps the separate kernels, which for the value layers, the orbital GEMMs of a value pass and the
-    mean product are slower at most sizes than what the library picks (8 electrons, 512 walkers: value pass 150 us with
-    64 x 64 tiles, 108 us with the library's choice)."""
-    return [
+def search_space(n_el: int, precision: str = "fp32", width1: int = 256) -> List[Tuple[str, Sequence[int], str]]:
+    """(field, candidates, pass it affects) in the order the sweep visits them, the library's own choice (-1 or 0) first: a
+    fixed tile keeps the separate kernels, which for the value layers, the orbital GEMMs of a value pass and the mean product
+    are slower at most sizes than what the library picks (8 electrons, 512 walkers: value pass 150 us with 64 x 64 tiles,
+    108 us with the library's choice).  Only what the precision form's kernels look at: the FP32 forms have one mean kernel
+    (at width 256), the BF16x3 form chooses between two."""
+    space = [
         ("fwd_main_tile", (-1,) + TILE_CHOICES + (3, 4), "value"),
         ("fwd_mu_split", SPLIT_CHOICES, "value"),
         ("fwd_orb_tile", (-1,) + TILE_CHOICES, "value"),
-        ("lap_cols", (128, 256), "lap"),
-        ("lap_electrons", lap_electron_choices(n_el), "lap"),
-        ("lap_mu_tile", (-1,) + TILE_CHOICES, "lap"),
-        ("lap_orb_tile", (-1,) + TILE_CHOICES, "lap"),
+        ("lap_cols", (0, 128, 256), "lap"),
+        ("lap_electrons", [0] + lap_electron_choices(n_el), "lap"),
     ]
+    if precision == "bf16x3":
+        space.append(("lap_mu_tile", (-1, 0), "lap"))
+    elif precision == "fp32" and width1 != 256:
+        space.append(("lap_mu_tile", (-1,) + TILE_CHOICES, "lap"))
+    space.append(("lap_orb_tile", (-1,) + TILE_CHOICES, "lap"))
+    return space
 
 
 def time_ms(fn: Callable[[], None], reps: int = 3) -> float:
@@ -77,16 +82,29 @@ def time_ms(fn: Callable[[], None], reps: int = 3) -> float:
 
 def autotune_model(model, r, R, Z, reps: int = 3, include_lap: bool = True) -> Tuple[Dict[str, int], List[dict]]:
     """One coordinate-descent sweep over the search space on the given walkers.  Leaves the best choices set
-    on `model` and returns them with the timing log."""
+    on `model` and returns them with the timing log.
+
+    The Laplacian pass of the FP32 form runs in two forms, split for energies and FP32 MFMA for the loss, whose kernels share
+    the fields: of each candidate the worse of its two times counts, each against the first candidate's (the library's
+    choice), so that a choice for one form does not slow the other."""
     import torch
+
+    from ._native import LAP_FP32, lap_form
 
     B = r.shape[0]
     lp = torch.empty(B, device=r.device)
     e = torch.empty(B, device=r.device)
-    passes = {"value": lambda: model.logpsi(r, R, Z, lp), "lap": lambda: model.local_energy(r, R, Z, e)}
+
+    def loss_energies():
+        with lap_form(LAP_FP32):
+            model.local_energy(r, R, Z, e)
+
+    passes = {"value": [lambda: model.logpsi(r, R, Z, lp)], "lap": [lambda: model.local_energy(r, R, Z, e)]}
+    if model.precision == "fp32":
+        passes["lap"].append(loss_energies)
     best = model.get_tuning()
     log = []
-    for name, cands, which in search_space(model.shape.n_el):
+    for name, cands, which in search_space(model.shape.n_el, model.precision, model.shape.width1):
         if which == "lap" and not include_lap:
             continue
         if name == "fwd_mu_split" and model.precision != "fp32":
@@ -94,11 +112,12 @@ def autotune_model(model, r, R, Z, reps: int = 3, include_lap: bool = True) -> T
         timings = {}
         for c in cands:
             model.set_tuning(**{**best, name: c})
-            timings[c] = time_ms(passes[which], reps)
-        choice = min(timings, key=timings.get)
+            timings[c] = [time_ms(fn, reps) for fn in passes[which]]
+        first = timings[cands[0]]
+        choice = min(timings, key=lambda c: max(t / t0 for t, t0 in zip(timings[c], first)))
         best[name] = choice
         model.set_tuning(**best)
-        log.append({"field": name, "pass": which, "ms": {str(k): round(v, 4) for k, v in timings.items()},
+        log.append({"field": name, "pass": which, "ms": {str(k): round(sum(v), 4) for k, v in timings.items()},
                     "choice": choice})
     return best, log
 

@@ -251,11 +251,14 @@ typedef struct dw_tuning {
   int32_t fwd_orb_tile;   /* orbital GEMMs of the value pass                                         */
   int32_t fwd_mu_split;   /* K-split (1, 2 or 4) of the spin-mean GEMMs of the value pass (FP32 form) */
   int32_t lap_orb_tile;   /* orbital GEMMs of the Laplacian pass                                     */
-  int32_t lap_mu_tile;    /* spin-mean GEMMs of the Laplacian pass                                   */
+  int32_t lap_mu_tile;    /* spin-mean GEMMs of the Laplacian pass: BF16X3, >= 0 keeps the kernels separate;
+                             FP32 MFMA at widths other than 256; the FP32 forms' fused kernels have one
+                             shape and do not look at it                                             */
   int32_t lap_electrons;  /* electrons per workgroup of the fused Laplacian GEMM (E * Cp <= 192); the
                              FP32 form takes its small tiles when that is fewer than its full tiles hold */
-  int32_t lap_cols;       /* output columns per workgroup of that GEMM (FP32 form): 0 by size, 128 or 256
-                             (E * Cp <= 96; larger tiles fall back to 128)                            */
+  int32_t lap_cols;       /* output columns per workgroup of that GEMM (FP32 forms): 0 by size, 128 or 256
+                             (E * Cp <= 96; larger tiles fall back to 128; 256 with fewer electrons than a
+                             full tile of the split form keeps its small tiles)                       */
 } dw_tuning;
 dw_status dw_model_set_tuning(dw_model* m, const dw_tuning* t);
 dw_status dw_model_get_tuning(const dw_model* m, dw_tuning* out);
