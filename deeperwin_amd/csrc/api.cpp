@@ -760,23 +760,29 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
       if (split) {
         // derivative channels of V, then the value channel (row 0 of each electron) with the value pass's
         // arithmetic, then the derivative channels of the layer
-        split_mean(X[l], m->Kx[l], m->Kh[l], W.WmuS[l].p, m->Km[l], ws.V, m->W1, sh, s);
         const int ldx = Cp * m->Kx[l], Km = m->Km[l];
+        const bool apart = !split_mean(X[l], m->Kx[l], m->Kh[l], W.WmuS[l].p, Km, ws.V, m->W1, sh, s);
+        if (apart) {  // ws.MU holds the means of every channel
+          launch_spin_mean<float>(X[l], m->Kx[l], m->Kh[l], ws.MU, Km, sh, s);
+          split_mean_product(ws.MU, Km, W.WmuS[l].p, ws.V, m->W1, sh, s);
+        }
         if (value_done <= l &&
             value_layer(X[l], ldx, m->Kx[l], m->Kh[l], W.WmainL[l].p, W.WmuL[l].p, Km, W.bias[l].as<float>(), 1, outp,
                         (long)Cp * ldo, last ? 1 : 0, (int)B, m->n, m->u, m->W1, s))
           value_done = l + 1;
         if (value_done <= l) value_done = l + value_layers(l, 1, Cp, true);
         if (value_done <= l) {
-          Shape s1 = sh;
-          s1.C = 1;
-          s1.Cp = 1;
-          launch_spin_mean<float>(X[l], ldx, m->Kh[l], ws.MU, Km, s1, s);
+          if (!apart) {
+            Shape s1 = sh;
+            s1.C = 1;
+            s1.Cp = 1;
+            launch_spin_mean<float>(X[l], ldx, m->Kh[l], ws.MU, Km, s1, s);
+          }
           GemmEpi ev;
           ev.bias = W.bias[l].as<float>();
           ev.nC = m->n;
-          gemm(GEMM_F32, ws.MU, Km, W.Wmu[l].as<float>(), nullptr, nullptr, Km, ws.V, Cp * m->W1, (int)B, m->W1, Km, ev,
-               s);  // over the value rows of V
+          gemm(GEMM_F32, ws.MU, apart ? Cp * Km : Km, W.Wmu[l].as<float>(), nullptr, nullptr, Km, ws.V, Cp * m->W1, (int)B,
+               m->W1, Km, ev, s);  // over the value rows of V
           GemmEpi em;
           em.V = ws.V;
           em.ldv = Cp * m->W1;

@@ -619,19 +619,18 @@ int split_lap(const float* X, int ldx, const void* P, int K, const float* amax, 
 // A workgroup forms the means of 48 rows x 128 k at a time and splits them straight into LDS (37 KB: four workgroups
 // per CU, whose load and MFMA phases overlap); the weights' parts come from L2.  Bound by the read of X's h columns
 // (1.41 GB for 2048 walkers of 14 electrons: 364 us = 3.9 TB/s against 471 us with FP32 MFMA; 26 electrons, 1024
-// walkers: 575 -> 461 us; 256 LiH walkers: 67 -> 28 us a layer with 64 columns per workgroup).
+// walkers: 575 -> 461 us).  Smaller batches form their means in k_spin_mean (split_mean says where).
 //
 // NP = 2 is the BF16x3 form: the first two parts and three products, every row (the value channel and its bias too), 64
 // rows.  Its sums are k_gemm_bf16's (v_mfma_f32_32x32x16_bf16 over 16 k at a time, low x high, high x low, high x high), so
 // results are bit-equal to the separate kernels (k_spin_mean and that GEMM), which small batches keep (launch_mean).
 // ------------------------------------------------------------------------------------------------
-template <int NQ, int NP, bool FEW>
+template <int NP>
 __global__ __launch_bounds__(256, NP == 2 ? 4 : 1) void k_split_mean(const float* __restrict__ X, int Kx, int Kh,
                                                     const uint4* __restrict__ P, int ncb, int Km,
                                                     const float* __restrict__ bias, float* __restrict__ V, int ldv,
                                                     Shape sh, int tilesN, int total) {
-  constexpr int RB = NP == 2 ? 4 : 3, CS = 4;  // row blocks, 32-wide slices per chunk
-  static_assert(NP == 3 || (NQ == 4 && !FEW), "the BF16x3 form takes 64 columns a wave");
+  constexpr int RB = NP == 2 ? 4 : 3, CS = 4, NQ = 4;  // row blocks, 32-wide slices per chunk, 16-column blocks of a wave
   __shared__ uint4 lds[CS][NP][RB][64];
   const int tile = tile_of(blockIdx.x, total);
   if (tile >= total) return;  // uniform over the workgroup, before any barrier
@@ -660,88 +659,37 @@ __global__ __launch_bounds__(256, NP == 2 ? 4 : 1) void k_split_mean(const float
     __syncthreads();  // the previous chunk's reads are done
     // consecutive lanes take consecutive quads of a row (coalesced); 4 quads a slice-row group
     auto put = [&](int rr, int qd, v4f v, float inv) {
-      if constexpr (NP == 2) {
-        v = scaled(v, inv);
-      } else {
-        v[0] *= inv;
-        v[1] *= inv;
-        v[2] *= inv;
-        v[3] *= inv;
-      }
       uint2 p[3];
-      split4(v, p);
+      split4(scaled(v, inv), p);
       const int quad = qd & 7;
 #pragma unroll
       for (int m = 0; m < NP; ++m)
         *((uint2*)&lds[qd >> 3][m][rr >> 4][(quad >> 1) * 16 + (rr & 15)] + (quad & 1)) = p[m];
     };
     const int units = 16 * RB * 8 * ns;
-    if constexpr (FEW) {
-      // up to four electrons of a spin: all of a thread's means together (one after another they wait for their few
-      // loads: 37 us a layer for 256 walkers of 4 electrons, 28 so; where there are workgroups enough to
-      // hide the wait, the registers cost more: 316 -> 450 us at 2,048 walkers of 14)
-      constexpr int TT = RB * 2;
-      const float* xp[TT];
-      v4f v[TT];
-      int cnt[TT], rr[TT], qd[TT];
-#pragma unroll
-      for (int a = 0; a < TT; ++a) {
-        const int t = tid + a * 256;
-        rr[a] = t / (8 * ns);
-        qd[a] = t - rr[a] * (8 * ns);
-        const long r = r0 + rr[a];
-        const int k = kc + 4 * qd[a];
-        v[a] = v4f{0.f, 0.f, 0.f, 0.f};
-        cnt[a] = 0;
-        xp[a] = X;
-        if (t < units && r < rows && k < 2 * Kh) {
-          const long b = div_idx(r, Cp);
-          const int s = k >= Kh ? 1 : 0;
-          cnt[a] = s ? n - u : u;
-          xp[a] = X + ((b * n + (s ? u : 0)) * Cp + (r - b * Cp)) * (long)Kx + (k - s * Kh);
-        }
-      }
-#pragma unroll 2
-      for (int i = 0; i < 4; ++i) {
-        v4f x[TT];
-#pragma unroll
-        for (int a = 0; a < TT; ++a) x[a] = i < cnt[a] ? *(const v4f*)(xp[a] + i * xstride) : v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int a = 0; a < TT; ++a) {
-          v[a][0] += x[a][0];
-          v[a][1] += x[a][1];
-          v[a][2] += x[a][2];
-          v[a][3] += x[a][3];
-        }
-      }
-#pragma unroll
-      for (int a = 0; a < TT; ++a)
-        if (tid + a * 256 < units) put(rr[a], qd[a], v[a], cnt[a] ? 1.f / (float)cnt[a] : 0.f);
-    } else {
-      for (int t = tid; t < units; t += 256) {
-        const int rr = t / (8 * ns), qd = t - rr * (8 * ns);
-        const long r = r0 + rr;
-        const int k = kc + 4 * qd;
-        v4f v = {0.f, 0.f, 0.f, 0.f};
-        float inv = 0.f;
-        if (r < rows && k < 2 * Kh) {
-          const long b = div_idx(r, Cp);
-          const int ch = (int)(r - b * Cp);
-          const int s = k >= Kh ? 1 : 0;
-          const int i0 = s ? u : 0, i1 = s ? n : u;
-          const float* xp = X + ((b * n + i0) * Cp + ch) * (long)Kx + (k - s * Kh);
+    for (int t = tid; t < units; t += 256) {
+      const int rr = t / (8 * ns), qd = t - rr * (8 * ns);
+      const long r = r0 + rr;
+      const int k = kc + 4 * qd;
+      v4f v = {0.f, 0.f, 0.f, 0.f};
+      float inv = 0.f;
+      if (r < rows && k < 2 * Kh) {
+        const long b = div_idx(r, Cp);
+        const int ch = (int)(r - b * Cp);
+        const int s = k >= Kh ? 1 : 0;
+        const int i0 = s ? u : 0, i1 = s ? n : u;
+        const float* xp = X + ((b * n + i0) * Cp + ch) * (long)Kx + (k - s * Kh);
 #pragma unroll 8
-          for (int i = i0; i < i1; ++i, xp += xstride) {
-            const v4f x = *(const v4f*)xp;
-            v[0] += x[0];
-            v[1] += x[1];
-            v[2] += x[2];
-            v[3] += x[3];
-          }
-          inv = 1.f / (float)(i1 - i0);
+        for (int i = i0; i < i1; ++i, xp += xstride) {
+          const v4f x = *(const v4f*)xp;
+          v[0] += x[0];
+          v[1] += x[1];
+          v[2] += x[2];
+          v[3] += x[3];
         }
-        put(rr, qd, v, inv);
+        inv = 1.f / (float)(i1 - i0);
       }
+      put(rr, qd, v, inv);
     }
     __syncthreads();
     for (int s = 0; s < ns; ++s) {
@@ -820,35 +768,82 @@ __global__ __launch_bounds__(256, NP == 2 ? 4 : 1) void k_split_mean(const float
   }
 }
 
-template <int NQ, bool FEW>
-static void mean_launch3(const float* X, int Kx, int Kh, const void* P, int ncb, int Km, float* V, int ldv, const Shape& sh,
-                         hipStream_t s) {
-  const int tilesN = sh.W1 / (64 * NQ), total = (int)(((long)sh.B * sh.Cp + 47) / 48 * tilesN);
-  hipLaunchKernelGGL((k_split_mean<NQ, 3, FEW>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh, (const uint4*)P, ncb,
-                     Km, (const float*)nullptr, V, ldv, sh, tilesN, total);
+// The product alone, from means that k_spin_mean has formed: C[M, 64 NQ tilesN columns] = A[M, K] B in BF16 parts, the sums of
+// k_split_mean.
+template <int RB, int NQ>
+__global__ __launch_bounds__(256) void k_split_gemm_mu(const float* __restrict__ A, int lda, SplitB W, float* __restrict__ C,
+                                                       int ldc, int M, int tilesN, int total) {
+  __shared__ SplitLds<RB, 3> lds;
+  const int tile = tile_of(blockIdx.x, total);
+  if (tile >= total) return;  // uniform over the workgroup, before any barrier
+  const long row0 = (long)(tile / tilesN) * (16 * RB);
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int cb0 = (tile % tilesN) * (4 * NQ) + wv * NQ;
+  const SplitUnits<RB> U(A, row0, M, lda);
+  v4f acc[RB][NQ];
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) acc[i][q] = v4f{0.f, 0.f, 0.f, 0.f};
+  split_main<RB, NQ>(U, W, cb0, lds, acc);
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const long r = row0 + i * 16 + 4 * (lane >> 4) + j;
+        if (r < M) C[r * ldc + (cb0 + q) * 16 + (lane & 15)] = acc[i][q][j];
+      }
 }
 
-void split_mean(const float* X, int Kx, int Kh, const void* P, int Km, float* V, int ldv, const Shape& sh, hipStream_t s) {
-  const int ncb = dw_pad(sh.W1, 256) / 16;
-  // 256 columns (X read once) where that gives two workgroups to every CU
-  if (sh.W1 % 256 == 0 && ((long)sh.B * sh.Cp + 47) / 48 * (sh.W1 / 256) >= 512)
-    mean_launch3<4, false>(X, Kx, Kh, P, ncb, Km, V, ldv, sh, s);
-  else if (sh.u <= 4 && sh.n - sh.u <= 4)
-    mean_launch3<1, true>(X, Kx, Kh, P, ncb, Km, V, ldv, sh, s);
+template <int RB, int NQ>
+static void mu_launch(const float* MU, const void* P, int Km, float* V, int ldv, const Shape& sh, hipStream_t s) {
+  const SplitB W{(const uint4*)P, dw_pad(sh.W1, 256) / 16, Km / 32};
+  const int M = sh.B * sh.Cp, tilesN = sh.W1 / (64 * NQ), total = (M + 16 * RB - 1) / (16 * RB) * tilesN;
+  hipLaunchKernelGGL((k_split_gemm_mu<RB, NQ>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, MU, Km, W, V, ldv, M, tilesN,
+                     total);
+}
+
+// The smallest tiles whose workgroups come to about four per CU: 16 or 32 rows x 64 columns, then 48 or 96 x 128.
+void split_mean_product(const float* MU, int Km, const void* P, float* V, int ldv, const Shape& sh, hipStream_t s) {
+  const long M = (long)sh.B * sh.Cp;
+  if ((M + 15) / 16 * (sh.W1 / 64) <= 1024)
+    mu_launch<1, 1>(MU, P, Km, V, ldv, sh, s);
+  else if ((M + 31) / 32 * (sh.W1 / 64) <= 1024)
+    mu_launch<2, 1>(MU, P, Km, V, ldv, sh, s);
+  else if ((M + 47) / 48 * (sh.W1 / 128) <= 768)
+    mu_launch<3, 2>(MU, P, Km, V, ldv, sh, s);
   else
-    mean_launch3<1, false>(X, Kx, Kh, P, ncb, Km, V, ldv, sh, s);
+    mu_launch<6, 2>(MU, P, Km, V, ldv, sh, s);
 }
 
-// From 600 tiles of 64 rows up, where the fused kernel keeps every CU busy; below, its few workgroups form their means one
+// 256 columns a workgroup (X read once) where that gives two workgroups to every CU; below that its few workgroups form
+// their means one after another, and two kernels win.  E_loc fused / apart, us: 14 electrons 473 / 317 (10 walkers), 765 / 619
+// (125), 2,096 / 1,780 (500), 3,297 / 3,372 (1,000: fused); 4 electrons 291 / 259 (93), 1,338 / 1,395 (3,000: fused); 42
+// electrons 1,160 / 994 (11); width 512, 14 electrons 877 / 542 (10), 4,182 / 4,118 (500: fused); other widths have 64-column
+// workgroups only (width 384, 14 electrons, 500 walkers 4,143 / 3,320).
+bool split_mean(const float* X, int Kx, int Kh, const void* P, int Km, float* V, int ldv, const Shape& sh, hipStream_t s) {
+  const long tilesM = ((long)sh.B * sh.Cp + 47) / 48;
+  if (sh.W1 % 256 != 0 || tilesM * (sh.W1 / 256) < 512) return false;
+  const int tilesN = sh.W1 / 256, total = (int)(tilesM * tilesN);
+  hipLaunchKernelGGL((k_split_mean<3>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh, (const uint4*)P,
+                     dw_pad(sh.W1, 256) / 16, Km, (const float*)nullptr, V, ldv, sh, tilesN, total);
+  return true;
+}
+
+// From 600 tiles of 64 rows up the fused kernel keeps every CU busy; below, its few workgroups form their means one
 // after another and the two separate kernels win.  E_loc, separate / fused: 14 electrons 510 / 702 us (85 walkers, 64
 // tiles), 1,939 / 2,052 (583, 438), 2,794 / 2,766 (833, 625), 3,306 / 3,236 (1,000, 750), 4,384 / 4,225 (1,365, 1,024); 8
-// electrons 1,184 / 1,262 (438 tiles), 1,739 / 1,705 (625); 26 electrons 1,287 / 1,460 (128), 5,350 / 5,189 (625).
+// electrons 1,184 / 1,262 (438 tiles), 1,739 / 1,705 (625).  From 20 electrons (longer sums to form a mean, which the fused
+// kernel does not store) from 400 tiles: 20 electrons 2,622 / 2,595 (375), 3,504 / 3,436 (512); 26 electrons 1,287 / 1,460
+// (128), 3,813 / 3,779 (438), 5,350 / 5,189 (625); 42 electrons 4,000 / 3,999 (256), 7,476 / 7,366 (512).
 bool mean_bf16x3(const float* X, int Kx, int Kh, const void* P, int Km, const float* bias, float* V, int ldv, const Shape& sh,
                  hipStream_t s) {
   const long tilesM = ((long)sh.B * sh.Cp + 63) / 64;
-  if (sh.W1 % 256 != 0 || tilesM * (sh.W1 / 256) < 600) return false;
+  if (sh.W1 % 256 != 0 || tilesM * (sh.W1 / 256) < (sh.n >= 20 ? 400 : 600)) return false;
   const int tilesN = sh.W1 / 256, total = (int)(tilesM * tilesN);
-  hipLaunchKernelGGL((k_split_mean<4, 2, false>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh, (const uint4*)P,
+  hipLaunchKernelGGL((k_split_mean<2>), dim3((total + 7) / 8 * 8), dim3(256), 0, s, X, Kx, Kh, (const uint4*)P,
                      dw_pad(sh.W1, 256) / 16, Km, bias, V, ldv, sh, tilesN, total);
   return true;
 }

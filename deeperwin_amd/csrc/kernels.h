@@ -70,8 +70,10 @@ void launch_split_pack16(const float* Bt, int ldb, int cols, int K, void* out, h
 void split_gemm(const float* A, int lda, const void* P16, const float* amax, int np, int ms, int rbe, float* C,
                 int ldc, int M, int N, int K, int tile, hipStream_t s);
 // V[(b Cp + ch), o] of the derivative channels: spin means of X's first Kh columns times W_mu (no bias), from three BF16 parts
-// of each (FP32 accuracy).
-void split_mean(const float* X, int Kx, int Kh, const void* P, int Km, float* V, int ldv, const Shape& sh, hipStream_t s);
+// of each (FP32 accuracy); false, launching nothing, where the batch is too small to gain against launch_spin_mean and
+// split_mean_product (V = MU times W_mu, the same sums).
+bool split_mean(const float* X, int Kx, int Kh, const void* P, int Km, float* V, int ldv, const Shape& sh, hipStream_t s);
+void split_mean_product(const float* MU, int Km, const void* P, float* V, int ldv, const Shape& sh, hipStream_t s);
 // The same for the BF16x3 form, all channels and the bias, bit-equal to launch_spin_mean and its GEMM; false, launching
 // nothing, where the batch is too small to gain.
 bool mean_bf16x3(const float* X, int Kx, int Kh, const void* P, int Km, const float* bias, float* V, int ldv, const Shape& sh,
