@@ -212,7 +212,7 @@ def grad_bench(args):
     gradient by autograd) in FP32 PyTorch on a walker sample."""
     import torch
 
-    from deeperwin_amd._native import NativeModel, clip_energies
+    from deeperwin_amd._native import LAP_FP32, NativeModel, clip_energies, lap_form
     from deeperwin_amd.batching import executed_forward_flops
     from deeperwin_amd.params import ModelShape, init_params
     from deeperwin_amd.physics import generate_el_ion_mapping, geometry_n2, init_walkers_gaussian
@@ -233,7 +233,8 @@ def grad_bench(args):
     state = torch.tensor([0.0, 1e12], dtype=torch.float64, device="cuda")
 
     def step():
-        m.local_energy(r, Rd, Zd, e)
+        with lap_form(LAP_FP32):  # the energies that the loss takes (deeperwin_amd/loss.py)
+            m.local_energy(r, Rd, Zd, e)
         w, _, stats = clip_energies(e, state)
         return m.param_grad(r, Rd, Zd, w), w
 
@@ -262,8 +263,8 @@ def grad_bench(args):
            "ms_per_step": round(dt * 1e3, 3), "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
            "dtype": args.precision, "data": "synthetic",
            "config": {"workload": ("N2, 14 electrons, 16 dets, " + ("dpe4 model" if dpe4 else "256/32 widths")
-                                   + ", seed 1; one optimisation step's gradient (E_loc with the full Laplacian, "
-                                     "tanh clipping, parameter gradient)"),
+                                   + ", seed 1; one optimisation step's gradient (E_loc with the full Laplacian on FP32 MFMA "
+                                     "as the loss takes it, tanh clipping, parameter gradient)"),
                       "walkers": B, "n_params": int(m.lib.dw_param_count(m.handle))},
            "gradient_pass_ms": round(g_ms, 3),
            "gradient_pass_tflops": tflops,

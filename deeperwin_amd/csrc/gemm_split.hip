@@ -1,21 +1,24 @@
 // FP32 GEMMs of the Laplacian pass's derivative channels on 16-bit MFMA with FP32 sums.
 //
 // Two forms.  BF16 parts: an FP32 operand is the exact sum of three BF16 numbers (x = h + m + l: h = bf16(x),
-// m = bf16(x - h), l = x - h - m; 8 + 8 + 8 significant bits), so a product is the sum of nine BF16 products; the three
-// below 2^-26 |a b| (m l, l m, l l) are left out.  FP16 parts: x = h + m with 11 + 11 bits and a rest below 2^-23 |x|,
-// three products (m m, below 2^-24 |a b|, left out); it needs operands near the top of FP16's range, so a row block (one
-// electron's channels) and each column of the weights are scaled by powers of two, and an element keeps those bits down to
-// 2^-17 of its block's or column's largest (below that its absolute error is 2^-39 of the largest).  In both a 32-wide K slice rounds the
-// accumulator six or three times, where the FP32 MFMA (16x16x4) rounds it at least eight times; over 320 products of
-// random operands that leaves 1.3e-7 (BF16) and 1.2e-7 (FP16) of the norm against 1.6e-7 for FP32.
+// m = bf16(x - h), l = x - h - m; 8 + 8 + 8 significant bits, m up to 2^-8 |x|, l up to 2^-17 |x|), so a product is the sum
+// of nine BF16 products; three (m l and l m, up to 2^-25 |a b|, and l l) are left out.  FP16 parts: x = h + m with 11 + 11
+// bits, m up to 2^-11 |x|, and a rest up to 2^-23 |x|; three products (m m, up to 2^-22 |a b|, left out).  It needs operands
+// near the top of FP16's range, so a row block (one electron's channels) and each column of the weights are scaled by powers
+// of two, and an element keeps those bits down to 2^-17 of its block's or column's largest (below that its absolute error is
+// 2^-39 of the largest).  A single product is thus less exact than FP32's (whose products the FP32 MFMA does not round); sums
+// are not: a 32-wide K slice rounds the accumulator six or three times, where the FP32 MFMA (16x16x4) rounds it at least
+// eight times, and over 320 products of random operands that leaves 1.3e-7 (BF16) and 1.2e-7 (FP16) of the norm against
+// 1.6e-7 for FP32.
 // The 16-bit MFMA runs at 16 times the FP32 rate: 6 / 16 and 3 / 16 of the FP32 form's time.
 //
 // FP16 parts are taken where the largest magnitudes are known: the layer's kernel leaves the maxima of what it writes,
 // and the columns of other kernels (pair features, the last slices) are looked at while they wait in registers.
 // Layer 0 (K of a few features) and the mean product, bound by memory, use BF16 parts.
 //
-// Measured against 64 bits (E_loc of 256 to 2048 walkers, 4 to 42 electrons, both models): the same relative
-// error as the FP32 form to two digits (4e-6 to 6e-5, set by the value channel), 2e-7 to 6e-7 between the two.
+// Measured against 64 bits (E_loc of 48 to 2048 walkers, 4 to 60 electrons, both models): the same relative error as the
+// FP32 form to a few per cent (5e-7 to 6e-5 of the norm, 9e-7 to 8e-4 for the median of unequilibrated walkers: set by the
+// value channel), between the two 1e-7 to 2e-6 of the norm, a quarter of that error or less.
 //
 // Only derivative channels (tangents, Laplacian) come from here.  The value channel of the pass (the first row
 // of an electron) keeps the FP32 MFMA of the value pass: log|psi|, the orbital matrices and their inverses
