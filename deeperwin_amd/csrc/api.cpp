@@ -897,7 +897,7 @@ dw_status run_pass(dw_model* m, const PassBufs<T>& ws, const float* r, long B, c
   {
     Timed t(m, C > 1 ? DW_TIMER_DET_LAP : -1, s);
     const CombineValue cv{out_lp, out_phase, out_flags, out_kappa, cond_thr, 0};
-    combined = launch_det<T>(ws.A, src, ws.minv, ws.ld, ws.sd, ws.g, ws.lap, ws.dcond, sh, s, C == 1 ? &cv : nullptr);
+    combined = launch_det<T>(ws.A, src, ws.minv, ws.ld, ws.sd, ws.g, ws.lap, ws.dcond, sh, s, C == 1 ? &cv : nullptr, !split);
   }
   if (!combined)
     launch_combine(ws.ld, ws.sd, ws.g, ws.lap, ws.dcond, cond_thr, r, R, Z, out_lp, out_phase, out_eloc, out_flags,

@@ -5,9 +5,8 @@
 // determinant) is never stored.
 //
 // 16,384 matrices of 26 (1024 walkers): 4.17 ms for the determinants and 1.99 ms for the stored product before, 0.73 ms
-// (inverses) + 2.30 ms (channels) here; 3,072 matrices of 42: 0.70 + 2.13 ms; 32,768 matrices of 14: 1.14 ms (one
-// wavefront per matrix) before, 0.13 + 0.60 ms here.  The fixed order of the channels' sums takes 0.24, 0.19 and 0.10 ms of
-// that, against each wave adding up its own channels.  Above 16 electrons the channel passes run at half the FP64 matrix
+// (inverses) + 2.06 ms (channels; 2.30 in the old order of sums) here; 3,072 matrices of 42: 0.70 + 1.94 (2.13) ms; 32,768
+// matrices of 14: 1.14 ms (one wavefront per matrix) before, 0.13 + 0.50 (0.60) ms here.  Above 16 electrons the channel passes run at half the FP64 matrix
 // rate, padding to 16 x 16 blocks counted.
 #include <utility>
 
@@ -353,24 +352,27 @@ __global__ __launch_bounds__(64) void k_det_inv_lds(OrbSrc<TA> src, Shape sh, do
 // of being computed a second time as (dM^T M^-T), so a channel is NB^3 x 4 MFMAs of 64 cycles, half of what two
 // products take.
 //
-// Order of the sums (fixed: an ill-conditioned walker's E_loc, and with it the FP64 loss, turns a rounding here into a
-// last bit): lane l of block (I, J) forms s_IJ = sum_e Y_IJ[4 e + g][c] Y_JI[c][4 e + g]; a chain per lane (NB <= 2) or
+// KEEP, order of the sums (an ill-conditioned walker's E_loc, and with it the FP64 loss, turns a rounding here into a last
+// bit; the loss and every form that was there before the split one keep it): lane l of block (I, J) forms s_IJ = sum_e Y_IJ[4 e + g][c] Y_JI[c][4 e + g]; a chain per lane (NB <= 2) or
 // per lane and J (NB > 2) adds them channel by channel, (I, J) in order, then the lanes meet.  The channels of a round
 // lie in different waves, so they leave their s_IJ in LDS and every wave continues a part of the chains: a barrier or two
 // a round of 4 channels (16 for NB = 1, whose channels are short).  tr Y is one chain of the operands' products per lane.
+// Otherwise (energies of the split form, whose channels are rounded in another way already) each wave adds up its own
+// channels, off-diagonal pairs once and doubled, tr Y from the diagonal that the transposition tile holds: 16,384 matrices of
+// 26 2.06 ms against 2.30, 3,072 of 42 1.94 against 2.13, 32,768 of 14 0.50 against 0.60.
 // ------------------------------------------------------------------------------------------------
-template <int NB>
+template <int NB, bool KEEP>
 constexpr int chan_region() {  // doubles of LDS per wave: transposition tiles, behind or over them the s_IJ of a round
-  return NB == 1 ? 16 * 17 + 4 * 64 : NB == 2 ? 16 * 17 + 2 * 4 * 64 : NB * NB * 64;
+  return !KEEP ? 16 * 17 : NB == 1 ? 16 * 17 + 4 * 64 : NB == 2 ? 16 * 17 + 2 * 4 * 64 : NB * NB * 64;
 }
 
-template <int NB, typename TA>
+template <int NB, typename TA, bool KEEP>
 __global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof(TA) == 4 ? 3 : 2)) void k_det_chan(OrbSrc<TA> src, Shape sh,
                                                                                const double* __restrict__ Minv,
                                                                                double* __restrict__ g,
                                                                                double* __restrict__ lapd, int nmat) {
   extern __shared__ double sm[];
-  constexpr int NP = 16 * NB, PM = NP + 1, REGION = chan_region<NB>(), RC = NB == 1 ? 4 : 1, NT = NB * NB;
+  constexpr int NP = 16 * NB, PM = NP + 1, REGION = chan_region<NB, KEEP>(), RC = NB == 1 && KEEP ? 4 : 1, NT = NB * NB;
   constexpr bool TWO = NB == 2;  // two buffers of s_IJ: one barrier a round
   const int n = sh.n, nd = 3 * n, C = sh.C;
   double* sM = sm;                        // M^-1, NP x PM, zero outside n x n
@@ -389,9 +391,14 @@ __global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, gq = lane >> 4, cl = lane & 15;
 
   TA* const sL = (TA*)sT;
+  double tp = 0.0;  // tr(M^-1 Lap M); KEEP: a row of M^-1 per lane, or elements 256 apart per thread
   for (int e = tid; e < NP * NP; e += 256) {
     const int i = e / NP, c = e - (e / NP) * NP;
     sM[i * PM + c] = (i < n && c < n) ? Minv[(long)bd * n * n + i * n + c] : 0.0;
+  }
+  if constexpr (!KEEP) __syncthreads();
+  for (int e = tid; e < NP * NP; e += 256) {
+    const int i = e / NP, c = e - (e / NP) * NP;
     TA env = TA(0), b0 = TA(0), b1 = TA(0), b2 = TA(0);
     if (i < n && c < n) {
       TA g0, g1, g2, le;
@@ -404,7 +411,11 @@ __global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof
       b0 = g0 * bf0;
       b1 = g1 * bf0;
       b2 = g2 * bf0;
-      sL[e] = le * bf0 + env * Oi[(long)(C - 1) * src.ldo] + TA(2) * (g0 * t0 + g1 * t1 + g2 * t2);
+      const TA lp = le * bf0 + env * Oi[(long)(C - 1) * src.ldo] + TA(2) * (g0 * t0 + g1 * t1 + g2 * t2);
+      if constexpr (KEEP)
+        sL[e] = lp;
+      else
+        tp += sM[c * PM + i] * (double)lp;
     }
     sE[e] = env;
     if constexpr (TABLE) {
@@ -414,17 +425,16 @@ __global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof
     }
   }
   __syncthreads();
-  double tp = 0.0;  // tr(M^-1 Lap M): a row of M^-1 per lane, or elements 256 apart per thread
-  if constexpr (NB <= 2) {
+  if constexpr (KEEP && NB <= 2) {
     if (tid < n)
       for (int e = 0; e < n; ++e) tp += sM[tid * PM + e] * (double)sL[e * NP + tid];
-  } else {
+  } else if constexpr (KEEP) {
     for (int e = tid; e < n * n; e += 256) {
       const int a = e / n, q = e - (e / n) * n;
       tp += sM[a * PM + q] * (double)sL[q * NP + a];
     }
   }
-  __syncthreads();  // sL has been read
+  if constexpr (KEEP) __syncthreads();  // sL has been read
 
   constexpr bool REG = NB <= 2;
   double mi[REG ? NB : 1][REG ? NB : 1][4];
@@ -467,9 +477,9 @@ __global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof
   constexpr int S0 = NB <= 2 ? 16 * 17 : 0;
   int buf = 0;
   constexpr bool AHEAD = sizeof(TA) == 4;  // FP64 orbitals: no registers for a second channel
-  double qacc = 0.0;  // NB <= 2: chain of lane 16 wv + lane (lanes 0 to 15); NB > 2: chain of (J = wv, lane)
+  double qacc = 0.0;  // KEEP: NB <= 2, chain of lane 16 wv + lane (lanes 0 to 15); NB > 2, chain of (J = wv, lane)
   if (AHEAD && wv < nd) load(wv);
-  for (int k0 = 0; k0 < nd; k0 += 4 * RC) {  // every wave takes every round (barriers)
+  for (int k0 = 0; k0 < nd; k0 += 4 * RC) {  // every wave takes every round (KEEP's barriers)
     double gp[4];  // NB > 2: tr Y's chains
     gp[3] = 0.0;
 #pragma unroll
@@ -509,16 +519,16 @@ __global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof
 #pragma unroll
         for (int J = I; J < NB; ++J) {
           v4d y = {0.0, 0.0, 0.0, 0.0}, z = y;
-          if (NB > 2 && J == I) t = 0.0;
+          if (KEEP && NB > 2 && J == I) t = 0.0;
 #pragma unroll
           for (int K = 0; K < NB; ++K)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               y = __builtin_amdgcn_mfma_f64_16x16x4f64(mia(I, K, q), dm[K][J][q], y, 0, 0, 0);
               if (J > I) z = __builtin_amdgcn_mfma_f64_16x16x4f64(mia(J, K, q), dm[K][I][q], z, 0, 0, 0);
-              if (J == I) t += mia(I, K, q) * dm[K][I][q];
+              if (KEEP && J == I) t += mia(I, K, q) * dm[K][I][q];
             }
-          if constexpr (NB > 2)
+          if constexpr (KEEP && NB > 2)
             if (J == I) gp[I] = t;
           // lane l, element e: row 4 e + g, column c of the block (LDS accesses of one wave stay in order)
           auto against = [&](double* tile, const v4d& a, const v4d& other) {
@@ -529,7 +539,14 @@ __global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof
             for (int e = 0; e < 4; ++e) w[e] = tile[cl * 17 + 4 * e + gq];
             return a[0] * w[0] + a[1] * w[1] + a[2] * w[2] + a[3] * w[3];
           };
-          if (J == I) {
+          if constexpr (!KEEP) {
+            if (J == I) {
+              qacc += against(T, y, y);
+              t += T[cl * 18];
+            } else {
+              qacc += 2.0 * against(T, y, z);
+            }
+          } else if (J == I) {
             st[I * NB + I] = against(T, y, y);
           } else {
             st[I * NB + J] = against(T, y, z);
@@ -537,6 +554,11 @@ __global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof
           }
           __builtin_amdgcn_sched_barrier(0);
         }
+      if constexpr (!KEEP) {
+        const double g_k = row_sum_dpp(t);
+        if (lane == 0) g[(long)bd * nd + k] = g_k;
+        continue;
+      }
 #pragma unroll
       for (int x = 0; x < NT; ++x) T[S0 + buf + (rc * NT + x) * 64 + lane] = st[x];  // over the tiles (NB > 2), now read
       if constexpr (NB <= 2) {
@@ -548,6 +570,7 @@ __global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof
         if (lane == 0) g[(long)bd * nd + k] = ((s0 + s1) + s2) + s3;
       }
     }
+    if constexpr (!KEEP) continue;
     __syncthreads();  // every wave's s_IJ of the round are in LDS
     const int nc = min(4 * RC, nd - k0);
     if constexpr (NB <= 2) {
@@ -569,7 +592,7 @@ __global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof
     else
       __syncthreads();  // and have been read
   }
-  if constexpr (NB <= 2) {  // the 64 chains to the lanes of wave 0
+  if constexpr (KEEP && NB <= 2) {  // the 64 chains to the lanes of wave 0
     if (lane < 16) sT[16 * wv + lane] = qacc;
     __syncthreads();
     if (wv == 0) {
@@ -584,21 +607,31 @@ __global__ __launch_bounds__(256, NB == 1 ? 6 : NB == 4 ? 1 : (NB == 2 && sizeof
   }
 }
 
-template <int NB, typename TA>
+template <int NB, typename TA, bool KEEP>
 static void launch_chan(const OrbSrc<TA>& src, const Shape& sh, const double* Minv, double* g, double* lapd,
                         hipStream_t s) {
   constexpr int NP = 16 * NB;
-  const size_t shm = (size_t)(NP * (NP + 1) + 4 * chan_region<NB>() + 32) * sizeof(double) +
+  const size_t shm = (size_t)(NP * (NP + 1) + 4 * chan_region<NB, KEEP>() + 32) * sizeof(double) +
                      ((size_t)NP * NP + (NB < 4 || sizeof(TA) == 4 ? 3 * NP * NP : 4 * NP)) * sizeof(TA);
   if (shm > 65536)
-    (void)hipFuncSetAttribute((const void*)k_det_chan<NB, TA>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
+    (void)hipFuncSetAttribute((const void*)k_det_chan<NB, TA, KEEP>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
   const int nmat = sh.B * sh.D;
-  hipLaunchKernelGGL((k_det_chan<NB, TA>), dim3((nmat + 7) / 8 * 8), dim3(256), shm, s, src, sh, Minv, g, lapd, nmat);
+  hipLaunchKernelGGL((k_det_chan<NB, TA, KEEP>), dim3((nmat + 7) / 8 * 8), dim3(256), shm, s, src, sh, Minv, g, lapd, nmat);
+}
+
+template <typename TA, bool KEEP>
+static void dispatch_chan(const OrbSrc<TA>& src, const Shape& sh, const double* Minv, double* g, double* lapd, hipStream_t s) {
+  switch ((sh.n + 15) / 16) {
+    case 1: launch_chan<1, TA, KEEP>(src, sh, Minv, g, lapd, s); break;
+    case 2: launch_chan<2, TA, KEEP>(src, sh, Minv, g, lapd, s); break;
+    case 3: launch_chan<3, TA, KEEP>(src, sh, Minv, g, lapd, s); break;
+    default: launch_chan<4, TA, KEEP>(src, sh, Minv, g, lapd, s); break;
+  }
 }
 
 template <typename TA>
 void launch_det_lap(const OrbSrc<TA>& src, double* Minv, double* ld, double* sd, double* g, double* lapd,
-                          float* dcond, const Shape& sh, hipStream_t s) {
+                          float* dcond, const Shape& sh, bool keep_order, hipStream_t s) {
   const int n = sh.n;
   const long nmat = (long)sh.B * sh.D;
   if (n <= 16) {
@@ -613,16 +646,17 @@ void launch_det_lap(const OrbSrc<TA>& src, double* Minv, double* ld, double* sd,
       (void)hipFuncSetAttribute((const void*)k_det_inv_lds<TA>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
     hipLaunchKernelGGL((k_det_inv_lds<TA>), dim3((unsigned)nmat), dim3(64), shm, s, src, sh, Minv, ld, sd, dcond);
   }
-  switch ((n + 15) / 16) {
-    case 1: launch_chan<1, TA>(src, sh, Minv, g, lapd, s); break;
-    case 2: launch_chan<2, TA>(src, sh, Minv, g, lapd, s); break;
-    case 3: launch_chan<3, TA>(src, sh, Minv, g, lapd, s); break;
-    default: launch_chan<4, TA>(src, sh, Minv, g, lapd, s); break;
+  if constexpr (sizeof(TA) == 4) {
+    if (!keep_order) {
+      dispatch_chan<TA, false>(src, sh, Minv, g, lapd, s);
+      return;
+    }
   }
+  dispatch_chan<TA, true>(src, sh, Minv, g, lapd, s);
 }
 template void launch_det_lap<float>(const OrbSrc<float>&, double*, double*, double*, double*, double*, float*,
-                                          const Shape&, hipStream_t);
+                                          const Shape&, bool, hipStream_t);
 template void launch_det_lap<double>(const OrbSrc<double>&, double*, double*, double*, double*, double*, float*,
-                                           const Shape&, hipStream_t);
+                                           const Shape&, bool, hipStream_t);
 
 }  // namespace dwmi

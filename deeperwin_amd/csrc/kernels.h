@@ -174,11 +174,11 @@ struct CombineValue {
 // determinants per workgroup); the caller then skips launch_combine.
 template <typename TA>
 bool launch_det(const TA* A, const OrbSrc<TA>& src, double* minv, double* ld, double* sd, double* g, double* lapd, float* dcond,
-                const Shape& sh, hipStream_t s, const CombineValue* combine = nullptr);
-// Its part for the Laplacian pass (det_lap.hip).
+                const Shape& sh, hipStream_t s, const CombineValue* combine = nullptr, bool keep_order = true);
+// Its part for the Laplacian pass (det_lap.hip, which says what keep_order keeps).
 template <typename TA>
 void launch_det_lap(const OrbSrc<TA>& src, double* minv, double* ld, double* sd, double* g, double* lapd,
-                          float* dcond, const Shape& sh, hipStream_t s);
+                          float* dcond, const Shape& sh, bool keep_order, hipStream_t s);
 void launch_combine(const double* ld, const double* sd, const double* g, const double* lapd, const float* dcond,
                     float cond_thr, const float* r, const float* R, const float* Z, float* out_lp, float* out_phase,
                     float* out_eloc, uint32_t* out_flags, float* out_kappa, const Shape& sh, hipStream_t s);

@@ -1066,12 +1066,12 @@ __global__ __launch_bounds__(64) void k_det_value_lds(const TA* __restrict__ A, 
 
 template <typename TA>
 bool launch_det(const TA* A, const OrbSrc<TA>& src, double* minv, double* ld, double* sd, double* g, double* lapd, float* dcond,
-                const Shape& sh, hipStream_t s, const CombineValue* combine) {
+                const Shape& sh, hipStream_t s, const CombineValue* combine, bool keep_order) {
   const int n = sh.n;
   const long nmat = (long)sh.B * sh.D;
   const long stride = (long)sh.C * n * n;
   if (sh.C > 1) {
-    launch_det_lap<TA>(src, minv, ld, sd, g, lapd, dcond, sh, s);
+    launch_det_lap<TA>(src, minv, ld, sd, g, lapd, dcond, sh, keep_order, s);
     return false;
   }
   if (n > 32) {
@@ -1079,29 +1079,27 @@ bool launch_det(const TA* A, const OrbSrc<TA>& src, double* minv, double* ld, do
     hipLaunchKernelGGL((k_det_value_lds<TA>), dim3((unsigned)nmat), dim3(64), shv, s, A, ld, sd, dcond, n, stride);
     return false;
   }
-  if (sh.C == 1) {
-    // 4 wavefronts per workgroup, 64 / NMAX matrices per wavefront; the envelope is applied as O is read.
-    // When D divides the matrices per workgroup, the walkers' combine runs at the end of the same kernel.
-    const int mpw = n <= 8 ? 32 : (n <= 16 ? 16 : 8);
-    CombineValue co{};
-    if (combine && mpw % sh.D == 0) {
-      co = *combine;
-      co.fuse = 1;
-    }
-    const dim3 grid((unsigned)((nmat + mpw - 1) / mpw));
-    if (n <= 8)
-      hipLaunchKernelGGL((k_det_value<8, TA>), grid, dim3(256), 0, s, src, ld, sd, dcond, nmat, n, sh, co);
-    else if (n <= 16)
-      hipLaunchKernelGGL((k_det_value<16, TA>), grid, dim3(256), 0, s, src, ld, sd, dcond, nmat, n, sh, co);
-    else
-      hipLaunchKernelGGL((k_det_value<32, TA>), grid, dim3(256), 0, s, src, ld, sd, dcond, nmat, n, sh, co);
-    return co.fuse != 0;
+  // 4 wavefronts per workgroup, 64 / NMAX matrices per wavefront; the envelope is applied as O is read.
+  // When D divides the matrices per workgroup, the walkers' combine runs at the end of the same kernel.
+  const int mpw = n <= 8 ? 32 : (n <= 16 ? 16 : 8);
+  CombineValue co{};
+  if (combine && mpw % sh.D == 0) {
+    co = *combine;
+    co.fuse = 1;
   }
+  const dim3 grid((unsigned)((nmat + mpw - 1) / mpw));
+  if (n <= 8)
+    hipLaunchKernelGGL((k_det_value<8, TA>), grid, dim3(256), 0, s, src, ld, sd, dcond, nmat, n, sh, co);
+  else if (n <= 16)
+    hipLaunchKernelGGL((k_det_value<16, TA>), grid, dim3(256), 0, s, src, ld, sd, dcond, nmat, n, sh, co);
+  else
+    hipLaunchKernelGGL((k_det_value<32, TA>), grid, dim3(256), 0, s, src, ld, sd, dcond, nmat, n, sh, co);
+  return co.fuse != 0;
 }
 template bool launch_det<float>(const float*, const OrbSrc<float>&, double*, double*, double*, double*, double*, float*,
-                                const Shape&, hipStream_t, const CombineValue*);
+                                const Shape&, hipStream_t, const CombineValue*, bool);
 template bool launch_det<double>(const double*, const OrbSrc<double>&, double*, double*, double*, double*, double*, float*,
-                                 const Shape&, hipStream_t, const CombineValue*);
+                                 const Shape&, hipStream_t, const CombineValue*, bool);
 
 // ------------------------------------------------------------------------------------------------
 // Per-walker combination (FP64).  Sum of determinants with max shift and LOG_EPSILON
