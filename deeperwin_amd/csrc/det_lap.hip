@@ -6,8 +6,8 @@
 //
 // 16,384 matrices of 26 (1024 walkers): 4.17 ms for the determinants and 1.99 ms for the stored product before, 0.73 ms
 // (inverses) + 2.06 ms (channels; 2.30 in the old order of sums) here; 3,072 matrices of 42: 0.70 + 1.94 (2.13) ms; 32,768
-// matrices of 14: 1.14 ms (one wavefront per matrix) before, 0.13 + 0.50 (0.60) ms here.  Above 16 electrons the channel passes run at half the FP64 matrix
-// rate, padding to 16 x 16 blocks counted.
+// matrices of 14: 1.14 ms (one wavefront per matrix) before, 0.13 + 0.50 (0.60) ms here.  Above 16 electrons the channel
+// passes run at half the FP64 matrix rate, padding to 16 x 16 blocks counted.
 #include <utility>
 
 #include "common.h"
@@ -353,7 +353,8 @@ __global__ __launch_bounds__(64) void k_det_inv_lds(OrbSrc<TA> src, Shape sh, do
 // products take.
 //
 // KEEP, order of the sums (an ill-conditioned walker's E_loc, and with it the FP64 loss, turns a rounding here into a last
-// bit; the loss and every form that was there before the split one keep it): lane l of block (I, J) forms s_IJ = sum_e Y_IJ[4 e + g][c] Y_JI[c][4 e + g]; a chain per lane (NB <= 2) or
+// bit; the loss and every form that was there before the split one keep it): lane l of block (I, J) forms
+// s_IJ = sum_e Y_IJ[4 e + g][c] Y_JI[c][4 e + g]; a chain per lane (NB <= 2) or
 // per lane and J (NB > 2) adds them channel by channel, (I, J) in order, then the lanes meet.  The channels of a round
 // lie in different waves, so they leave their s_IJ in LDS and every wave continues a part of the chains: a barrier or two
 // a round of 4 channels (16 for NB = 1, whose channels are short).  tr Y is one chain of the operands' products per lane.
